@@ -60,8 +60,10 @@ enum {
     SCANSCAM_MODE_SMALL = 1,   /* T <= 64*vec: several rows per wave, no carries */
     SCANSCAM_MODE_ROW = 2,     /* a workgroup (or part of one) walks a whole row */
     SCANSCAM_MODE_LOOKBACK = 3, /* rows cut into tiles over workgroups, decoupled look-back carries */
-    SCANSCAM_MODE_FLAT = 4      /* dense tensors, 16/sizeof(storage) <= T <= 64 * that: all rows scanned as one
+    SCANSCAM_MODE_FLAT = 4,     /* dense tensors, 16/sizeof(storage) <= T <= 64 * that: all rows scanned as one
                                    stream of aligned vectors with a reset at every row start (unroll 2 or 4) */
+    SCANSCAM_MODE_STAGED = 5   /* channels-last only, dense tensors on 16-byte borders, C <= 256: contiguous tiles of a
+                                   batch element staged through LDS; the plan's other shape fields must be zero */
 };
 
 /*
@@ -182,7 +184,8 @@ int scanscam_scan_bwd_timed(const void *a, const void *h, const void *gh, void *
  * GPU, time is also cut into tiles over workgroups, carried by a look-back
  * chain, which needs a workspace (scanscam_workspace_bytes_cl, same rules as
  * above); mode = SCANSCAM_MODE_ROW forbids that split, SCANSCAM_MODE_LOOKBACK
- * forces it. A time step (C channels, or the time stride of a strided call)
+ * forces it. Many batch elements of few
+ * or oddly many channels take SCANSCAM_MODE_STAGED by themselves. A time step (C channels, or the time stride of a strided call)
  * must stay below 4 GiB / 18 = 227 MiB (the kernels address a wave's steps with
  * 32-bit offsets from its first one): larger ones return SCANSCAM_EINVAL.
  */
@@ -255,7 +258,8 @@ int scanscam_resolve_plan(int64_t rows, int64_t T, int dtype, int direction, con
  * The same for the channels-last calls on dense [batch, T, C] tensors whose bases are 16-byte
  * aligned: mode SCANSCAM_MODE_ROW where a workgroup walks all of T, SCANSCAM_MODE_LOOKBACK where
  * tiles of time steps chain through the workspace; vec channels per lane, unroll time steps per
- * wave and tile, waves per workgroup. No counterpart in the reference, whose kernel has one launch
+ * wave and tile, waves per workgroup. (A call that takes SCANSCAM_MODE_STAGED by itself has this plan, and its
+ * workspace, in reserve for tensors the staged kernel cannot run.) No counterpart in the reference, whose kernel has one launch
  * shape (scanscam/cuda.py:69-95 passes channels_per_block only).
  */
 int scanscam_resolve_plan_cl(int64_t batch, int64_t T, int64_t C, int dtype, int direction,

@@ -22,6 +22,7 @@ using scanscam::kModeFlat;
 using scanscam::kModeLookback;
 using scanscam::kModeRow;
 using scanscam::kModeSmall;
+using scanscam::kModeStaged;
 using scanscam::kWave;
 using scanscam::Launch;
 using scanscam::ScanArgs;
@@ -690,6 +691,52 @@ int resolve_cl(const scanscam_plan *user, int64_t batch, int64_t T, int64_t C, i
     return SCANSCAM_OK;
 }
 
+// Channels-last tiles staged through LDS (scan_staged_kernels.hpp): whether that kernel can run the call, and its tile.
+// Dense tensors on 16-byte borders, all channels of a batch element in one workgroup.
+bool resolve_staged(int64_t batch, int64_t T, int64_t C, int esize, const void *const ptrs[5], const int64_t sB[5],
+                    const int64_t sT[5], scanscam::StagedArgs *out)
+{
+    for (int k = 0; k < 5; k++)
+        if (!aligned_to(ptrs[k], 16) || (T > 1 && sT[k] != C) || (batch > 1 && sB[k] != T * C)) return false;
+    if (C > scanscam::kStagedThreads || batch >= (int64_t(1) << 31)) return false;
+    // Steps per tile: what its vectors hold and what the threads' spans cover; then tiles of equal size, in spans of at
+    // least half the steps a thread can take (every span costs every thread a read and an FMA for its carry).
+    const int most_seg = scanscam::staged_steps(esize);
+    const int64_t spans = scanscam::kStagedThreads / C;
+    int64_t most = ((int64_t)scanscam::kStagedThreads * scanscam::kStagedVectors * 16 - 16) / (C * esize);
+    if (most > spans * most_seg) most = spans * most_seg;
+    const int64_t tiles = (T + most - 1) / most, rows = (T + tiles - 1) / tiles;
+    int64_t seg = (rows + spans - 1) / spans;
+    if (seg < (most_seg + 1) / 2) seg = (most_seg + 1) / 2;
+    out->T = (int32_t)T;
+    out->C = (int32_t)C;
+    out->seg = (int32_t)seg;
+    out->spans = (int32_t)((rows + seg - 1) / seg);
+    const int64_t whole = out->spans * seg;  // (no span is cut short but those of the last tile)
+    out->rows = (int32_t)(whole < most ? whole : most);
+    return true;
+}
+
+// Whether an automatic plan takes that kernel. Measured against the plans of scan_cl_plan.hpp (forward / backward, us):
+//   few channels in lanes they do not fill, fp32 [1000, 1023, 17] 73.5 / 138 -> 43.3 / 79.3, [851, 467, 27] 41.2 / 69.2 ->
+//   28.6 / 48.6, bf16 [1000, 1023, 17] 56.3 / 102 -> 23.1 / 40.1, [2048, 512, 40] 65.2 / 105 -> 48.6 / 83.8, fp64
+//   [1000, 1023, 17] 115 / 209 -> 86.1 / 156; it ends where
+//   - time steps are whole 128-byte lines (the walk streams them: fp32 [256, 1024, 128] 74.7 / 127 against 83.3 / 124) or
+//     fill the lanes of the packed kernel (fp32 [512, 4096, 8] 39.5 / 68.9 against 45.8 / 63.0; 16-bit lanes do not);
+//   - there are more channels, which fill the walk's lanes well (bf16 [1076, 490, 91] 79.1 / 138 against 85.8 / 147), but for
+//     fp32 steps off the 16-byte border and fp64 (fp32 [1076, 490, 91] 131 / 217 -> 114 / 202, fp64 [1024, 90, 130] 72.4 /
+//     129 -> 61.3 / 102);
+//   - batch elements are too few workgroups (fp32, C = 33: 320 of them 44.8 / 64.5 -> 40.3 / 65.5 us, 192 of them 46.2 /
+//     66.0 against 57.5 / 78.1; C = 130: 512 level, 320 37.4 / 60.7 against 51.9 / 87.8) or less than a tile and a half each
+//     (fp32 [3000, 16, 24] 5.5 / 7.8 against 7.9 / 12.3).
+bool staged_is_better(int64_t batch, int64_t T, int64_t C, int esize)
+{
+    const int64_t step = C * esize;
+    if (step % 128 == 0 || (esize >= 4 && step <= 64 && 64 % step == 0)) return false;
+    if (!(C <= 80 || esize == 8 || (esize == 4 && step % 16 != 0))) return false;
+    return (batch >= 512 || (batch >= 320 && C <= 80)) && T * step >= 12 * 1024;
+}
+
 int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void *y1,
            const scanscam_strides *const st[5], int64_t batch, int64_t T, int64_t C, int dtype, void *workspace,
            size_t workspace_bytes, void *stream, const scanscam_plan *plan)
@@ -713,6 +760,28 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         if (!aligned_to(ptrs[k], (size_t)esize)) return SCANSCAM_EALIGN;
         while (align > esize && !(aligned_to(ptrs[k], (size_t)align) && (sB[k] * esize) % align == 0 && (sT[k] * esize) % align == 0))
             align >>= 1;
+    }
+    auto run_staged = [&](scanscam::StagedArgs st) {
+        st.a = a;
+        st.x = x;
+        st.h = rev ? h : a;  // never read in the forward pass
+        st.y0 = y0;
+        st.y1 = rev ? y1 : y0;
+        hipError_t e = hipErrorInvalidValue;
+        hipStream_t s = static_cast<hipStream_t>(stream);
+        switch (dtype) {
+        case SCANSCAM_F32: e = scanscam::launch_scan_staged<float>(st, batch, rev, s); break;
+        case SCANSCAM_BF16: e = scanscam::launch_scan_staged<__bf16>(st, batch, rev, s); break;
+        case SCANSCAM_F16: e = scanscam::launch_scan_staged<_Float16>(st, batch, rev, s); break;
+        case SCANSCAM_F64: e = scanscam::launch_scan_staged<double>(st, batch, rev, s); break;
+        }
+        return e == hipSuccess ? SCANSCAM_OK : SCANSCAM_ELAUNCH;
+    };
+    scanscam::StagedArgs staged;
+    if (plan && plan->mode == kModeStaged) {
+        if (plan->vec || plan->unroll || plan->waves || !resolve_staged(batch, T, C, esize, ptrs, sB, sT, &staged))
+            return SCANSCAM_EPLAN;
+        return run_staged(staged);
     }
     scanscam::ClLaunch l;
     const int rc = resolve_cl(plan, batch, T, C, dtype, align, rev, &l);
@@ -771,6 +840,11 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     if (l.kind != 0) {
         if (!workspace || workspace_bytes < l.ws_bytes) return SCANSCAM_EWORKSPACE;
         if (!aligned_to(workspace, 8)) return SCANSCAM_EALIGN;
+    }
+    const bool free_plan = !plan || (plan->mode == SCANSCAM_MODE_AUTO && !plan->vec && !plan->unroll && !plan->waves);
+    if (free_plan && staged_is_better(batch, T, C, esize) && resolve_staged(batch, T, C, esize, ptrs, sB, sT, &staged))
+        return run_staged(staged);
+    if (l.kind != 0) {
         args.ws = static_cast<uint64_t *>(workspace);
         const int64_t words = (int64_t)(l.ws_bytes / sizeof(uint64_t));
         const int64_t rowgroups = batch * ((C + (int64_t)kWave * l.vec - 1) / ((int64_t)kWave * l.vec));

@@ -6,10 +6,11 @@
 #include "scan_cl_kernels.hpp"
 #include "scan_flat_kernels.hpp"
 #include "scan_kernels.hpp"
+#include "scan_staged_kernels.hpp"
 
 namespace scanscam {
 
-enum Mode { kModeSmall = 1, kModeRow = 2, kModeLookback = 3, kModeFlat = 4 };
+enum Mode { kModeSmall = 1, kModeRow = 2, kModeLookback = 3, kModeFlat = 4, kModeStaged = 5 };
 
 // A fully resolved launch: which kernel, with which shape.
 struct Launch {
@@ -199,6 +200,18 @@ hipError_t launch_scan_cl(const ClArgs &args, const ClLaunch &l, bool rev, hipSt
             SCANSCAM_CL_CASE(ST, HALF, 16)                                                             \
         }                                                                                              \
         return hipErrorInvalidValue;                                                                   \
+    }
+
+// The staged channels-last kernel: one workgroup per batch element.
+template <typename ST> hipError_t launch_scan_staged(const StagedArgs &args, int64_t batch, bool rev, hipStream_t stream);
+
+#define SCANSCAM_DEFINE_STAGED_LAUNCH(ST)                                                              \
+    template <>                                                                                        \
+    hipError_t launch_scan_staged<ST>(const StagedArgs &args, int64_t batch, bool rev, hipStream_t stream) \
+    {                                                                                                  \
+        const dim3 grid((unsigned)batch), block(kStagedThreads);                                       \
+        if (rev) return launch_kernel(scan_cl_staged_kernel<ST, true>, grid, block, 0, stream, nullptr, nullptr, args); \
+        return launch_kernel(scan_cl_staged_kernel<ST, false>, grid, block, 0, stream, nullptr, nullptr, args);         \
     }
 
 }  // namespace scanscam

@@ -1,0 +1,102 @@
+"""
+The channels-last kernel that stages contiguous tiles through LDS: parity with the CPU oracle at the edges of its
+tiles (256 threads x 2 vectors; spans of at most 32 / element size - 1 steps), through the C ABI.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from scanscam_amd import hip
+from test_hip_channels_last import as_rows, prev_abs, rel_err
+
+STAGED = hip.Plan(mode=hip.MODE_STAGED)
+# fp32 chains differ from the oracle's by a few roundings per step that the gates (below 1) do not amplify; results of
+# 16-bit storage by one rounding of the type, and the gate gradient by that of the stored output as well.
+BAR = {torch.float32: 1e-5, torch.float64: 1e-13, torch.bfloat16: 1e-2, torch.float16: 2e-3}
+
+
+def scan_pair(gpu, shape, dtype, plan, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    wide = torch.float64 if dtype == torch.float64 else torch.float32
+    a = torch.rand(shape, generator=g, dtype=wide).to(dtype)
+    b, gh = (torch.randn(shape, generator=g, dtype=wide).to(dtype) for _ in range(2))
+    da, db, dgh = a.to(gpu), b.to(gpu), gh.to(gpu)
+    h = hip.transposed_linear_scan_forward(da, db, plan=plan)
+    ga, gb = hip.transposed_linear_scan_backward(da, h, dgh, plan=plan)
+    return (a, b, gh), (da, db, dgh), (h, ga, gb)
+
+
+def check(inputs, results, dtype):
+    a, b, gh = (as_rows(t) for t in inputs)
+    h, ga, gb = (as_rows(t) for t in results)
+    assert rel_err(h, oracle.fwd(a, b)) <= BAR[dtype]
+    want_ga, want_gb = oracle.bwd(a, h, gh)
+    assert rel_err(gb, want_gb) <= BAR[dtype]
+    assert rel_err(ga, want_ga, prev_abs(h)) <= BAR[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", list(BAR))
+@pytest.mark.parametrize("C", [2, 3, 17, 40, 91, 127, 129, 255, 256])
+def test_edges_of_tiles_and_spans(gpu, dtype, C):
+    esize = torch.empty(0, dtype=dtype).element_size()
+    steps = 32 // esize - 1
+    tile = min((256 * 2 * 16 - 16) // (C * esize), 256 // C * steps)  # the longest tile
+    for T in sorted({2, steps, steps + 1, tile - 1, tile, tile + 1, 2 * tile + 1, 3 * tile + steps // 2}):
+        if T < 2:
+            continue
+        print(f"case staged {dtype} C={C} T={T}", flush=True)
+        inputs, _, results = scan_pair(gpu, (3, T, C), dtype, STAGED, seed=T)
+        check(inputs, results, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,shape", [(torch.float32, (600, 333, 33)), (torch.bfloat16, (2048, 167, 40)),
+                                         (torch.float16, (513, 400, 19)), (torch.float64, (520, 70, 130)),
+                                         (torch.float32, (512, 512, 12))])
+def test_automatic_route(gpu, dtype, shape):
+    """Calls whose automatic plan is this kernel give its very results, and agree with the other kernels."""
+    inputs, device, results = scan_pair(gpu, shape, dtype, None)
+    _, _, forced = scan_pair(gpu, shape, dtype, STAGED)
+    for x, y in zip(results, forced):
+        assert torch.equal(x, y)
+    few = [t[:7].contiguous() for t in inputs]
+    check(few, [t[:7] for t in results], dtype)
+    other = hip.resolve_plan_cl(*shape, dtype, hip.FORWARD)
+    h = hip.transposed_linear_scan_forward(device[0], device[1], plan=other)
+    assert rel_err(as_rows(results[0]), as_rows(h)) <= BAR[dtype]
+    # An output in place of an input, and bases off the 16-byte border (which this kernel leaves to the others).
+    L, code = hip.lib(), hip._dtype_code(dtype)
+    ws = torch.empty(max(8, hip.workspace_bytes_cl(*shape, dtype)), dtype=torch.uint8, device=gpu)
+    stream = torch.cuda.current_stream().cuda_stream
+    b = device[1].clone()
+    assert L.scanscam_scan_fwd_cl(device[0].data_ptr(), b.data_ptr(), b.data_ptr(), *shape, code, ws.data_ptr(), ws.numel(),
+                                  stream, None) == 0
+    assert torch.equal(b, results[0])
+    off = torch.empty(b.numel() + 1, dtype=dtype, device=gpu)[1:].view(shape)
+    off.copy_(device[1])
+    h = hip.transposed_linear_scan_forward(device[0], off)
+    assert rel_err(as_rows(results[0]), as_rows(h)) <= BAR[dtype]
+    with pytest.raises(RuntimeError):
+        hip.transposed_linear_scan_forward(device[0], off, plan=STAGED)
+
+
+@pytest.mark.gpu
+def test_nonfinite_values_stay_in_their_channel_and_batch_element(gpu):
+    shape = (3, 700, 33)
+    (a, b, gh), _, clean = scan_pair(gpu, shape, torch.float32, STAGED)
+    b[1, 350, 7] = np.nan
+    a, b, gh = a.to(gpu), b.to(gpu), gh.to(gpu)
+    h = hip.transposed_linear_scan_forward(a, b, plan=STAGED)
+    hit = torch.zeros(shape, dtype=torch.bool)
+    hit[1, 350:, 7] = True
+    assert torch.equal(torch.isnan(h).cpu(), hit)
+    assert torch.equal(h.cpu()[~hit], clean[0].cpu()[~hit])
+
+
+def test_only_channels_last_calls_take_it():
+    with pytest.raises(RuntimeError):
+        hip.resolve_plan(64, 4096, torch.float32, hip.FORWARD, STAGED)
+    with pytest.raises(RuntimeError):
+        hip.resolve_plan_cl(64, 4096, 40, torch.float32, hip.FORWARD, STAGED)
