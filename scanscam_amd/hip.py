@@ -130,6 +130,23 @@ except (OSError, AttributeError) as exc:  # not built, or built for another ABI
 has_hip_ops = _lib is not None
 
 
+def _bind_native(lib: ctypes.CDLL):
+    """The op's host path in native code (csrc/torch_binding.cpp) on this library's entry points, or ``None`` if it is
+    not built: the same calls then go through the Python functions below, three times as slowly on the host."""
+    try:
+        from . import _binding
+    except ImportError:
+        return None
+    _binding.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (
+        lib.scanscam_scan_fwd_strided, lib.scanscam_scan_bwd_strided, lib.scanscam_scan_fwd_cl_strided,
+        lib.scanscam_scan_bwd_cl_strided, lib.scanscam_workspace_bytes, lib.scanscam_workspace_bytes_cl,
+        lib.scanscam_strerror)))
+    return _binding
+
+
+_native = _bind_native(_lib) if _lib is not None else None
+
+
 def lib() -> ctypes.CDLL:
     """The loaded library; raises if it is not there (there is no substitute)."""
     if _lib is None:
@@ -775,6 +792,10 @@ def scan_forward(gate: torch.Tensor, value: torch.Tensor, plan: Optional[Plan] =
     reference's ``op.py:28-29``). Otherwise the row kernels on every tensor whose
     last dimension is unit-stride as it is (others are copied), result contiguous.
     """
+    if _native is not None and plan is None and not _check and _spin_limit == 0 and _lib is not None:
+        out = _native.forward(gate, value)  # None: a call it leaves to the code below
+        if out is not None:
+            return out
     _check_same(gate, value)
     if _is_cl_view(gate) and _is_cl_view(value):
         return _run_cl([gate, value], 1, FORWARD, plan)[0]
@@ -785,6 +806,10 @@ def scan_forward(gate: torch.Tensor, value: torch.Tensor, plan: Optional[Plan] =
 def scan_backward(gate: torch.Tensor, output: torch.Tensor, out_grad: torch.Tensor,
                   plan: Optional[Plan] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     """``(gate_grad, value_grad)`` for tensors of any strides; the counterpart of ``scan_forward``."""
+    if _native is not None and plan is None and not _check and _spin_limit == 0 and _lib is not None:
+        grads = _native.backward(gate, output, out_grad)
+        if grads is not None:
+            return grads
     _check_same(gate, output, out_grad)
     if _is_cl_view(gate) and _is_cl_view(output):
         ga, gb = _run_cl([gate, output, _to_cl(out_grad)], 2, BACKWARD, plan)
