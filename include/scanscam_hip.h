@@ -63,7 +63,9 @@ enum {
     SCANSCAM_MODE_FLAT = 4,     /* dense tensors, 16/sizeof(storage) <= T <= 64 * that: all rows scanned as one
                                    stream of aligned vectors with a reset at every row start (unroll 2 or 4) */
     SCANSCAM_MODE_STAGED = 5   /* channels-last only, dense tensors on 16-byte borders, C <= 256: contiguous tiles of a
-                                   batch element staged through LDS; the plan's other shape fields must be zero */
+                                   batch element staged through LDS; unroll = parts that its time is cut
+                                   into, each for a workgroup of its own (0: one; more need a workspace),
+                                   the plan's other shape fields must be zero */
 };
 
 /*
@@ -184,8 +186,9 @@ int scanscam_scan_bwd_timed(const void *a, const void *h, const void *gh, void *
  * GPU, time is also cut into tiles over workgroups, carried by a look-back
  * chain, which needs a workspace (scanscam_workspace_bytes_cl, same rules as
  * above); mode = SCANSCAM_MODE_ROW forbids that split, SCANSCAM_MODE_LOOKBACK
- * forces it. Many batch elements of few
- * or oddly many channels take SCANSCAM_MODE_STAGED by themselves. A time step (C channels, or the time stride of a strided call)
+ * forces it. Few channels, or oddly many
+ * of many batch elements, take SCANSCAM_MODE_STAGED by themselves, in parts only where the
+ * workspace is of the size that scanscam_workspace_bytes_cl gives. A time step (C channels, or the time stride of a strided call)
  * must stay below 4 GiB / 18 = 227 MiB (the kernels address a wave's steps with
  * 32-bit offsets from its first one): larger ones return SCANSCAM_EINVAL.
  */

@@ -693,11 +693,15 @@ int resolve_cl(const scanscam_plan *user, int64_t batch, int64_t T, int64_t C, i
 
 // Channels-last tiles staged through LDS (scan_staged_kernels.hpp): whether that kernel can run the call, and its tile.
 // Dense tensors on 16-byte borders, all channels of a batch element in one workgroup.
-bool resolve_staged(int64_t batch, int64_t T, int64_t C, int esize, const void *const ptrs[5], const int64_t sB[5],
-                    const int64_t sT[5], scanscam::StagedArgs *out)
+bool staged_fits(int64_t batch, int64_t T, int64_t C, const void *const ptrs[5], const int64_t sB[5], const int64_t sT[5])
 {
     for (int k = 0; k < 5; k++)
         if (!aligned_to(ptrs[k], 16) || (T > 1 && sT[k] != C) || (batch > 1 && sB[k] != T * C)) return false;
+    return true;
+}
+
+bool resolve_staged(int64_t batch, int64_t T, int64_t C, int esize, int64_t parts, scanscam::StagedArgs *out)
+{
     if (C > scanscam::kStagedThreads || batch >= (int64_t(1) << 31)) return false;
     // Steps per tile: what its vectors hold and what the threads' spans cover; then tiles of equal size, in spans of at
     // least half the steps a thread can take (every span costs every thread a read and an FMA for its carry).
@@ -714,27 +718,58 @@ bool resolve_staged(int64_t batch, int64_t T, int64_t C, int esize, const void *
     out->spans = (int32_t)((rows + seg - 1) / seg);
     const int64_t whole = out->spans * seg;  // (no span is cut short but those of the last tile)
     out->rows = (int32_t)(whole < most ? whole : most);
-    return true;
+    // Parts of equal numbers of tiles.
+    const int64_t all = (T + out->rows - 1) / out->rows;
+    if (parts > all) parts = all;
+    out->tiles = (int32_t)((all + parts - 1) / parts);
+    out->parts = (int32_t)((all + out->tiles - 1) / out->tiles);
+    out->pairs = nullptr;
+    return batch * out->parts < (int64_t(1) << 31);
 }
 
-// Whether an automatic plan takes that kernel. Measured against the plans of scan_cl_plan.hpp (forward / backward, us):
-//   few channels in lanes they do not fill, fp32 [1000, 1023, 17] 73.5 / 138 -> 43.3 / 79.3, [851, 467, 27] 41.2 / 69.2 ->
-//   28.6 / 48.6, bf16 [1000, 1023, 17] 56.3 / 102 -> 23.1 / 40.1, [2048, 512, 40] 65.2 / 105 -> 48.6 / 83.8, fp64
-//   [1000, 1023, 17] 115 / 209 -> 86.1 / 156; it ends where
+size_t staged_bytes(int64_t batch, int64_t C, int esize, const scanscam::StagedArgs &st)
+{
+    return st.parts > 1 ? (size_t)(batch * st.parts * C) * (esize == 8 ? 16 : 8) : 0;
+}
+
+// Into how many parts an automatic plan of that kernel cuts a batch element's time (1: one workgroup each, one launch);
+// 0: the plan is one of scan_cl_plan.hpp. Measured against those (forward / backward, us of GPU time).
+// Whole batch elements, for few channels in lanes they do not fill: fp32 [1000, 1023, 17] 73.5 / 138 -> 43.3 / 79.3,
+// [851, 467, 27] 41.2 / 69.2 -> 28.6 / 48.6, bf16 [1000, 1023, 17] 56.3 / 102 -> 23.1 / 40.1, [2048, 512, 40] 65.2 / 105 ->
+// 48.6 / 83.8, fp64 [1000, 1023, 17] 115 / 209 -> 86.1 / 156. It ends where
 //   - time steps are whole 128-byte lines (the walk streams them: fp32 [256, 1024, 128] 74.7 / 127 against 83.3 / 124) or
 //     fill the lanes of the packed kernel (fp32 [512, 4096, 8] 39.5 / 68.9 against 45.8 / 63.0; 16-bit lanes do not);
 //   - there are more channels, which fill the walk's lanes well (bf16 [1076, 490, 91] 79.1 / 138 against 85.8 / 147), but for
 //     fp32 steps off the 16-byte border and fp64 (fp32 [1076, 490, 91] 131 / 217 -> 114 / 202, fp64 [1024, 90, 130] 72.4 /
 //     129 -> 61.3 / 102);
-//   - batch elements are too few workgroups (fp32, C = 33: 320 of them 44.8 / 64.5 -> 40.3 / 65.5 us, 192 of them 46.2 /
-//     66.0 against 57.5 / 78.1; C = 130: 512 level, 320 37.4 / 60.7 against 51.9 / 87.8) or less than a tile and a half each
-//     (fp32 [3000, 16, 24] 5.5 / 7.8 against 7.9 / 12.3).
-bool staged_is_better(int64_t batch, int64_t T, int64_t C, int esize)
+//   - batch elements are too few workgroups (fp32, C = 33: 320 of them 44.8 / 64.5 -> 40.3 / 65.5, 192 of them 46.2 /
+//     66.0 against 57.5 / 78.1; C = 130: 512 level, 320 37.4 / 60.7 against 51.9 / 87.8) or less than a tile each (fp32
+//     [3000, 16, 24] 5.5 / 7.8 against 7.9 / 12.3; fp16 [5299, 101, 49], 10 KB each, 44.7 / 86.7 -> 40.0 / 61.4).
+// Parts, two launches that read gate and value twice but wait for nothing, for the fewer batch elements: fp32 [14, 13990,
+// 24] 32.0 / 44.8 -> 21.1 / 29.5, [1, 250000, 8] 92 / 98 -> 19 / 25, bf16 [39, 11559, 30] 57 / 81 -> 32 / 46, fp64 [3, 200000, 24]
+// 211 / 270 -> 105 / 160, small calls ([4, 458, 48] fp32 10.8 / 11.6 -> 8.0 / 8.8). 1280 workgroups, at most 256 parts (fp32
+// [1, 600000, 24] with 64 / 128 / 256 parts 309 / 159 / 86 us forwards; each workgroup folds the pairs before it). More channels
+// fill the lanes of the one-pass tiles, the sooner the more batch elements there are: fp32 [4, 100000, 40] 71 / 97 -> 65 /
+// 100, [16, 25000, 40] 61 / 84 against 63 / 98; bf16 [100, 3137, 51] level / 1.17 x, [100, 2500, 64] 31 / 47 against 37 / 52.
+int staged_parts(int64_t batch, int64_t T, int64_t C, int esize)
 {
-    const int64_t step = C * esize;
-    if (step % 128 == 0 || (esize >= 4 && step <= 64 && 64 % step == 0)) return false;
-    if (!(C <= 80 || esize == 8 || (esize == 4 && step % 16 != 0))) return false;
-    return (batch >= 512 || (batch >= 320 && C <= 80)) && T * step >= 12 * 1024;
+    const int64_t step = C * esize, elements = batch * T * C;
+    if (C > scanscam::kStagedThreads) return 0;
+    int64_t most;  // channels up to which time in parts is ahead
+    if (batch < 128) {
+        if (elements <= (int64_t(1) << 19)) most = 80;
+        else if (esize == 2) most = 52;
+        else most = batch <= (esize == 4 ? 8 : 16) ? 40 : 28;
+    } else {
+        most = batch < 320 && esize == 2 && elements >= (int64_t(1) << 23) ? 40 : 0;
+    }
+    if (C <= most && T * step >= 16 * 1024) {
+        const int64_t parts = (1280 + batch - 1) / batch;
+        return (int)(parts < 256 ? parts : 256);
+    }
+    if (step % 128 == 0 || (esize >= 4 && step <= 64 && 64 % step == 0)) return 0;
+    if (!(C <= 80 || esize == 8 || (esize == 4 && step % 16 != 0))) return 0;
+    return (batch >= 512 || (batch >= 320 && C <= 80)) && T * step >= 7680 ? 1 : 0;
 }
 
 int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void *y1,
@@ -779,8 +814,13 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     };
     scanscam::StagedArgs staged;
     if (plan && plan->mode == kModeStaged) {
-        if (plan->vec || plan->unroll || plan->waves || !resolve_staged(batch, T, C, esize, ptrs, sB, sT, &staged))
+        if (plan->vec || plan->waves || plan->unroll < 0 || !staged_fits(batch, T, C, ptrs, sB, sT) ||
+            !resolve_staged(batch, T, C, esize, plan->unroll ? plan->unroll : 1, &staged))
             return SCANSCAM_EPLAN;
+        const size_t need = staged_bytes(batch, C, esize, staged);
+        if (need != 0 && (!workspace || workspace_bytes < need)) return SCANSCAM_EWORKSPACE;
+        if (need != 0 && !aligned_to(workspace, 8)) return SCANSCAM_EALIGN;
+        staged.pairs = workspace;
         return run_staged(staged);
     }
     scanscam::ClLaunch l;
@@ -842,8 +882,14 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         if (!aligned_to(workspace, 8)) return SCANSCAM_EALIGN;
     }
     const bool free_plan = !plan || (plan->mode == SCANSCAM_MODE_AUTO && !plan->vec && !plan->unroll && !plan->waves);
-    if (free_plan && staged_is_better(batch, T, C, esize) && resolve_staged(batch, T, C, esize, ptrs, sB, sT, &staged))
-        return run_staged(staged);
+    const int parts = free_plan ? staged_parts(batch, T, C, esize) : 0;
+    if (parts > 0 && staged_fits(batch, T, C, ptrs, sB, sT) && resolve_staged(batch, T, C, esize, parts, &staged)) {
+        const size_t need = staged_bytes(batch, C, esize, staged);
+        if (need == 0 || (workspace && workspace_bytes >= need && aligned_to(workspace, 8))) {
+            staged.pairs = workspace;
+            return run_staged(staged);
+        }
+    }
     if (l.kind != 0) {
         args.ws = static_cast<uint64_t *>(workspace);
         const int64_t words = (int64_t)(l.ws_bytes / sizeof(uint64_t));
@@ -955,11 +1001,22 @@ size_t scanscam_workspace_bytes_cl(int64_t batch, int64_t T, int64_t C, int dtyp
     const int esize = elem_size(dtype);
     if (esize == 0 || batch <= 0 || T <= 0 || C <= 0 || T >= kMaxT || C >= kMaxT) return 0;
     size_t need = 0;
+    if (plan && plan->mode == kModeStaged) {
+        scanscam::StagedArgs st;
+        return resolve_staged(batch, T, C, esize, plan->unroll > 0 ? plan->unroll : 1, &st) ? staged_bytes(batch, C, esize, st) : 0;
+    }
     // The caller's pointers are not known yet: every alignment the tensors may turn out to have.
     for (int align = 16; align >= esize; align >>= 1) {
         scanscam::ClLaunch l;
         if (resolve_cl(plan, batch, T, C, dtype, align, direction == SCANSCAM_BACKWARD, &l) == SCANSCAM_OK && l.ws_bytes > need)
             need = l.ws_bytes;
+    }
+    const int parts = !plan || (plan->mode == SCANSCAM_MODE_AUTO && !plan->vec && !plan->unroll && !plan->waves)
+                          ? staged_parts(batch, T, C, esize) : 0;
+    scanscam::StagedArgs st;
+    if (parts > 1 && resolve_staged(batch, T, C, esize, parts, &st)) {
+        const size_t staged = staged_bytes(batch, C, esize, st);
+        if (staged > need) need = staged;
     }
     return need;
 }

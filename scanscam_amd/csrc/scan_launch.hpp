@@ -202,16 +202,21 @@ hipError_t launch_scan_cl(const ClArgs &args, const ClLaunch &l, bool rev, hipSt
         return hipErrorInvalidValue;                                                                   \
     }
 
-// The staged channels-last kernel: one workgroup per batch element.
+// The staged channels-last kernels: one workgroup per batch element, or one per part of it in two launches.
 template <typename ST> hipError_t launch_scan_staged(const StagedArgs &args, int64_t batch, bool rev, hipStream_t stream);
+
+#define SCANSCAM_STAGED_PASS(ST, PASS)                                                                 \
+    (rev ? launch_kernel(scan_cl_staged_kernel<ST, true, PASS>, grid, block, 0, stream, nullptr, nullptr, args)    \
+         : launch_kernel(scan_cl_staged_kernel<ST, false, PASS>, grid, block, 0, stream, nullptr, nullptr, args))
 
 #define SCANSCAM_DEFINE_STAGED_LAUNCH(ST)                                                              \
     template <>                                                                                        \
     hipError_t launch_scan_staged<ST>(const StagedArgs &args, int64_t batch, bool rev, hipStream_t stream) \
     {                                                                                                  \
-        const dim3 grid((unsigned)batch), block(kStagedThreads);                                       \
-        if (rev) return launch_kernel(scan_cl_staged_kernel<ST, true>, grid, block, 0, stream, nullptr, nullptr, args); \
-        return launch_kernel(scan_cl_staged_kernel<ST, false>, grid, block, 0, stream, nullptr, nullptr, args);         \
+        const dim3 grid((unsigned)(batch * args.parts)), block(kStagedThreads);                        \
+        if (args.parts == 1) return SCANSCAM_STAGED_PASS(ST, kWhole);                                  \
+        const hipError_t e = SCANSCAM_STAGED_PASS(ST, kReduce);                                        \
+        return e != hipSuccess ? e : SCANSCAM_STAGED_PASS(ST, kApply);                                 \
     }
 
 }  // namespace scanscam

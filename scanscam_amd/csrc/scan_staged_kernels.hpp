@@ -46,7 +46,14 @@ struct StagedArgs {
     int32_t rows;   // time steps per tile
     int32_t seg;    // time steps per thread and tile
     int32_t spans;  // spans of `seg` steps in a tile, at most kStagedThreads / C
+    int32_t parts;  // parts of a batch element's tiles, one workgroup each (1: the whole)
+    int32_t tiles;  // tiles per part
+    void *pairs;    // parts > 1: the parts' affine pairs, [B, parts, C]
 };
+
+// What a launch does: all of a batch element in one workgroup; or, with time in parts over workgroups, first every
+// part's affine pairs (kReduce), then the scan of every part from the composition of the pairs before it (kApply).
+enum StagedPass { kWhole, kReduce, kApply };
 
 constexpr int kStagedThreads = 256;
 constexpr int kStagedVectors = 2;  // 16-byte vectors per thread, tile and tensor
@@ -55,7 +62,7 @@ constexpr int kStagedVectors = 2;  // 16-byte vectors per thread, tile and tenso
 // different spans meet in different LDS banks.
 constexpr int staged_steps(int esize) { return 16 * kStagedVectors / esize - 1; }
 
-template <typename ST, bool REV>
+template <typename ST, bool REV, int PASS>
 __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const StagedArgs p)
 {
     using CT = typename ComputeOf<ST>::type;
@@ -64,7 +71,7 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
     using W = Vec<ST, 1>;
     using word_t = typename W::raw_t;  // one element as it is stored
     constexpr int NT = kStagedThreads, U = kStagedVectors, E = (int)sizeof(ST), VEC = 16 / E, SEG = staged_steps(E);
-    constexpr int NS = REV ? 3 : 2;       // tensors in: a, x, h
+    constexpr int NS = REV && PASS != kReduce ? 3 : 2;  // tensors in: a, x, h
     struct Pair { CT A, B; };
     __shared__ raw_t stage[NS][NT * U];
     __shared__ Pair ex[NT];
@@ -73,9 +80,14 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
     const int C = p.C, Q = p.spans;
     const int q = tid / C, c = tid - q * C;  // this thread's span and channel
     const bool active = q < Q;
-    const int64_t start = (int64_t)blockIdx.x * p.T * p.C * E;  // first byte of the batch element
+    const int64_t batch = PASS == kWhole ? blockIdx.x : blockIdx.x / p.parts;
+    const int part = PASS == kWhole ? 0 : (int)(blockIdx.x % p.parts);
+    if (PASS == kReduce && part == (REV ? 0 : p.parts - 1)) return;  // no part comes after it in scan order
+    const int64_t start = batch * p.T * p.C * E;  // first byte of the batch element
     const int step = p.C * E;             // bytes from time step to time step
-    const int ntiles = (p.T + p.rows - 1) / p.rows;
+    const int all_tiles = (p.T + p.rows - 1) / p.rows;
+    const int tile0 = PASS == kWhole ? 0 : part * p.tiles;  // tiles [tile0, tile1) are this workgroup's
+    const int tile1 = PASS == kWhole || all_tiles - tile0 < p.tiles ? all_tiles : tile0 + p.tiles;
 
     auto widen = [](word_t w) { CT f[1]; W::unpack(w, f); return f[0]; };
     auto narrow = [](CT v) { const CT f[1] = {v}; return W::pack(f); };
@@ -96,15 +108,51 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
                 reg[s][u] = V::load(reinterpret_cast<const ST *>(base + (off < end ? off : 0)));
             }
         }
-        if (REV) {
+        if (NS == 3) {
             edge_h = zero;
             if (q == 0 && t0 > 0)
                 edge_h = reinterpret_cast<const word_t *>(static_cast<const char *>(p.h) + (at - step))[c];
         }
     };
 
-    CT carry = CT(0);
+    CT carry = CT(0), product = CT(1);  // (product: kReduce, the composition of all gates)
     word_t a_next = zero;  // backwards: a of the step just after the tile (0 past the end)
+    if (REV && PASS != kWhole && active && tile1 < all_tiles)
+        a_next = reinterpret_cast<const word_t *>(static_cast<const char *>(p.a) + start + (int64_t)tile1 * p.rows * step)[c];
+    load(REV ? tile1 - 1 : tile0);
+    if (PASS == kApply) {
+        // The carry into this part: the pairs of the parts before it in scan order, in as many runs as there are threads
+        // for each channel.
+        const int before = REV ? p.parts - 1 - part : part;
+        const int runs = NT / C, run = (before + runs - 1) / runs;
+        const Pair *pairs = static_cast<const Pair *>(p.pairs) + batch * p.parts * C + c;
+        Pair sum = {CT(1), CT(0)};
+        if (q < runs) {
+            const int last = (q + 1) * run < before ? (q + 1) * run : before;
+            for (int i = q * run; i < last; i += 4) {
+                Pair e[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const int n = i + k < last ? i + k : last - 1;
+                    e[k] = pairs[(int64_t)(REV ? p.parts - 1 - n : n) * C];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    if (i + k < last) {
+                        sum.B = fma_(e[k].A, sum.B, e[k].B);
+                        sum.A = sum.A * e[k].A;
+                    }
+                }
+            }
+        }
+        ex[tid] = sum;
+        __syncthreads();
+        for (int i = 0; i < runs; i++) {
+            const Pair e = ex[i * C + c];
+            carry = fma_(e.A, carry, e.B);
+        }
+        // (ex is written again after the barriers of the first tile.)
+    }
     auto to_lds = [&]() {
 #pragma unroll
         for (int s = 0; s < NS; s++)
@@ -112,13 +160,13 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
             for (int u = 0; u < U; u++) stage[s][tid + u * NT] = reg[s][u];
     };
 
-    load(REV ? ntiles - 1 : 0);
     to_lds();
     __syncthreads();
+    const int ntiles = tile1 - tile0;
     for (int it = 0; it < ntiles; it++) {
-        const int tile = REV ? ntiles - 1 - it : it;
+        const int tile = REV ? tile1 - 1 - it : tile0 + it;
         const int t0 = tile * p.rows, n = p.T - t0 < p.rows ? p.T - t0 : p.rows;
-        const word_t edge0 = edge_h;
+        const word_t edge0 = NS == 3 ? edge_h : zero;
         if (it + 1 < ntiles) load(REV ? tile - 1 : tile + 1);
 
         // Byte of this thread's channels at step r of the tile, the same in every slot.
@@ -134,7 +182,7 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
         // The thread's steps in scan order, packed as they are stored: gate (backwards a of the step after) and
         // value, the identity past `cnt`, and backwards h of the step before. All reads are under way before the
         // first is used, and are kept for the replay.
-        word_t wa[SEG], wx[SEG], wh[REV ? SEG : 1];
+        word_t wa[SEG], wx[SEG], wh[NS == 3 ? SEG : 1];
         if (cnt == SEG) {
 #pragma unroll
             for (int i = 0; i < SEG; i++) {
@@ -142,20 +190,20 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
                 if (!REV) wa[i] = *at(0, r);
                 else if (i > 0) wa[i] = *at(0, r + 1);
                 wx[i] = *at(1, r);
-                if (REV && i + 1 < SEG) wh[i] = *at(2, r - 1);
+                if (NS == 3 && i + 1 < SEG) wh[i] = *at(2, r - 1);
             }
         } else {
 #pragma unroll
             for (int i = 0; i < SEG; i++) {
                 wa[i] = one;
                 wx[i] = zero;
-                if (REV) wh[i] = zero;
+                if (NS == 3) wh[i] = zero;
                 if (i < cnt) {
                     const int r = REV ? r1 - 1 - i : r0 + i;
                     if (!REV) wa[i] = *at(0, r);
                     else if (i > 0) wa[i] = *at(0, r + 1);
                     wx[i] = *at(1, r);
-                    if (REV && i + 1 < cnt) wh[i] = *at(2, r - 1);
+                    if (NS == 3 && i + 1 < cnt) wh[i] = *at(2, r - 1);
                 }
             }
         }
@@ -164,8 +212,9 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
             // a of this tile's first step.
             if (cnt > 0) {
                 wa[0] = r1 < n ? *at(0, r1) : a_next;
-                const word_t before = r0 > 0 ? *at(2, r0 - 1) : edge0;
-                if (cnt == SEG) {
+                const word_t before = NS == 3 && r0 > 0 ? *at(2, r0 - 1) : edge0;
+                if (NS < 3) {
+                } else if (cnt == SEG) {
                     wh[SEG - 1] = before;
                 } else {
 #pragma unroll
@@ -192,9 +241,17 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
                 const Pair e = ex[qq * C + c];
                 if (qq == q) mine = carry;
                 carry = fma_(e.A, carry, e.B);
+                if (PASS == kReduce) product = product * e.A;
             }
         } else {
             carry = fma_(A, carry, B);
+            if (PASS == kReduce) product = product * A;
+        }
+        if (PASS == kReduce) {
+            __syncthreads();
+            if (it + 1 < ntiles) to_lds();
+            __syncthreads();
+            continue;
         }
 
         // Backwards the results of a step go over gh and h of that step; the neighbours' border steps were read before
@@ -205,7 +262,7 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
             if (cnt == SEG || i < cnt) {
                 const int r = REV ? r1 - 1 - i : r0 + i;
                 *at(1, r) = narrow(mine);
-                if (REV) *at(2, r) = narrow(mine * widen(wh[i]));
+                if (NS == 3) *at(2, r) = narrow(mine * widen(wh[i]));
             }
         }
         __syncthreads();
@@ -239,6 +296,8 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
         }
         __syncthreads();
     }
+    if (PASS == kReduce && q == 0)
+        static_cast<Pair *>(p.pairs)[(batch * p.parts + part) * C + c] = Pair{product, carry};
 }
 
 }  // namespace scanscam

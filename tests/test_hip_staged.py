@@ -52,13 +52,46 @@ def test_edges_of_tiles_and_spans(gpu, dtype, C):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", list(BAR))
+@pytest.mark.parametrize("C", [2, 24, 64, 91, 129, 256])
+def test_time_in_parts(gpu, dtype, C):
+    """Two launches: the parts' pairs, then every part from the pairs before it. Parts of one and of several tiles, the
+    last one short, more parts than tiles, and as many as the runs of threads that fold the pairs do not divide."""
+    esize = torch.empty(0, dtype=dtype).element_size()
+    tile = min((256 * 2 * 16 - 16) // (C * esize), 256 // C * (32 // esize - 1))
+    for T, parts in ((tile + 1, 2), (5 * tile + 3, 2), (5 * tile + 3, 5), (7 * tile, 64), (67 * tile + 1, 66)):
+        print(f"case staged in parts {dtype} C={C} T={T} parts={parts}", flush=True)
+        inputs, _, results = scan_pair(gpu, (2, T, C), dtype, hip.Plan(mode=hip.MODE_STAGED, unroll=parts), seed=T)
+        check(inputs, results, dtype)
+
+
+@pytest.mark.gpu
+def test_a_short_workspace_leaves_the_other_kernels(gpu):
+    """A workspace below the size asked for is no error where the one-pass kernels can do with it, as ever."""
+    B, T, C = 100, 400, 24
+    a, b = torch.rand(B, T, C, device=gpu), torch.rand(B, T, C, device=gpu)
+    want = hip.transposed_linear_scan_forward(a, b)
+    L, stream = hip.lib(), torch.cuda.current_stream().cuda_stream
+    other = hip.resolve_plan_cl(B, T, C, torch.float32, hip.FORWARD)
+    need = hip.workspace_bytes_cl(B, T, C, torch.float32, hip.FORWARD, other)
+    assert need < hip.workspace_bytes_cl(B, T, C, torch.float32, hip.FORWARD) or need > 0
+    out, ws = torch.empty_like(a), torch.empty(max(need, 8), dtype=torch.uint8, device=gpu)
+    assert L.scanscam_scan_fwd_cl(a.data_ptr(), b.data_ptr(), out.data_ptr(), B, T, C, 0, ws.data_ptr(), need, stream, None) == 0
+    assert rel_err(as_rows(out), as_rows(want)) <= 1e-5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype,shape", [(torch.float32, (600, 333, 33)), (torch.bfloat16, (2048, 167, 40)),
                                          (torch.float16, (513, 400, 19)), (torch.float64, (520, 70, 130)),
-                                         (torch.float32, (512, 512, 12))])
+                                         (torch.float32, (512, 512, 12)), (torch.float32, (14, 2000, 24)),
+                                         (torch.bfloat16, (100, 900, 33)), (torch.float64, (1, 30000, 8)),
+                                         (torch.float16, (150, 1700, 37))])
 def test_automatic_route(gpu, dtype, shape):
     """Calls whose automatic plan is this kernel give its very results, and agree with the other kernels."""
     inputs, device, results = scan_pair(gpu, shape, dtype, None)
-    _, _, forced = scan_pair(gpu, shape, dtype, STAGED)
+    parts = 1 if shape[0] >= 320 else min(256, -(-1280 // shape[0]))
+    staged = hip.Plan(mode=hip.MODE_STAGED, unroll=parts)
+    _, _, forced = scan_pair(gpu, shape, dtype, staged)
     for x, y in zip(results, forced):
         assert torch.equal(x, y)
     few = [t[:7].contiguous() for t in inputs]
@@ -79,16 +112,17 @@ def test_automatic_route(gpu, dtype, shape):
     h = hip.transposed_linear_scan_forward(device[0], off)
     assert rel_err(as_rows(results[0]), as_rows(h)) <= BAR[dtype]
     with pytest.raises(RuntimeError):
-        hip.transposed_linear_scan_forward(device[0], off, plan=STAGED)
+        hip.transposed_linear_scan_forward(device[0], off, plan=staged)
 
 
 @pytest.mark.gpu
-def test_nonfinite_values_stay_in_their_channel_and_batch_element(gpu):
-    shape = (3, 700, 33)
-    (a, b, gh), _, clean = scan_pair(gpu, shape, torch.float32, STAGED)
+@pytest.mark.parametrize("parts", [1, 6])
+def test_nonfinite_values_stay_in_their_channel_and_batch_element(gpu, parts):
+    shape, plan = (3, 700, 33), hip.Plan(mode=hip.MODE_STAGED, unroll=parts)
+    (a, b, gh), _, clean = scan_pair(gpu, shape, torch.float32, plan)
     b[1, 350, 7] = np.nan
     a, b, gh = a.to(gpu), b.to(gpu), gh.to(gpu)
-    h = hip.transposed_linear_scan_forward(a, b, plan=STAGED)
+    h = hip.transposed_linear_scan_forward(a, b, plan=plan)
     hit = torch.zeros(shape, dtype=torch.bool)
     hit[1, 350:, 7] = True
     assert torch.equal(torch.isnan(h).cpu(), hit)
