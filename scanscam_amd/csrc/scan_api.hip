@@ -747,7 +747,8 @@ size_t staged_bytes(int64_t batch, int64_t C, int esize, const scanscam::StagedA
 //     [3000, 16, 24] 5.5 / 7.8 against 7.9 / 12.3; fp16 [5299, 101, 49], 10 KB each, 44.7 / 86.7 -> 40.0 / 61.4).
 // Parts, two launches that read gate and value twice but wait for nothing, for the fewer batch elements: fp32 [14, 13990,
 // 24] 32.0 / 44.8 -> 21.1 / 29.5, [1, 250000, 8] 92 / 98 -> 19 / 25, bf16 [39, 11559, 30] 57 / 81 -> 32 / 46, fp64 [3, 200000, 24]
-// 211 / 270 -> 105 / 160, small calls ([4, 458, 48] fp32 10.8 / 11.6 -> 8.0 / 8.8). 1280 workgroups, at most 256 parts (fp32
+// 211 / 270 -> 105 / 160, small calls ([4, 458, 48] fp32 10.8 / 11.6 -> 8.0 / 8.8; from 64 channels on a wave's lanes are
+// full in one pass, and the plan that resolve_plan_cl reports is the one that runs). 1280 workgroups, at most 256 parts (fp32
 // [1, 600000, 24] with 64 / 128 / 256 parts 309 / 159 / 86 us forwards; each workgroup folds the pairs before it). More channels
 // fill the lanes of the one-pass tiles, the sooner the more batch elements there are: fp32 [4, 100000, 40] 71 / 97 -> 65 /
 // 100, [16, 25000, 40] 61 / 84 against 63 / 98; bf16 [100, 3137, 51] level / 1.17 x, [100, 2500, 64] 31 / 47 against 37 / 52.
@@ -757,7 +758,7 @@ int staged_parts(int64_t batch, int64_t T, int64_t C, int esize)
     if (C > scanscam::kStagedThreads) return 0;
     int64_t most;  // channels up to which time in parts is ahead
     if (batch < 128) {
-        if (elements <= (int64_t(1) << 19)) most = 80;
+        if (elements <= (int64_t(1) << 19)) most = 63;
         else if (esize == 2) most = 52;
         else most = batch <= (esize == 4 ? 8 : 16) ? 40 : 28;
     } else {
