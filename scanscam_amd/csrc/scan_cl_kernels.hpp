@@ -219,6 +219,14 @@ struct ClSteps {
     // other lane and only its stores are masked, so no per-lane mask is kept per step.
     raw_t ra[S], rx[S];  // what issue() brought; dead once fold() has run
 
+    // Element-aligned 4-byte types load through the caches' normal policy (0; otherwise 2, non-temporal): a lane's 16 bytes
+    // straddle a line border that the next lane, wave or workgroup needs again, and non-temporal lines are the first to
+    // go. fp32 [64, 2048, 1001] 363 / 608 -> 350 / 575 us, a forward and a backward pass over buffers in rotation 969 -> 909
+    // us; [16, 4096, 1999] 977 -> 902 us, [256, 500, 513] 473 -> 444 us. 16-bit types lose as often as they gain (bf16 [64, 2048,
+    // 1001] 185 / 353 against 194 / 314 us, [400, 700, 203] 96 / 157 against 101 / 166 us), and on natural alignment it costs 7 %
+    // of what does not fit the last-level cache (fp32 [64, 2048, 1024] 263 / 439 against 280 / 474 us).
+    static constexpr int LOADS = RAGGED && sizeof(ST) == 4 ? 0 : 2;
+
     // Issues every load of the wave's S steps; nothing waits for them here.
     __device__ __forceinline__ void issue(const ClLane<ST> &ln, int T, int first_step, int limit_)
     {
@@ -245,9 +253,9 @@ struct ClSteps {
             const unsigned off_x = in ? step_off(t, ln.px) : 0u;
             const unsigned off_a = a_in ? step_off(REV ? t + 1 : t, ln.pa) : 0u;
             if (APPLY) {
-                ra[s] = BV::template load<2>(res_a, ln.c, off_a);
-                rx[s] = BV::template load<2>(res_x, ln.c, off_x);
-                if (REV) n_rh[s] = BV::template load<2>(res_h, ln.c, h_in ? step_off(t - 1, ln.ph) : 0u);
+                ra[s] = BV::template load<LOADS>(res_a, ln.c, off_a);
+                rx[s] = BV::template load<LOADS>(res_x, ln.c, off_x);
+                if (REV) n_rh[s] = BV::template load<LOADS>(res_h, ln.c, h_in ? step_off(t - 1, ln.ph) : 0u);
             } else {
                 ra[s] = BV::template load<0>(res_a, ln.c, off_a);
                 rx[s] = BV::template load<0>(res_x, ln.c, off_x);
