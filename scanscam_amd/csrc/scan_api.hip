@@ -723,13 +723,13 @@ bool resolve_staged(int64_t batch, int64_t T, int64_t C, int esize, int64_t part
     if (parts > all) parts = all;
     out->tiles = (int32_t)((all + parts - 1) / parts);
     out->parts = (int32_t)((all + out->tiles - 1) / out->tiles);
-    out->pairs = nullptr;
+    out->ws = nullptr;
     return batch * out->parts < (int64_t(1) << 31);
 }
 
 size_t staged_bytes(int64_t batch, int64_t C, int esize, const scanscam::StagedArgs &st)
 {
-    return st.parts > 1 ? (size_t)(batch * st.parts * C) * (esize == 8 ? 16 : 8) : 0;
+    return st.parts > 1 ? scanscam::kStagedHeader * sizeof(uint64_t) + (size_t)(batch * st.parts * C) * (esize == 8 ? 16 : 8) : 0;
 }
 
 // Into how many parts an automatic plan of that kernel cuts a batch element's time (1: one workgroup each, one launch);
@@ -803,6 +803,9 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         st.h = rev ? h : a;  // never read in the forward pass
         st.y0 = y0;
         st.y1 = rev ? y1 : y0;
+        // Any workspace with room for the flag word is one scanscam_workspace_timed_out may be asked about.
+        if (workspace && workspace_bytes >= scanscam::kStagedHeader * sizeof(uint64_t) && aligned_to(workspace, 8))
+            st.ws = static_cast<uint64_t *>(workspace);
         hipError_t e = hipErrorInvalidValue;
         hipStream_t s = static_cast<hipStream_t>(stream);
         switch (dtype) {
@@ -821,7 +824,6 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         const size_t need = staged_bytes(batch, C, esize, staged);
         if (need != 0 && (!workspace || workspace_bytes < need)) return SCANSCAM_EWORKSPACE;
         if (need != 0 && !aligned_to(workspace, 8)) return SCANSCAM_EALIGN;
-        staged.pairs = workspace;
         return run_staged(staged);
     }
     scanscam::ClLaunch l;
@@ -887,8 +889,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     if (parts > 0 && staged_fits(batch, T, C, ptrs, sB, sT) && resolve_staged(batch, T, C, esize, parts, &staged)) {
         const size_t need = staged_bytes(batch, C, esize, staged);
         if (need == 0 || (workspace && workspace_bytes >= need && aligned_to(workspace, 8))) {
-            staged.pairs = workspace;
-            return run_staged(staged);
+                return run_staged(staged);
         }
     }
     if (l.kind != 0) {

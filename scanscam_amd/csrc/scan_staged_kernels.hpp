@@ -48,8 +48,10 @@ struct StagedArgs {
     int32_t spans;  // spans of `seg` steps in a tile, at most kStagedThreads / C
     int32_t parts;  // parts of a batch element's tiles, one workgroup each (1: the whole)
     int32_t tiles;  // tiles per part
-    void *pairs;    // parts > 1: the parts' affine pairs, [B, parts, C]
+    uint64_t *ws;   // workspace, or null where a call in one part has none: two words, the second of them the flag of
+                    // an expired wait (kTimeoutWord), then, parts > 1, the parts' affine pairs, [B, parts, C]
 };
+constexpr int kStagedHeader = 2;  // words of the workspace before the pairs
 
 // What a launch does: all of a batch element in one workgroup; or, with time in parts over workgroups, first every
 // part's affine pairs (kReduce), then the scan of every part from the composition of the pairs before it (kApply).
@@ -82,6 +84,8 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
     const bool active = q < Q;
     const int64_t batch = PASS == kWhole ? blockIdx.x : blockIdx.x / p.parts;
     const int part = PASS == kWhole ? 0 : (int)(blockIdx.x % p.parts);
+    // No workgroup waits for another here, so the flag says so, whatever the workspace held before.
+    if (PASS != kApply && p.ws && blockIdx.x == 0 && tid == 0) p.ws[kTimeoutWord] = 0;
     if (PASS == kReduce && part == (REV ? 0 : p.parts - 1)) return;  // no part comes after it in scan order
     const int64_t start = batch * p.T * p.C * E;  // first byte of the batch element
     const int step = p.C * E;             // bytes from time step to time step
@@ -125,7 +129,7 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
         // for each channel.
         const int before = REV ? p.parts - 1 - part : part;
         const int runs = NT / C, run = (before + runs - 1) / runs;
-        const Pair *pairs = static_cast<const Pair *>(p.pairs) + batch * p.parts * C + c;
+        const Pair *pairs = reinterpret_cast<const Pair *>(p.ws + kStagedHeader) + batch * p.parts * C + c;
         Pair sum = {CT(1), CT(0)};
         if (q < runs) {
             const int last = (q + 1) * run < before ? (q + 1) * run : before;
@@ -297,7 +301,7 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
         __syncthreads();
     }
     if (PASS == kReduce && q == 0)
-        static_cast<Pair *>(p.pairs)[(batch * p.parts + part) * C + c] = Pair{product, carry};
+        reinterpret_cast<Pair *>(p.ws + kStagedHeader)[(batch * p.parts + part) * C + c] = Pair{product, carry};
 }
 
 }  // namespace scanscam

@@ -2,11 +2,14 @@
 The channels-last kernel that stages contiguous tiles through LDS: parity with the CPU oracle at the edges of its
 tiles (256 threads x 2 vectors; spans of at most 32 / element size - 1 steps), through the C ABI.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
+import scanscam_amd
 from scanscam_amd import hip
 from test_hip_channels_last import as_rows, prev_abs, rel_err
 
@@ -113,6 +116,44 @@ def test_automatic_route(gpu, dtype, shape):
     assert rel_err(as_rows(results[0]), as_rows(h)) <= BAR[dtype]
     with pytest.raises(RuntimeError):
         hip.transposed_linear_scan_forward(device[0], off, plan=staged)
+
+
+# In parts in both directions; in one launch beside a look-back workspace in reserve (backwards), and without any.
+FLAG_SHAPES = [(torch.float32, (14, 2000, 24)), (torch.float64, (1, 30000, 8)), (torch.bfloat16, (100, 900, 33)),
+               (torch.float16, (1, 4000, 5)), (torch.float32, (600, 333, 33)), (torch.bfloat16, (2048, 167, 40))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,shape", FLAG_SHAPES)
+def test_no_expired_wait_is_reported(gpu, dtype, shape):
+    """This kernel waits for no other workgroup: whatever the workspace held before, its flag says so after the call."""
+    inputs, (a, b, gh), _ = scan_pair(gpu, shape, dtype, None)
+    L, code, stream = hip.lib(), hip._dtype_code(dtype), torch.cuda.current_stream().cuda_stream
+    h, g0, g1 = (torch.empty_like(a) for _ in range(3))
+    for direction in (hip.FORWARD, hip.BACKWARD):
+        need = max(16, hip.workspace_bytes_cl(*shape, dtype, direction))
+        ws = torch.full((need,), 255, dtype=torch.uint8, device=gpu)
+        print(f"case flag {dtype} {shape} direction={direction} workspace={need}", flush=True)
+        if direction == hip.FORWARD:
+            rc = L.scanscam_scan_fwd_cl(a.data_ptr(), b.data_ptr(), h.data_ptr(), *shape, code, ws.data_ptr(), need, stream, None)
+        else:
+            rc = L.scanscam_scan_bwd_cl(a.data_ptr(), h.data_ptr(), gh.data_ptr(), g0.data_ptr(), g1.data_ptr(), *shape, code,
+                                        ws.data_ptr(), need, stream, None)
+        assert rc == 0
+        flag = ctypes.c_int(-1)
+        assert L.scanscam_workspace_timed_out(ws.data_ptr(), stream, ctypes.byref(flag)) == 0 and flag.value == 0
+    check([t[:2].contiguous() for t in inputs], [t[:2] for t in (h, g0, g1)], dtype)
+    # The same through the op, with checking on; the allocator hands it memory that held something.
+    hip.check_waits(True)
+    try:
+        x, y = a.mT.requires_grad_(), b.mT.requires_grad_()
+        torch.full((4 << 20,), 255, dtype=torch.uint8, device=gpu)
+        out = scanscam_amd.scan(x, y)
+        grads = torch.autograd.grad(out, (x, y), gh.mT)
+    finally:
+        hip.check_waits(False)
+    for got, want in zip((out, *grads), (h, g0, g1)):
+        assert torch.equal(got.mT, want)
 
 
 @pytest.mark.gpu
