@@ -245,7 +245,10 @@ int scanscam_scan_bwd_cl_strided(const void *a, const void *h, const void *gh, v
  * Whether a wait for another workgroup's carry expired in a call that used this workspace (see
  * spin_limit in scanscam_plan): waits for the work on `stream` to finish, reads the workspace's flag
  * word and writes 1 or 0 to *timed_out. A correct launch never sets it; where it is set, the
- * affected outputs hold NaN. Meant for debugging and tests: it blocks the host. No counterpart in
+ * affected outputs hold NaN. Calls that look back (SCANSCAM_MODE_LOOKBACK) and staged ones
+ * (SCANSCAM_MODE_STAGED) clear the word first; a plan of another family waits for nothing and leaves the
+ * workspace as it is, also where scanscam_workspace_bytes() is not 0 (it covers tensors of other
+ * alignments): zero word 1 before the call where that may be. Meant for debugging and tests: it blocks the host. No counterpart in
  * the reference.
  */
 int scanscam_workspace_timed_out(const void *workspace, void *stream, int *timed_out);

@@ -233,12 +233,18 @@ def _raise_if_wait_expired(ws: Optional[torch.Tensor], what: str) -> None:
         raise RuntimeError(f"{what}: a wait for another workgroup's carry expired; the affected outputs hold NaN")
 
 
+def _new_workspace(n: int, device: torch.device) -> torch.Tensor:
+    """A workspace; with checking on its flag word is zero to begin with, because a plan that waits for nothing leaves
+    it as it is (the size covers every alignment the tensors may have, also those whose plan needs no workspace)."""
+    return (torch.zeros if _check else torch.empty)(n, dtype=torch.uint8, device=device)
+
+
 def _workspace(rows: int, T: int, dtype: torch.dtype, direction: int, plan: Optional[Plan],
                device: torch.device) -> Tuple[Optional[torch.Tensor], int, int]:
     n = workspace_bytes(rows, T, dtype, direction, plan)
     if n == 0:
         return None, 0, 0
-    ws = torch.empty(n, dtype=torch.uint8, device=device)
+    ws = _new_workspace(n, device)
     return ws, ws.data_ptr(), n
 
 
@@ -511,7 +517,7 @@ def _workspace_cl(L, batch: int, T: int, C: int, dtype: torch.dtype, direction: 
     n = workspace_bytes_cl(batch, T, C, dtype, direction, plan)
     if n == 0:
         return None, 0, 0
-    ws = torch.empty(n, dtype=torch.uint8, device=device)
+    ws = _new_workspace(n, device)
     return ws, ws.data_ptr(), n
 
 

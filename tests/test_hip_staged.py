@@ -147,7 +147,7 @@ def test_no_expired_wait_is_reported(gpu, dtype, shape):
     hip.check_waits(True)
     try:
         x, y = a.mT.requires_grad_(), b.mT.requires_grad_()
-        torch.full((4 << 20,), 255, dtype=torch.uint8, device=gpu)
+        torch.full((hip.workspace_bytes_cl(*shape, dtype),), 255, dtype=torch.uint8, device=gpu)
         out = scanscam_amd.scan(x, y)
         grads = torch.autograd.grad(out, (x, y), gh.mT)
     finally:

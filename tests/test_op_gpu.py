@@ -280,3 +280,23 @@ def test_expired_wait_raises_through_the_op_when_checking_is_on(gpu):
         torch.cuda.synchronize()
     finally:
         hip.check_waits(False)
+
+
+@pytest.mark.parametrize("direction", [hip.FORWARD, hip.BACKWARD])
+def test_checking_a_plan_that_leaves_its_workspace_alone(gpu, direction):
+    """Rows of 16128 on 16-byte borders are walked; the workspace is sized for those that are not, and holds what the
+    memory held before. Nothing waited, so nothing expired."""
+    shape = (20, 16128)
+    need = hip.workspace_bytes(*shape, torch.float32, direction)
+    assert need > 0
+    assert hip.resolve_plan(*shape, torch.float32, direction).mode != hip.MODE_LOOKBACK
+    a, b = torch.rand(shape, device=gpu), torch.randn(shape, device=gpu)
+    h = hip.scan_forward(a, b)
+    want = h if direction == hip.FORWARD else hip.scan_backward(a, h, b)[1]
+    torch.full((need,), 255, dtype=torch.uint8, device=gpu)
+    hip.check_waits(True)
+    try:
+        got = hip.scan_forward(a, b) if direction == hip.FORWARD else hip.scan_backward(a, h, b)[1]
+    finally:
+        hip.check_waits(False)
+    assert torch.equal(got, want)
