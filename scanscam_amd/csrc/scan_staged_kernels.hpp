@@ -64,6 +64,49 @@ constexpr int kStagedVectors = 2;  // 16-byte vectors per thread, tile and tenso
 // different spans meet in different LDS banks.
 constexpr int staged_steps(int esize) { return 16 * kStagedVectors / esize - 1; }
 
+// A product of a part's gates spans any number of steps, so it is kept as m * 2^e. In fp32 alone 1.02 to the 8000th is
+// infinite, and infinity times a carry of zero NaN where the recurrence itself stays finite (the other kernels compose
+// at most about a thousand steps before they go on from a value). Scaling by a power of two rounds nothing, so where fp32
+// holds the product, results have the bits they would have with it. It costs 1 to 5 % of a call in parts, 6 to 14 % with
+// two or three channels, whose tiles have the most spans (forward / backward, us: fp32 [14, 13990, 24] 21.2 / 29.7 ->
+// 21.5 / 29.9, [1, 250000, 8] 19.1 / 24.8 -> 20.2 / 25.7, [1, 1000000, 2] 36.0 / 47.6 -> 40.9 / 51.0).
+__device__ __forceinline__ float frexp_m(float v) { return __builtin_amdgcn_frexp_mantf(v); }
+__device__ __forceinline__ double frexp_m(double v) { return __builtin_amdgcn_frexp_mant(v); }
+__device__ __forceinline__ int frexp_e(float v) { return __builtin_amdgcn_frexp_expf(v); }
+__device__ __forceinline__ int frexp_e(double v) { return __builtin_amdgcn_frexp_exp(v); }
+__device__ __forceinline__ float scale2(float v, int e) { return __builtin_ldexpf(v, e); }
+__device__ __forceinline__ double scale2(double v, int e) { return __builtin_ldexp(v, e); }
+
+template <typename CT>
+struct GateProduct {
+    static constexpr int FAR = 1 << 22;  // nothing but zero survives 2^FAR, and no sum of a few hundred leaves 32 bits
+    CT m;  // |m| <= 1 (or not finite) while gates are multiplied onto it: no product of it and a gate overflows
+    int e;
+    __device__ __forceinline__ void times(CT g)
+    {
+        const CT v = m * g;
+        m = frexp_m(v);
+        e += frexp_e(v);
+    }
+    __device__ __forceinline__ void bound() { e = e < -FAR ? -FAR : (e > FAR ? FAR : e); }
+    __device__ __forceinline__ void normalise()  // 1 <= |m| < 2, or zero times 2^0
+    {
+        e += frexp_e(m) - 1;
+        m = CT(2) * frexp_m(m);
+        bound();
+        if (m == CT(0)) e = 0;
+    }
+};
+
+// What a part does to the value entering it: B + m * 2^e * value, m normalised (so that the scaled value overflows only
+// where the product does, and is subnormal only where the product is below twice the smallest normal number).
+template <typename CT>
+struct PartPair {
+    CT m, B;
+    int e;
+    __device__ __forceinline__ CT after(CT value) const { return fma_(m, scale2(value, e), B); }
+};
+
 template <typename ST, bool REV, int PASS>
 __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const StagedArgs p)
 {
@@ -75,8 +118,10 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
     constexpr int NT = kStagedThreads, U = kStagedVectors, E = (int)sizeof(ST), VEC = 16 / E, SEG = staged_steps(E);
     constexpr int NS = REV && PASS != kReduce ? 3 : 2;  // tensors in: a, x, h
     struct Pair { CT A, B; };
+    using Part = PartPair<CT>;
     __shared__ raw_t stage[NS][NT * U];
     __shared__ Pair ex[NT];
+    __shared__ int ex_e[PASS == kApply ? NT : 1];
 
     const int tid = threadIdx.x;
     const int C = p.C, Q = p.spans;
@@ -119,7 +164,8 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
         }
     };
 
-    CT carry = CT(0), product = CT(1);  // (product: kReduce, the composition of all gates)
+    CT carry = CT(0);
+    GateProduct<CT> product = {CT(1), 0};  // kReduce: of all gates
     word_t a_next = zero;  // backwards: a of the step just after the tile (0 past the end)
     if (REV && PASS != kWhole && active && tile1 < all_tiles)
         a_next = reinterpret_cast<const word_t *>(static_cast<const char *>(p.a) + start + (int64_t)tile1 * p.rows * step)[c];
@@ -129,12 +175,13 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
         // for each channel.
         const int before = REV ? p.parts - 1 - part : part;
         const int runs = NT / C, run = (before + runs - 1) / runs;
-        const Pair *pairs = reinterpret_cast<const Pair *>(p.ws + kStagedHeader) + batch * p.parts * C + c;
-        Pair sum = {CT(1), CT(0)};
+        const Part *pairs = reinterpret_cast<const Part *>(p.ws + kStagedHeader) + batch * p.parts * C + c;
+        GateProduct<CT> gates = {CT(1), 0};
+        CT value = CT(0);
         if (q < runs) {
             const int last = (q + 1) * run < before ? (q + 1) * run : before;
             for (int i = q * run; i < last; i += 4) {
-                Pair e[4];
+                Part e[4];
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     const int n = i + k < last ? i + k : last - 1;
@@ -143,17 +190,20 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     if (i + k < last) {
-                        sum.B = fma_(e[k].A, sum.B, e[k].B);
-                        sum.A = sum.A * e[k].A;
+                        value = e[k].after(value);
+                        gates.m *= e[k].m;
+                        gates.e += e[k].e;
                     }
                 }
+                gates.normalise();
             }
         }
-        ex[tid] = sum;
+        ex[tid] = Pair{gates.m, value};
+        ex_e[tid] = gates.e;
         __syncthreads();
         for (int i = 0; i < runs; i++) {
             const Pair e = ex[i * C + c];
-            carry = fma_(e.A, carry, e.B);
+            carry = Part{e.A, e.B, ex_e[i * C + c]}.after(carry);
         }
         // (ex is written again after the barriers of the first tile.)
     }
@@ -240,18 +290,21 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
         if (Q > 1) {
             ex[tid] = Pair{A, B};
             __syncthreads();
-            for (int i = 0; i < Q; i++) {
-                const int qq = REV ? Q - 1 - i : i;
-                const Pair e = ex[qq * C + c];
-                if (qq == q) mine = carry;
-                carry = fma_(e.A, carry, e.B);
-                if (PASS == kReduce) product = product * e.A;
+            if (PASS != kReduce || q == 0) {  // (kReduce: only the threads that write the part's pair)
+                for (int i = 0; i < Q; i++) {
+                    const int qq = REV ? Q - 1 - i : i;
+                    const Pair e = ex[qq * C + c];
+                    if (qq == q) mine = carry;
+                    carry = fma_(e.A, carry, e.B);
+                    if (PASS == kReduce) product.times(e.A);
+                }
             }
         } else {
             carry = fma_(A, carry, B);
-            if (PASS == kReduce) product = product * A;
+            if (PASS == kReduce) product.times(A);
         }
         if (PASS == kReduce) {
+            product.bound();
             __syncthreads();
             if (it + 1 < ntiles) to_lds();
             __syncthreads();
@@ -300,8 +353,10 @@ __global__ __launch_bounds__(kStagedThreads) void scan_cl_staged_kernel(const St
         }
         __syncthreads();
     }
-    if (PASS == kReduce && q == 0)
-        reinterpret_cast<Pair *>(p.ws + kStagedHeader)[(batch * p.parts + part) * C + c] = Pair{product, carry};
+    if (PASS == kReduce && q == 0) {
+        product.normalise();
+        reinterpret_cast<Part *>(p.ws + kStagedHeader)[(batch * p.parts + part) * C + c] = Part{product.m, carry, product.e};
+    }
 }
 
 }  // namespace scanscam

@@ -118,6 +118,45 @@ def test_automatic_route(gpu, dtype, shape):
         hip.transposed_linear_scan_forward(device[0], off, plan=staged)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", list(BAR))
+@pytest.mark.parametrize("C,parts", [(2, 0), (8, 0), (8, 3), (24, 40), (130, 9)])
+def test_growing_gates_over_a_zero_carry_in_parts(gpu, dtype, C, parts):
+    """Gates of 1.5 over 3000 steps of zeros: their product is beyond every type (2 ** 1754), the recurrence stays zero."""
+    plan = hip.Plan(mode=hip.MODE_STAGED, unroll=parts) if parts else None
+    T, grown = 12000, 3000
+    g = torch.Generator().manual_seed(C)
+    wide = torch.float64 if dtype == torch.float64 else torch.float32
+    a = torch.rand((1, T, C), generator=g, dtype=wide).to(dtype)
+    b, h, gh = (torch.randn((1, T, C), generator=g, dtype=wide).to(dtype) for _ in range(3))
+    a[:, :grown], b[:, :grown] = 1.5, 0
+    print(f"case growing gates {dtype} C={C} parts={parts}", flush=True)
+    got = hip.transposed_linear_scan_forward(a.to(gpu), b.to(gpu), plan=plan)
+    assert rel_err(as_rows(got), oracle.fwd(as_rows(a), as_rows(b))) <= BAR[dtype]
+    # Backwards: the gates of the last steps, under no gradient.
+    a, gh = a.flip(1).contiguous(), gh.clone()
+    gh[:, -grown:] = 0
+    ga, gb = hip.transposed_linear_scan_backward(a.to(gpu), h.to(gpu), gh.to(gpu), plan=plan)
+    want_ga, want_gb = oracle.bwd(as_rows(a), as_rows(h), as_rows(gh))
+    assert rel_err(as_rows(gb), want_gb) <= BAR[dtype]
+    assert rel_err(as_rows(ga), want_ga, prev_abs(as_rows(h))) <= BAR[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_small_carry_through_a_part_that_grows_and_shrinks(gpu, dtype):
+    """2 ** -100, doubled 160 times and halved again inside every part: powers of two throughout, so nothing rounds."""
+    T, C = 6400, 24
+    a, b = torch.ones((1, T, C), dtype=dtype), torch.zeros((1, T, C), dtype=dtype)
+    for t in range(100, T - 400, 400):
+        a[:, t:t + 160], a[:, t + 160:t + 320] = 2.0, 0.5
+    b[:, 0] = 2.0 ** -100
+    want = torch.cumprod(a.double(), 1) * 2.0 ** -100
+    for parts in (2, 5, 100):
+        got = hip.transposed_linear_scan_forward(a.to(gpu), b.to(gpu), plan=hip.Plan(mode=hip.MODE_STAGED, unroll=parts))
+        assert torch.equal(got.cpu().double(), want), parts
+
+
 # In parts in both directions; in one launch beside a look-back workspace in reserve (backwards), and without any.
 FLAG_SHAPES = [(torch.float32, (14, 2000, 24)), (torch.float64, (1, 30000, 8)), (torch.bfloat16, (100, 900, 33)),
                (torch.float16, (1, 4000, 5)), (torch.float32, (600, 333, 33)), (torch.bfloat16, (2048, 167, 40))]
