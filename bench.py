@@ -598,7 +598,8 @@ def channels_last_table(args, hip, torch):
     for B, T, C, dtype in shapes:
         f_ms, b_ms, nsets = time_channels_last(B, T, C, dtype, max(20, args.steps // 2), max(3, args.warmup // 2), hip, torch)
         n, esize = B * T * C, torch.empty(0, dtype=dtype).element_size()
-        short = lambda p: f"mode={p.mode} vec={p.vec} steps={p.unroll} waves={p.waves}"
+        short = lambda p: (f"staged parts={p.waves_per_row}" if p.waves_per_row  # noqa: E731
+                           else f"mode={p.mode} vec={p.vec} steps={p.unroll} waves={p.waves}")
         out[f"{B}x{T}x{C}_{str(dtype).replace('torch.', '')}"] = {
             "fwd_us": round(f_ms * 1e3, 1), "bwd_us": round(b_ms * 1e3, 1),
             "fwd_frac": round(FWD_BYTES[esize] * n / (f_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),

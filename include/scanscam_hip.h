@@ -74,7 +74,9 @@ enum {
  *   vec            elements per lane per load: 16/sizeof(storage) or 1
  *   unroll         64-lane chunks per wave per tile: 1, 2, 3, 4 or 8 (1 or 4 when vec == 1)
  *   waves          waves per workgroup, 1..16 (at most 8 when unroll == 8)
- *   waves_per_row  ROW only: a divisor of `waves` (waves / waves_per_row rows share a workgroup)
+ *   waves_per_row  row layout, ROW only: a divisor of `waves` (waves / waves_per_row rows share a workgroup);
+ *                  channels-last: parts of time in which SCANSCAM_MODE_STAGED takes the call where it can,
+ *                  the other fields then being the plan where it cannot
  *   spin_limit     kernels that wait for another workgroup's carry poll at most this many times
  *                  (0 = 2^20, about a second); a wait that expires sets word 1 of the workspace to 1
  *                  and poisons the affected outputs with NaN instead of spinning for ever
@@ -187,8 +189,9 @@ int scanscam_scan_bwd_timed(const void *a, const void *h, const void *gh, void *
  * chain, which needs a workspace (scanscam_workspace_bytes_cl, same rules as
  * above); mode = SCANSCAM_MODE_ROW forbids that split, SCANSCAM_MODE_LOOKBACK
  * forces it. Few channels, or oddly many
- * of many batch elements, take SCANSCAM_MODE_STAGED by themselves, in parts only where the
- * workspace is of the size that scanscam_workspace_bytes_cl gives. A time step (C channels, or the time stride of a strided call)
+ * of many batch elements, take SCANSCAM_MODE_STAGED by themselves (dense tensors on 16-byte borders; in
+ * parts only where the workspace is of the size that scanscam_workspace_bytes_cl gives; otherwise the
+ * plan that the model chooses). A time step (C channels, or the time stride of a strided call)
  * must stay below 4 GiB / 18 = 227 MiB (the kernels address a wave's steps with
  * 32-bit offsets from its first one): larger ones return SCANSCAM_EINVAL.
  */
@@ -264,9 +267,11 @@ int scanscam_resolve_plan(int64_t rows, int64_t T, int dtype, int direction, con
  * The same for the channels-last calls on dense [batch, T, C] tensors whose bases are 16-byte
  * aligned: mode SCANSCAM_MODE_ROW where a workgroup walks all of T, SCANSCAM_MODE_LOOKBACK where
  * tiles of time steps chain through the workspace; vec channels per lane, unroll time steps per
- * wave and tile, waves per workgroup. (A call that takes SCANSCAM_MODE_STAGED by itself has this plan, and its
- * workspace, in reserve for tensors the staged kernel cannot run.) No counterpart in the reference, whose kernel has one launch
- * shape (scanscam/cuda.py:69-95 passes channels_per_block only).
+ * wave and tile, waves per workgroup. waves_per_row > 0: the call takes SCANSCAM_MODE_STAGED by itself, in that
+ * many parts, and the other fields are the plan in reserve for tensors the staged kernel cannot run (zero
+ * waves_per_row to force that one). Handed back, the plan runs what the automatic call runs, bit for bit. A
+ * SCANSCAM_MODE_STAGED plan has nothing to resolve and is refused. No counterpart in the reference, whose kernel has
+ * one launch shape (scanscam/cuda.py:69-95 passes channels_per_block only).
  */
 int scanscam_resolve_plan_cl(int64_t batch, int64_t T, int64_t C, int dtype, int direction,
                              const scanscam_plan *plan, scanscam_plan *out);
@@ -274,7 +279,8 @@ int scanscam_resolve_plan_cl(int64_t batch, int64_t T, int64_t C, int dtype, int
 /*
  * The duration in microseconds that the library's cost model estimates for a channels-last call on dense
  * [batch, T, C] tensors with this plan (NULL or zero fields: with what the model itself chooses for them, i.e.
- * the estimate behind scanscam_resolve_plan_cl). The automatic plan is the candidate with the smallest such
+ * the estimate behind scanscam_resolve_plan_cl; of the plan in reserve where that reports waves_per_row > 0, since the
+ * model does not know the staged kernel). The plan is the candidate with the smallest such
  * estimate; the model (a formula of a few physical terms and a learned correction on top of it) is fitted to
  * timings on one MI355X (scanscam_amd/plan_fit.py), so the figure is a ranking aid with an error of about 5 %,
  * not a promise. The first call for a (shape, plan) on a thread takes about 0.1 ms on the host (the choice is

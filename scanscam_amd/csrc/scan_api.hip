@@ -773,6 +773,16 @@ int staged_parts(int64_t batch, int64_t T, int64_t C, int esize)
     return (batch >= 512 || (batch >= 320 && C <= 80)) && T * step >= 7680 ? 1 : 0;
 }
 
+// The parts in which a call with this plan takes the staged kernel, 0 for none: what a resolved plan says
+// (scanscam_resolve_plan_cl writes it into waves_per_row), the automatic choice where the plan leaves everything open.
+int staged_parts_of(const scanscam_plan *plan, int64_t batch, int64_t T, int64_t C, int esize)
+{
+    if (plan && plan->mode == kModeStaged) return plan->unroll > 0 ? plan->unroll : 1;
+    if (plan && plan->waves_per_row > 0) return plan->waves_per_row;
+    const bool free_plan = !plan || (plan->mode == SCANSCAM_MODE_AUTO && !plan->vec && !plan->unroll && !plan->waves);
+    return free_plan ? staged_parts(batch, T, C, esize) : 0;
+}
+
 int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void *y1,
            const scanscam_strides *const st[5], int64_t batch, int64_t T, int64_t C, int dtype, void *workspace,
            size_t workspace_bytes, void *stream, const scanscam_plan *plan)
@@ -819,7 +829,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     scanscam::StagedArgs staged;
     if (plan && plan->mode == kModeStaged) {
         if (plan->vec || plan->waves || plan->unroll < 0 || !staged_fits(batch, T, C, ptrs, sB, sT) ||
-            !resolve_staged(batch, T, C, esize, plan->unroll ? plan->unroll : 1, &staged))
+            !resolve_staged(batch, T, C, esize, staged_parts_of(plan, batch, T, C, esize), &staged))
             return SCANSCAM_EPLAN;
         const size_t need = staged_bytes(batch, C, esize, staged);
         if (need != 0 && (!workspace || workspace_bytes < need)) return SCANSCAM_EWORKSPACE;
@@ -884,8 +894,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         if (!workspace || workspace_bytes < l.ws_bytes) return SCANSCAM_EWORKSPACE;
         if (!aligned_to(workspace, 8)) return SCANSCAM_EALIGN;
     }
-    const bool free_plan = !plan || (plan->mode == SCANSCAM_MODE_AUTO && !plan->vec && !plan->unroll && !plan->waves);
-    const int parts = free_plan ? staged_parts(batch, T, C, esize) : 0;
+    const int parts = staged_parts_of(plan, batch, T, C, esize);
     if (parts > 0 && staged_fits(batch, T, C, ptrs, sB, sT) && resolve_staged(batch, T, C, esize, parts, &staged)) {
         const size_t need = staged_bytes(batch, C, esize, staged);
         if (need == 0 || (workspace && workspace_bytes >= need && aligned_to(workspace, 8))) {
@@ -1003,22 +1012,15 @@ size_t scanscam_workspace_bytes_cl(int64_t batch, int64_t T, int64_t C, int dtyp
     const int esize = elem_size(dtype);
     if (esize == 0 || batch <= 0 || T <= 0 || C <= 0 || T >= kMaxT || C >= kMaxT) return 0;
     size_t need = 0;
-    if (plan && plan->mode == kModeStaged) {
-        scanscam::StagedArgs st;
-        return resolve_staged(batch, T, C, esize, plan->unroll > 0 ? plan->unroll : 1, &st) ? staged_bytes(batch, C, esize, st) : 0;
-    }
+    const int parts = staged_parts_of(plan, batch, T, C, esize);
+    scanscam::StagedArgs st;
+    if (parts > 1 && resolve_staged(batch, T, C, esize, parts, &st)) need = staged_bytes(batch, C, esize, st);
+    if (plan && plan->mode == kModeStaged) return need;
     // The caller's pointers are not known yet: every alignment the tensors may turn out to have.
     for (int align = 16; align >= esize; align >>= 1) {
         scanscam::ClLaunch l;
         if (resolve_cl(plan, batch, T, C, dtype, align, direction == SCANSCAM_BACKWARD, &l) == SCANSCAM_OK && l.ws_bytes > need)
             need = l.ws_bytes;
-    }
-    const int parts = !plan || (plan->mode == SCANSCAM_MODE_AUTO && !plan->vec && !plan->unroll && !plan->waves)
-                          ? staged_parts(batch, T, C, esize) : 0;
-    scanscam::StagedArgs st;
-    if (parts > 1 && resolve_staged(batch, T, C, esize, parts, &st)) {
-        const size_t staged = staged_bytes(batch, C, esize, st);
-        if (staged > need) need = staged;
     }
     return need;
 }
@@ -1115,11 +1117,13 @@ int scanscam_resolve_plan_cl(int64_t batch, int64_t T, int64_t C, int dtype, int
     scanscam::ClLaunch l;
     const int rc = resolve_cl(plan, batch, T, C, dtype, align, direction == SCANSCAM_BACKWARD, &l);
     if (rc != SCANSCAM_OK) return rc;
+    const int parts = staged_parts_of(plan, batch, T, C, esize);  // (`out` may be the plan itself)
+    scanscam::StagedArgs st;
     out->mode = l.kind == 2 ? kModeLookback : kModeRow;
     out->vec = l.vec;
     out->unroll = l.steps;
     out->waves = l.waves;
-    out->waves_per_row = 0;
+    out->waves_per_row = parts > 0 && resolve_staged(batch, T, C, esize, parts, &st) ? st.parts : 0;
     out->spin_limit = (plan && plan->spin_limit > 0) ? plan->spin_limit : scanscam::kSpinLimit;
     return SCANSCAM_OK;
 }

@@ -490,7 +490,9 @@ def workspace_bytes_cl(batch: int, T: int, C: int, dtype: torch.dtype, direction
 
 def resolve_plan_cl(batch: int, T: int, C: int, dtype: torch.dtype, direction: int = FORWARD,
                     plan: Optional[Plan] = None) -> Plan:
-    """The plan the channels-last calls would run for dense ``[batch, T, C]`` tensors (no GPU needed)."""
+    """The plan the channels-last calls would run for dense ``[batch, T, C]`` tensors (no GPU needed). ``waves_per_row`` > 0:
+    the kernel that stages tiles through LDS, in that many parts of time; the other fields are then the plan of tensors it
+    cannot run."""
     out = Plan()
     rc = lib().scanscam_resolve_plan_cl(batch, T, C, _dtype_code(dtype), direction, _plan_ref(plan), ctypes.byref(out))
     if rc != 0:
@@ -500,7 +502,8 @@ def resolve_plan_cl(batch: int, T: int, C: int, dtype: torch.dtype, direction: i
 
 def predict_cl(batch: int, T: int, C: int, dtype: torch.dtype, direction: int = FORWARD,
                plan: Optional[Plan] = None) -> float:
-    """Microseconds the library's cost model estimates for this channels-last call and plan (no GPU needed)."""
+    """Microseconds the library's cost model estimates for this channels-last call and plan (no GPU needed); it has no
+    estimate of the staged kernel, and gives that of the plan in reserve."""
     us = ctypes.c_double()
     rc = lib().scanscam_predict_cl(batch, T, C, _dtype_code(dtype), direction, _plan_ref_plain(plan), ctypes.byref(us))
     if rc != 0:

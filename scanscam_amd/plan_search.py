@@ -162,9 +162,11 @@ def _time(calls, reps, warm):
     return e0.elapsed_time(e1) / reps * 1e3
 
 
-def _short(plan):
+def _short(plan, layout="rows"):
     if plan is None:
         return "auto"
+    if layout == "cl" and plan.waves_per_row:
+        return f"staged x{plan.waves_per_row}"
     s = f"m{plan.mode} v{plan.vec} u{plan.unroll} w{plan.waves}"
     return s + (f" r{plan.waves_per_row}" if plan.waves_per_row else "")
 
@@ -217,7 +219,7 @@ def search(layout, shape, dtype, reps=24, warm=4, out=sys.stdout, every=False, d
         best, best_plan = min(times[name], key=lambda tp: tp[0])
         res[name] = (auto, best, best_plan)
         frac = per_elem * esize * n / (auto * 1e-6) / 1e9 / HBM_PEAK_GBPS
-        text.append(f"{name} auto [{_short(auto_plan):16s}] {auto:7.1f} us {100 * frac:4.1f} %  best {best:7.1f} {_short(best_plan):16s}"
+        text.append(f"{name} auto [{_short(auto_plan, layout):16s}] {auto:7.1f} us {100 * frac:4.1f} %  best {best:7.1f} {_short(best_plan):16s}"
                     + (" BEHIND" if auto > 1.08 * best else "       "))
     label = "x".join(str(d) for d in shape) + ":" + str(dtype).replace("torch.", "")
     print(f"{layout} {label:26s} {len(times['fwd']) - 2:2d} plans | " + " | ".join(text), file=out, flush=True)

@@ -293,6 +293,8 @@ int main(void)
     failures += check_case("long rows [3, 300000]", 3, 300000, 0, 0, stream);
     failures += check_case("channels-last [4, 999, 320]", 4 * 320, 999, 320, 1, stream);
     failures += check_case("channels-last [1, 2048, 64]", 64, 2048, 64, 1, stream);
+    failures += check_case("channels-last [14, 2000, 24]", 14 * 24, 2000, 24, 1, stream);
+    failures += check_case("channels-last [512, 100, 33]", 512 * 33, 100, 33, 1, stream);
     failures += check_strided("halves of x[6][2*40][1000]", 6, 40, 1000, 0, stream);
     failures += check_strided("halves of x[2][2*3][200000]", 2, 3, 200000, 0, stream);
     failures += check_strided("halves of x[5][777][2*192]", 5, 192, 777, 1, stream);

@@ -69,18 +69,32 @@ def test_time_in_parts(gpu, dtype, C):
 
 
 @pytest.mark.gpu
-def test_a_short_workspace_leaves_the_other_kernels(gpu):
-    """A workspace below the size asked for is no error where the one-pass kernels can do with it, as ever."""
-    B, T, C = 100, 400, 24
-    a, b = torch.rand(B, T, C, device=gpu), torch.rand(B, T, C, device=gpu)
-    want = hip.transposed_linear_scan_forward(a, b)
-    L, stream = hip.lib(), torch.cuda.current_stream().cuda_stream
-    other = hip.resolve_plan_cl(B, T, C, torch.float32, hip.FORWARD)
-    need = hip.workspace_bytes_cl(B, T, C, torch.float32, hip.FORWARD, other)
-    assert need < hip.workspace_bytes_cl(B, T, C, torch.float32, hip.FORWARD) or need > 0
-    out, ws = torch.empty_like(a), torch.empty(max(need, 8), dtype=torch.uint8, device=gpu)
-    assert L.scanscam_scan_fwd_cl(a.data_ptr(), b.data_ptr(), out.data_ptr(), B, T, C, 0, ws.data_ptr(), need, stream, None) == 0
-    assert rel_err(as_rows(out), as_rows(want)) <= 1e-5
+@pytest.mark.parametrize("dtype,shape", [(torch.bfloat16, (250, 1000, 39)), (torch.float32, (3, 4000, 40))])
+def test_a_short_workspace_leaves_the_other_kernels(gpu, dtype, shape):
+    """A workspace below the size asked for is no error where the plan in reserve, a walk or tiles, can do with it."""
+    code, L = hip._dtype_code(dtype), hip.lib()
+    _, (a, b, gh), (h, ga, gb) = scan_pair(gpu, shape, dtype, None)
+    stream = torch.cuda.current_stream().cuda_stream
+    for direction in (hip.FORWARD, hip.BACKWARD):
+        other = hip.resolve_plan_cl(*shape, dtype, direction)
+        assert other.waves_per_row > 1
+        other.waves_per_row = 0
+        need = hip.workspace_bytes_cl(*shape, dtype, direction, other)
+        assert need < hip.workspace_bytes_cl(*shape, dtype, direction)
+        ws = torch.empty(max(need, 8), dtype=torch.uint8, device=gpu)
+        x, y = torch.empty_like(a), torch.empty_like(a)
+        if direction == hip.FORWARD:
+            rc = L.scanscam_scan_fwd_cl(a.data_ptr(), b.data_ptr(), x.data_ptr(), *shape, code, ws.data_ptr(), need, stream, None)
+            got, auto = (x,), (h,)
+            want = (hip.transposed_linear_scan_forward(a, b, plan=other),)
+        else:
+            rc = L.scanscam_scan_bwd_cl(a.data_ptr(), h.data_ptr(), gh.data_ptr(), x.data_ptr(), y.data_ptr(), *shape, code,
+                                        ws.data_ptr(), need, stream, None)
+            got, auto = (x, y), (ga, gb)
+            want = hip.transposed_linear_scan_backward(a, h, gh, plan=other)
+        assert rc == 0
+        for g, w, s in zip(got, want, auto):
+            assert torch.equal(g, w) and rel_err(as_rows(g), as_rows(s)) <= BAR[dtype]
 
 
 @pytest.mark.gpu
@@ -92,16 +106,20 @@ def test_a_short_workspace_leaves_the_other_kernels(gpu):
 def test_automatic_route(gpu, dtype, shape):
     """Calls whose automatic plan is this kernel give its very results, and agree with the other kernels."""
     inputs, device, results = scan_pair(gpu, shape, dtype, None)
-    parts = 1 if shape[0] >= 320 else min(256, -(-1280 // shape[0]))
-    staged = hip.Plan(mode=hip.MODE_STAGED, unroll=parts)
+    plans = [hip.resolve_plan_cl(*shape, dtype, d) for d in (hip.FORWARD, hip.BACKWARD)]
+    assert plans[0].waves_per_row == plans[1].waves_per_row > 0
+    staged = hip.Plan(mode=hip.MODE_STAGED, unroll=plans[0].waves_per_row)
     _, _, forced = scan_pair(gpu, shape, dtype, staged)
-    for x, y in zip(results, forced):
-        assert torch.equal(x, y)
+    ga, gb = hip.transposed_linear_scan_backward(device[0], results[0], device[2], plan=plans[1])
+    resolved = (hip.transposed_linear_scan_forward(device[0], device[1], plan=plans[0]), ga, gb)
+    for x, y, z in zip(results, forced, resolved):
+        assert torch.equal(x, y) and torch.equal(x, z)
     few = [t[:7].contiguous() for t in inputs]
     check(few, [t[:7] for t in results], dtype)
-    other = hip.resolve_plan_cl(*shape, dtype, hip.FORWARD)
+    other = plans[0]
+    other.waves_per_row = 0
     h = hip.transposed_linear_scan_forward(device[0], device[1], plan=other)
-    assert rel_err(as_rows(results[0]), as_rows(h)) <= BAR[dtype]
+    assert rel_err(as_rows(results[0]), as_rows(h)) <= BAR[dtype] and not torch.equal(h, results[0])
     # An output in place of an input, and bases off the 16-byte border (which this kernel leaves to the others).
     L, code = hip.lib(), hip._dtype_code(dtype)
     ws = torch.empty(max(8, hip.workspace_bytes_cl(*shape, dtype)), dtype=torch.uint8, device=gpu)
@@ -113,7 +131,7 @@ def test_automatic_route(gpu, dtype, shape):
     off = torch.empty(b.numel() + 1, dtype=dtype, device=gpu)[1:].view(shape)
     off.copy_(device[1])
     h = hip.transposed_linear_scan_forward(device[0], off)
-    assert rel_err(as_rows(results[0]), as_rows(h)) <= BAR[dtype]
+    assert not torch.equal(h, results[0]) and rel_err(as_rows(results[0]), as_rows(h)) <= BAR[dtype]
     with pytest.raises(RuntimeError):
         hip.transposed_linear_scan_forward(device[0], off, plan=staged)
 
@@ -214,3 +232,27 @@ def test_only_channels_last_calls_take_it():
         hip.resolve_plan(64, 4096, torch.float32, hip.FORWARD, STAGED)
     with pytest.raises(RuntimeError):
         hip.resolve_plan_cl(64, 4096, 40, torch.float32, hip.FORWARD, STAGED)
+
+
+def test_a_resolved_plan_says_what_runs():
+    """What scanscam_resolve_plan_cl reports holds the staged kernel's parts as well; it resolves to itself, also in place,
+    and asks for the automatic call's workspace; without the parts it is the plan in reserve."""
+    L, staged = hip.lib(), 0
+    for dtype in BAR:
+        code = hip._dtype_code(dtype)
+        for batch, T, C in ((14, 2000, 24), (1, 30000, 8), (600, 333, 33), (2048, 512, 40), (200, 9000, 37), (8, 4096, 512),
+                            (64, 2048, 1001), (1, 4000, 64), (90, 700, 257)):
+            for direction in (hip.FORWARD, hip.BACKWARD):
+                plan, again, reserve = hip.resolve_plan_cl(batch, T, C, dtype, direction), hip.Plan(), hip.Plan()
+                staged += plan.waves_per_row > 0
+                need = hip.workspace_bytes_cl(batch, T, C, dtype, direction)
+                assert hip.workspace_bytes_cl(batch, T, C, dtype, direction, plan) <= need
+                ctypes.memmove(ctypes.byref(again), ctypes.byref(plan), ctypes.sizeof(hip.Plan))
+                ref = ctypes.byref(again)
+                assert L.scanscam_resolve_plan_cl(batch, T, C, code, direction, ref, ref) == 0
+                assert bytes(again) == bytes(plan)
+                ctypes.memmove(ctypes.byref(reserve), ctypes.byref(plan), ctypes.sizeof(hip.Plan))
+                reserve.waves_per_row = 0
+                back = hip.resolve_plan_cl(batch, T, C, dtype, direction, reserve)
+                assert bytes(back) == bytes(reserve)
+    assert staged >= 20
