@@ -45,6 +45,7 @@ struct ClArgs {
     int32_t group;      // packed kernel: lanes per time step (power of two below 64)
     int32_t xcd_order;  // scan_cl_kernel, scan_cl_lookback_kernel: consecutive (batch element, channel group) pairs share an XCD
     int32_t cached_stores;  // outputs through the caches' normal policy instead of non-temporal (the host decides, see run_cl)
+    int32_t cached_loads;    // element-aligned 8-byte lanes of 4-byte types: the same for loads
     uint64_t *ws;       // look-back kernel: ticket counters + published pairs
     int32_t spin_limit; // look-back kernel: polls before a wait gives up
 };
@@ -62,6 +63,7 @@ template <typename ST> struct ClLane {
     unsigned c;                // byte offset of the lane's first channel (0 for a lane without channels)
     bool c_ok;
     bool cached;               // ClArgs::cached_stores (the same in every wave of the launch)
+    bool cached_loads;         // ClArgs::cached_loads, likewise
     // Element-aligned lanes (RAGGED): C need not be a multiple of the lane's VEC channels, so the last lane of
     // a time step may own fewer. It loads the window of VEC channels that ends with the time step instead
     // (`c` points there) and moves its components down by `shift` places; its stores go out per channel.
@@ -219,16 +221,32 @@ struct ClSteps {
     // other lane and only its stores are masked, so no per-lane mask is kept per step.
     raw_t ra[S], rx[S];  // what issue() brought; dead once fold() has run
 
-    // Element-aligned 4-byte types load through the caches' normal policy (0; otherwise 2, non-temporal): a lane's 16 bytes
-    // straddle a line border that the next lane, wave or workgroup needs again, and non-temporal lines are the first to
-    // go. fp32 [64, 2048, 1001] 363 / 608 -> 350 / 575 us, a forward and a backward pass over buffers in rotation 969 -> 909
-    // us; [16, 4096, 1999] 977 -> 902 us, [256, 500, 513] 473 -> 444 us. 16-bit types lose as often as they gain (bf16 [64, 2048,
-    // 1001] 185 / 353 against 194 / 314 us, [400, 700, 203] 96 / 157 against 101 / 166 us), and on natural alignment it costs 7 %
-    // of what does not fit the last-level cache (fp32 [64, 2048, 1024] 263 / 439 against 280 / 474 us).
-    static constexpr int LOADS = RAGGED && sizeof(ST) == 4 ? 0 : 2;
+    // Loads through the caches' normal policy instead of non-temporal: element-aligned lanes of 4-byte types straddle line
+    // borders that the next lane, wave or workgroup needs again, and non-temporal lines are the first to go. 16-byte lanes
+    // always (buffers in rotation, us forward / backward: [64, 2048, 1001] 359 / 613 -> 347 / 580; 57 other shapes of 3 to
+    // 490 MB 0.94 to 1.05 x forwards, 0.86 to 1.02 x backwards), 8-byte lanes where the host asks for it. 16-bit types lose as
+    // often as they gain (bf16 [64, 2048, 1001] 185 / 353 against 194 / 314 us, [400, 700, 203] 96 / 157 against 101 / 166
+    // us), and on natural alignment it costs 7 % of what does not fit the last-level cache (fp32 [64, 2048, 1024] 263 / 439
+    // against 280 / 474 us).
+    static constexpr bool CACHED_LOADS = RAGGED && sizeof(ST) == 4 && sizeof(raw_t) == 16;
+    static constexpr bool CHOSEN_LOADS = RAGGED && sizeof(ST) == 4 && sizeof(raw_t) == 8;
 
     // Issues every load of the wave's S steps; nothing waits for them here.
     __device__ __forceinline__ void issue(const ClLane<ST> &ln, int T, int first_step, int limit_)
+    {
+        if constexpr (CHOSEN_LOADS) {
+            if (ln.cached_loads) {
+                // (The compiler would merge the two copies of the loads, and drop what tells them apart.)
+                asm volatile("" ::: "memory");
+                issue_as<0>(ln, T, first_step, limit_);
+                asm volatile("" ::: "memory");
+                return;
+            }
+        }
+        issue_as<CACHED_LOADS ? 0 : 2>(ln, T, first_step, limit_);
+    }
+
+    template <int LOADS> __device__ __forceinline__ void issue_as(const ClLane<ST> &ln, int T, int first_step, int limit_)
     {
         n_tau0 = first_step;
         n_limit = limit_;
@@ -393,6 +411,7 @@ __device__ __forceinline__ ClLane<ST> cl_lane(const ClArgs &p, int64_t batch_ind
     const int64_t c0 = ((int64_t)group * kWave + lane) * VEC;  // first channel of this lane
     ClLane<ST> ln;
     ln.cached = p.cached_stores != 0;
+    ln.cached_loads = p.cached_loads != 0;
     ln.c_ok = c0 < p.C;
     ln.shift = (RAGGED && ln.c_ok && c0 + VEC > p.C) ? (int)(c0 + VEC - p.C) : 0;  // C >= VEC: the host checks it
     ln.c = ln.c_ok ? (unsigned)((c0 - ln.shift) * sizeof(ST)) : 0u;

@@ -451,6 +451,24 @@ def test_automatic_plans_on_large_shapes(gpu, dtype, shape):
     assert rel_err(as_rows(got_ga.mT), ga, prev_abs(as_rows(hs))) <= bar
 
 
+@pytest.mark.parametrize("batch", [2, 21])
+def test_element_aligned_pairs_within_and_beyond_the_last_level_cache(gpu, batch):
+    """Element-aligned 8-byte fp32 lanes load by another policy once a call moves more than 256 MiB (21 elements: 279 MB
+    forwards, 464 backwards); the last lane's shifted window included. First and last batch elements against the oracle."""
+    shape, plan = (batch, 1100, 1003), hip.Plan(mode=hip.MODE_ROW, vec=2, unroll=8, waves=8)
+    g = torch.Generator(device=gpu).manual_seed(batch)
+    a = torch.rand(shape, generator=g, device=gpu)
+    b, gh = torch.randn(shape, generator=g, device=gpu), torch.randn(shape, generator=g, device=gpu)
+    print(f"case cl element-aligned pairs {shape}", flush=True)
+    h = hip.transposed_linear_scan_forward(a, b, plan=plan)
+    ga, gb = hip.transposed_linear_scan_backward(a, h, gh, plan=plan)
+    for i in (0, batch - 1):
+        ca, cb, cgh, ch, cga, cgb = (as_rows(t[i:i + 1]) for t in (a, b, gh, h, ga, gb))
+        assert rel_err(ch, oracle.fwd(ca, cb)) <= 1e-5
+        want_ga, want_gb = oracle.bwd(ca, ch, cgh)
+        assert rel_err(cgb, want_gb) <= 1e-5 and rel_err(cga, want_ga, prev_abs(ch)) <= 1e-5
+
+
 CHANNEL_EDGES = [1, 2, 3, 5, 8, 24, 31, 32, 33, 40, 63, 64, 65, 66, 77, 96, 100, 127, 128, 129, 130, 192, 200, 250, 256,
                  257, 300, 320, 333, 384, 448, 500, 511, 512, 513, 514, 600, 601, 640, 768, 777, 896, 1000, 1001, 1002,
                  1003, 1004, 1016, 1024, 1100]
