@@ -101,7 +101,7 @@ def test_a_short_workspace_leaves_the_other_kernels(gpu, dtype, shape):
 @pytest.mark.parametrize("dtype,shape", [(torch.float32, (600, 333, 33)), (torch.bfloat16, (2048, 167, 40)),
                                          (torch.float16, (513, 400, 19)), (torch.float64, (520, 70, 130)),
                                          (torch.float32, (512, 512, 12)), (torch.float32, (14, 2000, 24)),
-                                         (torch.bfloat16, (100, 900, 33)), (torch.float64, (1, 30000, 8)),
+                                         (torch.bfloat16, (100, 1100, 33)), (torch.float64, (1, 30000, 8)),
                                          (torch.float16, (150, 1700, 37))])
 def test_automatic_route(gpu, dtype, shape):
     """Calls whose automatic plan is this kernel give its very results, and agree with the other kernels."""
@@ -138,7 +138,7 @@ def test_automatic_route(gpu, dtype, shape):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", list(BAR))
-@pytest.mark.parametrize("C,parts", [(2, 0), (8, 0), (8, 3), (24, 40), (130, 9)])
+@pytest.mark.parametrize("C,parts", [(2, 16), (8, 0), (8, 3), (24, 40), (130, 9)])
 def test_growing_gates_over_a_zero_carry_in_parts(gpu, dtype, C, parts):
     """Gates of 1.5 over 3000 steps of zeros: their product is beyond every type (2 ** 1754), the recurrence stays zero."""
     plan = hip.Plan(mode=hip.MODE_STAGED, unroll=parts) if parts else None
@@ -176,7 +176,7 @@ def test_a_small_carry_through_a_part_that_grows_and_shrinks(gpu, dtype):
 
 
 # In parts in both directions; in one launch beside a look-back workspace in reserve (backwards), and without any.
-FLAG_SHAPES = [(torch.float32, (14, 2000, 24)), (torch.float64, (1, 30000, 8)), (torch.bfloat16, (100, 900, 33)),
+FLAG_SHAPES = [(torch.float32, (14, 2000, 24)), (torch.float64, (1, 30000, 8)), (torch.bfloat16, (100, 1100, 33)),
                (torch.float16, (1, 4000, 5)), (torch.float32, (600, 333, 33)), (torch.bfloat16, (2048, 167, 40))]
 
 
@@ -256,3 +256,17 @@ def test_a_resolved_plan_says_what_runs():
                 back = hip.resolve_plan_cl(batch, T, C, dtype, direction, reserve)
                 assert bytes(back) == bytes(reserve)
     assert staged >= 20
+
+
+@pytest.mark.parametrize("dtype,takes,leaves", [
+    (torch.float32, [(1000, 1023, 17), (851, 467, 27), (435, 988, 5), (14, 13990, 24), (1, 1000000, 2), (6, 607, 51)],
+     [(435, 988, 3), (423, 115, 30), (12, 95, 61), (4, 5315, 2), (2, 982, 5), (512, 4096, 8), (192, 2000, 33)]),
+    (torch.bfloat16, [(2048, 512, 40), (1000, 1023, 17), (39, 11559, 30), (2, 39951, 2), (250, 1000, 39)],
+     [(506, 4528, 2), (338, 2002, 4), (255, 54672, 2), (242, 68888, 8), (11, 188, 53), (8, 723, 23), (1, 7948, 2)]),
+    (torch.float64, [(1000, 1023, 17), (1024, 90, 130), (3, 200000, 24), (4, 222, 62)],
+     [(463, 14524, 3), (343, 8902, 5), (665, 246, 7), (125, 102, 35), (14, 4134, 38)])])
+def test_calls_that_take_it_and_calls_that_do_not(dtype, takes, leaves):
+    """Both sides of the automatic choice, each shape measured against the plan in reserve."""
+    parts = lambda s: [hip.resolve_plan_cl(*s, dtype, d).waves_per_row for d in (hip.FORWARD, hip.BACKWARD)]  # noqa: E731
+    assert all(p > 0 for s in takes for p in parts(s)), [s for s in takes if min(parts(s)) == 0]
+    assert all(p == 0 for s in leaves for p in parts(s)), [s for s in leaves if max(parts(s)) > 0]
