@@ -704,7 +704,7 @@ bool staged_fits(int64_t batch, int64_t T, int64_t C, const void *const ptrs[5],
 
 bool resolve_staged(int64_t batch, int64_t T, int64_t C, int esize, int64_t parts, scanscam::StagedArgs *out)
 {
-    if (C > scanscam::kStagedThreads || batch >= (int64_t(1) << 31)) return false;
+    if (C > scanscam::kStagedThreads || batch >= (int64_t(1) << 31)) return false;  // (the product below stays in range)
     // Steps per tile: what its vectors hold and what the threads' spans cover; then tiles of equal size, in spans of at
     // least half the steps a thread can take (every span costs every thread a read and an FMA for its carry).
     const int most_seg = scanscam::staged_steps(esize);
@@ -726,7 +726,7 @@ bool resolve_staged(int64_t batch, int64_t T, int64_t C, int esize, int64_t part
     out->tiles = (int32_t)((all + parts - 1) / parts);
     out->parts = (int32_t)((all + out->tiles - 1) / out->tiles);
     out->ws = nullptr;
-    return batch * out->parts < (int64_t(1) << 31);
+    return batch * out->parts <= ((int64_t(1) << 32) - 1) / scanscam::kStagedThreads;  // threads of one launch
 }
 
 size_t staged_bytes(int64_t batch, int64_t C, int esize, const scanscam::StagedArgs &st)
@@ -852,7 +852,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     };
     scanscam::StagedArgs staged;
     if (plan && plan->mode == kModeStaged) {
-        if (plan->vec || plan->waves || plan->unroll < 0 || !staged_fits(batch, T, C, ptrs, sB, sT) ||
+        if (plan->vec || plan->waves || plan->waves_per_row || plan->unroll < 0 || !staged_fits(batch, T, C, ptrs, sB, sT) ||
             !resolve_staged(batch, T, C, esize, staged_parts_of(plan, batch, T, C, esize), &staged))
             return SCANSCAM_EPLAN;
         const size_t need = staged_bytes(batch, C, esize, staged);

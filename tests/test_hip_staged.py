@@ -270,3 +270,18 @@ def test_calls_that_take_it_and_calls_that_do_not(dtype, takes, leaves):
     parts = lambda s: [hip.resolve_plan_cl(*s, dtype, d).waves_per_row for d in (hip.FORWARD, hip.BACKWARD)]  # noqa: E731
     assert all(p > 0 for s in takes for p in parts(s)), [s for s in takes if min(parts(s)) == 0]
     assert all(p == 0 for s in leaves for p in parts(s)), [s for s in leaves if max(parts(s)) > 0]
+
+
+def test_forced_plans_that_it_refuses():
+    """Refused before anything is launched, so made-up pointers will do: fields it has no use for, more threads than one
+    launch can have, more channels than a workgroup has threads, bases off the 16-byte border."""
+    L = hip.lib()
+
+    def call(plan, batch=4, T=100, C=8, base=4096):
+        return L.scanscam_scan_fwd_cl(base, base, base, batch, T, C, 0, None, 0, None, ctypes.byref(plan))
+
+    refused = [call(hip.Plan(mode=hip.MODE_STAGED, vec=1)), call(hip.Plan(mode=hip.MODE_STAGED, waves=4)),
+               call(hip.Plan(mode=hip.MODE_STAGED, waves_per_row=2)), call(hip.Plan(mode=hip.MODE_STAGED, unroll=-1)),
+               call(STAGED, C=257), call(STAGED, base=4100), call(STAGED, batch=1 << 24, T=1, C=1)]
+    assert refused == [4] * len(refused)
+    assert call(hip.Plan(mode=hip.MODE_STAGED, unroll=4), T=10000) == 5  # in parts: a workspace
