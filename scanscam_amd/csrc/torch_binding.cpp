@@ -15,6 +15,7 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <array>
@@ -203,8 +204,8 @@ PyObject *run(PyObject *const *args, Py_ssize_t nargs, int inputs, int outputs)
 {
     HANDLE_TH_ERRORS
     if (nargs != inputs || !fwd_rows) Py_RETURN_NONE;
-    // A Python-level function mode sees the calls of the Python path; leave them to it.
-    if (at::impl::PythonTorchFunctionTLS::stack_len() > 0) Py_RETURN_NONE;
+    // A Python-level function or dispatch mode sees the calls of the Python path; leave them to it.
+    if (at::impl::PythonTorchFunctionTLS::stack_len() > 0 || c10::impl::TorchDispatchModeTLS::any_modes_set()) Py_RETURN_NONE;
     Call c;
     c.inputs = inputs;
     c.outputs = outputs;

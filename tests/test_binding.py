@@ -43,6 +43,8 @@ def forms(dev, dtype):
     yield "empty", new(0, 6, 50), new(0, 6, 50), new(0, 6, 50)
     yield "workspace", new(2, 70000), new(2, 70000), new(2, 70000)
     yield "channels-last workspace", new(1, 4000, 64).mT, new(1, 4000, 64).mT, new(1, 4000, 64).mT
+    yield "channels-last staged in parts", new(14, 2000, 24).mT, new(14, 2000, 24).mT, new(14, 2000, 24).mT
+    yield "channels-last staged", new(600, 333, 33).mT, new(600, 333, 33).mT, new(600, 333, 33).mT
     if dtype != torch.float64:
         yield "off the vector border", rows().flatten()[1:1 + 4 * 6 * 49].view(4, 6, 49), new(4, 6, 49), new(4, 6, 49)
 
@@ -87,13 +89,63 @@ def test_left_to_the_python_path(gpu, monkeypatch):
     assert hip._native.forward(a) is None
     with pytest.raises(RuntimeError):
         torch.func.vmap(hip.scan_forward)(a[None], b[None])
-    # Tensors a hook hands back, and checking of waits, which is the Python path's.
+    # With checking of waits on, the native path is not entered at all.
+    class Untouched:
+        def forward(self, *args):
+            raise AssertionError("the native path was entered")
+
+        backward = forward
+
+    want = hip.scan_forward(a, b)
+    with monkeypatch.context() as m:
+        m.setattr(hip, "_native", Untouched())
+        with pytest.raises(AssertionError, match="native path"):
+            hip.scan_forward(a, b)
+        hip.check_waits(True)
+        try:
+            assert torch.equal(hip.scan_forward(a, b), want)
+            grads = hip.scan_backward(a, want, b)
+        finally:
+            hip.check_waits(False)
+    for x, y in zip(grads, hip.scan_backward(a, want, b)):
+        assert torch.equal(x, y)
+    # Tensors a hook hands back.
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(gpu)):
         x, y = a.clone().requires_grad_(), b.clone().requires_grad_()
         h = scan(x, y)
     h.sum().backward()
     want = hip.scan_backward(a, h.detach(), torch.ones_like(a))
     assert torch.equal(x.grad, want[0]) and torch.equal(y.grad, want[1])
+
+
+@pytest.mark.gpu
+def test_modes_are_left_to_the_python_path(gpu, monkeypatch):
+    """Under a function or a dispatch mode the calls go where the mode sees what the Python path does."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", str(func)))
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    a, b = torch.rand(4, 50, device=gpu), torch.rand(4, 50, device=gpu)
+    want = hip.scan_forward(a, b)
+    for mode in (Functions, Dispatch):
+        seen = []
+        with mode():
+            assert hip._native.forward(a, b) is None and hip._native.backward(a, b, b) is None
+            del seen[:]
+            got, calls = hip.scan_forward(a, b), list(seen)
+            del seen[:]
+            python_path(monkeypatch, hip.scan_forward, a, b)
+            assert calls == seen and len(calls) > 0
+        assert torch.equal(got, want)
 
 
 @pytest.mark.gpu
