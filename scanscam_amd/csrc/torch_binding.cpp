@@ -263,4 +263,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, methods, n
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__binding() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__binding()
+{
+    PyObject *m = PyModule_Create(&module);
+    // The PyTorch it was compiled against, for hip.py to compare: its C++ API is not stable between versions.
+    if (m && PyModule_AddStringConstant(m, "torch_version", SCANSCAM_TORCH_VERSION) != 0) Py_CLEAR(m);
+    return m;
+}

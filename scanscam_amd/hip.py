@@ -17,6 +17,7 @@ raise.
 import ctypes
 import functools
 import os
+import warnings
 from typing import Optional, Tuple
 
 import torch
@@ -132,10 +133,16 @@ has_hip_ops = _lib is not None
 
 def _bind_native(lib: ctypes.CDLL):
     """The op's host path in native code (csrc/torch_binding.cpp) on this library's entry points, or ``None`` if it is
-    not built: the same calls then go through the Python functions below, three times as slowly on the host."""
+    not built (``make -C scanscam_amd/csrc binding``) or was built against another PyTorch: the same calls then go through
+    the Python functions below, three times as slowly on the host."""
     try:
         from . import _binding
     except ImportError:
+        return None
+    built = getattr(_binding, "torch_version", None)
+    if built != str(torch.__version__):
+        warnings.warn(f"{_binding.__file__} was built against PyTorch {built}, not {torch.__version__}: not used; "
+                      "rebuild it with `make -C scanscam_amd/csrc binding`", RuntimeWarning, stacklevel=2)
         return None
     _binding.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (
         lib.scanscam_scan_fwd_strided, lib.scanscam_scan_bwd_strided, lib.scanscam_scan_fwd_cl_strided,

@@ -1,5 +1,6 @@
 import os
 import sys
+import sysconfig
 
 import pytest
 
@@ -11,6 +12,7 @@ if ROOT not in sys.path:
 BUILT = [
     os.path.join(ROOT, "scanscam_amd", "libscanscam_hip.so"),
     os.path.join(ROOT, "scanscam_amd", "libscanscam_cpu.so"),
+    os.path.join(ROOT, "scanscam_amd", "_binding" + sysconfig.get_config_var("EXT_SUFFIX")),
     os.path.join(ROOT, "oracle", "libscan_oracle.so"),
     os.path.join(ROOT, "tests", "c_abi", "abi_check"),
     os.path.join(ROOT, "tests", "c_abi", "cpu_abi_check"),

@@ -2,6 +2,8 @@
 The native host path of the op (csrc/torch_binding.cpp) against the Python path it stands in for: the same results in the
 same layout for every form it takes, and the same outcome for every form it leaves alone.
 """
+import os
+import subprocess
 import threading
 
 import pytest
@@ -175,7 +177,23 @@ def test_streams_and_threads(gpu):
 
 def test_declines_what_is_not_on_a_gpu():
     if hip._native is None:
-        pytest.skip("_binding.so is not built")
+        pytest.skip("the binding is not built")
     a = torch.rand(3, 4)
     assert hip._native.forward(a, a) is None and hip._native.backward(a, a, a) is None
     assert hip._native.forward(1, 2) is None
+
+
+def test_a_binding_of_another_pytorch_is_not_used(monkeypatch):
+    assert hip._bind_native(hip.lib()) is not None
+    with monkeypatch.context() as m:
+        m.setattr(torch, "__version__", "0.0")
+        with pytest.warns(RuntimeWarning, match="built against PyTorch"):
+            assert hip._bind_native(hip.lib()) is None
+
+
+def test_the_c_libraries_build_without_python():
+    """`make` alone names neither PyTorch nor a Python, only the compilers."""
+    csrc = os.path.join(os.path.dirname(os.path.abspath(hip.__file__)), "csrc")
+    done = subprocess.run(["make", "-C", csrc, "-n", "-B", "PYTHON=/nonexistent/python"], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stderr
+    assert "libscanscam_hip.so" in done.stdout and "libscanscam_cpu.so" in done.stdout and "torch" not in done.stdout
