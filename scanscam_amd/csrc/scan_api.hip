@@ -731,7 +731,9 @@ bool resolve_staged(int64_t batch, int64_t T, int64_t C, int esize, int64_t part
 
 size_t staged_bytes(int64_t batch, int64_t C, int esize, const scanscam::StagedArgs &st)
 {
-    return st.parts > 1 ? scanscam::kStagedHeader * sizeof(uint64_t) + (size_t)(batch * st.parts * C) * (esize == 8 ? sizeof(scanscam::PartPair<double>) : sizeof(scanscam::PartPair<float>)) : 0;
+    if (st.parts <= 1) return 0;
+    const size_t pair = esize == 8 ? sizeof(scanscam::PartPair<double>) : sizeof(scanscam::PartPair<float>);
+    return scanscam::kStagedHeader * sizeof(uint64_t) + (size_t)(batch * st.parts * C) * pair;
 }
 
 // Into how many parts an automatic plan of that kernel cuts a batch element's time (1: one workgroup each, one launch);
