@@ -738,65 +738,73 @@ size_t staged_bytes(int64_t batch, int64_t C, int esize, const scanscam::StagedA
 
 // Into how many parts an automatic plan of that kernel cuts a batch element's time (1: one workgroup each, one launch);
 // 0: the plan is one of scan_cl_plan.hpp. Measured against those (forward / backward, us of GPU time, buffers in rotation;
-// where the line lies is from some 1500 random shapes).
+// random shapes with both sides: profiles/staged_route_random_shapes.txt).
 // Whole batch elements, for few channels in lanes they do not fill: fp32 [1000, 1023, 17] 73.5 / 138 -> 41.0 / 74.5,
 // [851, 467, 27] 41.2 / 69.2 -> 28.6 / 48.6, bf16 [1000, 1023, 17] 56.3 / 102 -> 22.8 / 41.8, [2048, 512, 40] 65.2 / 105 ->
 // 46.2 / 80.0, fp64 [1000, 1023, 17] 115 / 209 -> 86.1 / 156. It ends where
 //   - time steps are whole 128-byte lines (the walk streams them: fp32 [256, 1024, 128] 74.7 / 127 against 83.3 / 124) or
 //     fill the lanes of the packed kernel: fp32 [512, 4096, 8] 39.5 / 68.9 against 45.8 / 63.0, bf16 [506, 4528, 2] 14.4 /
-//     17.9 against 18.2 / 25.3, [338, 2002, 4] 10.3 / 11.5 against 13.6 / 19.7, fp64 [463, 14524, 3] 124 / 223 against 223 /
-//     255 (eight 16-bit channels stay: a step 0.78 to 0.92 x, but 0.79 to 1.14 x below 25 MB per tensor);
+//     17.9 against 18.2 / 25.3, [338, 2002, 4] 10.3 / 11.5 against 13.6 / 19.7 (but [264, 119208, 4] 411 / 469 -> 273 / 376),
+//     fp64 [463, 14524, 3] 124 / 223 against 223 / 255, and eight 16-bit channels below 12 M elements (a step 0.81 to 1.23 x
+//     there, 0.78 to 0.92 x above);
 //   - there are more channels, which fill the walk's lanes well (bf16 [1076, 490, 91] 79.1 / 138 against 85.8 / 147), but for
 //     fp32 steps off the 16-byte border and fp64 (fp32 [1076, 490, 91] 131 / 217 -> 114 / 202, fp64 [1024, 90, 130] 72.4 /
 //     129 -> 61.3 / 102);
 //   - batch elements are too few workgroups (fp32, C = 33: 320 of them 44.8 / 64.5 -> 40.3 / 65.5, 192 of them 46.2 /
 //     66.0 against 57.5 / 78.1; C = 130: 512 level, 320 37.4 / 60.7 against 51.9 / 87.8), more of them for the fewest
 //     channels, whose tiles have the most spans (fp32 [435, 988, 3] 7.4 / 10.6 against 9.7 / 11.8, fp64 [343, 8902, 5] 131 /
-//     211 against 171 / 205), or less than a tile each, below 512 of them two (fp32 [3000, 16, 24] 5.5 / 7.8 against 7.9 /
-//     12.3, bf16 [358, 246, 16] 6.2 / 7.5 against 7.2 / 9.6; fp16 [5299, 101, 49], 10 KB each, 44.7 / 86.7 -> 40.0 / 61.4).
+//     211 against 171 / 205), or less than a tile each (fp32 [3000, 16, 24] 5.5 / 7.8 against 7.9 / 12.3; fp16 [5299, 101,
+//     49], 10 KB each, 44.7 / 86.7 -> 40.0 / 61.4), below 512 of them also few time steps (bf16 [358, 246, 16] 6.2 / 7.5 against
+//     7.2 / 9.6, fp32 [414, 345, 10] 10.3 / 13.0 -> 7.0 / 9.1).
 // Parts, two launches that read gate and value twice but wait for nothing, for the fewer batch elements: fp32 [14, 13990,
 // 24] 32.0 / 44.8 -> 21.5 / 29.9, [1, 250000, 8] 92 / 98 -> 20 / 26, bf16 [39, 11559, 30] 57 / 81 -> 34 / 45, fp64 [3, 200000, 24]
 // 211 / 270 -> 107 / 158. 1280 workgroups, at most 256 parts (fp32 [1, 600000, 24] with 64 / 128 / 256 parts 309 / 159 / 86 us
 // forwards; each workgroup folds the pairs before it). It ends where
-//   - the one-pass tiles' chain is short, which depends on the steps and not on the batch: bf16 [11, 188, 53] 7.6 / 8.7
-//     against 9.1 / 11.3, [8, 723, 23] 8.4 / 10.5 against 9.5 / 11.6, [15, 991, 47] 0.96 x, [12, 1989, 8] 0.94 x; fp32 [12, 95,
-//     61] 7.1 / 7.7 against 7.8 / 8.9, [22, 360, 19] 0.99 x, [6, 607, 51] 9.1 / 10.5 -> 8.1 / 9.2; fp64 [125, 102, 35] 1.07 x, [4,
-//     216, 12] 0.78 x; or short for the spans of a tile of very few channels (fp32 [4, 5315, 2] 11.1 / 12.8 against 14.6 /
-//     16.7, bf16 [1, 7948, 2] 11.4 / 14.8 against 13.2 / 16.2, [2, 39951, 2] 24.4 / 28.0 -> 14.2 / 17.2);
+//   - the one-pass tiles' chain is short: bf16 [11, 188, 53] 7.6 / 8.7 against 9.1 / 11.3, [8, 723, 23] 8.4 / 10.5 against 9.5 /
+//     11.6, [15, 991, 47] 0.96 x, of 32 batch elements on [46, 255, 34] 8.8 / 9.4 against 9.8 / 11.9, [52, 799, 14] 10.9 / 14.6 ->
+//     9.7 / 11.2; fp32 [12, 95, 61] 7.1 / 7.7 against 7.8 / 8.9, [22, 360, 19] 0.99 x, [6, 607, 51] 9.1 / 10.5 -> 8.1 / 9.2; fp64 [11, 49,
+//     44] 0.97 x, [34, 74, 32] 9.3 / 9.3 -> 7.4 / 8.2; or short for the spans of a tile of very few channels, below 16 batch elements,
+//     which the other kernels cut into tiles as well (fp32 [4, 5315, 2] 11.1 / 12.8 against 14.6 / 16.7, bf16 [1, 7948, 2] 11.4 /
+//     14.8 against 13.2 / 16.2, [3, 26492, 2] 20.6 / 26.6 -> 14.0 / 16.3; [16, 19488, 2] 39.2 / 56.3 -> 14.8 / 18.7);
 //   - more channels fill the lanes of the one-pass tiles, the sooner the more batch elements there are: fp32 [4, 100000, 40]
-//     71 / 97 -> 65 / 100, [16, 25000, 40] 61 / 84 against 63 / 98, fp64 [14, 4134, 38] 24.4 / 33.9 against 28.6 / 36.8; bf16 [100,
-//     3137, 51] level / 1.17 x, [100, 2500, 64] 31 / 47 against 37 / 52. Small calls up to 63 channels (fp32 [1, 3124, 61] 11.6 / 13.0
-//     -> 10.0 / 11.1, fp64 [4, 222, 62] 9.8 / 11.3 -> 7.7 / 8.5). Above 64 a tile has no four spans (fp32 [1, 4032, 65] 12.0 / 13.7
-//     against 14.0 / 15.5, fp64 [4, 2016, 65] 15.3 / 20.9 against 24.9 / 26.2); 64 itself would gain (fp32 [1, 4096, 64] 13.5 /
-//     15.6 against 10.8 / 12.0) and has only kept the plan, and the bits, that it had.
-//   - a walk of 128 batch elements or more keeps the memory busy: up to 320 only 16-bit calls of 8 M elements, not of 1, 2,
-//     4 or 8 channels (bf16 [255, 54672, 2] 59 / 98 against 93 / 130, [242, 68888, 8] 244 / 325 against 255 / 373).
+//     71 / 97 -> 65 / 100, [16, 25000, 40] 61 / 84 against 63 / 98, fp64 [14, 4134, 38] 24.4 / 33.9 against 28.6 / 36.8 ([13, 3223,
+//     36] 0.84 x); bf16 [40, 32409, 51] 0.95 / 0.79 x, [100, 2500, 64] 31 / 47 against 37 / 52. Small calls up to 63 channels (fp32 [1,
+//     3124, 61] 11.6 / 13.0 -> 10.0 / 11.1, fp64 [4, 222, 62] 9.8 / 11.3 -> 7.7 / 8.5). Above 64 a tile has no four spans (fp32 [1, 4032,
+//     65] 12.0 / 13.7 against 14.0 / 15.5, fp64 [4, 2016, 65] 15.3 / 20.9 against 24.9 / 26.2); 64 itself would gain (fp32 [1, 4096,
+//     64] 13.5 / 15.6 against 10.8 / 12.0) and has only kept the plan, and the bits, that it had.
+//   - a walk of 128 batch elements or more keeps the memory busy: up to 320 only 16-bit calls of 8 M elements that the packed
+//     kernel does not serve (bf16 [255, 54672, 2] 59 / 98 against 93 / 130, [242, 68888, 8] 244 / 325 against 255 / 373).
 int staged_parts(int64_t batch, int64_t T, int64_t C, int esize)
 {
     if (C > scanscam::kStagedThreads) return 0;
     const int64_t step = C * esize, elements = batch * T * C;
-    // Steps that fill the packed kernel's lanes: 16-bit pairs and quads, fp32 and fp64 whose steps divide 64 bytes, and
-    // three fp64 channels (three of four lanes).
-    const bool packed = esize == 2 ? C <= 4 && 4 % C == 0 : (step <= 64 && 64 % step == 0) || (esize == 8 && C == 3);
-    int64_t most;  // channels up to which time in parts is ahead
+    // Steps that fill the packed kernel's lanes: 16-bit pairs, quads of few time steps, eights in small calls; fp32 and fp64
+    // whose steps divide 64 bytes, and three fp64 channels (three of four lanes).
+    const bool packed = esize == 2 ? C <= 2 || (C == 4 && T < 8192) || (C == 8 && elements < 12 << 20)
+                                   : (step <= 64 && 64 % step == 0) || (esize == 8 && C == 3);
+    int64_t most = 0;  // channels up to which time in parts is ahead
     if (batch < 128) {
-        const int64_t steps = esize == 2 ? 1024 : (esize == 4 ? 448 : 128);
-        const int64_t bytes = (C <= 2 ? 256 / C : (C <= 4 ? 64 : (C < 8 ? 24 : 16))) * 1024;
-        if (T < steps || T * step < bytes) most = 0;
-        else if (elements <= (int64_t(1) << 19)) most = 63;
-        else if (esize == 2) most = 52;
-        else most = batch <= 8 ? 40 : 28;
-    } else {
-        most = batch < 320 && esize == 2 && 8 % C != 0 && elements >= (int64_t(1) << 23) ? 40 : 0;
+        const int64_t steps = esize == 2 ? (batch < 32 ? 1024 : 512) : (esize == 4 ? 448 : 64);
+        int64_t kib = 16;  // of a batch element
+        if (batch < 32 && C < 8) kib = 24;
+        if (batch < 16 && C < 5 && (C < 4 || esize == 2) && esize != 8) kib = C == 2 && esize == 4 ? 128 : 64;
+        if (batch < 16 && C == 1) kib = 256;
+        if (T >= steps && T * step >= kib * 1024) {
+            if (elements <= (int64_t(1) << 19)) most = 63;
+            else if (esize == 2) most = 52;
+            else most = batch <= 8 ? 40 : (esize == 8 && batch <= 16 ? 36 : 28);
+        }
+    } else if (batch < 320 && esize == 2 && !packed && elements >= (int64_t(1) << 23) && (C != 8 || elements < 64 << 20)) {
+        most = 40;
     }
     if (C <= most) {
         const int64_t parts = (1280 + batch - 1) / batch;
         return (int)(parts < 256 ? parts : 256);
     }
     if (step % 128 == 0 || packed) return 0;
-    if (!(C <= 80 || esize == 8 || (esize == 4 && step % 16 != 0))) return 0;
-    if (batch < 512) return batch >= 320 && C <= 80 && T * step >= 16 * 1024 && (esize == 2 || C >= (esize == 4 ? 4 : 8)) ? 1 : 0;
-    return T * step >= 7680 && (esize != 8 || C >= 8 || batch >= 768) ? 1 : 0;
+    if (!(C <= 80 || esize == 8 || (esize == 4 && step % 16 != 0)) || T * step < 7680) return 0;
+    if (batch < 512) return batch >= 320 && C <= 80 && T >= 256 && (esize == 2 || C >= (esize == 4 ? 4 : 8)) ? 1 : 0;
+    return esize != 8 || C >= 8 || batch >= 768 ? 1 : 0;
 }
 
 // The parts in which a call with this plan takes the staged kernel, 0 for none: what a resolved plan says
@@ -913,9 +921,10 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     args.cached_stores = (!lines && lane_bytes <= 8 && esize <= 4 &&
                           (esize == 2 ? (lane_bytes > 2 || !rev) : (!rev || l.kind == 2))) ? 1 : 0;
     // Loads through the caches' normal policy in element-aligned 8-byte lanes of fp32, once the call does not fit the
-    // last-level cache. Against non-temporal ones, buffers in rotation: 64 calls beyond it 0.87 to 1.02 x, 0.94 x in the mean
-    // ([16, 4096, 1999] forwards 340 -> 298 us, [256, 500, 513] backwards 296 -> 267 us), 97 calls within it 0.91 to 1.21 x,
-    // 1.03 x in the mean ([39, 32, 1823] 7.6 / 11.8 -> 9.2 / 13.8 us, [238, 32, 733] 14.2 / 24.0 -> 16.1 / 26.3 us).
+    // last-level cache. Against non-temporal ones, buffers in rotation (profiles/element_aligned_loads_random_shapes.txt): 64
+    // calls beyond it 0.87 to 1.02 x, 0.94 x in the mean ([16, 4096, 1999] forwards 340 -> 298 us, [256, 500, 513] backwards
+    // 296 -> 267 us), 97 calls within it 0.91 to 1.21 x, 1.03 x in the mean ([39, 32, 1823] 7.6 / 11.8 -> 9.2 / 13.8 us, [238,
+    // 32, 733] 14.2 / 24.0 -> 16.1 / 26.3 us).
     args.cached_loads = (rev ? 5 : 3) * batch * T * C * esize > kLastLevelCache ? 1 : 0;
     args.ws = nullptr;
     args.spin_limit = (plan && plan->spin_limit > 0) ? plan->spin_limit : scanscam::kSpinLimit;

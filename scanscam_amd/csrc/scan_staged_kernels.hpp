@@ -20,10 +20,10 @@
 // 15, of the same 16-byte block, never used. The host sends only tensors whose base is a 16-byte border, so no
 // block begins before the tensor and corresponding runs of all tensors have one phase against the border.
 //
-// In a kernel trace 53 to 65 % of 8 TB/s (bf16 [2048, 512, 40] 48.4 / 83.6 us forwards / backwards, fp32 [1000, 1023, 17] 43.6 /
-// 82.7 us), at 1.01 to 1.03 times the bytes it has to move. Bound by a tile's chain of four barriers and two LDS passes
+// In a kernel trace 53 to 65 % of 8 TB/s (bf16 [2048, 512, 40] 48.5 / 83.8 us forwards / backwards, fp32 [1000, 1023, 17] 44.0 /
+// 82.2 us), at 1.01 to 1.03 times the bytes it has to move. Bound by a tile's chain of four barriers and two LDS passes
 // against the workgroups in flight: the waves wait half of their cycles and another quarter to third for an instruction to
-// issue; bank conflicts are 26 to 29 % of the LDS cycles. Registers allow 6 workgroups per CU forwards and 4 backwards in
+// issue; bank conflicts are 23 to 29 % of the LDS cycles. Registers allow 6 workgroups per CU forwards and 4 backwards in
 // fp32, 4 and 4 in 16-bit storage (3 backwards in parts), 8 and 5 in fp64 (7 and 4). Two vectors per thread (8 KiB tiles),
 // because with four the registers halve the workgroups per CU (bf16 [851, 467, 27] 16.6 / 27.7 us against 24.5 / 37.9), and
 // one 16-bit channel per thread, not two, because that halves the spans each thread folds its carry over ([1024, 2048, 16]
