@@ -76,7 +76,9 @@ enum {
  *   waves          waves per workgroup, 1..16 (at most 8 when unroll == 8)
  *   waves_per_row  row layout, ROW only: a divisor of `waves` (waves / waves_per_row rows share a workgroup);
  *                  channels-last: parts of time in which SCANSCAM_MODE_STAGED takes the call where it can,
- *                  the other fields then being the plan where it cannot
+ *                  the other fields then being the plan where it cannot; below zero: the negative of
+ *                  64 * steps + 2 * waves + (1: tiles of time, 0: a walk), the launch in which lanes move channels
+ *                  between each other (odd C) takes the call where it can
  *   spin_limit     kernels that wait for another workgroup's carry poll at most this many times
  *                  (0 = 2^20, about a second); a wait that expires sets word 1 of the workspace to 1
  *                  and poisons the affected outputs with NaN instead of spinning for ever
@@ -269,7 +271,8 @@ int scanscam_resolve_plan(int64_t rows, int64_t T, int dtype, int direction, con
  * tiles of time steps chain through the workspace; vec channels per lane, unroll time steps per
  * wave and tile, waves per workgroup. waves_per_row > 0: the call takes SCANSCAM_MODE_STAGED by itself, in that
  * many parts, and the other fields are the plan in reserve for tensors the staged kernel cannot run (zero
- * waves_per_row to force that one). Handed back, the plan runs what the automatic call runs, bit for bit. A
+ * waves_per_row to force that one). waves_per_row < 0: the call moves channels between neighbouring lanes (odd C of
+ * large dense tensors; struct scanscam_plan), with the same meaning of the other fields. Handed back, the plan runs what the automatic call runs, bit for bit. A
  * SCANSCAM_MODE_STAGED plan has nothing to resolve and is refused. No counterpart in the reference, whose kernel has
  * one launch shape (scanscam/cuda.py:69-95 passes channels_per_block only).
  */
@@ -279,8 +282,8 @@ int scanscam_resolve_plan_cl(int64_t batch, int64_t T, int64_t C, int dtype, int
 /*
  * The duration in microseconds that the library's cost model estimates for a channels-last call on dense
  * [batch, T, C] tensors with this plan (NULL or zero fields: with what the model itself chooses for them, i.e.
- * the estimate behind scanscam_resolve_plan_cl; of the plan in reserve where that reports waves_per_row > 0, since the
- * model does not know the staged kernel). The plan is the candidate with the smallest such
+ * the estimate behind scanscam_resolve_plan_cl; of the plan in reserve where that reports another waves_per_row than 0,
+ * since the model knows neither the staged kernel nor the moved channels). The plan is the candidate with the smallest such
  * estimate; the model (a formula of a few physical terms and a learned correction on top of it) is fitted to
  * timings on one MI355X (scanscam_amd/plan_fit.py), so the figure is a ranking aid with an error of about 5 %,
  * not a promise. The first call for a (shape, plan) on a thread takes about 0.1 ms on the host (the choice is

@@ -620,6 +620,33 @@ int run(bool rev, const void *a, const void *x, const void *h, void *y0, void *y
     return SCANSCAM_OK;
 }
 
+// Grid, LDS and workspace of a chosen launch; `virtual_steps`: steps before the first one that the tiles cover as well.
+int size_cl(int64_t batch, int64_t T, int dtype, int virtual_steps, scanscam::ClLaunch *l)
+{
+    const int64_t rowgroups = batch * l->groups;
+    const int64_t tile_steps = (int64_t)l->waves * l->steps;
+    const int64_t tiles = (T + virtual_steps + tile_steps - 1) / tile_steps;
+    const int64_t vals = (int64_t)l->vec * kWave * value_words(dtype);  // words of one [vec][64] array of values
+    l->lds_bytes = (size_t)(l->kind == 2 ? 7 : 4) * l->waves * l->vec * kWave * compute_size(dtype);
+    l->ws_bytes = 0;
+    l->segments = 1;
+    if (l->kind == 2) {
+        if (tiles >= (int64_t(1) << 31)) return SCANSCAM_EINVAL;
+        l->segments = (int)tiles;  // the kernel's tiles per row-group
+        const int64_t supers = (tiles + l->waves - 1) / l->waves;
+        const int64_t pairs = (int64_t)l->vec * kWave * tile_words(dtype);  // words of one [vec][64] array of pairs
+        l->ws_bytes = (size_t)(rowgroups * kCounterStride + rowgroups * tiles * pairs + rowgroups * supers * (pairs + vals)) *
+                      sizeof(uint64_t);
+    }
+    if (l->segments <= 1) {  // a forced time split of a single tile: nothing to split after all
+        l->kind = 0;
+        l->ws_bytes = 0;
+    }
+    l->grid = rowgroups * l->segments;
+    if (l->grid >= (int64_t(1) << 31)) return SCANSCAM_EINVAL;
+    return SCANSCAM_OK;
+}
+
 // Channels-last: the launch plan. `align`: the largest of 16, 8, 4 and the element size that every tensor's base
 // and strides are multiples of (bytes). The choice itself is the cost model of scan_cl_plan.hpp: every field the
 // caller's plan leaves at zero is chosen by the smallest estimated duration; this function turns the chosen
@@ -669,33 +696,15 @@ int resolve_cl(const scanscam_plan *user, int64_t batch, int64_t T, int64_t C, i
     l->kind = c.kind;
     l->group = c.group;
     l->ragged = c.ragged;
-    const int64_t rowgroups = batch * scanscam::cl_groups(C, c.vec);
-    const int64_t tile_steps = (int64_t)l->waves * l->steps;
-    const int64_t tiles = (T + tile_steps - 1) / tile_steps;
-    const int64_t vals = (int64_t)l->vec * kWave * value_words(dtype);  // words of one [vec][64] array of values
-    l->lds_bytes = (size_t)(l->kind == 2 ? 7 : 4) * l->waves * l->vec * kWave * compute_size(dtype);
-    l->ws_bytes = 0;
-    l->segments = 1;
-    if (l->kind == 2) {
-        if (tiles >= (int64_t(1) << 31)) return SCANSCAM_EINVAL;
-        l->segments = (int)tiles;  // the kernel's tiles per row-group
-        const int64_t supers = (tiles + l->waves - 1) / l->waves;
-        const int64_t pairs = (int64_t)l->vec * kWave * tile_words(dtype);  // words of one [vec][64] array of pairs
-        l->ws_bytes = (size_t)(rowgroups * kCounterStride + rowgroups * tiles * pairs + rowgroups * supers * (pairs + vals)) *
-                      sizeof(uint64_t);
-    }
-    if (l->segments <= 1) {  // a forced time split of a single tile: nothing to split after all
-        l->kind = 0;
-        l->ws_bytes = 0;
-    }
-    l->grid = rowgroups * l->segments;
-    if (l->grid >= (int64_t(1) << 31)) return SCANSCAM_EINVAL;
-    return SCANSCAM_OK;
+    l->shift = 0;
+    l->groups = (int)scanscam::cl_groups(C, c.vec);
+    l->vectors = kWave;
+    return size_cl(batch, T, dtype, 0, l);
 }
 
 // Channels-last tiles staged through LDS (scan_staged_kernels.hpp): whether that kernel can run the call, and its tile.
 // Dense tensors on 16-byte borders, all channels of a batch element in one workgroup.
-bool staged_fits(int64_t batch, int64_t T, int64_t C, const void *const ptrs[5], const int64_t sB[5], const int64_t sT[5])
+bool cl_dense(int64_t batch, int64_t T, int64_t C, const void *const ptrs[5], const int64_t sB[5], const int64_t sT[5])
 {
     for (int k = 0; k < 5; k++)
         if (!aligned_to(ptrs[k], 16) || (T > 1 && sT[k] != C) || (batch > 1 && sB[k] != T * C)) return false;
@@ -817,6 +826,76 @@ int staged_parts_of(const scanscam_plan *plan, int64_t batch, int64_t T, int64_t
     return free_plan ? staged_parts(batch, T, C, esize) : 0;
 }
 
+// Channels moved between neighbouring lanes (scan_cl_shift.hpp), for odd channel counts: which of its launches a call takes,
+// as one number -- 64 * time steps per wave + 2 * waves + (1: tiles of time over workgroups, 0: a walk) --, 0 for none.
+int shift_code(int steps, int waves, bool tiles) { return 64 * steps + 2 * waves + (tiles ? 1 : 0); }
+
+int shift_vec(int esize) { return esize == 8 ? 2 : 4; }
+
+// Fills a launch from that number; false where the kernels cannot run it.
+bool resolve_shift(int64_t batch, int64_t T, int64_t C, int dtype, int code, scanscam::ClLaunch *l)
+{
+    const int esize = elem_size(dtype);
+    l->vec = shift_vec(esize);
+    l->steps = code / 64;
+    l->waves = code / 2 % 32;
+    l->kind = code % 2 == 1 ? 2 : 0;
+    l->group = kWave;
+    l->ragged = false;
+    l->shift = (int)(C % l->vec);
+    // The vector after a group's last one is loaded by a lane of its own; a time step's last group has at least one whole.
+    const int64_t all = (C + l->vec - 1) / l->vec;
+    l->groups = (int)((all + kWave - 2) / (kWave - 1));
+    l->vectors = (int)((all + l->groups - 1) / l->groups);
+    if (l->shift % 2 == 0 || T < 2 || C <= (int64_t)(kWave - 1) * l->vec || all - (int64_t)(l->groups - 1) * l->vectors < 2) return false;
+    if (!scanscam::cl_shift_built(esize, l->vec, l->steps, l->kind) || l->waves < 1 ||
+        l->waves > scanscam::cl_max_waves(l->vec, l->steps, l->kind, compute_size(dtype)))
+        return false;
+    return size_cl(batch, T, dtype, l->vec - 1, l) == SCANSCAM_OK && scanscam::cl_shift_built(esize, l->vec, l->steps, l->kind);  // (one tile: a walk)
+}
+
+// When an automatic call takes them. What it does without them is the cost model's plan: lanes of one channel, or wide ones
+// that load and store at any element. Measured against that plan (forward / backward, x of its time, or us; buffers in
+// rotation), in calls that do not fit the last-level cache -- within it the two are level or up to 1.3 x behind (bf16 [61,
+// 333, 1471] 1.07 / 1.04, fp32 [8, 1198, 831] 1.02 / 1.04) -- of 256 time steps or more:
+//   A walk, for 192 workgroups or more (up to 512 in fp32 and 16 bits): fp32 [64, 2048, 1001] 342 / 569 -> 304 / 509 us, [117,
+//   1055, 363] 0.82 / 0.85, [134, 354, 659] 0.97 / 0.87; bf16 [64, 2048, 1001] 197 / 342 -> 155 / 274 us, [28, 2048, 1777] 0.92 /
+//   0.82, [52, 407, 2265] 0.95 / 0.90; fp64 [39, 491, 1169] 0.87 / 0.89, [10, 669, 3709] 0.96 / 1.01, [6, 609, 3921] 0.98 / 0.83.
+//   With 840 workgroups fp32 [280, 372, 599] 1.06 / 1.13, bf16 [421, 343, 269] 1.03 / 1.13; with groups of fewer than 44 of 64
+//   lanes bf16 [144, 1447, 275] 1.25 / 1.13, fp64 [131, 353, 167] 0.99 / 1.06.
+//   Tiles, for fewer. fp32 up to 96 (batch element, channel group) pairs: [1, 9006, 3361] 0.79 / 0.71, [4, 5636, 1993] 0.91 /
+//   0.93, [28, 2754, 721] 0.93 / 0.98 ([59, 2896, 365], 118 pairs, 1.00 / 1.15; [7, 738, 2803] 290 MB backwards 1.05). 16 bits
+//   backwards, which is bound by its accesses more than by bytes, from 64 MiB on: bf16 [5, 2172, 741] 0.66, [14, 1649, 1119]
+//   0.79, [11, 669, 3295] 0.79, [9, 1598, 2353] 0.91 (from 96 to 143 pairs 0.99 to 1.10; [2, 17252, 285], 4 pairs, 1.14; [31, 1342,
+//   275], 35 lanes, 1.08); forwards they lose (0.92 to 1.4). fp64 has no fewer accesses per byte to gain (1.0 to 1.5).
+int shift_choice(int64_t batch, int64_t T, int64_t C, int esize, bool rev)
+{
+    const int vec = shift_vec(esize);
+    if (C % 2 == 0 || C <= (kWave - 1) * vec || T < 256) return 0;
+    const int64_t bytes = batch * T * C * esize * (rev ? 5 : 3);
+    const int64_t all = (C + vec - 1) / vec, groups = (all + kWave - 2) / (kWave - 1), pairs = batch * groups;
+    const bool filled = all >= 44 * groups;
+    if (pairs >= 192) {
+        if (bytes <= kLastLevelCache || !filled || (pairs > 512 && esize != 8)) return 0;
+        return esize == 2 ? shift_code(rev ? 4 : 8, 8, false) : shift_code(8, 4, false);
+    }
+    if (esize == 2) {
+        if (!rev || bytes <= kLastLevelCache / 4 || pairs < 8 || (pairs >= 96 && pairs < 144)) return 0;
+        return pairs < 40 ? shift_code(16, 8, true) : (filled ? shift_code(16, 4, true) : 0);
+    }
+    if (esize == 4) return filled && pairs <= 96 && bytes > (rev ? kLastLevelCache / 4 * 5 : kLastLevelCache) ? shift_code(8, 8, true) : 0;
+    return 0;
+}
+
+// The same for a call's plan: what a resolved plan says (scanscam_resolve_plan_cl writes the number's negative into
+// waves_per_row), the automatic choice where the plan leaves everything open.
+int shift_code_of(const scanscam_plan *plan, int64_t batch, int64_t T, int64_t C, int esize, bool rev)
+{
+    if (plan && plan->waves_per_row < 0) return plan->waves_per_row > -4096 ? -plan->waves_per_row : 0;
+    const bool free_plan = !plan || (plan->mode == SCANSCAM_MODE_AUTO && !plan->vec && !plan->unroll && !plan->waves && !plan->waves_per_row);
+    return free_plan ? shift_choice(batch, T, C, esize, rev) : 0;
+}
+
 int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void *y1,
            const scanscam_strides *const st[5], int64_t batch, int64_t T, int64_t C, int dtype, void *workspace,
            size_t workspace_bytes, void *stream, const scanscam_plan *plan)
@@ -841,6 +920,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         while (align > esize && !(aligned_to(ptrs[k], (size_t)align) && (sB[k] * esize) % align == 0 && (sT[k] * esize) % align == 0))
             align >>= 1;
     }
+    const bool dense = cl_dense(batch, T, C, ptrs, sB, sT);
     auto run_staged = [&](scanscam::StagedArgs st) {
         st.a = a;
         st.x = x;
@@ -862,7 +942,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     };
     scanscam::StagedArgs staged;
     if (plan && plan->mode == kModeStaged) {
-        if (plan->vec || plan->waves || plan->waves_per_row || plan->unroll < 0 || !staged_fits(batch, T, C, ptrs, sB, sT) ||
+        if (plan->vec || plan->waves || plan->waves_per_row || plan->unroll < 0 || !dense ||
             !resolve_staged(batch, T, C, esize, staged_parts_of(plan, batch, T, C, esize), &staged))
             return SCANSCAM_EPLAN;
         const size_t need = staged_bytes(batch, C, esize, staged);
@@ -877,6 +957,13 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     // offsets from its first one, the lane's channel included.
     for (int k = 0; k < 5; k++)
         if ((uint64_t)sT[k] * (uint64_t)esize * 18u + (uint64_t)C * (uint64_t)esize >= (uint64_t(1) << 32)) return SCANSCAM_EINVAL;
+
+    const int parts = staged_parts_of(plan, batch, T, C, esize);
+    const int code = parts > 0 ? 0 : shift_code_of(plan, batch, T, C, esize, rev);
+    scanscam::ClLaunch shifted;
+    if (code != 0 && dense && resolve_shift(batch, T, C, dtype, code, &shifted) &&
+        (shifted.ws_bytes == 0 || (workspace && workspace_bytes >= shifted.ws_bytes && aligned_to(workspace, 8))))
+        l = shifted;
 
     scanscam::ClArgs args;
     args.a = a;
@@ -893,6 +980,8 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     args.C = (int32_t)C;
     args.segments = l.segments;
     args.group = l.group;
+    args.groups = l.groups;
+    args.vectors = l.vectors;
     // Time steps that are not whole 128-byte lines: neighbouring channel groups on one XCD (see the kernel).
     bool lines = true;
     for (int k = 0; k < 5; k++) lines = lines && (sT[k] * esize) % 128 == 0 && aligned_to(ptrs[k], 128) && (sB[k] * esize) % 128 == 0;
@@ -934,8 +1023,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         if (!workspace || workspace_bytes < l.ws_bytes) return SCANSCAM_EWORKSPACE;
         if (!aligned_to(workspace, 8)) return SCANSCAM_EALIGN;
     }
-    const int parts = staged_parts_of(plan, batch, T, C, esize);
-    if (parts > 0 && staged_fits(batch, T, C, ptrs, sB, sT) && resolve_staged(batch, T, C, esize, parts, &staged)) {
+    if (parts > 0 && dense && resolve_staged(batch, T, C, esize, parts, &staged)) {
         const size_t need = staged_bytes(batch, C, esize, staged);
         if (need == 0 || (workspace && workspace_bytes >= need && aligned_to(workspace, 8))) {
                 return run_staged(staged);
@@ -944,7 +1032,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     if (l.kind != 0) {
         args.ws = static_cast<uint64_t *>(workspace);
         const int64_t words = (int64_t)(l.ws_bytes / sizeof(uint64_t));
-        const int64_t rowgroups = batch * ((C + (int64_t)kWave * l.vec - 1) / ((int64_t)kWave * l.vec));
+        const int64_t rowgroups = batch * l.groups;
         if (clear_workspace(args.ws, words, rowgroups * kCounterStride, s) != hipSuccess) return SCANSCAM_ELAUNCH;
     }
     hipError_t e = hipErrorInvalidValue;
@@ -1056,6 +1144,9 @@ size_t scanscam_workspace_bytes_cl(int64_t batch, int64_t T, int64_t C, int dtyp
     scanscam::StagedArgs st;
     if (parts > 1 && resolve_staged(batch, T, C, esize, parts, &st)) need = staged_bytes(batch, C, esize, st);
     if (plan && plan->mode == kModeStaged) return need;
+    const int code = parts > 0 ? 0 : shift_code_of(plan, batch, T, C, esize, direction == SCANSCAM_BACKWARD);
+    scanscam::ClLaunch shifted;
+    if (code != 0 && resolve_shift(batch, T, C, dtype, code, &shifted)) need = shifted.ws_bytes;
     // The caller's pointers are not known yet: every alignment the tensors may turn out to have.
     for (int align = 16; align >= esize; align >>= 1) {
         scanscam::ClLaunch l;
@@ -1158,12 +1249,14 @@ int scanscam_resolve_plan_cl(int64_t batch, int64_t T, int64_t C, int dtype, int
     const int rc = resolve_cl(plan, batch, T, C, dtype, align, direction == SCANSCAM_BACKWARD, &l);
     if (rc != SCANSCAM_OK) return rc;
     const int parts = staged_parts_of(plan, batch, T, C, esize);  // (`out` may be the plan itself)
+    const int code = parts > 0 ? 0 : shift_code_of(plan, batch, T, C, esize, direction == SCANSCAM_BACKWARD);
     scanscam::StagedArgs st;
     out->mode = l.kind == 2 ? kModeLookback : kModeRow;
     out->vec = l.vec;
     out->unroll = l.steps;
     out->waves = l.waves;
     out->waves_per_row = parts > 0 && resolve_staged(batch, T, C, esize, parts, &st) ? st.parts : 0;
+    if (code != 0 && resolve_shift(batch, T, C, dtype, code, &l)) out->waves_per_row = -code;
     out->spin_limit = (plan && plan->spin_limit > 0) ? plan->spin_limit : scanscam::kSpinLimit;
     return SCANSCAM_OK;
 }

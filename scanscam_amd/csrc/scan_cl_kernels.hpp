@@ -43,6 +43,8 @@ struct ClArgs {
     int32_t C;
     int32_t segments;   // look-back kernel: tiles per (batch element, channel group)
     int32_t group;      // packed kernel: lanes per time step (power of two below 64)
+    int32_t groups;     // channel groups (workgroups side by side) of a time step
+    int32_t vectors;    // scan_cl_shift.hpp: vectors of channels per group
     int32_t xcd_order;  // scan_cl_kernel, scan_cl_lookback_kernel: consecutive (batch element, channel group) pairs share an XCD
     int32_t cached_stores;  // outputs through the caches' normal policy instead of non-temporal (the host decides, see run_cl)
     int32_t cached_loads;    // element-aligned 8-byte lanes of 4-byte types: the same for loads
@@ -68,6 +70,13 @@ template <typename ST> struct ClLane {
     // a time step may own fewer. It loads the window of VEC channels that ends with the time step instead
     // (`c` points there) and moves its components down by `shift` places; its stores go out per channel.
     int shift;
+    // Lanes that move elements between neighbours (scan_cl_shift.hpp): the lane's number, the group's last one with channels
+    // and whether that holds fewer than VEC (a time step's last group), lane offsets of loads, and where the scan's virtual
+    // origin lies.
+    int lane, last;
+    bool tail;
+    unsigned c_few, c_all;  // `c`, and one vector further for the lane after the last: in all groups but a tail, in all
+    int phase0, k0;         // elements the batch element's first step lies after a vector border; virtual steps before it
 
     // base + elems elements + the lane's channel offset. The lane part enters as a zero-extended 32-bit
     // byte count, the form the scalar-base addressing mode takes.
@@ -405,6 +414,43 @@ __device__ __forceinline__ int xcd_contiguous(int r, int n)
     return xcd < rem ? xcd * per + slot : rem * per + (xcd - rem) * (per - 1) + slot;
 }
 
+}  // namespace scanscam
+#include "scan_cl_shift.hpp"  // (on top of ClLane and ClAccess)
+namespace scanscam {
+
+// The lane's view for ClShiftSteps: a group is p.vectors vectors of channels, the last group of a time step what is left.
+template <typename ST, int VEC, bool REV, int M>
+__device__ __forceinline__ ClLane<ST> cl_shift_lane(const ClArgs &p, int64_t batch_index, int group, int lane)
+{
+    constexpr unsigned LB = VEC * sizeof(ST);
+    const int c0 = group * p.vectors * VEC;  // a multiple of VEC: the phase of a time step is the same in all its groups
+    const int left = (p.C - c0 + VEC - 1) / VEC;
+    ClLane<ST> ln;
+    ln.cached = ln.cached_loads = false;
+    ln.c_ok = true;
+    ln.shift = 0;
+    ln.lane = lane;
+    ln.tail = left <= p.vectors;
+    ln.last = (ln.tail ? left : p.vectors) - 1;
+    ln.c = (lane < ln.last ? lane : ln.last) * LB;
+    ln.c_all = (lane < ln.last + 1 ? lane : ln.last + 1) * LB;
+    ln.c_few = ln.tail ? ln.c : ln.c_all;
+    const int64_t first = batch_index * p.sB[0] + c0;  // dense: the same for all tensors
+    ln.phase0 = (int)(first & (VEC - 1));
+    const int at = REV ? (VEC - (ln.phase0 + (p.T - 1) % VEC * M) % VEC) % VEC : ln.phase0;  // k0 * M mod VEC
+    ln.k0 = 0;
+#pragma unroll
+    for (int k = VEC - 1; k >= 0; k--)
+        if (k * M % VEC == at) ln.k0 = k;
+    ln.a = static_cast<const ST *>(p.a) + first;
+    ln.x = static_cast<const ST *>(p.x) + first;
+    ln.h = static_cast<const ST *>(p.h) + first;
+    ln.y0 = static_cast<ST *>(p.y0) + first;
+    ln.y1 = static_cast<ST *>(p.y1) + first;
+    ln.pa = ln.px = ln.ph = ln.py0 = ln.py1 = p.C;
+    return ln;
+}
+
 template <typename ST, int VEC, bool RAGGED = false>
 __device__ __forceinline__ ClLane<ST> cl_lane(const ClArgs &p, int64_t batch_index, int group, int lane)
 {
@@ -428,8 +474,22 @@ __device__ __forceinline__ ClLane<ST> cl_lane(const ClArgs &p, int64_t batch_ind
     return ln;
 }
 
+template <typename ST, int VEC, bool REV, bool RAGGED, int M>
+__device__ __forceinline__ ClLane<ST> cl_lane_of(const ClArgs &p, int64_t batch_index, int group, int lane)
+{
+    if constexpr (M != 0) return cl_shift_lane<ST, VEC, REV, M>(p, batch_index, group, lane);
+    else return cl_lane<ST, VEC, RAGGED>(p, batch_index, group, lane);
+}
+template <typename ST, int VEC, int S, bool REV, int M, typename CT, bool SPLIT, bool RAGGED> struct ClStepsOf {
+    using type = ClShiftSteps<ST, VEC, S, REV, M, CT, SPLIT>;
+};
+template <typename ST, int VEC, int S, bool REV, typename CT, bool SPLIT, bool RAGGED> struct ClStepsOf<ST, VEC, S, REV, 0, CT, SPLIT, RAGGED> {
+    using type = ClSteps<ST, VEC, S, REV, true, CT, SPLIT, RAGGED>;
+};
+
 // Dynamic LDS: two buffers (tiles alternate) of A and B, each [W][VEC][64] values.
-template <typename ST, int VEC, int S, bool REV, int MAXT, bool RAGGED = false>
+// M: channels beyond whole vectors, moved as scan_cl_shift.hpp says (0: not).
+template <typename ST, int VEC, int S, bool REV, int MAXT, bool RAGGED = false, int M = 0>
 __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
 {
     using CT = typename ComputeOf<ST>::type;
@@ -439,17 +499,17 @@ __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // wave-uniform: kept in a scalar register
     const int W = blockDim.x / kWave;
-    const int groups = (p.C + kWave * VEC - 1) / (kWave * VEC);  // channel groups per batch element
+    const int groups = p.groups;
     // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2. When a time step of C
     // channels is not a whole number of 128-byte lines, neighbouring channel groups share a line at
     // every time step; handled by different XCDs that line is fetched twice and written in two parts.
     // xcd_order gives each XCD a contiguous run of (batch element, channel group) pairs instead, so that
     // neighbours meet in one L2.
     const int bid = p.xcd_order ? xcd_contiguous((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
-    const ClLane<ST> ln = cl_lane<ST, VEC, RAGGED>(p, bid / groups, bid % groups, lane);
+    const ClLane<ST> ln = cl_lane_of<ST, VEC, REV, RAGGED, M>(p, bid / groups, bid % groups, lane);
 
     const int tile_steps = W * S;
-    const int ntiles = (p.T + tile_steps - 1) / tile_steps;
+    const int ntiles = (p.T + (M != 0 ? ln.k0 : 0) + tile_steps - 1) / tile_steps;
     const int plane = W * VEC * kWave;  // values per LDS array
     CT carry[VEC];
 #pragma unroll
@@ -463,7 +523,7 @@ __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
     // [8, 4096, 2048] forward 93 -> 90 us. fp32 pays 30 to 120 registers for it and is level on average (+28 % to -10 %),
     // 16-byte lanes of 16-bit storage spill.
     constexpr bool AHEAD = sizeof(ST) == 2 && VEC <= 4 && VEC * S <= 32;
-    ClSteps<ST, VEC, S, REV, true, CT, false, RAGGED> steps;
+    typename ClStepsOf<ST, VEC, S, REV, M, CT, false, RAGGED>::type steps;
     if (AHEAD) steps.issue(ln, p.T, wave * S, p.T);
     for (int it = 0; it < ntiles; it++) {
         CT *lds_A = lds + (it & 1) * 2 * plane, *lds_B = lds_A + plane;
@@ -736,7 +796,7 @@ __device__ __forceinline__ void cl_publish_pair(uint64_t *dst, int lane, const C
     for (int k = 0; k < VEC; k++) D::store_pair(dst + (k * kWave + lane) * D::PAIR, a[k], b[k]);
 }
 
-template <typename ST, int VEC, int S, bool REV, int MAXT>
+template <typename ST, int VEC, int S, bool REV, int MAXT, int M = 0>
 __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
 {
     using CT = typename ComputeOf<ST>::type;
@@ -749,7 +809,7 @@ __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // wave-uniform: kept in a scalar register
     const int W = blockDim.x / kWave;
-    const int groups = (p.C + kWave * VEC - 1) / (kWave * VEC);
+    const int groups = p.groups;
     const int64_t rowgroups = p.batch * groups;
     const int tpr = p.segments;              // tiles per row-group
     const int spr = (tpr + W - 1) / W;       // super-tiles per row-group
@@ -786,13 +846,13 @@ __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     const int tile = (int)__builtin_amdgcn_readfirstlane((int)lds_ticket);
-    const ClLane<ST> ln = cl_lane<ST, VEC>(p, rg / groups, (int)(rg % groups), lane);
+    const ClLane<ST> ln = cl_lane_of<ST, VEC, REV, false, M>(p, rg / groups, (int)(rg % groups), lane);
     uint64_t *tiles = p.ws + rowgroups * kCounterStride + rg * (int64_t)tpr * kPairs;
     uint64_t *supers = p.ws + rowgroups * kCounterStride + rowgroups * (int64_t)tpr * kPairs +
                        rg * (int64_t)spr * kSup;
     const int j = tile % W, m = tile / W;
 
-    ClSteps<ST, VEC, S, REV, true, CT, true> cur;
+    typename ClStepsOf<ST, VEC, S, REV, M, CT, true, false>::type cur;
     CT A[VEC], B[VEC];
     cur.load_fold(ln, p.T, tile * W * S + wave * S, p.T, A, B);
 #pragma unroll

@@ -142,6 +142,9 @@ struct ClLaunch {
     int segments;   // kind 2: tiles per row-group
     bool ragged;    // kind 0, full lanes of a wave: lanes of vec channels on time steps that are only element-aligned,
                     // or whose C is no multiple of vec
+    int shift;      // channels beyond whole lanes that are moved between neighbouring lanes (scan_cl_shift.hpp); 0: none
+    int groups;     // workgroups side by side for a time step
+    int vectors;    // shift: vectors of channels per group
     int64_t grid;
     size_t lds_bytes;
     size_t ws_bytes;
@@ -152,10 +155,37 @@ constexpr int cl_max_threads(int vec, int steps) { return (vec > 1 && steps >= 8
 template <typename ST>
 hipError_t launch_scan_cl(const ClArgs &args, const ClLaunch &l, bool rev, hipStream_t stream);
 
+// Lanes that move elements between neighbours (scan_cl_shift.hpp): four channels of 4- and 2-byte types, two of fp64, and
+// spans of whole cycles of the phase.
+constexpr bool cl_shift_built(int esize, int vec, int steps, int kind)
+{
+    return vec == (esize == 8 ? 2 : 4) && (steps == 4 || steps == 8 || (steps == 16 && esize == 2 && kind == 2));
+}
+
+template <typename ST, int VEC, int S, int M>
+inline hipError_t launch_cl_shift(const ClArgs &args, const ClLaunch &l, bool rev, dim3 grid, dim3 block, hipStream_t stream)
+{
+    constexpr int MAXT = cl_max_threads(VEC, S);
+    if (l.kind == 2)
+        return rev ? launch_kernel(scan_cl_lookback_kernel<ST, VEC, S, true, MAXT, M>, grid, block, l.lds_bytes, stream, nullptr, nullptr, args)
+                   : launch_kernel(scan_cl_lookback_kernel<ST, VEC, S, false, MAXT, M>, grid, block, l.lds_bytes, stream, nullptr, nullptr, args);
+    if constexpr (cl_shift_built(sizeof(ST), VEC, S, 0))
+        return rev ? launch_kernel(scan_cl_kernel<ST, VEC, S, true, MAXT, false, M>, grid, block, l.lds_bytes, stream, nullptr, nullptr, args)
+                   : launch_kernel(scan_cl_kernel<ST, VEC, S, false, MAXT, false, M>, grid, block, l.lds_bytes, stream, nullptr, nullptr, args);
+    return hipErrorInvalidValue;
+}
+
 #define SCANSCAM_CL_CASE(ST, VEC, S)                                                                   \
     if (l.vec == (VEC) && l.steps == (S)) {                                                            \
         constexpr int MAXT = cl_max_threads(VEC, S);                                                   \
         hipError_t err = hipErrorInvalidValue;                                                         \
+        if constexpr (cl_shift_built(sizeof(ST), VEC, S, 2)) {                                            \
+            if (l.shift == 1) return launch_cl_shift<ST, VEC, S, 1>(args, l, rev, grid, block, stream);        \
+            if constexpr ((VEC) == 4) {                                                                \
+                if (l.shift == 3) return launch_cl_shift<ST, VEC, S, 3>(args, l, rev, grid, block, stream);    \
+            }                                                                                          \
+        }                                                                                              \
+        if (l.shift != 0) return hipErrorInvalidValue;                                                 \
         if (l.kind == 2) {                                                                             \
             if (rev) err = launch_kernel(scan_cl_lookback_kernel<ST, VEC, S, true, MAXT>, grid, block, l.lds_bytes, stream, nullptr, nullptr, args);  \
             else     err = launch_kernel(scan_cl_lookback_kernel<ST, VEC, S, false, MAXT>, grid, block, l.lds_bytes, stream, nullptr, nullptr, args); \

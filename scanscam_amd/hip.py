@@ -498,8 +498,9 @@ def workspace_bytes_cl(batch: int, T: int, C: int, dtype: torch.dtype, direction
 def resolve_plan_cl(batch: int, T: int, C: int, dtype: torch.dtype, direction: int = FORWARD,
                     plan: Optional[Plan] = None) -> Plan:
     """The plan the channels-last calls would run for dense ``[batch, T, C]`` tensors (no GPU needed). ``waves_per_row`` > 0:
-    the kernel that stages tiles through LDS, in that many parts of time; the other fields are then the plan of tensors it
-    cannot run."""
+    the kernel that stages tiles through LDS, in that many parts of time; below 0: lanes that move channels between each
+    other, in the launch ``-waves_per_row`` = 64 * steps + 2 * waves + (1 for tiles). The other fields are then the plan of
+    tensors these cannot run."""
     out = Plan()
     rc = lib().scanscam_resolve_plan_cl(batch, T, C, _dtype_code(dtype), direction, _plan_ref(plan), ctypes.byref(out))
     if rc != 0:

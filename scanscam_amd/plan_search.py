@@ -166,6 +166,9 @@ def _short(plan, layout="rows"):
     if plan is None:
         return "auto"
     if layout == "cl" and plan.waves_per_row:
+        if plan.waves_per_row < 0:
+            code = -plan.waves_per_row
+            return f"shifted {'tiles' if code % 2 else 'walk'} s{code // 64} w{code // 2 % 32}"
         return f"staged x{plan.waves_per_row}"
     s = f"m{plan.mode} v{plan.vec} u{plan.unroll} w{plan.waves}"
     return s + (f" r{plan.waves_per_row}" if plan.waves_per_row else "")

@@ -1,0 +1,91 @@
+"""
+Channels-last calls of odd channel counts whose channels move between neighbouring lanes: parity with the CPU oracle at
+the edges of its groups (63 vectors of 4 channels, 2 in float64), spans and tiles, and its route.
+"""
+import pytest
+import torch
+
+from scanscam_amd import hip
+from test_hip_channels_last import as_rows, rel_err
+from test_hip_staged import BAR, check, scan_pair
+
+
+def forced(steps, waves, tiles):
+    return hip.Plan(waves_per_row=-(64 * steps + 2 * waves + tiles))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", list(BAR))
+@pytest.mark.parametrize("steps,waves,tiles", [(4, 1, 0), (4, 3, 0), (8, 8, 0), (4, 2, 1), (8, 8, 1), (16, 4, 1)])  # (16: 16-bit types, others the plan in reserve)
+def test_edges_of_groups_and_spans(gpu, dtype, steps, waves, tiles):
+    """Either odd remainder of C, a last group of two vectors up to a whole one, every phase of a batch element's first
+    step, two time steps up to several tiles; outputs of nothing but their own elements."""
+    vec = 2 if dtype == torch.float64 else 4
+    plan = forced(steps, waves, tiles)
+    tile = steps * waves
+    for C in (63 * vec + 1, 63 * vec + 3, 70 * vec - 1, 126 * vec - 1, 126 * vec + 1):
+        if C % 2 == 0:
+            continue
+        for batch, T in ((5, 2), (3, tile - 1), (2, tile + 1), (1, 3 * tile + 2)):
+            print(f"case shift {dtype} C={C} batch={batch} T={T} {steps}x{waves} tiles={tiles}", flush=True)
+            inputs, (a, b, gh), results = scan_pair(gpu, (batch, T, C), dtype, plan, seed=C + T)
+            check(inputs, results, dtype)
+    # The last shape again, into the middle of buffers, and a forward pass in place.
+    n, L, code, stream = a.numel(), hip.lib(), hip._dtype_code(dtype), torch.cuda.current_stream().cuda_stream
+    pad = 16 * vec
+    for direction, count in ((hip.FORWARD, 1), (hip.BACKWARD, 2)):
+        ws = torch.empty(max(8, hip.workspace_bytes_cl(*a.shape, dtype, direction, plan)), dtype=torch.uint8, device=gpu)
+        out = [torch.full((n + 2 * pad,), 77.0, dtype=dtype, device=gpu) for _ in range(count)]
+        p = [o[pad:].data_ptr() for o in out]
+        if direction == hip.FORWARD:
+            rc = L.scanscam_scan_fwd_cl(a.data_ptr(), b.data_ptr(), p[0], *a.shape, code, ws.data_ptr(), ws.numel(), stream, plan)
+        else:
+            rc = L.scanscam_scan_bwd_cl(a.data_ptr(), results[0].data_ptr(), gh.data_ptr(), p[0], p[1], *a.shape, code,
+                                        ws.data_ptr(), ws.numel(), stream, plan)
+        assert rc == 0
+        for o, want in zip(out, results[:1] if count == 1 else results[1:]):
+            assert torch.equal(o[pad:pad + n].view(a.shape), want)
+            assert (o[:pad] == 77).all() and (o[pad + n:] == 77).all()
+    ws = torch.empty(max(8, hip.workspace_bytes_cl(*a.shape, dtype, hip.FORWARD, plan)), dtype=torch.uint8, device=gpu)
+    for place in (a, b):
+        x, y = a.clone(), b.clone()
+        target = x if place is a else y
+        assert L.scanscam_scan_fwd_cl(x.data_ptr(), y.data_ptr(), target.data_ptr(), *a.shape, code, ws.data_ptr(), ws.numel(),
+                                      stream, plan) == 0
+        assert torch.equal(target, results[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,shape", [(torch.float32, (64, 600, 1001)), (torch.bfloat16, (64, 1100, 1003)),
+                                         (torch.float64, (60, 300, 701)), (torch.float32, (2, 8000, 1601))])
+def test_automatic_route(gpu, dtype, shape):
+    """Calls that take these lanes by themselves give the results of the plan they report, bit for bit, and those of the plan
+    in reserve to within the bar; tensors off the vector border, or not dense, keep the plan in reserve."""
+    _, (a, b, gh), results = scan_pair(gpu, shape, dtype, None)
+    plans = [hip.resolve_plan_cl(*shape, dtype, d) for d in (hip.FORWARD, hip.BACKWARD)]
+    assert plans[0].waves_per_row < 0 and plans[1].waves_per_row < 0
+    call = lambda x, h, g, p: (hip.transposed_linear_scan_forward(x, b, plan=p[0]),  # noqa: E731
+                               *hip.transposed_linear_scan_backward(x, h, g, plan=p[1]))
+    same = call(a, results[0], gh, plans)
+    reserve = [hip.Plan(mode=p.mode, vec=p.vec, unroll=p.unroll, waves=p.waves) for p in plans]
+    other = call(a, results[0], gh, reserve)
+    for got, x, y in zip(results, same, other):
+        assert torch.equal(got, x)
+        assert rel_err(as_rows(got[:2]), as_rows(y[:2])) <= 2 * BAR[dtype]
+    # One element off the border: the same results as the plan in reserve gives there.
+    off = torch.empty(a.numel() + 1, dtype=dtype, device=gpu)[1:].view(shape)
+    off.copy_(a)
+    got = hip.transposed_linear_scan_forward(off, b)
+    assert torch.equal(got, hip.transposed_linear_scan_forward(off, b, plan=plans[0]))
+    assert rel_err(as_rows(got[:2]), as_rows(results[0][:2])) <= 2 * BAR[dtype]
+
+
+def test_where_the_route_lies():
+    """Even or few channels, short or small calls keep the cost model's plan; the numbers that are no launch are not taken."""
+    code = lambda b, T, C, dt, d: hip.resolve_plan_cl(b, T, C, dt, d).waves_per_row  # noqa: E731
+    f32, bf16 = torch.float32, torch.bfloat16
+    assert code(64, 2048, 1001, f32, hip.FORWARD) < 0 and code(64, 2048, 1001, bf16, hip.BACKWARD) < 0
+    for shape in ((64, 2048, 1000), (64, 2048, 1002), (300, 2048, 251), (512, 255, 1001), (8, 256, 1001)):
+        assert code(*shape, f32, hip.FORWARD) == 0, shape
+    for bad in (-1, -(64 * 5 + 2 * 4), -(64 * 12 + 8), -(64 * 16 + 9), -(64 * 8), -(64 * 8 + 2 * 16), -(1 << 20)):
+        assert hip.resolve_plan_cl(64, 2048, 1001, f32, hip.FORWARD, hip.Plan(waves_per_row=bad)).waves_per_row == 0, bad
