@@ -620,6 +620,24 @@ int run(bool rev, const void *a, const void *x, const void *h, void *y0, void *y
     return SCANSCAM_OK;
 }
 
+// Whether every tile of a time split takes the aggregates of all tiles before it instead of waiting for the chain of
+// super-tiles. A tile then waits for nothing but its predecessors' folds, one memory round trip, where the chain takes one
+// more per super-tile; each of its waves reads up to 8 aggregates of every channel. In calls of few rounds of workgroups
+// that wait is most of the time (GPU time, us forward / backward, buffers in rotation): fp32 [1, 2541, 295] 12.7 / 13.9 -> 10.2 /
+// 11.4, [10, 1083, 128] 12.8 / 14.7 -> 10.0 / 12.0, [3, 2000, 512] 14.5 / 18.7 -> 13.1 / 17.3, bf16 [2, 1643, 96] 12.4 / 13.9 ->
+// 9.6 / 10.8, [6, 574, 256] 9.6 / 10.6 -> 8.3 / 8.6; of 60 calls in fp32 and 16 bits none is slower by more than 2 %, and
+// larger ones are level ([8, 4096, 512] 45.3 / 73.8 -> 44.7 / 73.8). It ends where
+//   - a wave's aggregates span more than 1024 steps, or number more than 8: the product of a wave's gates is a plain number,
+//     and the chain composes no more;
+//   - a lane holds 64 elements, one workgroup per CU (bf16 [8, 4096, 512] backward, 4 channels x 16 steps, 39.3 against 41.5);
+//   - pairs are four words each: fp64 would lose as often as it gains ([4, 1489, 832] forward 45.1 against 57.1, [9, 599, 320] 17.0
+//     / 21.2 against 18.1 / 23.1, [1, 2754, 250] 16.2 / 21.5 -> 13.5 / 19.2).
+bool direct_lookback(const scanscam::ClLaunch &l, int esize)
+{
+    const int per_wave = (l.segments + l.waves - 1) / l.waves;  // tiles
+    return scanscam::cl_direct_built(esize, l.vec, l.steps) && per_wave <= 8 && per_wave * l.waves * l.steps <= 1024;
+}
+
 // Grid, LDS and workspace of a chosen launch; `virtual_steps`: steps before the first one that the tiles cover as well.
 int size_cl(int64_t batch, int64_t T, int dtype, int virtual_steps, scanscam::ClLaunch *l)
 {
@@ -642,6 +660,7 @@ int size_cl(int64_t batch, int64_t T, int dtype, int virtual_steps, scanscam::Cl
         l->kind = 0;
         l->ws_bytes = 0;
     }
+    l->direct = l->kind == 2 && l->shift == 0 && direct_lookback(*l, elem_size(dtype));
     l->grid = rowgroups * l->segments;
     if (l->grid >= (int64_t(1) << 31)) return SCANSCAM_EINVAL;
     return SCANSCAM_OK;

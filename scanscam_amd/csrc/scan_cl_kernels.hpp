@@ -751,6 +751,8 @@ __global__ __launch_bounds__(MAXT) void scan_cl_packed_kernel(const ClArgs p)
 //   carry   from S_m through the aggregates of tiles 0..j-1.
 // The last tile of a super-tile publishes (SA, SB) as soon as it holds all W
 // tile aggregates, and SI = fma(SA, S_m, SB) once S_m is known.
+// With DIRECT (few tiles per row-group, a kernel of its own: the code beside the chain costs that up to 7 %) there are no super-tiles: the waves share out ALL tiles before this one, each
+// composes its run of aggregates, and every lane folds the waves' pairs in order.
 //
 // Workspace, in 64-bit words: ticket counter of row-group r at word
 // r * kCounterStride, word 1 raised on a timed-out wait; then per (row-group,
@@ -796,7 +798,7 @@ __device__ __forceinline__ void cl_publish_pair(uint64_t *dst, int lane, const C
     for (int k = 0; k < VEC; k++) D::store_pair(dst + (k * kWave + lane) * D::PAIR, a[k], b[k]);
 }
 
-template <typename ST, int VEC, int S, bool REV, int MAXT, int M = 0>
+template <typename ST, int VEC, int S, bool REV, int MAXT, int M = 0, bool DIRECT = false>
 __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
 {
     using CT = typename ComputeOf<ST>::type;
@@ -880,7 +882,63 @@ __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
 #pragma unroll
     for (int k = 0; k < VEC; k++) carry[k] = CT(0);
 
-    if (tpr > 1) {
+    if constexpr (DIRECT) {
+        // Every tile takes the aggregates of all tiles before it, an equal run of them per wave.
+        if (wave == 0 && tile + 1 < tpr) cl_publish_pair<CT, VEC>(tiles + (int64_t)tile * kPairs, lane, TA, TB);
+        constexpr int NB = VEC <= 2 ? 4 : 2;  // in flight at a time
+        const int per = (tile + W - 1) / W, lo = wave * per, hi = lo + per < tile ? lo + per : tile;
+        CT RA[VEC], RB[VEC];
+#pragma unroll
+        for (int k = 0; k < VEC; k++) {
+            RA[k] = CT(1);
+            RB[k] = CT(0);
+        }
+        bool ready = true;
+        for (int i = lo, polls = p.spin_limit; i < hi && ready; i += NB) {
+            CT ta[NB][VEC], tb[NB][VEC];
+            for (;;) {
+                ready = true;
+#pragma unroll
+                for (int n = 0; n < NB; n++) {
+                    const uint64_t *src = tiles + (int64_t)(i + n < hi ? i + n : hi - 1) * kPairs;
+#pragma unroll
+                    for (int k = 0; k < VEC; k++) ready = D::load_pair(src + (k * kWave + lane) * D::PAIR, ta[n][k], tb[n][k]) && ready;
+                }
+                ready = __ballot(ready) == ~0ull;
+                if (ready || --polls <= 0) break;
+                __builtin_amdgcn_s_sleep(1);
+            }
+#pragma unroll
+            for (int n = 0; n < NB; n++) {
+                if (i + n < hi) {
+#pragma unroll
+                    for (int k = 0; k < VEC; k++) {
+                        RB[k] = fma_(ta[n][k], RB[k], tb[n][k]);
+                        RA[k] = ta[n][k] * RA[k];
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < VEC; k++) {
+            AT(tA, wave, k) = RA[k];
+            AT(tB, wave, k) = RB[k];
+        }
+        if (lane == 0) lds_flags[0][wave] = ready ? 1 : 0;
+        __syncthreads();
+        bool expired = false;
+        for (int w = 0; w < W; w++) {
+            expired = expired || lds_flags[0][w] == 0;
+#pragma unroll
+            for (int k = 0; k < VEC; k++) carry[k] = fma_(AT(tA, w, k), carry[k], AT(tB, w, k));
+        }
+        if (expired) {
+            if (threadIdx.x == 0)
+                __hip_atomic_store(p.ws + kTimeoutWord, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int k = 0; k < VEC; k++) carry[k] = CT(__builtin_nanf(""));
+        }
+    } else if (tpr > 1) {
         const bool closes = (j == W - 1) && (m + 1 < spr);
         if (wave == 0 && j < W - 1 && tile + 1 < tpr) cl_publish_pair<CT, VEC>(tiles + (int64_t)tile * kPairs, lane, TA, TB);
         // Wave w is responsible for tile w of this super-tile (if w < j) and for super-tile m-1-w.

@@ -144,6 +144,7 @@ struct ClLaunch {
                     // or whose C is no multiple of vec
     int shift;      // channels beyond whole lanes that are moved between neighbouring lanes (scan_cl_shift.hpp); 0: none
     int groups;     // workgroups side by side for a time step
+    bool direct;    // kind 2: every tile takes the aggregates of all tiles before it
     int vectors;    // shift: vectors of channels per group
     int64_t grid;
     size_t lds_bytes;
@@ -161,6 +162,9 @@ constexpr bool cl_shift_built(int esize, int vec, int steps, int kind)
 {
     return vec == (esize == 8 ? 2 : 4) && (steps == 4 || steps == 8 || (steps == 16 && esize == 2 && kind == 2));
 }
+
+// Lanes whose time split may look back over all tiles at once (ClLaunch::direct).
+constexpr bool cl_direct_built(int esize, int vec, int steps) { return esize != 8 && vec * steps < 64; }
 
 template <typename ST, int VEC, int S, int M>
 inline hipError_t launch_cl_shift(const ClArgs &args, const ClLaunch &l, bool rev, dim3 grid, dim3 block, hipStream_t stream)
@@ -186,6 +190,11 @@ inline hipError_t launch_cl_shift(const ClArgs &args, const ClLaunch &l, bool re
             }                                                                                          \
         }                                                                                              \
         if (l.shift != 0) return hipErrorInvalidValue;                                                 \
+        if constexpr (cl_direct_built(sizeof(ST), VEC, S)) {                                           \
+            if (l.kind == 2 && l.direct)                                                               \
+                return rev ? launch_kernel(scan_cl_lookback_kernel<ST, VEC, S, true, MAXT, 0, true>, grid, block, l.lds_bytes, stream, nullptr, nullptr, args)   \
+                           : launch_kernel(scan_cl_lookback_kernel<ST, VEC, S, false, MAXT, 0, true>, grid, block, l.lds_bytes, stream, nullptr, nullptr, args); \
+        }                                                                                              \
         if (l.kind == 2) {                                                                             \
             if (rev) err = launch_kernel(scan_cl_lookback_kernel<ST, VEC, S, true, MAXT>, grid, block, l.lds_bytes, stream, nullptr, nullptr, args);  \
             else     err = launch_kernel(scan_cl_lookback_kernel<ST, VEC, S, false, MAXT>, grid, block, l.lds_bytes, stream, nullptr, nullptr, args); \
