@@ -131,6 +131,13 @@ except (OSError, AttributeError) as exc:  # not built, or built for another ABI
 has_hip_ops = _lib is not None
 
 
+def _backward_in_python(gate: torch.Tensor, output: torch.Tensor, out_grad: torch.Tensor):
+    """What the native op's backward pass hands back: gradients to be copied first, tensors that hooks moved elsewhere."""
+    from .op import scan_gradients
+
+    return scan_gradients(gate, output, out_grad)
+
+
 def _bind_native(lib: ctypes.CDLL):
     """The op's host path in native code (csrc/torch_binding.cpp) on this library's entry points, or ``None`` if it is
     not built (``make -C scanscam_amd/csrc binding``) or was built against another PyTorch: the same calls then go through
@@ -147,7 +154,7 @@ def _bind_native(lib: ctypes.CDLL):
     _binding.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (
         lib.scanscam_scan_fwd_strided, lib.scanscam_scan_bwd_strided, lib.scanscam_scan_fwd_cl_strided,
         lib.scanscam_scan_bwd_cl_strided, lib.scanscam_workspace_bytes, lib.scanscam_workspace_bytes_cl,
-        lib.scanscam_strerror)))
+        lib.scanscam_strerror)), _backward_in_python)
     return _binding
 
 
@@ -223,10 +230,23 @@ _check = os.environ.get("SCANSCAM_DEBUG", "") not in ("", "0")
 _spin_limit = int(os.environ.get("SCANSCAM_SPIN_LIMIT", "0") or 0)
 
 
+_binding_module = _native
+
+
+def _leave_native() -> None:
+    """Tells the native op, whose backward pass does not come by here, when calls have to take the Python path."""
+    if _binding_module is not None:
+        _binding_module.leave_to_python(_check or _spin_limit > 0)
+
+
+_leave_native()
+
+
 def check_waits(on: bool, spin_limit: int = 0) -> None:
     """Turn the check for expired carry waits on or off (it blocks the host after every such launch)."""
     global _check, _spin_limit
     _check, _spin_limit = bool(on), int(spin_limit)
+    _leave_native()
 
 
 def _raise_if_wait_expired(ws: Optional[torch.Tensor], what: str) -> None:

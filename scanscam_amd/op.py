@@ -1,5 +1,6 @@
 """
-The user-facing op: ``scan(gate, value)`` and its ``torch.autograd.Function``.
+The user-facing op: ``scan(gate, value)`` and its ``torch.autograd.Function``, which plain GPU tensors pass by where the
+native binding is built (``csrc/torch_binding.cpp``: the same op with an autograd node in C++).
 
 Same surface as the reference's ``scanscam/op.py:9-55``: ``scan`` applies
 ``Scan``; ``Scan.forward`` saves ``(gate, output)``; ``Scan.backward`` returns
@@ -36,6 +37,10 @@ def scan(gate: torch.Tensor, value: torch.Tensor) -> torch.Tensor:
     :param value: [N x ... x T] tensor of values
     :return: an [N x ... x T] tensor of accumulated values.
     """
+    if hip._native is not None and hip._lib is not None and not torch.compiler.is_compiling():
+        output = hip._native.scan(gate, value)  # None: a call it leaves to the function below
+        if output is not None:
+            return output
     return Scan.apply(gate, value)
 
 
@@ -64,10 +69,15 @@ class Scan(torch.autograd.Function):
     @staticmethod
     def backward(ctx: Any, output_grad: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         gate, output = ctx.saved_tensors
-        if _on_gpu(output_grad):
-            # Channels-last when gate and output are: what op.py:45-49 of the reference means to
-            # do (its call has one argument too many).
-            return hip.scan_backward(gate, output, output_grad)
-        if cpu.supports(gate) and cpu.supports(output) and cpu.supports(output_grad):
-            return cpu.simple_linear_scan_backward(gate, output, output_grad)
-        return naive_linear_scan_backward(gate, output, output_grad)
+        return scan_gradients(gate, output, output_grad)
+
+
+def scan_gradients(gate: torch.Tensor, output: torch.Tensor, output_grad: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``(grad_gate, grad_value)``, dispatched as the forward pass is."""
+    if _on_gpu(output_grad):
+        # Channels-last when gate and output are: what op.py:45-49 of the reference means to
+        # do (its call has one argument too many).
+        return hip.scan_backward(gate, output, output_grad)
+    if cpu.supports(gate) and cpu.supports(output) and cpu.supports(output_grad):
+        return cpu.simple_linear_scan_backward(gate, output, output_grad)
+    return naive_linear_scan_backward(gate, output, output_grad)

@@ -1,0 +1,179 @@
+"""
+The op's native autograd node (csrc/torch_binding.cpp) against the Python function it stands in for: the same gradients, and
+the same outcome of everything the engine, hooks and modes do to a node.
+"""
+import threading
+
+import pytest
+import torch
+
+from scanscam_amd import hip, op, scan
+from test_binding import forms
+
+
+def leaves(*tensors):
+    return [t.detach().requires_grad_() for t in tensors]
+
+
+def is_native(h):
+    return h.grad_fn is not None and not isinstance(h.grad_fn, torch.autograd.function.BackwardCFunction)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+def test_same_gradients_as_the_python_function(gpu, dtype):
+    native = 0
+    for name, a, b, gh in forms(gpu, dtype):
+        print(f"case {name} {dtype}", flush=True)
+        results = []
+        for fn in (scan, op.Scan.apply):
+            x, y = leaves(a, b)
+            h = fn(x, y)
+            native += is_native(h)
+            results.append((h.detach(), *torch.autograd.grad(h, (x, y), gh)))
+        for got, want in zip(*results):
+            assert torch.equal(got, want) and got.stride() == want.stride() and got.dtype == want.dtype, name
+        for mask in ((True, False), (False, True)):
+            x, y = a.detach().requires_grad_(mask[0]), b.detach().requires_grad_(mask[1])
+            scan(x, y).backward(gh)
+            for leaf, want, on in zip((x, y), results[0][1:], mask):
+                assert (leaf.grad is None) if not on else torch.equal(leaf.grad, want)
+    assert native >= 15
+
+
+def outcome(fn):
+    try:
+        r = fn()
+        return tuple(t.cpu().tolist() for t in r) if isinstance(r, tuple) else r
+    except Exception as e:  # noqa: BLE001
+        return type(e), str(e).split("\n")[0][:60]
+
+
+@pytest.mark.gpu
+def test_same_outcomes_as_the_python_function(gpu):
+    g = torch.Generator(device=gpu).manual_seed(5)
+    a, b, gh = (torch.rand(4, 50, generator=g, device=gpu) for _ in range(3))
+
+    def twice(fn, retain):
+        x, y = leaves(a, b)
+        h = fn(x, y)
+        torch.autograd.grad(h, (x, y), gh, retain_graph=retain)
+        return torch.autograd.grad(h, (x, y), gh)
+
+    def changed(fn, which):
+        x, y = leaves(a, b)
+        x1 = x * 1
+        h = fn(x1, y)
+        with torch.no_grad():
+            (x1 if which == 0 else h).add_(1)
+        return torch.autograd.grad(h, (x, y), gh)
+
+    def second_order(fn):
+        x, y = leaves(a, b)
+        ga, _ = torch.autograd.grad(fn(x, y), (x, y), gh, create_graph=True)
+        return torch.autograd.grad(ga.sum(), (x,))
+
+    def saved_elsewhere(fn):
+        seen = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(t.shape), t.cpu())[1], lambda t: t.to(gpu)):
+            x, y = leaves(a, b)
+            h = fn(x, y)
+        assert len(seen) == 2
+        return torch.autograd.grad(h, (x, y), gh)
+
+    def left_on_the_cpu(fn):  # an error in both: the output gradient is on the GPU
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t):
+            x, y = leaves(a, b)
+            h = fn(x, y)
+        return torch.autograd.grad(h, (x, y), gh)
+
+    def hooked(fn):
+        x, y = leaves(a, b)
+        h = fn(x, y)
+        h.register_hook(lambda t: 2 * t)
+        h.grad_fn.register_hook(lambda gin, gout: (gin[0] + 1, gin[1]))
+        return torch.autograd.grad(h, (x, y), gh)
+
+    def checkpointed(fn):
+        x, y = leaves(a, b)
+        return torch.autograd.grad(torch.utils.checkpoint.checkpoint(fn, x, y, use_reentrant=False), (x, y), gh)
+
+    def checked(fn):  # switched on between the two passes
+        x, y = leaves(a, b)
+        h = fn(x, y)
+        hip.check_waits(True)
+        try:
+            return torch.autograd.grad(h, (x, y), gh)
+        finally:
+            hip.check_waits(False)
+
+    def vmapped(fn):
+        return torch.func.vmap(fn)(a[None], b[None])
+
+    def inside_a_transform(fn):
+        return torch.func.grad(lambda t: t.sum() + fn(a, b).sum())(a)
+
+    def dual(fn):
+        with torch.autograd.forward_ad.dual_level():
+            return fn(torch.autograd.forward_ad.make_dual(a, b), b)
+
+    def unused(fn):  # no gradient reaches the output of the inner call
+        x, y = leaves(a, b)
+        h = fn(x, y)
+        return torch.autograd.grad((h * 0).sum() + x.sum(), (x, y))
+
+    def grads_off(fn):
+        x, y = leaves(a, b)
+        with torch.no_grad():
+            h = fn(x, y)
+        with torch.inference_mode():
+            i = fn(x, y)
+        return h.requires_grad, h.grad_fn, i.is_inference(), h.is_inference()
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    def under_a_mode(fn):
+        x, y = leaves(a, b)
+        with Mode():
+            h = fn(x, y)
+            assert not is_native(h)
+            return torch.autograd.grad(h, (x, y), gh)
+
+    calls = [lambda f: twice(f, True), lambda f: twice(f, False), lambda f: changed(f, 0), lambda f: changed(f, 1), second_order,
+             saved_elsewhere, left_on_the_cpu, hooked, checkpointed, checked, vmapped, inside_a_transform, dual, unused, under_a_mode]
+    for i, call in enumerate(calls):
+        got, want = outcome(lambda: call(scan)), outcome(lambda: call(op.Scan.apply))
+        assert got == want, (i, got if isinstance(got[0], type) else "values", want if isinstance(want[0], type) else "values")
+    assert grads_off(scan) == grads_off(op.Scan.apply)
+    assert is_native(scan(*leaves(a, b)))
+
+
+@pytest.mark.gpu
+def test_threads_and_streams(gpu):
+    """Steps of several threads, each on a stream of its own, and an error of the library raised from the engine's thread."""
+    g = torch.Generator(device=gpu).manual_seed(6)
+    sets = [[torch.rand(8, 64, 4096, generator=g, device=gpu) for _ in range(3)] for _ in range(4)]
+    want = []
+    for a, b, gh in sets:
+        x, y = leaves(a, b)
+        want.append(torch.autograd.grad(op.Scan.apply(x, y), (x, y), gh))
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()) as _:
+            for _ in range(5):
+                x, y = leaves(*sets[i][:2])
+                got = torch.autograd.grad(scan(x, y), (x, y), sets[i][2])
+                torch.cuda.current_stream().synchronize()
+                if not all(torch.equal(p, q) for p, q in zip(got, want[i])):
+                    bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
