@@ -627,6 +627,9 @@ int run(bool rev, const void *a, const void *x, const void *h, void *y0, void *y
 // 11.4, [10, 1083, 128] 12.8 / 14.7 -> 10.0 / 12.0, [3, 2000, 512] 14.5 / 18.7 -> 13.1 / 17.3, bf16 [2, 1643, 96] 12.4 / 13.9 ->
 // 9.6 / 10.8, [6, 574, 256] 9.6 / 10.6 -> 8.3 / 8.6; of 60 calls in fp32 and 16 bits none is slower by more than 2 %, and
 // larger ones are level ([8, 4096, 512] 45.3 / 73.8 -> 44.7 / 73.8). It ends where
+//   - more workgroups cover each other's waits, and the aggregates they read are what is left: [25, 1696, 384], 2100 workgroups,
+//     0.97 / 0.99 x, [64, 1024, 333] backward, 3072 of them, 1.06 x, [24, 2048, 3072] backward, 18432, 543 -> 569, bf16 [90, 2048,
+//     514] backward, 14400, 243 -> 256 us: 2048 at most;
 //   - a wave's aggregates span more than 1024 steps, or number more than 8: the product of a wave's gates is a plain number,
 //     and the chain composes no more;
 //   - a lane holds 64 elements, one workgroup per CU (bf16 [8, 4096, 512] backward, 4 channels x 16 steps, 39.3 against 41.5);
@@ -635,7 +638,8 @@ int run(bool rev, const void *a, const void *x, const void *h, void *y0, void *y
 bool direct_lookback(const scanscam::ClLaunch &l, int esize)
 {
     const int per_wave = (l.segments + l.waves - 1) / l.waves;  // tiles
-    return scanscam::cl_direct_built(esize, l.vec, l.steps) && per_wave <= 8 && per_wave * l.waves * l.steps <= 1024;
+    return scanscam::cl_direct_built(esize, l.vec, l.steps) && l.grid <= 2048 && per_wave <= 8 &&
+           per_wave * l.waves * l.steps <= 1024;
 }
 
 // Grid, LDS and workspace of a chosen launch; `virtual_steps`: steps before the first one that the tiles cover as well.
@@ -660,8 +664,8 @@ int size_cl(int64_t batch, int64_t T, int dtype, int virtual_steps, scanscam::Cl
         l->kind = 0;
         l->ws_bytes = 0;
     }
-    l->direct = l->kind == 2 && l->shift == 0 && direct_lookback(*l, elem_size(dtype));
     l->grid = rowgroups * l->segments;
+    l->direct = l->kind == 2 && l->shift == 0 && direct_lookback(*l, elem_size(dtype));
     if (l->grid >= (int64_t(1) << 31)) return SCANSCAM_EINVAL;
     return SCANSCAM_OK;
 }

@@ -43,13 +43,13 @@ struct ClArgs {
     int32_t C;
     int32_t segments;   // look-back kernel: tiles per (batch element, channel group)
     int32_t group;      // packed kernel: lanes per time step (power of two below 64)
-    int32_t groups;     // channel groups (workgroups side by side) of a time step
-    int32_t vectors;    // scan_cl_shift.hpp: vectors of channels per group
     int32_t xcd_order;  // scan_cl_kernel, scan_cl_lookback_kernel: consecutive (batch element, channel group) pairs share an XCD
     int32_t cached_stores;  // outputs through the caches' normal policy instead of non-temporal (the host decides, see run_cl)
     int32_t cached_loads;    // element-aligned 8-byte lanes of 4-byte types: the same for loads
     uint64_t *ws;       // look-back kernel: ticket counters + published pairs
     int32_t spin_limit; // look-back kernel: polls before a wait gives up
+    int32_t groups;     // scan_cl_shift.hpp: channel groups (workgroups side by side) of a time step
+    int32_t vectors;    // scan_cl_shift.hpp: vectors of channels per group
 };
 
 // One workgroup's view of its channels: pointers offset to the batch element
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // wave-uniform: kept in a scalar register
     const int W = blockDim.x / kWave;
-    const int groups = p.groups;
+    const int groups = M != 0 ? p.groups : (p.C + kWave * VEC - 1) / (kWave * VEC);  // channel groups per batch element
     // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2. When a time step of C
     // channels is not a whole number of 128-byte lines, neighbouring channel groups share a line at
     // every time step; handled by different XCDs that line is fetched twice and written in two parts.
@@ -811,7 +811,7 @@ __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // wave-uniform: kept in a scalar register
     const int W = blockDim.x / kWave;
-    const int groups = p.groups;
+    const int groups = M != 0 ? p.groups : (p.C + kWave * VEC - 1) / (kWave * VEC);
     const int64_t rowgroups = p.batch * groups;
     const int tpr = p.segments;              // tiles per row-group
     const int spr = (tpr + W - 1) / W;       // super-tiles per row-group
