@@ -626,7 +626,7 @@ int run(bool rev, const void *a, const void *x, const void *h, void *y0, void *y
 // that wait is most of the time (GPU time, us forward / backward, buffers in rotation): fp32 [1, 2541, 295] 12.7 / 13.9 -> 10.2 /
 // 11.4, [10, 1083, 128] 12.8 / 14.7 -> 10.0 / 12.0, [3, 2000, 512] 14.5 / 18.7 -> 13.1 / 17.3, bf16 [2, 1643, 96] 12.4 / 13.9 ->
 // 9.6 / 10.8, [6, 574, 256] 9.6 / 10.6 -> 8.3 / 8.6; of 60 calls in fp32 and 16 bits none is slower by more than 2 %, and
-// larger ones are level ([8, 4096, 512] 45.3 / 73.8 -> 44.7 / 73.8). It ends where
+// larger ones gain little ([8, 4096, 512] 45.0 / 73.0 -> 43.7 / 72.5). It ends where
 //   - more workgroups cover each other's waits, and the aggregates they read are what is left: [25, 1696, 384], 2100 workgroups,
 //     0.97 / 0.99 x, [64, 1024, 333] backward, 3072 of them, 1.06 x, [24, 2048, 3072] backward, 18432, 543 -> 569, bf16 [90, 2048,
 //     514] backward, 14400, 243 -> 256 us: 2048 at most;

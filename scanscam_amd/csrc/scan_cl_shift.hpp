@@ -16,7 +16,7 @@
 //
 // fp32 [64, 2048, 1001], 4 waves of 8 steps, forward / backward: 342 / 569 us at any element, 304 / 509 us here (bf16 197 / 342 ->
 // 155 / 274 us), where the bytes take 257 / 433 us at C = 1024. Reads are those of the algorithm to 0.1 % and writes 3 % more
-// (FETCH_SIZE, WRITE_SIZE); a wave issues 0.9 / 1.5 times the vector instructions. What is left is the wave's accesses, still
+// (FETCH_SIZE, WRITE_SIZE); a wave issues 1.3 / 1.5 times the vector instructions. What is left is the wave's accesses, still
 // nine lines for the bytes of eight (C = 992, on whole lines, takes 288 / 497 us as well). Loads go through the caches' normal
 // policy, because the line that two channel groups share is in the L2 when the second one asks for it (313 / 528 us with
 // non-temporal ones); stores of whole vectors are non-temporal in fp32 (341 / 565 us with cached loads and stores) and fp64
