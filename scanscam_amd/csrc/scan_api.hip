@@ -630,8 +630,7 @@ int run(bool rev, const void *a, const void *x, const void *h, void *y0, void *y
 //   - more workgroups cover each other's waits, and the aggregates they read are what is left: [25, 1696, 384], 2100 workgroups,
 //     0.97 / 0.99 x, [64, 1024, 333] backward, 3072 of them, 1.06 x, [24, 2048, 3072] backward, 18432, 543 -> 569, bf16 [90, 2048,
 //     514] backward, 14400, 243 -> 256 us: 2048 at most;
-//   - a wave's aggregates span more than 1024 steps, or number more than 8: the product of a wave's gates is a plain number,
-//     and the chain composes no more;
+//   - a wave's aggregates span more than 1024 steps, or number more than 8: beyond what was measured;
 //   - a lane holds 64 elements, one workgroup per CU (bf16 [8, 4096, 512] backward, 4 channels x 16 steps, 39.3 against 41.5);
 //   - pairs are four words each: fp64 would lose as often as it gains ([4, 1489, 832] forward 45.1 against 57.1, [9, 599, 320] 17.0
 //     / 21.2 against 18.1 / 23.1, [1, 2754, 250] 16.2 / 21.5 -> 13.5 / 19.2).

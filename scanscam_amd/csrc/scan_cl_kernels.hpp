@@ -924,13 +924,33 @@ __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
             AT(tA, wave, k) = RA[k];
             AT(tB, wave, k) = RB[k];
         }
-        if (lane == 0) lds_flags[0][wave] = ready ? 1 : 0;
+        // A run's product of gates spans more than any that the chain multiplies together (8 tiles against W, and not on the
+        // super-tiles' borders). Where it is infinite the recurrence may still be finite (infinity times a value of zero is
+        // NaN), and the carry goes through the tiles one by one.
+        bool finite = true;
+#pragma unroll
+        for (int k = 0; k < VEC; k++) finite = finite && __builtin_isfinite(RA[k]);
+        finite = __ballot(finite) == ~0ull;
+        if (lane == 0) lds_flags[0][wave] = (ready ? 1 : 0) | (finite ? 2 : 0);
         __syncthreads();
-        bool expired = false;
-        for (int w = 0; w < W; w++) {
-            expired = expired || lds_flags[0][w] == 0;
+        int flags = 3;
+#pragma unroll 4
+        for (int w = 0; w < W; w++) {  // (unrolled further, 2 x 16 16-bit elements lose a workgroup's registers)
+            flags &= lds_flags[0][w];
 #pragma unroll
             for (int k = 0; k < VEC; k++) carry[k] = fma_(AT(tA, w, k), carry[k], AT(tB, w, k));
+        }
+        bool expired = !(flags & 1);
+        if (!(flags & 2)) {
+#pragma unroll
+            for (int k = 0; k < VEC; k++) carry[k] = CT(0);
+#pragma unroll 1
+            for (int i = 0; i < tile; i++) {  // (published: the waves have seen them all)
+                CT ta[VEC], tb[VEC];
+                expired = !cl_fetch_pair<CT, VEC>(tiles + (int64_t)i * kPairs, lane, ta, tb) || expired;
+#pragma unroll
+                for (int k = 0; k < VEC; k++) carry[k] = fma_(ta[k], carry[k], tb[k]);
+            }
         }
         if (expired) {
             if (threadIdx.x == 0)
