@@ -890,32 +890,40 @@ bool resolve_shift(int64_t batch, int64_t T, int64_t C, int dtype, int code, sca
 //   backwards, which is bound by its accesses more than by bytes, from 64 MiB on: bf16 [5, 2172, 741] 0.66, [14, 1649, 1119]
 //   0.79, [11, 669, 3295] 0.79, [9, 1598, 2353] 0.91 (from 96 to 143 pairs 0.99 to 1.10; [2, 17252, 285], 4 pairs, 1.14; [31, 1342,
 //   275], 35 lanes, 1.08); forwards they lose (0.92 to 1.4). fp64 has no fewer accesses per byte to gain (1.0 to 1.5).
-int shift_choice(int64_t batch, int64_t T, int64_t C, int esize, bool rev)
+//
+// Tiles multiply the gates of their super-tiles together, waves^2 * steps of them, and a product that leaves fp32's range
+// makes NaN of a scan value of zero (gates above one before the first value). `reserve`, the cost model's plan, is what the
+// call ran without them: they take it only where that multiplies as many together, in 16 bits with fewer waves where it
+// multiplies 128 (0.82 to 0.93 x backwards) and not at all where it is a walk, whose waves multiply 16 gates at most (tiles
+// 0.68 to 1.25 x of its time there). From 144 pairs on 16 bits backwards are a walk of these lanes instead (0.80 to 0.98 x).
+int shift_choice(int64_t batch, int64_t T, int64_t C, int esize, bool rev, const scanscam::ClLaunch &reserve)
 {
     const int vec = shift_vec(esize);
     if (C % 2 == 0 || C <= (kWave - 1) * vec || T < 256) return 0;
     const int64_t bytes = batch * T * C * esize * (rev ? 5 : 3);
     const int64_t all = (C + vec - 1) / vec, groups = (all + kWave - 2) / (kWave - 1), pairs = batch * groups;
     const bool filled = all >= 44 * groups;
-    if (pairs >= 192) {
-        if (bytes <= kLastLevelCache || !filled || (pairs > 512 && esize != 8)) return 0;
+    const int product = reserve.kind == 2 ? reserve.waves * reserve.waves * reserve.steps : 0;
+    if (pairs >= (esize == 2 && rev ? 144 : 192)) {
+        if (bytes <= (pairs < 192 ? kLastLevelCache / 4 : kLastLevelCache) || !filled || (pairs > 512 && esize != 8)) return 0;
         return esize == 2 ? shift_code(rev ? 4 : 8, 8, false) : shift_code(8, 4, false);
     }
     if (esize == 2) {
-        if (!rev || bytes <= kLastLevelCache / 4 || pairs < 8 || (pairs >= 96 && pairs < 144)) return 0;
-        return pairs < 40 ? shift_code(16, 8, true) : (filled ? shift_code(16, 4, true) : 0);
+        if (!rev || bytes <= kLastLevelCache / 4 || pairs < 8 || pairs >= 96 || (pairs >= 40 && !filled)) return 0;
+        return product >= 256 ? shift_code(16, 4, true) : (product >= 128 ? shift_code(8, 4, true) : 0);
     }
-    if (esize == 4) return filled && pairs <= 96 && bytes > (rev ? kLastLevelCache / 4 * 5 : kLastLevelCache) ? shift_code(8, 8, true) : 0;
+    if (esize == 4 && filled && pairs <= 96 && bytes > (rev ? kLastLevelCache / 4 * 5 : kLastLevelCache))
+        return product >= 512 ? shift_code(8, 8, true) : (product >= 256 && rev ? shift_code(4, 8, true) : 0);
     return 0;
 }
 
 // The same for a call's plan: what a resolved plan says (scanscam_resolve_plan_cl writes the number's negative into
 // waves_per_row), the automatic choice where the plan leaves everything open.
-int shift_code_of(const scanscam_plan *plan, int64_t batch, int64_t T, int64_t C, int esize, bool rev)
+int shift_code_of(const scanscam_plan *plan, int64_t batch, int64_t T, int64_t C, int esize, bool rev, const scanscam::ClLaunch &reserve)
 {
     if (plan && plan->waves_per_row < 0) return plan->waves_per_row > -4096 ? -plan->waves_per_row : 0;
     const bool free_plan = !plan || (plan->mode == SCANSCAM_MODE_AUTO && !plan->vec && !plan->unroll && !plan->waves && !plan->waves_per_row);
-    return free_plan ? shift_choice(batch, T, C, esize, rev) : 0;
+    return free_plan ? shift_choice(batch, T, C, esize, rev, reserve) : 0;
 }
 
 int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void *y1,
@@ -981,7 +989,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         if ((uint64_t)sT[k] * (uint64_t)esize * 18u + (uint64_t)C * (uint64_t)esize >= (uint64_t(1) << 32)) return SCANSCAM_EINVAL;
 
     const int parts = staged_parts_of(plan, batch, T, C, esize);
-    const int code = parts > 0 ? 0 : shift_code_of(plan, batch, T, C, esize, rev);
+    const int code = parts > 0 ? 0 : shift_code_of(plan, batch, T, C, esize, rev, l);
     scanscam::ClLaunch shifted;
     if (code != 0 && dense && resolve_shift(batch, T, C, dtype, code, &shifted) &&
         (shifted.ws_bytes == 0 || (workspace && workspace_bytes >= shifted.ws_bytes && aligned_to(workspace, 8))))
@@ -1166,14 +1174,14 @@ size_t scanscam_workspace_bytes_cl(int64_t batch, int64_t T, int64_t C, int dtyp
     scanscam::StagedArgs st;
     if (parts > 1 && resolve_staged(batch, T, C, esize, parts, &st)) need = staged_bytes(batch, C, esize, st);
     if (plan && plan->mode == kModeStaged) return need;
-    const int code = parts > 0 ? 0 : shift_code_of(plan, batch, T, C, esize, direction == SCANSCAM_BACKWARD);
-    scanscam::ClLaunch shifted;
-    if (code != 0 && resolve_shift(batch, T, C, dtype, code, &shifted)) need = shifted.ws_bytes;
     // The caller's pointers are not known yet: every alignment the tensors may turn out to have.
+    const bool rev = direction == SCANSCAM_BACKWARD;
     for (int align = 16; align >= esize; align >>= 1) {
-        scanscam::ClLaunch l;
-        if (resolve_cl(plan, batch, T, C, dtype, align, direction == SCANSCAM_BACKWARD, &l) == SCANSCAM_OK && l.ws_bytes > need)
-            need = l.ws_bytes;
+        scanscam::ClLaunch l, shifted;
+        if (resolve_cl(plan, batch, T, C, dtype, align, rev, &l) != SCANSCAM_OK) continue;
+        if (l.ws_bytes > need) need = l.ws_bytes;
+        const int code = align == esize && parts == 0 ? shift_code_of(plan, batch, T, C, esize, rev, l) : 0;  // (odd channel counts)
+        if (code != 0 && resolve_shift(batch, T, C, dtype, code, &shifted) && shifted.ws_bytes > need) need = shifted.ws_bytes;
     }
     return need;
 }
@@ -1271,7 +1279,7 @@ int scanscam_resolve_plan_cl(int64_t batch, int64_t T, int64_t C, int dtype, int
     const int rc = resolve_cl(plan, batch, T, C, dtype, align, direction == SCANSCAM_BACKWARD, &l);
     if (rc != SCANSCAM_OK) return rc;
     const int parts = staged_parts_of(plan, batch, T, C, esize);  // (`out` may be the plan itself)
-    const int code = parts > 0 ? 0 : shift_code_of(plan, batch, T, C, esize, direction == SCANSCAM_BACKWARD);
+    const int code = parts > 0 ? 0 : shift_code_of(plan, batch, T, C, esize, direction == SCANSCAM_BACKWARD, l);
     scanscam::StagedArgs st;
     out->mode = l.kind == 2 ? kModeLookback : kModeRow;
     out->vec = l.vec;

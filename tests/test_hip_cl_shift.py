@@ -2,11 +2,14 @@
 Channels-last calls of odd channel counts whose channels move between neighbouring lanes: parity with the CPU oracle at
 the edges of its groups (63 vectors of 4 channels, 2 in float64), spans and tiles, and its route.
 """
+import random
+
 import pytest
 import torch
 
+import oracle
 from scanscam_amd import hip
-from test_hip_channels_last import as_rows, rel_err
+from test_hip_channels_last import as_rows, prev_abs, rel_err
 from test_hip_staged import BAR, check, scan_pair
 
 
@@ -89,3 +92,38 @@ def test_where_the_route_lies():
         assert code(*shape, f32, hip.FORWARD) == 0, shape
     for bad in (-1, -(64 * 5 + 2 * 4), -(64 * 12 + 8), -(64 * 16 + 9), -(64 * 8), -(64 * 8 + 2 * 16), -(1 << 20)):
         assert hip.resolve_plan_cl(64, 2048, 1001, f32, hip.FORWARD, hip.Plan(waves_per_row=bad)).waves_per_row == 0, bad
+
+
+def test_tiles_multiply_no_more_gates_than_the_plan_in_reserve():
+    """A super-tile's product of gates is a plain number: where the plan in reserve multiplies fewer, gates above one would
+    take it out of range earlier (a walk multiplies a wave's own steps)."""
+    rng, taken = random.Random(3), 0
+    for _ in range(4000):
+        dtype = rng.choice((torch.float32, torch.bfloat16, torch.float64))
+        C = int(2 ** rng.uniform(8, 12)) | 1
+        T = int(2 ** rng.uniform(8, 15))
+        batch = max(1, int(2 ** rng.uniform(22, 27)) // (C * T))
+        p = hip.resolve_plan_cl(batch, T, C, dtype, rng.randrange(2))
+        if p.waves_per_row >= 0 or p.waves_per_row % 2 == 0:
+            continue
+        taken += 1
+        steps, waves = -p.waves_per_row // 64, -p.waves_per_row // 2 % 32
+        assert p.mode == hip.MODE_LOOKBACK and waves * waves * steps <= p.waves * p.waves * p.unroll, (batch, T, C, dtype, p)
+    assert taken > 100
+
+
+@pytest.mark.gpu
+def test_gates_above_one_after_the_last_gradient(gpu):
+    """Backwards over 563 steps of gates of 1.5 before the first output gradient other than zero: the gradients stay zero
+    there, also in calls wide enough for tiles."""
+    shape, last = (5, 683, 2421), 120
+    print(f"case {shape} {hip.resolve_plan_cl(*shape, torch.bfloat16, hip.BACKWARD)}", flush=True)
+    g = torch.Generator().manual_seed(8)
+    a = torch.rand(shape, generator=g)
+    h, gh = torch.randn(shape, generator=g).bfloat16(), torch.randn(shape, generator=g)
+    a[:, last:], gh[:, last:] = 1.5, 0
+    a, gh = a.bfloat16(), gh.bfloat16()
+    ga, gb = hip.transposed_linear_scan_backward(a.to(gpu), h.to(gpu), gh.to(gpu))
+    want_ga, want_gb = oracle.bwd(as_rows(a), as_rows(h), as_rows(gh))
+    assert rel_err(as_rows(gb), want_gb) <= BAR[torch.bfloat16]
+    assert rel_err(as_rows(ga), want_ga, prev_abs(as_rows(h))) <= BAR[torch.bfloat16]
