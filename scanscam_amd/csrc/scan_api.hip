@@ -876,26 +876,28 @@ bool resolve_shift(int64_t batch, int64_t T, int64_t C, int dtype, int code, sca
     return size_cl(batch, T, dtype, l->vec - 1, l) == SCANSCAM_OK && scanscam::cl_shift_built(esize, l->vec, l->steps, l->kind);  // (one tile: a walk)
 }
 
-// When an automatic call takes them. What it does without them is the cost model's plan: lanes of one channel, or wide ones
-// that load and store at any element. Measured against that plan (forward / backward, x of its time, or us; buffers in
-// rotation), in calls that do not fit the last-level cache -- within it the two are level or up to 1.3 x behind (bf16 [61,
-// 333, 1471] 1.07 / 1.04, fp32 [8, 1198, 831] 1.02 / 1.04) -- of 256 time steps or more:
-//   A walk, for 192 workgroups or more (up to 512 in fp32 and 16 bits): fp32 [64, 2048, 1001] 342 / 569 -> 304 / 509 us, [117,
-//   1055, 363] 0.82 / 0.85, [134, 354, 659] 0.97 / 0.87; bf16 [64, 2048, 1001] 197 / 342 -> 155 / 274 us, [28, 2048, 1777] 0.92 /
-//   0.82, [52, 407, 2265] 0.95 / 0.90; fp64 [39, 491, 1169] 0.87 / 0.89, [10, 669, 3709] 0.96 / 1.01, [6, 609, 3921] 0.98 / 0.83.
-//   With 840 workgroups fp32 [280, 372, 599] 1.06 / 1.13, bf16 [421, 343, 269] 1.03 / 1.13; with groups of fewer than 44 of 64
-//   lanes bf16 [144, 1447, 275] 1.25 / 1.13, fp64 [131, 353, 167] 0.99 / 1.06.
-//   Tiles, for fewer. fp32 up to 96 (batch element, channel group) pairs: [1, 9006, 3361] 0.79 / 0.71, [4, 5636, 1993] 0.91 /
-//   0.93, [28, 2754, 721] 0.93 / 0.98 ([59, 2896, 365], 118 pairs, 1.00 / 1.15; [7, 738, 2803] 290 MB backwards 1.05). 16 bits
-//   backwards, which is bound by its accesses more than by bytes, from 64 MiB on: bf16 [5, 2172, 741] 0.66, [14, 1649, 1119]
-//   0.79, [11, 669, 3295] 0.79, [9, 1598, 2353] 0.91 (from 96 to 143 pairs 0.99 to 1.10; [2, 17252, 285], 4 pairs, 1.14; [31, 1342,
-//   275], 35 lanes, 1.08); forwards they lose (0.92 to 1.4). fp64 has no fewer accesses per byte to gain (1.0 to 1.5).
+// When an automatic call takes them. `reserve` is what it does without them, the cost model's plan: lanes of one channel, or
+// wide ones that load and store at any element. Times of 1134 calls against that plan, buffers in rotation
+// (profiles/moved_channels_random_shapes.txt): calls of 256 time steps or more that do not fit the last-level cache -- within it
+// the two are level or up to 1.3 x behind --, by their (batch element, channel group) pairs:
+//   A walk, a workgroup per pair, for 192 (16 bits backwards 144) to 512 of them (fp64 any number), whose groups fill 44 of 64
+//   lanes. Up to 256, one per CU: 16 bits 0.76 to 0.98 forwards and 0.67 to 0.98 backwards, fp64 0.84 to 1.04 and 0.73 to 0.95,
+//   fp32 backwards 0.79 to 1.05; forwards in fp32 only from 1 GiB of tensors on (0.87 to 1.03; below, where the reserve moves
+//   up to 5.3 TB/s, 0.88 to 1.20, slower in three of four). From 257 to 320 a second round of workgroups is nearly empty
+//   (16 bits up to 1.31 and 1.19, fp32 1.28 and 1.21, fp64 1.13; up to 384 16 bits forwards 0.76 to 1.12, fp32 0.87 to 1.04 and
+//   0.85 to 1.11). Beyond, 16 bits 0.76 to 1.04 and 0.74 to 1.01, fp32 0.84 to 0.98 and 0.84 to 1.04, fp64 0.76 to 1.06 and
+//   0.76 to 1.08.
+//   fp32 [64, 2048, 1001] 345 / 567 -> 304 / 507 us, bf16 199 / 333 -> 151 / 263.
+//   Tiles, for fewer. fp32 below 40 pairs, 8 steps x 8 waves: 0.70 to 1.05 forwards (with 24 pairs and more from 512 MiB on;
+//   below up to 1.14), 0.68 to 1.02 backwards; up to 96 backwards, 4 x 8 where the reserve has 16 steps a wave 0.83 to 1.01 (8
+//   steps, 0.88 to 1.08; forwards 0.89 to 1.29). 16 bits backwards, which is bound by its accesses more than by bytes, from 96
+//   MiB on, 8 to 95 pairs: 0.57 to 1.06 (from 64 MiB on 0.71 to 1.16, with 97 to 143 pairs 0.65 to 1.23, below 8 0.74 to 1.29);
+//   forwards they lose (0.92 to 1.4). fp64 has no fewer accesses per byte to gain (1.0 to 1.5).
 //
 // Tiles multiply the gates of their super-tiles together, waves^2 * steps of them, and a product that leaves fp32's range
-// makes NaN of a scan value of zero (gates above one before the first value). `reserve`, the cost model's plan, is what the
-// call ran without them: they take it only where that multiplies as many together, in 16 bits with fewer waves where it
-// multiplies 128 (0.82 to 0.93 x backwards) and not at all where it is a walk, whose waves multiply 16 gates at most (tiles
-// 0.68 to 1.25 x of its time there). From 144 pairs on 16 bits backwards are a walk of these lanes instead (0.80 to 0.98 x).
+// makes NaN of a scan value of zero (gates above one before the first value). They are taken only where the reserve
+// multiplies as many together, in 16 bits with fewer steps where it multiplies 128 (0.70 to 1.00) and not at all where it is a
+// walk, whose waves multiply 16 gates at most (tiles 0.68 to 1.25 there).
 int shift_choice(int64_t batch, int64_t T, int64_t C, int esize, bool rev, const scanscam::ClLaunch &reserve)
 {
     const int vec = shift_vec(esize);
@@ -904,16 +906,21 @@ int shift_choice(int64_t batch, int64_t T, int64_t C, int esize, bool rev, const
     const int64_t all = (C + vec - 1) / vec, groups = (all + kWave - 2) / (kWave - 1), pairs = batch * groups;
     const bool filled = all >= 44 * groups;
     const int product = reserve.kind == 2 ? reserve.waves * reserve.waves * reserve.steps : 0;
+    const int64_t cache = kLastLevelCache;
     if (pairs >= (esize == 2 && rev ? 144 : 192)) {
-        if (bytes <= (pairs < 192 ? kLastLevelCache / 4 : kLastLevelCache) || !filled || (pairs > 512 && esize != 8)) return 0;
+        const int64_t least = pairs < 192 ? cache / 8 * 3 : (esize == 4 && !rev && pairs <= 256 ? 4 * cache : cache);
+        const bool second_round = pairs > 256 && pairs <= (esize == 4 || (esize == 2 && !rev) ? 384 : 320);
+        if (bytes <= least || !filled || second_round || (pairs > 512 && esize != 8)) return 0;
         return esize == 2 ? shift_code(rev ? 4 : 8, 8, false) : shift_code(8, 4, false);
     }
     if (esize == 2) {
-        if (!rev || bytes <= kLastLevelCache / 4 || pairs < 8 || pairs >= 96 || (pairs >= 40 && !filled)) return 0;
+        if (!rev || bytes <= cache / 8 * 3 || pairs < 8 || pairs >= 96 || (pairs >= 40 && !filled)) return 0;
         return product >= 256 ? shift_code(16, 4, true) : (product >= 128 ? shift_code(8, 4, true) : 0);
     }
-    if (esize == 4 && filled && pairs <= 96 && bytes > (rev ? kLastLevelCache / 4 * 5 : kLastLevelCache))
-        return product >= 512 ? shift_code(8, 8, true) : (product >= 256 && rev ? shift_code(4, 8, true) : 0);
+    if (esize == 4 && filled && bytes > (rev ? cache / 4 * 5 : cache)) {
+        if (pairs < (rev || bytes > 2 * cache ? 40 : 24)) return product >= 512 ? shift_code(8, 8, true) : 0;
+        if (rev && pairs <= 96) return product >= 256 && reserve.steps >= 16 ? shift_code(4, 8, true) : 0;
+    }
     return 0;
 }
 

@@ -59,7 +59,7 @@ def test_edges_of_groups_and_spans(gpu, dtype, steps, waves, tiles):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype,shape", [(torch.float32, (64, 600, 1001)), (torch.bfloat16, (64, 1100, 1003)),
+@pytest.mark.parametrize("dtype,shape", [(torch.float32, (100, 300, 1001)), (torch.bfloat16, (64, 1100, 1003)),
                                          (torch.float64, (60, 300, 701)), (torch.float32, (2, 8000, 1601))])
 def test_automatic_route(gpu, dtype, shape):
     """Calls that take these lanes by themselves give the results of the plan they report, bit for bit, and those of the plan
@@ -92,6 +92,21 @@ def test_where_the_route_lies():
         assert code(*shape, f32, hip.FORWARD) == 0, shape
     for bad in (-1, -(64 * 5 + 2 * 4), -(64 * 12 + 8), -(64 * 16 + 9), -(64 * 8), -(64 * 8 + 2 * 16), -(1 << 20)):
         assert hip.resolve_plan_cl(64, 2048, 1001, f32, hip.FORWARD, hip.Plan(waves_per_row=bad)).waves_per_row == 0, bad
+
+
+def test_calls_that_the_cost_model_s_plan_runs_faster_keep_it():
+    """Walks whose second round of workgroups is nearly empty, fp32 forwards below 1 GiB, tiles against a walk."""
+    code = lambda b, T, C, dt, d: hip.resolve_plan_cl(b, T, C, dt, d).waves_per_row  # noqa: E731
+    f32, f64, bf16, fwd, bwd = torch.float32, torch.float64, torch.bfloat16, hip.FORWARD, hip.BACKWARD
+    for call in ((90, 1064, 531, bf16, fwd), (19, 831, 3293, bf16, fwd), (19, 831, 3293, bf16, bwd), (30, 857, 2161, bf16, bwd),
+                 (32, 505, 2851, bf16, fwd), (29, 415, 2021, f32, fwd), (29, 415, 2021, f32, bwd), (88, 1133, 689, f32, bwd),
+                 (44, 1080, 723, f64, bwd), (16, 1000, 3225, f32, fwd), (56, 1000, 993, f32, fwd), (9, 2173, 1651, f32, fwd),
+                 (3, 4153, 2549, f32, fwd), (26, 260, 3223, f32, bwd), (1, 2361, 3531, bf16, bwd), (54, 368, 441, bf16, bwd)):
+        assert code(*call) == 0, call
+    for call in ((64, 1000, 977, bf16, fwd), (64, 1000, 977, bf16, bwd), (104, 1370, 965, bf16, fwd), (60, 600, 1001, f32, bwd),
+                 (64, 2048, 1001, f32, fwd), (100, 300, 1001, f32, fwd), (42, 600, 741, f64, bwd), (2, 15698, 1589, f32, fwd),
+                 (23, 1442, 871, f32, bwd), (36, 1357, 923, bf16, bwd), (11, 3192, 813, bf16, bwd)):
+        assert code(*call) < 0, call
 
 
 def test_tiles_multiply_no_more_gates_than_the_plan_in_reserve():
