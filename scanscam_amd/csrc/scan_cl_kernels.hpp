@@ -941,7 +941,7 @@ __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
             for (int k = 0; k < VEC; k++) carry[k] = fma_(AT(tA, w, k), carry[k], AT(tB, w, k));
         }
         bool expired = !(flags & 1);
-        if (!(flags & 2)) {
+        if (__builtin_expect(!(flags & 2), 0)) {
 #pragma unroll
             for (int k = 0; k < VEC; k++) carry[k] = CT(0);
 #pragma unroll 1
