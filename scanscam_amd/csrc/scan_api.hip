@@ -625,24 +625,27 @@ int run(bool rev, const void *a, const void *x, const void *h, void *y0, void *y
 // more per super-tile; each of its waves reads up to 8 aggregates of every channel. In calls of few rounds of workgroups
 // that wait is most of the time (GPU time, us forward / backward, buffers in rotation): fp32 [1, 2541, 295] 12.7 / 13.9 -> 10.2 /
 // 11.4, [10, 1083, 128] 12.8 / 14.7 -> 10.0 / 12.0, [3, 2000, 512] 14.5 / 18.7 -> 13.1 / 17.3, bf16 [2, 1643, 96] 12.4 / 13.9 ->
-// 9.6 / 10.8, [6, 574, 256] 9.6 / 10.6 -> 8.3 / 8.6; of 60 calls in fp32 and 16 bits none is slower by more than 2 %, and
-// larger ones gain little ([8, 4096, 512] 45.0 / 73.0 -> 43.7 / 72.5). It ends where
+// 9.6 / 10.8, [6, 574, 256] 9.6 / 10.6 -> 8.3 / 8.6; 225 and 192 calls in fp32 and 16 bits 0.87 and 0.89 x in the mean, at most 1.04 and 1.06
+// (profiles/direct_lookback_random_shapes.txt), and larger ones gain little ([8, 4096, 512] 45.0 / 73.0 -> 43.7 / 72.5). It
+// ends where
 //   - more workgroups cover each other's waits, and the aggregates they read are what is left: [25, 1696, 384], 2100 workgroups,
 //     0.97 / 0.99 x, [64, 1024, 333] backward, 3072 of them, 1.06 x, [24, 2048, 3072] backward, 18432, 543 -> 569, bf16 [90, 2048,
-//     514] backward, 14400, 243 -> 256 us: 2048 at most;
+//     514] backward, 14400, 243 -> 256 us: 2048 at most, and 896 for 16 single 16-bit channels backwards (30 calls with fewer
+//     0.78 to 1.03 x, 19 with more 0.98 to 1.10 x: [18, 1242, 151] 21.4 -> 23.4 us);
 //   - a wave's aggregates span more than 1024 steps, or number more than 8: beyond what was measured;
 //   - a lane holds 64 elements, one workgroup per CU (bf16 [8, 4096, 512] backward, 4 channels x 16 steps, 39.3 against 41.5);
 //   - pairs are four words each: fp64 would lose as often as it gains ([4, 1489, 832] forward 45.1 against 57.1, [9, 599, 320] 17.0
 //     / 21.2 against 18.1 / 23.1, [1, 2754, 250] 16.2 / 21.5 -> 13.5 / 19.2).
-bool direct_lookback(const scanscam::ClLaunch &l, int esize)
+bool direct_lookback(const scanscam::ClLaunch &l, int esize, bool rev)
 {
     const int per_wave = (l.segments + l.waves - 1) / l.waves;  // tiles
-    return scanscam::cl_direct_built(esize, l.vec, l.steps) && l.grid <= 2048 && per_wave <= 8 &&
+    const int most = esize == 2 && rev && l.vec == 1 && l.steps == 16 ? 896 : 2048;  // workgroups
+    return scanscam::cl_direct_built(esize, l.vec, l.steps) && l.grid <= most && per_wave <= 8 &&
            per_wave * l.waves * l.steps <= 1024;
 }
 
 // Grid, LDS and workspace of a chosen launch; `virtual_steps`: steps before the first one that the tiles cover as well.
-int size_cl(int64_t batch, int64_t T, int dtype, int virtual_steps, scanscam::ClLaunch *l)
+int size_cl(int64_t batch, int64_t T, int dtype, bool rev, int virtual_steps, scanscam::ClLaunch *l)
 {
     const int64_t rowgroups = batch * l->groups;
     const int64_t tile_steps = (int64_t)l->waves * l->steps;
@@ -664,7 +667,7 @@ int size_cl(int64_t batch, int64_t T, int dtype, int virtual_steps, scanscam::Cl
         l->ws_bytes = 0;
     }
     l->grid = rowgroups * l->segments;
-    l->direct = l->kind == 2 && l->shift == 0 && direct_lookback(*l, elem_size(dtype));
+    l->direct = l->kind == 2 && l->shift == 0 && direct_lookback(*l, elem_size(dtype), rev);
     if (l->grid >= (int64_t(1) << 31)) return SCANSCAM_EINVAL;
     return SCANSCAM_OK;
 }
@@ -721,7 +724,7 @@ int resolve_cl(const scanscam_plan *user, int64_t batch, int64_t T, int64_t C, i
     l->shift = 0;
     l->groups = (int)scanscam::cl_groups(C, c.vec);
     l->vectors = kWave;
-    return size_cl(batch, T, dtype, 0, l);
+    return size_cl(batch, T, dtype, rev, 0, l);
 }
 
 // Channels-last tiles staged through LDS (scan_staged_kernels.hpp): whether that kernel can run the call, and its tile.
@@ -873,7 +876,7 @@ bool resolve_shift(int64_t batch, int64_t T, int64_t C, int dtype, int code, sca
     if (!scanscam::cl_shift_built(esize, l->vec, l->steps, l->kind) || l->waves < 1 ||
         l->waves > scanscam::cl_max_waves(l->vec, l->steps, l->kind, compute_size(dtype)))
         return false;
-    return size_cl(batch, T, dtype, l->vec - 1, l) == SCANSCAM_OK && scanscam::cl_shift_built(esize, l->vec, l->steps, l->kind);  // (one tile: a walk)
+    return size_cl(batch, T, dtype, false, l->vec - 1, l) == SCANSCAM_OK && scanscam::cl_shift_built(esize, l->vec, l->steps, l->kind);  // (one tile: a walk)
 }
 
 // When an automatic call takes them. `reserve` is what it does without them, the cost model's plan: lanes of one channel, or

@@ -11,6 +11,38 @@ from test_hip_channels_last import as_rows, prev_abs, rel_err
 from test_hip_staged import BAR, check, scan_pair
 
 
+def through_super_tiles(gpu, shape, dtype, direction, plan):
+    """Whether a call of more tiles than waves goes through the chain of super-tiles: it publishes their aggregates, in the
+    last words of the workspace, all of which are alike to begin with."""
+    batch, T, C = shape
+    tiles, L = -(-T // (plan.unroll * plan.waves)), hip.lib()
+    assert tiles > plan.waves
+    supers = batch * -(-C // (64 * plan.vec)) * -(-tiles // plan.waves) * 64 * plan.vec * (6 if dtype == torch.float64 else 2)
+    n = hip.workspace_bytes_cl(*shape, dtype, direction, plan)
+    ws, t = torch.empty(n, dtype=torch.uint8, device=gpu), [torch.rand(shape, device=gpu).to(dtype) for _ in range(5)]
+    p, tail = [x.data_ptr() for x in t], (*shape, hip._dtype_code(dtype), ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream, plan)
+    rc = L.scanscam_scan_fwd_cl(*p[:3], *tail) if direction == hip.FORWARD else L.scanscam_scan_bwd_cl(*p, *tail)
+    assert rc == 0
+    words = ws.view(torch.int64)[-supers:]
+    return bool((words != words[-1]).any())
+
+
+@pytest.mark.gpu
+def test_where_the_chain_takes_over(gpu):
+    """8 tiles per wave, 1024 steps per wave, 2048 workgroups (16 single 16-bit channels backwards: 896), no fp64."""
+    f32, bf16, f64, fwd, bwd = torch.float32, torch.bfloat16, torch.float64, hip.FORWARD, hip.BACKWARD
+    for shape, dtype, steps, waves, chain in [
+            ((2, 2048, 70), f32, 4, 8, (False, False)), ((2, 2049, 70), f32, 4, 8, (True, True)),
+            ((1, 8192, 64), f32, 16, 8, (False, False)), ((1, 8193, 64), bf16, 16, 8, (True, True)),
+            ((227, 288, 64), f32, 4, 8, (False, False)), ((228, 288, 64), f32, 4, 8, (True, True)),
+            ((99, 576, 64), bf16, 16, 4, (False, False)), ((100, 576, 64), bf16, 16, 4, (False, True)),
+            ((100, 576, 64), f32, 16, 4, (False, False)), ((100, 288, 64), bf16, 8, 4, (False, False)),
+            ((2, 2048, 70), f64, 4, 8, (True, True))]:
+        plan = hip.Plan(mode=hip.MODE_LOOKBACK, vec=1, unroll=steps, waves=waves)
+        print(f"case {shape} {dtype} {plan}", flush=True)
+        assert tuple(through_super_tiles(gpu, shape, dtype, d, plan) for d in (fwd, bwd)) == chain, (shape, dtype, steps, waves)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", list(BAR))
 @pytest.mark.parametrize("vec,steps,waves", [(1, 4, 8), (1, 4, 3), (2, 4, 4), (1, 8, 1)])
