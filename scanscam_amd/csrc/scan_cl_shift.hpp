@@ -192,7 +192,8 @@ struct ClShiftSteps {
         // Whole vectors: up to the group's last, of which a tail group (M elements in the last lane) holds only so many.
         const int whole_end = ln.tail && PH < VEC - M ? ln.last : ln.last + 1;
         if (ln.lane >= (PH == 0 ? 0 : 1) && ln.lane < whole_end) {
-            if constexpr (CACHED_STORES) BV::store_cached(whole, res, ln.c, off);
+            if constexpr (CACHED_STORES && !BUF) BV::store_cached_elem_aligned(whole, res, ln.c, off);  // (no resource: see lead_at)
+            else if constexpr (CACHED_STORES) BV::store_cached(whole, res, ln.c, off);
             else BV::store(whole, res, ln.c, off);
         }
         if (PH != 0 || ln.tail) {

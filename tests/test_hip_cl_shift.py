@@ -2,7 +2,10 @@
 Channels-last calls of odd channel counts whose channels move between neighbouring lanes: parity with the CPU oracle at
 the edges of its groups (63 vectors of 4 channels, 2 in float64), spans and tiles, and its route.
 """
+import os
 import random
+import shutil
+import subprocess
 
 import pytest
 import torch
@@ -92,6 +95,29 @@ def test_where_the_route_lies():
         assert code(*shape, f32, hip.FORWARD) == 0, shape
     for bad in (-1, -(64 * 5 + 2 * 4), -(64 * 12 + 8), -(64 * 16 + 9), -(64 * 8), -(64 * 8 + 2 * 16), -(1 << 20)):
         assert hip.resolve_plan_cl(64, 2048, 1001, f32, hip.FORWARD, hip.Plan(waves_per_row=bad)).waves_per_row == 0, bad
+
+
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="no hipcc")
+def test_no_buffer_resource_starts_between_vectors(tmp_path):
+    """The walk backwards addresses its tensors from a constant number of elements before a time step, i.e. from any element:
+    buffer instructions, which want their resource to start on 4 bytes at least, have no place there."""
+    csrc = os.path.join(os.path.dirname(os.path.abspath(hip.__file__)), "csrc")
+    kernel = "template __global__ void scanscam::scan_cl_kernel<{}, {}, {}, true, scanscam::cl_max_threads({}, {}), false, {}>(scanscam::ClArgs);\n"
+    source = tmp_path / "walks.hip"
+    source.write_text('#include "scan_launch.hpp"\n' + "".join(
+        kernel.format(t, v, s, v, s, m) for t, v, ms in (("__bf16", 4, (1, 3)), ("_Float16", 4, (1,)), ("float", 4, (1,)), ("double", 2, (1,)))
+        for s in (4, 8) for m in ms))
+    done = subprocess.run([HIPCC, "-O3", "-std=c++17", "--offload-arch=gfx950", "--offload-device-only", "-S", "-Xclang", "-target-feature",
+                           "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument", f"-I{csrc}",
+                           f"-I{os.path.join(csrc, '../../include')}", str(source), "-o", str(tmp_path / "walks.s")],
+                          capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0, done.stderr
+    code = (tmp_path / "walks.s").read_text()
+    assert code.count("global_load") > 100 and code.count("global_store") > 100
+    assert "buffer_load" not in code and "buffer_store" not in code
 
 
 def test_calls_that_the_cost_model_s_plan_runs_faster_keep_it():
