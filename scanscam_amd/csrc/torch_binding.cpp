@@ -16,11 +16,13 @@
 // runs.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/record_function.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -286,6 +288,7 @@ struct ScanBackward : torch::autograd::Function<ScanBackward> {
     }
     static variable_list backward(torch::autograd::AutogradContext *ctx, variable_list out_grads)
     {
+        RECORD_FUNCTION("ScanBackward", c10::ArrayRef<const c10::IValue>{});
         const variable_list saved = ctx->get_saved_variables();
         variable_list grads;
         Call c;
@@ -300,6 +303,36 @@ struct ScanBackward : torch::autograd::Function<ScanBackward> {
         return grads;
     }
 };
+
+// What Python sees of the node (output.grad_fn): the name and the attributes that a Python function's node has, on top of a
+// C++ node's.
+using ScanNode = torch::autograd::CppNode<ScanBackward>;
+
+ScanNode *scan_node(PyObject *self) { return static_cast<ScanNode *>(reinterpret_cast<torch::autograd::THPCppFunction *>(self)->cdata.get()); }
+
+PyObject *node_name(PyObject *, PyObject *) { return PyUnicode_FromString("ScanBackward"); }
+
+PyObject *node_saved_tensors(PyObject *self, void *)
+{
+    HANDLE_TH_ERRORS
+    const variable_list saved = scan_node(self)->ctx_.get_saved_variables();
+    pybind11::tuple out(saved.size());
+    for (size_t i = 0; i < saved.size(); i++) out[i] = pybind11::reinterpret_steal<pybind11::object>(THPVariable_Wrap(saved[i]));
+    return out.release().ptr();
+    END_HANDLE_TH_ERRORS
+}
+
+PyObject *node_needs_input_grad(PyObject *self, void *)
+{
+    ScanNode *node = scan_node(self);
+    return PyTuple_Pack(2, node->should_compute_output(0) ? Py_True : Py_False, node->should_compute_output(1) ? Py_True : Py_False);
+}
+
+PyMethodDef node_methods[] = {{"name", node_name, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyGetSetDef node_properties[] = {{"saved_tensors", node_saved_tensors, nullptr, nullptr, nullptr},
+                                 {"needs_input_grad", node_needs_input_grad, nullptr, nullptr, nullptr},
+                                 {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyTypeObject node_type;
 
 PyObject *scan(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 {
@@ -318,6 +351,7 @@ PyObject *scan(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     bool covered;
     {
         pybind11::gil_scoped_release no_gil;
+        RECORD_FUNCTION("Scan", c10::ArrayRef<const c10::IValue>{});
         {
             const at::AutoGradMode no_grad(false);
             covered = execute(c);
@@ -340,7 +374,7 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t nargs) { return 
 PyObject *backward(PyObject *, PyObject *const *args, Py_ssize_t nargs) { return run(args, nargs, 3, 2); }
 
 // bind(fwd_rows, bwd_rows, fwd_cl, bwd_cl, ws_rows, ws_cl, strerror, backward): addresses of the library's entry points, and
-// the Python function (gate, output, out_grad) -> (gate_grad, value_grad).
+// the Python function (gate, output, out_grad) -> (gate_grad, value_grad). Returns the type of the autograd nodes.
 PyObject *bind(PyObject *, PyObject *args)
 {
     unsigned long long a[7];
@@ -355,7 +389,20 @@ PyObject *bind(PyObject *, PyObject *args)
     ws_cl = reinterpret_cast<decltype(ws_cl)>(a[5]);
     error_text = reinterpret_cast<decltype(error_text)>(a[6]);
     fwd_rows = reinterpret_cast<decltype(fwd_rows)>(a[0]);
-    Py_RETURN_NONE;
+    static const bool registered = [] {
+        // The type of a node whose class has none of its own.
+        const std::shared_ptr<torch::autograd::Node> node(new ScanNode, torch::autograd::deleteNode);
+        PyObject *plain_node = torch::autograd::functionToPyObject(node);
+        node_type.tp_base = Py_TYPE(plain_node);
+        Py_INCREF(node_type.tp_base);
+        Py_DECREF(plain_node);
+        torch::autograd::_initFunctionPyTypeObject(node_type, "ScanBackward", node_properties, node_methods);
+        torch::autograd::registerCppFunction(typeid(ScanNode), &node_type);
+        return true;
+    }();
+    (void)registered;
+    Py_INCREF(&node_type);
+    return reinterpret_cast<PyObject *>(&node_type);
 }
 
 PyMethodDef methods[] = {{"scan", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan)), METH_FASTCALL, nullptr},

@@ -151,10 +151,11 @@ def _bind_native(lib: ctypes.CDLL):
         warnings.warn(f"{_binding.__file__} was built against PyTorch {built}, not {torch.__version__}: not used; "
                       "rebuild it with `make -C scanscam_amd/csrc binding`", RuntimeWarning, stacklevel=2)
         return None
-    _binding.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (
+    node_type = _binding.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (
         lib.scanscam_scan_fwd_strided, lib.scanscam_scan_bwd_strided, lib.scanscam_scan_fwd_cl_strided,
         lib.scanscam_scan_bwd_cl_strided, lib.scanscam_workspace_bytes, lib.scanscam_workspace_bytes_cl,
         lib.scanscam_strerror)), _backward_in_python)
+    torch.autograd.graph.Node.register(node_type)
     return _binding
 
 

@@ -151,6 +151,52 @@ def test_same_outcomes_as_the_python_function(gpu):
 
 
 @pytest.mark.gpu
+def test_the_node_shows_what_the_python_function_s_shows(gpu):
+    """Name, saved tensors and which inputs need gradients; what a profile calls the two passes."""
+    a, b, gh = (torch.rand(4, 50, device=gpu) for _ in range(3))
+    for mask in ((True, True), (True, False), (False, True)):
+        seen = []
+        for fn in (scan, op.Scan.apply):
+            x, y = a.detach().requires_grad_(mask[0]), b.detach().requires_grad_(mask[1])
+            h = fn(x, y)
+            node = h.grad_fn
+            gate, output = node.saved_tensors
+            assert gate is x and torch.equal(output, h) and output.grad_fn is node
+            assert isinstance(node, torch.autograd.graph.Node) and repr(h).endswith("grad_fn=<ScanBackward>)")
+            edges = [None if n is None else type(n).__name__ for n, _ in node.next_functions]
+            shown = [type(node).__name__, node.name(), node.needs_input_grad, node.metadata, edges]
+            h.backward(gh)
+            with pytest.raises(RuntimeError, match="second time"):
+                node.saved_tensors
+            seen.append(shown)
+        assert seen[0] == seen[1]
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(gpu)):
+        h = scan(*leaves(a, b))
+    assert is_native(h) and all(t.is_cuda for t in h.grad_fn.saved_tensors)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as profile:
+        x, y = leaves(a, b)
+        torch.autograd.grad(scan(x, y), (x, y), gh)
+    assert {"Scan", "ScanBackward"} <= {e.name for e in profile.events()}
+
+
+@pytest.mark.gpu
+def test_compiled_autograd(gpu):
+    """A backward pass that is traced into a graph calls the node as it is."""
+    from torch._dynamo import compiled_autograd
+
+    a, b, gh = (torch.rand(4, 50, device=gpu) for _ in range(3))
+    results = []
+    for fn in (scan, op.Scan.apply):
+        torch._dynamo.reset()
+        x, y = leaves(a, b)
+        h = fn(x, y)
+        with compiled_autograd._enable(torch.compile(backend="eager")):
+            h.backward(gh)
+        results.append((x.grad, y.grad))
+    assert all(torch.equal(p, q) for p, q in zip(*results))
+
+
+@pytest.mark.gpu
 def test_threads_and_streams(gpu):
     """Steps of several threads, each on a stream of its own, and an error of the library raised from the engine's thread."""
     g = torch.Generator(device=gpu).manual_seed(6)
