@@ -65,6 +65,8 @@ HBM_PEAK_GBPS = 8000.0
 # kernel sources it was taken with (a digest); with other sources the figure is reported as null.
 TRAFFIC_PROFILE = os.path.join("profiles", "scan_row_f32_fwd_bwd_8x2048x4096_pmc_traffic.txt")
 KERNEL_SOURCES = ("scan_kernels.hpp", "scan_launch.hpp", "scan_api.hip", "scan_f32.hip")
+CHANNELS_LAST_SOURCES = ("scan_kernels.hpp", "scan_cl_kernels.hpp", "scan_cl_shift.hpp", "scan_staged_kernels.hpp", "scan_cl_plan.hpp",
+                         "scan_cl_model.inc", "scan_launch.hpp", "scan_api.hip", "scan_f32.hip", "scan_bf16.hip", "scan_f16.hip", "scan_f64.hip")
 METRIC = "scan HBM GB/s and % of MI355X peak, fwd and fwd+bwd, fp32 [B,C,T]"
 FWD_BYTES = {8: 24, 4: 12, 2: 6}
 BWD_BYTES = {8: 40, 4: 20, 2: 10}
@@ -72,12 +74,13 @@ BWD_BYTES = {8: 40, 4: 20, 2: 10}
 GRAPH_BELOW_MS = 0.025
 
 
-def kernel_sources_digest():
-    """sha256 over the sources the row kernels are built from (what a traffic profile is valid for)."""
+def kernel_sources_digest(names=KERNEL_SOURCES):
+    """sha256 over the sources the row kernels are built from (what a traffic profile is valid for), or over those of the
+    channels-last kernels."""
     import hashlib
 
     d = hashlib.sha256()
-    for name in KERNEL_SOURCES:
+    for name in names:
         with open(os.path.join(ROOT, "scanscam_amd", "csrc", name), "rb") as f:
             d.update(f.read())
     return d.hexdigest()
@@ -585,6 +588,16 @@ def channels_last_workload(spec, args, hip, torch):
     }))
 
 
+def plan_text(p):
+    """A resolved channels-last plan in words: the kernel that runs, not the plan in reserve beside it."""
+    if p.waves_per_row > 0:
+        return f"staged parts={p.waves_per_row}"
+    if p.waves_per_row < 0:
+        code = -p.waves_per_row
+        return f"moved {'tiles' if code % 2 else 'walk'} steps={code // 64} waves={code // 2 % 32}"
+    return f"mode={p.mode} vec={p.vec} steps={p.unroll} waves={p.waves}"
+
+
 def channels_last_table(args, hip, torch):
     """Contiguous [B, T, C] tensors scanned along T (the layout of the reference's transposed kernels,
     scanscam/cuda.py:69-95): its timing shape, many-channel and many-batch shapes in fp32 and bf16, channel
@@ -598,15 +611,13 @@ def channels_last_table(args, hip, torch):
     for B, T, C, dtype in shapes:
         f_ms, b_ms, nsets = time_channels_last(B, T, C, dtype, max(20, args.steps // 2), max(3, args.warmup // 2), hip, torch)
         n, esize = B * T * C, torch.empty(0, dtype=dtype).element_size()
-        short = lambda p: (f"staged parts={p.waves_per_row}" if p.waves_per_row  # noqa: E731
-                           else f"mode={p.mode} vec={p.vec} steps={p.unroll} waves={p.waves}")
         out[f"{B}x{T}x{C}_{str(dtype).replace('torch.', '')}"] = {
             "fwd_us": round(f_ms * 1e3, 1), "bwd_us": round(b_ms * 1e3, 1),
             "fwd_frac": round(FWD_BYTES[esize] * n / (f_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),
             "bwd_frac": round(BWD_BYTES[esize] * n / (b_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),
             "buffer_sets": nsets,
-            "plan_fwd": short(hip.resolve_plan_cl(B, T, C, dtype, hip.FORWARD)),
-            "plan_bwd": short(hip.resolve_plan_cl(B, T, C, dtype, hip.BACKWARD)),
+            "plan_fwd": plan_text(hip.resolve_plan_cl(B, T, C, dtype, hip.FORWARD)),
+            "plan_bwd": plan_text(hip.resolve_plan_cl(B, T, C, dtype, hip.BACKWARD)),
         }
     return out
 

@@ -78,7 +78,8 @@ enum {
  *                  channels-last: parts of time in which SCANSCAM_MODE_STAGED takes the call where it can,
  *                  the other fields then being the plan where it cannot; below zero: the negative of
  *                  64 * steps + 2 * waves + (1: tiles of time, 0: a walk), the launch in which lanes move channels
- *                  between each other (odd C) takes the call where it can
+ *                  between each other (odd C) takes the call where it can, whatever the other fields
+ *                  force, and they are again the plan where it cannot (also where the number is no launch)
  *   spin_limit     kernels that wait for another workgroup's carry poll at most this many times
  *                  (0 = 2^20, about a second); a wait that expires sets word 1 of the workspace to 1
  *                  and poisons the affected outputs with NaN instead of spinning for ever
@@ -272,9 +273,9 @@ int scanscam_resolve_plan(int64_t rows, int64_t T, int dtype, int direction, con
  * wave and tile, waves per workgroup. waves_per_row > 0: the call takes SCANSCAM_MODE_STAGED by itself, in that
  * many parts, and the other fields are the plan in reserve for tensors the staged kernel cannot run (zero
  * waves_per_row to force that one). waves_per_row < 0: the call moves channels between neighbouring lanes (odd C of
- * large dense tensors; struct scanscam_plan), with the same meaning of the other fields. Handed back, the plan runs what the automatic call runs, bit for bit. A
- * SCANSCAM_MODE_STAGED plan has nothing to resolve and is refused. No counterpart in the reference, whose kernel has
- * one launch shape (scanscam/cuda.py:69-95 passes channels_per_block only).
+ * large dense tensors; struct scanscam_plan), with the same meaning of the other fields. Handed back, the plan runs
+ * what the automatic call runs, bit for bit. A SCANSCAM_MODE_STAGED plan has nothing to resolve and is refused. No counterpart in the reference,
+ * whose kernel has one launch shape (scanscam/cuda.py:69-95 passes channels_per_block only).
  */
 int scanscam_resolve_plan_cl(int64_t batch, int64_t T, int64_t C, int dtype, int direction,
                              const scanscam_plan *plan, scanscam_plan *out);

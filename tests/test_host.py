@@ -327,3 +327,13 @@ def test_the_learned_correction_is_trained_printed_and_read_back(tmp_path):
     assert abs(float(r.correct(x)[0]) - np.log(1.2)) < 0.05
     wild = [1e9] * plan_fit.N_FEATURES
     assert abs(float(r.correct(wild)[0])) <= plan_fit.RESIDUAL_LIMIT
+
+
+def test_bench_names_the_channels_last_kernel_that_runs():
+    import bench
+
+    plan = lambda *s: bench.plan_text(hip.resolve_plan_cl(*s, torch.float32, hip.FORWARD))  # noqa: E731
+    assert plan(64, 2048, 1001) == "moved walk steps=8 waves=4" and plan(2, 15698, 1589) == "moved tiles steps=8 waves=8"
+    assert plan(2048, 512, 40).startswith("staged parts=") and plan(64, 2048, 1024).startswith("mode=2 vec=4 ")
+    digests = {bench.kernel_sources_digest(), bench.kernel_sources_digest(bench.CHANNELS_LAST_SOURCES)}
+    assert len(digests) == 2
