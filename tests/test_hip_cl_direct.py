@@ -8,7 +8,7 @@ import torch
 import oracle
 from scanscam_amd import hip
 from test_hip_channels_last import as_rows, prev_abs, rel_err
-from test_hip_staged import BAR, check, scan_pair
+from test_hip_staged import BAR, check, check_special_values, scan_pair
 
 
 def through_super_tiles(gpu, shape, dtype, direction, plan):
@@ -47,7 +47,8 @@ def test_where_the_chain_takes_over(gpu):
 @pytest.mark.parametrize("dtype", list(BAR))
 @pytest.mark.parametrize("vec,steps,waves", [(1, 4, 8), (1, 4, 3), (2, 4, 4), (1, 8, 1)])
 def test_runs_of_tiles(gpu, dtype, vec, steps, waves):
-    """2 tiles to 8 per wave and one more, the last one whole, of one step, and short; the same bits every time."""
+    """2 tiles to 8 per wave and one more, the last one whole, of one step, and short; the same bits every time. The chain
+    takes the count beyond, and all of fp64."""
     plan = hip.Plan(mode=hip.MODE_LOOKBACK, vec=vec, unroll=steps, waves=waves)
     tile = steps * waves
     for tiles in sorted({2, 9, waves, waves + 1, 2 * waves + 1, 5 * waves, 8 * waves, 8 * waves + 1} - {1}):
@@ -85,3 +86,35 @@ def test_gates_above_one_before_the_first_value(gpu, dtype, steps, waves, tiles,
     want_ga, want_gb = oracle.bwd(as_rows(a), as_rows(h), as_rows(x))
     assert rel_err(as_rows(gb), want_gb) <= BAR[dtype]
     assert rel_err(as_rows(ga), want_ga, prev_abs(as_rows(h))) <= BAR[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("vec,steps,waves,tiles", [(1, 4, 8, 20), (2, 4, 4, 9), (4, 4, 8, 3)])
+def test_values_that_are_no_numbers(gpu, dtype, vec, steps, waves, tiles):
+    plan = hip.Plan(mode=hip.MODE_LOOKBACK, vec=vec, unroll=steps, waves=waves)
+    check_special_values(gpu, (3, tiles * steps * waves - 1, 132), dtype, plan, [0, 1, 63, 64, 65, 70, 127, 128, 130, 131])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_an_expired_wait_ends_and_is_reported(gpu, dtype):
+    """One poll per wait: every wave still ends, and either no wait expired and the result is the usual one, or the flag is
+    raised and there are NaN; what is neither NaN nor the usual result there is none."""
+    shape, L = (4, 2048, 256), hip.lib()
+    g = torch.Generator(device=gpu).manual_seed(29)
+    x, y = (torch.rand(shape, generator=g, device=gpu).to(dtype) for _ in range(2))
+    plan = hip.Plan(mode=hip.MODE_LOOKBACK, vec=1, unroll=4, waves=8)
+    assert not through_super_tiles(gpu, shape, dtype, hip.FORWARD, plan)
+    good = hip.transposed_linear_scan_forward(x, y, plan=plan)
+    once = hip.Plan(mode=hip.MODE_LOOKBACK, vec=1, unroll=4, waves=8, spin_limit=1)
+    n = hip.workspace_bytes_cl(*shape, dtype, hip.FORWARD, once)
+    ws, out = torch.empty(n, dtype=torch.uint8, device=gpu), torch.empty_like(x)
+    rc = L.scanscam_scan_fwd_cl(x.data_ptr(), y.data_ptr(), out.data_ptr(), *shape, hip._dtype_code(dtype), ws.data_ptr(), n,
+                                torch.cuda.current_stream().cuda_stream, once)
+    assert rc == 0
+    expired = int(ws.view(torch.int64)[1].item()) != 0
+    print(f"case one poll {dtype}: {'expired' if expired else 'no wait expired'}", flush=True)
+    assert bool(torch.isnan(out).any()) == expired
+    assert torch.equal(out[~torch.isnan(out)], good[~torch.isnan(out)])
+    assert torch.equal(hip.transposed_linear_scan_forward(x, y, plan=plan), good)

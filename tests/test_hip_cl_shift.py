@@ -13,16 +13,23 @@ import torch
 import oracle
 from scanscam_amd import hip
 from test_hip_channels_last import as_rows, prev_abs, rel_err
-from test_hip_staged import BAR, check, scan_pair
+from test_hip_staged import BAR, check, check_special_values, scan_pair
 
 
 def forced(steps, waves, tiles):
     return hip.Plan(waves_per_row=-(64 * steps + 2 * waves + tiles))
 
 
+def runs(dtype, steps, waves, tiles, T):
+    """Whether these lanes are built for the launch: 16 steps only for 16-bit types, and only in tiles, two of them at least
+    (the tiles start up to a vector's channels in steps early)."""
+    vec = 2 if dtype == torch.float64 else 4
+    return steps < 16 or (dtype in (torch.bfloat16, torch.float16) and tiles == 1 and T + vec - 1 > steps * waves)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", list(BAR))
-@pytest.mark.parametrize("steps,waves,tiles", [(4, 1, 0), (4, 3, 0), (8, 8, 0), (4, 2, 1), (8, 8, 1), (16, 4, 1)])  # (16: 16-bit types, others the plan in reserve)
+@pytest.mark.parametrize("steps,waves,tiles", [(4, 1, 0), (4, 3, 0), (8, 8, 0), (4, 2, 1), (8, 8, 1), (16, 4, 1), (16, 8, 1), (8, 4, 1), (4, 8, 1)])
 def test_edges_of_groups_and_spans(gpu, dtype, steps, waves, tiles):
     """Either odd remainder of C, a last group of two vectors up to a whole one, every phase of a batch element's first
     step, two time steps up to several tiles; outputs of nothing but their own elements."""
@@ -30,10 +37,11 @@ def test_edges_of_groups_and_spans(gpu, dtype, steps, waves, tiles):
     plan = forced(steps, waves, tiles)
     tile = steps * waves
     for C in (63 * vec + 1, 63 * vec + 3, 70 * vec - 1, 126 * vec - 1, 126 * vec + 1):
-        if C % 2 == 0:
-            continue
         for batch, T in ((5, 2), (3, tile - 1), (2, tile + 1), (1, 3 * tile + 2)):
             print(f"case shift {dtype} C={C} batch={batch} T={T} {steps}x{waves} tiles={tiles}", flush=True)
+            for direction in (hip.FORWARD, hip.BACKWARD):  # (others run the plan in reserve)
+                taken = hip.resolve_plan_cl(batch, T, C, dtype, direction, plan).waves_per_row
+                assert taken == (plan.waves_per_row if runs(dtype, steps, waves, tiles, T) else 0)
             inputs, (a, b, gh), results = scan_pair(gpu, (batch, T, C), dtype, plan, seed=C + T)
             check(inputs, results, dtype)
     # The last shape again, into the middle of buffers, and a forward pass in place.
@@ -84,6 +92,35 @@ def test_automatic_route(gpu, dtype, shape):
     got = hip.transposed_linear_scan_forward(off, b)
     assert torch.equal(got, hip.transposed_linear_scan_forward(off, b, plan=plans[0]))
     assert rel_err(as_rows(got[:2]), as_rows(results[0][:2])) <= 2 * BAR[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,shape,code", [(torch.bfloat16, (8, 3000, 741), -1033), (torch.float16, (3, 1497, 2345), -521),
+                                              (torch.bfloat16, (36, 290, 1003), -272), (torch.float32, (6, 1087, 3393), -273)])
+def test_automatic_route_backwards(gpu, dtype, shape, code):
+    """Calls that take these lanes backwards only."""
+    plans = [hip.resolve_plan_cl(*shape, dtype, d) for d in (hip.FORWARD, hip.BACKWARD)]
+    assert [p.waves_per_row for p in plans] == [0, code]
+    print(f"case automatic {dtype} {shape} {plans[1]}", flush=True)
+    _, (a, b, gh), results = scan_pair(gpu, shape, dtype, None)
+    reserve = hip.Plan(mode=plans[1].mode, vec=plans[1].vec, unroll=plans[1].unroll, waves=plans[1].waves)
+    same = hip.transposed_linear_scan_backward(a, results[0], gh, plan=plans[1])
+    other = hip.transposed_linear_scan_backward(a, results[0], gh, plan=reserve)
+    for got, x, y in zip(results[1:], same, other):
+        assert torch.equal(got, x)
+        floor = prev_abs(as_rows(results[0][:2])) if got is results[1] else None
+        assert rel_err(as_rows(got[:2]), as_rows(y[:2]), floor) <= 2 * BAR[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", list(BAR))
+@pytest.mark.parametrize("steps,waves,tiles", [(4, 8, 0), (8, 4, 0), (8, 4, 1)])
+def test_values_that_are_no_numbers_stay_in_their_channels(gpu, dtype, steps, waves, tiles):
+    """At the edges of groups, lanes and steps, whose vectors neighbours load as well."""
+    vec = 2 if dtype == torch.float64 else 4
+    shape = (3, 3 * steps * waves + 2, 126 * vec + 1)  # three groups of 43 vectors, the last of 41
+    channels = [0, 1, vec, 43 * vec - 1, 43 * vec, 86 * vec - 1, 86 * vec, shape[2] - 2, shape[2] - 1]
+    check_special_values(gpu, shape, dtype, forced(steps, waves, tiles), channels)
 
 
 def test_where_the_route_lies():
@@ -157,7 +194,7 @@ def test_tiles_multiply_no_more_gates_than_the_plan_in_reserve():
 def test_gates_above_one_after_the_last_gradient(gpu):
     """Backwards over 563 steps of gates of 1.5 before the first output gradient other than zero: the gradients stay zero
     there, also in calls wide enough for tiles."""
-    shape, last = (5, 683, 2421), 120
+    shape, last = (4, 1228, 2937), 665
     print(f"case {shape} {hip.resolve_plan_cl(*shape, torch.bfloat16, hip.BACKWARD)}", flush=True)
     g = torch.Generator().manual_seed(8)
     a = torch.rand(shape, generator=g)

@@ -39,6 +39,33 @@ def check(inputs, results, dtype):
     assert rel_err(ga, want_ga, prev_abs(h)) <= BAR[dtype]
 
 
+def check_special_values(gpu, shape, dtype, plan, channels):
+    """Infinities and NaN in one step each of some channels: the outputs that are no numbers are those of the recurrence, and
+    all others as with numbers in their place. Gates of 0.95 and more: no product over the time steps is zero, which times an
+    infinity is NaN where the recurrence stays infinite."""
+    print(f"case special {dtype} {shape} {plan}", flush=True)
+    g, T = torch.Generator().manual_seed(4), shape[1]
+    a = (0.95 + 0.05 * torch.rand(shape, generator=g, dtype=torch.float64)).to(dtype)
+    b, h, gh = (torch.randn(shape, generator=g, dtype=torch.float64).to(dtype) for _ in range(3))
+    for i, c in enumerate(channels):
+        value, t = (float("nan"), float("inf"), float("-inf"))[i % 3], (0, 1, T // 2, T - 2, T - 1)[i % 5]
+        b[0, t, c] = gh[0, t, c] = value
+        a[1, t, c] = float("nan")
+        h[2, t, c] = value
+    with np.errstate(invalid="ignore"):
+        want_h, (want_ga, want_gb) = oracle.fwd(as_rows(a), as_rows(b)), oracle.bwd(as_rows(a), as_rows(h), as_rows(gh))
+    got_h = hip.transposed_linear_scan_forward(a.to(gpu), b.to(gpu), plan=plan)
+    got_ga, got_gb = hip.transposed_linear_scan_backward(a.to(gpu), h.to(gpu), gh.to(gpu), plan=plan)
+    for got, want in ((got_h, want_h), (got_ga, want_ga), (got_gb, want_gb)):
+        got = as_rows(got)
+        numbers = np.isfinite(want)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isfinite(got), numbers)
+        assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        floor = prev_abs(as_rows(h))[numbers] if want is want_ga else None
+        # (gates near 1 add up the roundings of a thousand steps and more)
+        assert rel_err(got[numbers], want[numbers], None if floor is None else np.where(np.isfinite(floor), floor, 1)) <= 4 * BAR[dtype]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", list(BAR))
 @pytest.mark.parametrize("C", [2, 3, 17, 40, 91, 127, 129, 255, 256])

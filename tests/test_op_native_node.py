@@ -2,6 +2,7 @@
 The op's native autograd node (csrc/torch_binding.cpp) against the Python function it stands in for: the same gradients, and
 the same outcome of everything the engine, hooks and modes do to a node.
 """
+import ctypes
 import threading
 
 import pytest
@@ -42,11 +43,14 @@ def test_same_gradients_as_the_python_function(gpu, dtype):
 
 
 def outcome(fn):
+    """("values", the tensors' values) or ("raises", type and message); a test's own assertions are not an outcome."""
     try:
         r = fn()
-        return tuple(t.cpu().tolist() for t in r) if isinstance(r, tuple) else r
+        return "values", tuple(t.cpu().tolist() for t in r) if isinstance(r, tuple) else r
+    except AssertionError:
+        raise
     except Exception as e:  # noqa: BLE001
-        return type(e), str(e).split("\n")[0][:60]
+        return "raises", type(e), str(e).split("\n")[0][:60]
 
 
 @pytest.mark.gpu
@@ -141,11 +145,14 @@ def test_same_outcomes_as_the_python_function(gpu):
             assert not is_native(h)
             return torch.autograd.grad(h, (x, y), gh)
 
-    calls = [lambda f: twice(f, True), lambda f: twice(f, False), lambda f: changed(f, 0), lambda f: changed(f, 1), second_order,
-             saved_elsewhere, left_on_the_cpu, hooked, checkpointed, checked, vmapped, inside_a_transform, dual, unused, under_a_mode]
-    for i, call in enumerate(calls):
-        got, want = outcome(lambda: call(scan)), outcome(lambda: call(op.Scan.apply))
-        assert got == want, (i, got if isinstance(got[0], type) else "values", want if isinstance(want[0], type) else "values")
+    calls = {"values": [lambda f: twice(f, True), saved_elsewhere, hooked, checkpointed, checked, unused, under_a_mode],
+             "raises": [lambda f: twice(f, False), lambda f: changed(f, 0), lambda f: changed(f, 1), second_order, left_on_the_cpu,
+                        vmapped, inside_a_transform, dual]}
+    for kind, cases in calls.items():
+        for i, call in enumerate(cases):
+            got, want = outcome(lambda: call(scan)), outcome(lambda: call(op.Scan.apply))
+            assert got[0] == want[0] == kind, (kind, i, got[:2] if got[0] == "raises" else "", want[:2] if want[0] == "raises" else "")
+            assert got == want, (kind, i, got if kind == "raises" else "values", want if kind == "raises" else "values")
     assert grads_off(scan) == grads_off(op.Scan.apply)
     assert is_native(scan(*leaves(a, b)))
 
@@ -197,8 +204,45 @@ def test_compiled_autograd(gpu):
 
 
 @pytest.mark.gpu
+def test_errors_on_the_engine_s_thread(gpu):
+    """The library's errors, and memory that cannot be had, in a backward pass: exceptions of the caller, as the Python function
+    raises them; the next pass works."""
+    a, b, gh = (torch.rand(4, 50, device=gpu) for _ in range(3))
+    lib = hip.lib()
+    names = ["scan_fwd_strided", "scan_bwd_strided", "scan_fwd_cl_strided", "scan_bwd_cl_strided", "workspace_bytes",
+             "workspace_bytes_cl", "strerror"]
+    entries = [ctypes.cast(getattr(lib, f"scanscam_{n}"), ctypes.c_void_p).value for n in names]
+    refuse = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: 1)  # an error code for every call
+    x, y = leaves(a, b)
+    h = scan(x, y)
+    try:
+        hip._native.bind(entries[0], ctypes.cast(refuse, ctypes.c_void_p).value, *entries[2:], hip._backward_in_python)
+        with pytest.raises(RuntimeError) as raised:
+            torch.autograd.grad(h, (x, y), gh, retain_graph=True)
+    finally:
+        hip._native.bind(*entries, hip._backward_in_python)
+    assert str(raised.value).startswith(f"scanscam_scan_bwd_strided: {hip.strerror(1)}")
+    want = torch.autograd.grad(op.Scan.apply(x, y), (x, y), gh)
+    assert all(torch.equal(p, q) for p, q in zip(torch.autograd.grad(h, (x, y), gh), want))
+
+    x, y = (torch.rand(64, 1 << 20, device=gpu).requires_grad_() for _ in range(2))
+    steps = [(fn(x, y), torch.rand_like(x)) for fn in (scan, op.Scan.apply)]
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)
+    try:
+        for h, g in steps:
+            with pytest.raises(torch.OutOfMemoryError):
+                torch.autograd.grad(h, (x, y), g)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    x, y = leaves(a, b)
+    assert all(torch.equal(p, q) for p, q in zip(torch.autograd.grad(scan(x, y), (x, y), gh), want))
+
+
+@pytest.mark.gpu
 def test_threads_and_streams(gpu):
-    """Steps of several threads, each on a stream of its own, and an error of the library raised from the engine's thread."""
+    """Steps of several threads, each on a stream of its own."""
     g = torch.Generator(device=gpu).manual_seed(6)
     sets = [[torch.rand(8, 64, 4096, generator=g, device=gpu) for _ in range(3)] for _ in range(4)]
     want = []
@@ -209,13 +253,16 @@ def test_threads_and_streams(gpu):
     bad = []
 
     def work(i):
-        with torch.cuda.stream(torch.cuda.Stream()) as _:
-            for _ in range(5):
-                x, y = leaves(*sets[i][:2])
-                got = torch.autograd.grad(scan(x, y), (x, y), sets[i][2])
-                torch.cuda.current_stream().synchronize()
-                if not all(torch.equal(p, q) for p, q in zip(got, want[i])):
-                    bad.append(i)
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(5):
+                    x, y = leaves(*sets[i][:2])
+                    got = torch.autograd.grad(scan(x, y), (x, y), sets[i][2])
+                    torch.cuda.current_stream().synchronize()
+                    if not all(torch.equal(p, q) for p, q in zip(got, want[i])):
+                        bad.append(i)
+        except BaseException as e:  # noqa: BLE001
+            bad.append((i, e))
 
     threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
     for t in threads:
