@@ -274,8 +274,8 @@ int scanscam_resolve_plan(int64_t rows, int64_t T, int dtype, int direction, con
  * many parts, and the other fields are the plan in reserve for tensors the staged kernel cannot run (zero
  * waves_per_row to force that one). waves_per_row < 0: the call moves channels between neighbouring lanes (odd C of
  * large dense tensors; struct scanscam_plan), with the same meaning of the other fields. Handed back, the plan runs
- * what the automatic call runs, bit for bit. A SCANSCAM_MODE_STAGED plan has nothing to resolve and is refused. No counterpart in the reference,
- * whose kernel has one launch shape (scanscam/cuda.py:69-95 passes channels_per_block only).
+ * what the automatic call runs, bit for bit. A SCANSCAM_MODE_STAGED plan has nothing to resolve and is refused. No
+ * counterpart in the reference, whose kernel has one launch shape (scanscam/cuda.py:69-95 passes channels_per_block only).
  */
 int scanscam_resolve_plan_cl(int64_t batch, int64_t T, int64_t C, int dtype, int direction,
                              const scanscam_plan *plan, scanscam_plan *out);

@@ -625,9 +625,9 @@ int run(bool rev, const void *a, const void *x, const void *h, void *y0, void *y
 // more per super-tile; each of its waves reads up to 8 aggregates of every channel. In calls of few rounds of workgroups
 // that wait is most of the time (GPU time, us forward / backward, buffers in rotation): fp32 [1, 2541, 295] 12.7 / 13.9 -> 10.2 /
 // 11.4, [10, 1083, 128] 12.8 / 14.7 -> 10.0 / 12.0, [3, 2000, 512] 14.5 / 18.7 -> 13.1 / 17.3, bf16 [2, 1643, 96] 12.4 / 13.9 ->
-// 9.6 / 10.8, [6, 574, 256] 9.6 / 10.6 -> 8.3 / 8.6; 225 and 192 calls in fp32 and 16 bits 0.87 and 0.89 x in the mean, at most 1.04 and 1.06
-// (profiles/direct_lookback_random_shapes.txt), and larger ones gain little ([8, 4096, 512] 45.0 / 73.0 -> 43.7 / 72.5). It
-// ends where
+// 9.6 / 10.8, [6, 574, 256] 9.6 / 10.6 -> 8.3 / 8.6; 225 and 192 calls in fp32 and 16 bits 0.87 and 0.89 x in the mean, at most
+// 1.04 and 1.06 (profiles/direct_lookback_random_shapes.txt), and larger ones gain little ([8, 4096, 512] 45.7 / 74.4 -> 44.0 /
+// 73.0). It ends where
 //   - more workgroups cover each other's waits, and the aggregates they read are what is left: [25, 1696, 384], 2100 workgroups,
 //     0.97 / 0.99 x, [64, 1024, 333] backward, 3072 of them, 1.06 x, [24, 2048, 3072] backward, 18432, 543 -> 569, bf16 [90, 2048,
 //     514] backward, 14400, 243 -> 256 us: 2048 at most, and 896 for 16 single 16-bit channels backwards (30 calls with fewer
@@ -890,7 +890,7 @@ bool resolve_shift(int64_t batch, int64_t T, int64_t C, int dtype, int code, sca
 //   (16 bits up to 1.31 and 1.19, fp32 1.28 and 1.21, fp64 1.13; up to 384 16 bits forwards 0.76 to 1.12, fp32 0.87 to 1.04 and
 //   0.85 to 1.11). Beyond, 16 bits 0.76 to 1.04 and 0.74 to 1.01, fp32 0.84 to 0.98 and 0.84 to 1.04, fp64 0.76 to 1.06 and
 //   0.76 to 1.08.
-//   fp32 [64, 2048, 1001] 345 / 567 -> 304 / 507 us, bf16 199 / 333 -> 151 / 263.
+//   fp32 [64, 2048, 1001] 346 / 573 -> 299 / 505 us, bf16 197 / 344 -> 158 / 263 us.
 //   Tiles, for fewer. fp32 below 40 pairs, 8 steps x 8 waves: 0.70 to 1.05 forwards (with 24 pairs and more from 512 MiB on;
 //   below up to 1.14), 0.68 to 1.02 backwards; up to 96 backwards, 4 x 8 where the reserve has 16 steps a wave 0.83 to 1.01 (8
 //   steps, 0.88 to 1.08; forwards 0.89 to 1.29). 16 bits backwards, which is bound by its accesses more than by bytes, from 96

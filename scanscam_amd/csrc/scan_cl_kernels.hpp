@@ -751,8 +751,9 @@ __global__ __launch_bounds__(MAXT) void scan_cl_packed_kernel(const ClArgs p)
 //   carry   from S_m through the aggregates of tiles 0..j-1.
 // The last tile of a super-tile publishes (SA, SB) as soon as it holds all W
 // tile aggregates, and SI = fma(SA, S_m, SB) once S_m is known.
-// With DIRECT (few tiles per row-group, a kernel of its own: the code beside the chain costs that up to 7 %) there are no super-tiles: the waves share out ALL tiles before this one, each
-// composes its run of aggregates, and every lane folds the waves' pairs in order.
+// With DIRECT (few tiles per row-group, a kernel of its own: the code beside the chain costs that up to 7 %) there are no
+// super-tiles: the waves share out ALL tiles before this one, each composes its run of aggregates, and every lane folds the
+// waves' pairs in order (or, where a run's product of gates is not finite, the tiles' one by one).
 //
 // Workspace, in 64-bit words: ticket counter of row-group r at word
 // r * kCounterStride, word 1 raised on a timed-out wait; then per (row-group,

@@ -14,13 +14,14 @@
 // phases whichever span it is, known at compile time from M = C mod VEC: no shift amount is ever a register. The
 // virtual steps are the identity, like those past the end.
 //
-// fp32 [64, 2048, 1001], 4 waves of 8 steps, forward / backward: 342 / 569 us at any element, 304 / 509 us here (bf16 197 / 342 ->
-// 155 / 274 us), where the bytes take 257 / 433 us at C = 1024. Reads are those of the algorithm to 0.1 % and writes 3 % more
-// (FETCH_SIZE, WRITE_SIZE); a wave issues 1.3 / 1.5 times the vector instructions. What is left is the wave's accesses, still
-// nine lines for the bytes of eight (C = 992, on whole lines, takes 288 / 497 us as well). Loads go through the caches' normal
-// policy, because the line that two channel groups share is in the L2 when the second one asks for it (313 / 528 us with
-// non-temporal ones); stores of whole vectors are non-temporal in fp32 (341 / 565 us with cached loads and stores) and fp64
-// and cached in 16 bits (164 / 286 -> 155 / 270 us). Loading a tile ahead is level in fp32 (298 / 519 us).
+// fp32 [64, 2048, 1001], 4 waves of 8 steps, forward / backward: 346 / 573 us at any element, 299 / 505 us here (bf16 197 / 344 ->
+// 158 / 263 us; GPU time, buffers in rotation), where the bytes take 275 / 435 us at C = 1024. Reads are those of the algorithm
+// to 0.1 % and writes 3 % more (FETCH_SIZE, WRITE_SIZE); a wave issues 1.3 / 1.5 times the vector instructions. What is left is
+// the wave's accesses, still nine lines for the bytes of eight (C = 992, on whole lines, takes 289 / 493 us as well). Loads go
+// through the caches' normal policy, because the line that two channel groups share is in the L2 when the second one asks for it
+// (in one run with 304 / 509 us: 313 / 528 with non-temporal ones); stores of whole vectors are non-temporal in fp32 (there 341
+// / 565 with cached loads and stores) and fp64 and cached in 16 bits (bf16 in one run 164 / 286 -> 155 / 270 us). Loading a tile
+// ahead is level in fp32 (there 298 / 519).
 //
 // The vector after a group's last one is needed too, so a wave owns at most 63 vectors of channels per step. Vectors that
 // hold foreign elements are only ever read, and only those with an element of the tensor in them (the host sends dense
@@ -89,7 +90,7 @@ struct ClShiftSteps {
     }
     // A tensor's base for a span whose first step is t lies `lead` elements before that step: on the vector border before it
     // for buffer instructions; for global ones, whose base may be any address, a constant number that keeps every offset
-    // from being negative (one scalar addition fewer per access: bf16 [64, 2048, 1001] backward 280 -> 265 us).
+    // from being negative (one scalar addition fewer per access: bf16 [64, 2048, 1001] backward in one run 280 -> 265 us).
     static __device__ __forceinline__ int phase_at(const ClLane<ST> &ln, int t) { return (ln.phase0 + t % VEC * M) % VEC; }
     static __device__ __forceinline__ int lead_at(const ClLane<ST> &ln, int t)
     {
