@@ -222,10 +222,9 @@ bool modes_active()
     return at::impl::PythonTorchFunctionTLS::stack_len() > 0 || c10::impl::TorchDispatchModeTLS::any_modes_set();
 }
 
-// Runs a call whose inputs are in c.t; false if it is not covered. The library's errors are exceptions.
-bool execute(Call &c)
+// Runs an accepted call; false if it is not covered after all. The library's errors are exceptions.
+bool perform(Call &c)
 {
-    if (!c.accept()) return false;
     const c10::DeviceGuard guard(c.t[0].device());
     c.allocate();
     if (!c.lay_out()) return false;
@@ -234,6 +233,9 @@ bool execute(Call &c)
         throw std::runtime_error(std::string("scanscam_scan_") + (c.inputs == 2 ? "fwd" : "bwd") + (c.cl ? "_cl" : "") + "_strided: " + error_text(rc));
     return true;
 }
+
+// The same for a call of which only the inputs are there, in c.t.
+bool execute(Call &c) { return c.accept() && perform(c); }
 
 PyObject *run(PyObject *const *args, Py_ssize_t nargs, int inputs, int outputs)
 {
@@ -348,13 +350,14 @@ PyObject *scan(PyObject *, PyObject *const *args, Py_ssize_t nargs)
         c.t[i] = THPVariable_Unpack(args[i]);
         if (c.t[i]._fw_grad(/*level=*/0).defined()) Py_RETURN_NONE;
     }
+    if (!c.accept()) Py_RETURN_NONE;
     bool covered;
     {
         pybind11::gil_scoped_release no_gil;
         RECORD_FUNCTION("Scan", c10::ArrayRef<const c10::IValue>{});
         {
             const at::AutoGradMode no_grad(false);
-            covered = execute(c);
+            covered = perform(c);
         }
         if (covered && at::GradMode::is_enabled() && (c.t[0].requires_grad() || c.t[1].requires_grad()))
             c.t[2] = ScanBackward::apply(c.t[0], c.t[1], &c);

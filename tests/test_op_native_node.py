@@ -186,6 +186,14 @@ def test_the_node_shows_what_the_python_function_s_shows(gpu):
     assert {"Scan", "ScanBackward"} <= {e.name for e in profile.events()}
 
 
+def test_calls_left_to_python_are_profiled_once():
+    x, y = (torch.rand(4, 50, requires_grad=True) for _ in range(2))
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as profile:
+        scan(x, y).sum().backward()
+    names = [e.name for e in profile.events()]
+    assert names.count("Scan") == 1 and names.count("ScanBackward") == 1
+
+
 @pytest.mark.gpu
 def test_compiled_autograd(gpu):
     """A backward pass that is traced into a graph calls the node as it is."""
