@@ -651,7 +651,6 @@ int size_cl(int64_t batch, int64_t T, int dtype, bool rev, int virtual_steps, sc
     const int64_t tile_steps = (int64_t)l->waves * l->steps;
     const int64_t tiles = (T + virtual_steps + tile_steps - 1) / tile_steps;
     const int64_t vals = (int64_t)l->vec * kWave * value_words(dtype);  // words of one [vec][64] array of values
-    l->lds_bytes = (size_t)(l->kind == 2 ? 7 : 4) * l->waves * l->vec * kWave * compute_size(dtype);
     l->ws_bytes = 0;
     l->segments = 1;
     if (l->kind == 2) {
@@ -668,6 +667,8 @@ int size_cl(int64_t batch, int64_t T, int dtype, bool rev, int virtual_steps, sc
     }
     l->grid = rowgroups * l->segments;
     l->direct = l->kind == 2 && l->shift == 0 && direct_lookback(*l, elem_size(dtype), rev);
+    const int arrays = l->kind == 2 ? scanscam::cl_lookback_arrays(l->direct) : 4;
+    l->lds_bytes = (size_t)arrays * l->waves * l->vec * kWave * compute_size(dtype);
     if (l->grid >= (int64_t(1) << 31)) return SCANSCAM_EINVAL;
     return SCANSCAM_OK;
 }

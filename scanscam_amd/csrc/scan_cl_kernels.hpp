@@ -133,16 +133,19 @@ template <typename ST, int VEC> struct ClAccess<ST, VEC, true> {
         else if constexpr (kBytes == 4) return __builtin_amdgcn_raw_buffer_load_b32(r, lane_off, step_off, AUX);
         else return __builtin_amdgcn_raw_buffer_load_b16(r, lane_off, step_off, AUX);
     }
+    // 16-byte stores take no scalar offset: the compiler counts such a store's data as read by the time the next vector
+    // instruction writes the registers that hold it, and it was not (8 x 4 and 8 x 8 16-bit elements forwards, the next
+    // step's values copied over them by v_mov_b64: single vectors of single steps wrong in two of their words).
     static __device__ __forceinline__ void store_cached(raw_t v, Base r, unsigned lane_off, unsigned step_off)
     {
-        if constexpr (kBytes == 16) __builtin_amdgcn_raw_buffer_store_b128(v, r, lane_off, step_off, 0);
+        if constexpr (kBytes == 16) __builtin_amdgcn_raw_buffer_store_b128(v, r, lane_off + step_off, 0, 0);
         else if constexpr (kBytes == 8) __builtin_amdgcn_raw_buffer_store_b64(v, r, lane_off, step_off, 0);
         else if constexpr (kBytes == 4) __builtin_amdgcn_raw_buffer_store_b32(v, r, lane_off, step_off, 0);
         else __builtin_amdgcn_raw_buffer_store_b16(v, r, lane_off, step_off, 0);
     }
     static __device__ __forceinline__ void store(raw_t v, Base r, unsigned lane_off, unsigned step_off)
     {
-        if constexpr (kBytes == 16) __builtin_amdgcn_raw_buffer_store_b128(v, r, lane_off, step_off, 2);
+        if constexpr (kBytes == 16) __builtin_amdgcn_raw_buffer_store_b128(v, r, lane_off + step_off, 0, 2);
         else if constexpr (kBytes == 8) __builtin_amdgcn_raw_buffer_store_b64(v, r, lane_off, step_off, 2);
         else if constexpr (kBytes == 4) __builtin_amdgcn_raw_buffer_store_b32(v, r, lane_off, step_off, 2);
         else __builtin_amdgcn_raw_buffer_store_b16(v, r, lane_off, step_off, 2);
@@ -200,6 +203,9 @@ __device__ __forceinline__ typename Vec<ST, VEC>::raw_t cl_shift_down(typename V
     }
 }
 
+// Whether a walk issues the next tile's loads as soon as this tile is folded (see scan_cl_kernel).
+template <typename ST, int VEC, int S> constexpr bool cl_ahead() { return sizeof(ST) == 2 && VEC <= 4 && VEC * S <= 32; }
+
 template <typename ST, int VEC, int S, bool REV, bool APPLY, typename CT, bool SPLIT = false, bool RAGGED = false>
 struct ClSteps {
     using V = Vec<ST, VEC>;
@@ -208,27 +214,54 @@ struct ClSteps {
     using BV = ClAccess<ST, VEC, !RAGGED && cl_buffered<ST, VEC, S, REV, SPLIT>()>;
     using Base = typename BV::Base;
 
-    CT g[S][VEC], v[S][VEC];
-    raw_t rh[(REV && APPLY) ? S : 1];
-    int tau0;   // scan position of the first step
-    int limit;  // scan positions from here on do not exist
-    int tb;     // time step the resources' bases point at: no access of this wave lies before it
-    // issue() may run for the next span of steps while the folded one still awaits apply(): what it sets is kept
-    // apart (n_*) until fold() takes it over. The raw gates and values need no second copy, fold() has used them up.
-    raw_t n_rh[(REV && APPLY) ? S : 1];
-    int n_tau0, n_limit, n_tb;
+    // PACKED: 16-bit gates and values stay as they are stored from fold() to apply(), each of which widens them, in half the
+    // registers of the widened ones. In tiles of time where that lets a second workgroup of 8 waves onto a CU: 32 elements per
+    // lane backwards (130 -> 102 registers; bf16 [8, 4096, 2048] 2 x 16: 176 -> 155 us, fp16 [1, 18877, 1920] 97 -> 76 us) and 64
+    // forwards (192 -> 126; 4 x 16: 98 -> 87 us, 68 -> 58 us); 32 forwards (104 -> 72, no whole workgroup more) run 1.0 to 1.13 x
+    // and 64 backwards (222 -> 158) 1.0 to 1.09 x with it. In walks that do not load ahead, 16-byte lanes 0.94 to 1.0 x.
+    static constexpr bool PACKED = sizeof(ST) == 2 && VEC > 1 && (SPLIT ? VEC * S == (REV ? 32 : 64) : !cl_ahead<ST, VEC, S>());
+    raw_t ra[S], rx[S], rh[(REV && APPLY) ? S : 1];
+    CT g[PACKED ? 1 : S][VEC], v[PACKED ? 1 : S][VEC];
+    int tau0;  // scan position of the first step
+    // issue() may run for the next span of steps while the folded one still awaits apply(): what it brings is kept apart until
+    // fold() takes it over.
+    raw_t n_ra[S], n_rx[S], n_rh[(REV && APPLY) ? S : 1];
+    int n_tau0;
 
-    // Byte distance of time step t from the base, for a tensor with `stride` elements per step.
-    __device__ __forceinline__ unsigned step_off(int t, int stride) const
+    // Every access of a span lies a whole number of time steps from the span's base: step s, `d` steps later in time, lies
+    // rel(s, d) of them after it. A step that does not exist (past the row's end; backwards also a[t+1] at the first step and
+    // h[t-1] at the last) reads the nearest one that does and is put right in fold(), so an access takes two scalar
+    // instructions, a product with a constant and a minimum or maximum, where each step's own conditions, selects and offsets
+    // took 8 to 14 (16 x 1 fp32 elements backwards: 1662 -> 880 scalar instructions in the kernel). Over 160 random calls of 4 M
+    // elements and more, buffers in rotation, with PACKED: 0.98 x forwards (0.82 to 1.03), 0.97 x backwards (0.77 to 1.08).
+    static constexpr int rel(int s, int d = 0) { return (REV ? S - s : s) + d; }
+    static __device__ __forceinline__ int base_step(int first, int T)
     {
-        return (unsigned)(t - tb) * (unsigned)stride * (unsigned)sizeof(ST);
+        if (!REV) return first < T - 1 ? first : T - 1;
+        const int low = T - 1 - first - S;  // h[t-1] of the last step
+        return low > -(S + 1) ? low : -(S + 1);
     }
+    // Steps from the base that exist: forwards up to `most`, backwards from `least` on (and a[t+1] up to `most`).
+    struct Range { int least, most; };
+    static __device__ __forceinline__ Range range(int tb, int T)
+    {
+        const int left = T - 1 - tb;
+        return {tb < 0 ? -tb : 0, left < S + 1 ? left : S + 1};
+    }
+    // Byte offset from the base for a tensor with `stride` elements per step.
+    static __device__ __forceinline__ unsigned clamped(int s, int d, int stride, Range r)
+    {
+        const unsigned step = (unsigned)stride * (unsigned)sizeof(ST);
+        const unsigned at = (unsigned)rel(s, d) * step, least = (unsigned)r.least * step, most = (unsigned)r.most * step;
+        if (!REV) return at < most ? at : most;
+        if (s == 0 && d > 0) return at < most ? at : most;  // (least <= S, or the whole span does not exist and least == most)
+        return at > least ? at : least;
+    }
+    // How many of the span's steps exist.
+    static __device__ __forceinline__ int count(int first, int T) { return T - first < S ? T - first : S; }
 
-    // Whether a step exists, and whether its shifted operands do, is the same for every lane of the
-    // wave (tau0 and limit are wave-uniform): scalar conditions, scalar offsets. A lane without
-    // channels (C no multiple of the workgroup's channels) computes on channel 0's data like any
-    // other lane and only its stores are masked, so no per-lane mask is kept per step.
-    raw_t ra[S], rx[S];  // what issue() brought; dead once fold() has run
+    // A lane without channels (C no multiple of the workgroup's channels) computes on channel 0's data like any
+    // other lane and only its stores are masked.
 
     // Loads through the caches' normal policy instead of non-temporal: element-aligned lanes of 4-byte types straddle line
     // borders that the next lane, wave or workgroup needs again, and non-temporal lines are the first to go. 16-byte lanes
@@ -241,64 +274,53 @@ struct ClSteps {
     static constexpr bool CHOSEN_LOADS = RAGGED && sizeof(ST) == 4 && sizeof(raw_t) == 8;
 
     // Issues every load of the wave's S steps; nothing waits for them here.
-    __device__ __forceinline__ void issue(const ClLane<ST> &ln, int T, int first_step, int limit_)
+    __device__ __forceinline__ void issue(const ClLane<ST> &ln, int T, int first_step)
     {
         if constexpr (CHOSEN_LOADS) {
             if (ln.cached_loads) {
                 // (The compiler would merge the two copies of the loads, and drop what tells them apart.)
                 asm volatile("" ::: "memory");
-                issue_as<0>(ln, T, first_step, limit_);
+                issue_as<0>(ln, T, first_step);
                 asm volatile("" ::: "memory");
                 return;
             }
         }
-        issue_as<CACHED_LOADS ? 0 : 2>(ln, T, first_step, limit_);
+        issue_as<CACHED_LOADS ? 0 : 2>(ln, T, first_step);
     }
 
-    template <int LOADS> __device__ __forceinline__ void issue_as(const ClLane<ST> &ln, int T, int first_step, int limit_)
+    template <int LOADS> __device__ __forceinline__ void issue_as(const ClLane<ST> &ln, int T, int first_step)
     {
         n_tau0 = first_step;
-        n_limit = limit_;
-        // Forwards the wave touches times tau0 ... tau0+S-1; backwards T-1-tau for the same tau, plus
-        // a[t+1] and h[t-1]: nothing before T-1-(tau0+S-1)-1. Clamped into the tensor.
-        const int lowest = REV ? T - 1 - (n_tau0 + S - 1) - 1 : n_tau0;
-        n_tb = lowest < 0 ? 0 : (lowest > T - 1 ? T - 1 : lowest);
-        const int tb = n_tb, tau0 = n_tau0, limit = n_limit;  // this function's own view (step_off below takes tb from here)
-        auto step_off = [tb](int t, int stride) { return (unsigned)(t - tb) * (unsigned)stride * (unsigned)sizeof(ST); };
+        const int tb = base_step(first_step, T);
+        const Range in = range(tb, T);
         const Base res_a = BV::base(ln.a + (int64_t)tb * ln.pa), res_x = BV::base(ln.x + (int64_t)tb * ln.px);
         const Base res_h = BV::base(ln.h + (int64_t)tb * ln.ph);
-        // Every load is issued unconditionally (a step that does not exist reads the base): no
-        // branch separates the loads, so all of a wave's S x streams loads are in flight before the
-        // first one is waited for.
+        // Every load is issued unconditionally: no branch separates the loads, so all of a wave's S x streams loads are
+        // in flight before the first one is waited for.
 #pragma unroll
         for (int s = 0; s < S; s++) {
-            const int tau = tau0 + s;
-            const int t = REV ? T - 1 - tau : tau;
-            const bool in = tau < limit;
-            // The gate of step t is a[t] forwards and a[t+1] backwards (0 past the end); h[-1] = 0.
-            const bool a_in = in && (!REV || t + 1 < T), h_in = in && t > 0;
-            const unsigned off_x = in ? step_off(t, ln.px) : 0u;
-            const unsigned off_a = a_in ? step_off(REV ? t + 1 : t, ln.pa) : 0u;
+            // The gate of step t is a[t] forwards and a[t+1] backwards.
+            const unsigned off_a = clamped(s, REV ? 1 : 0, ln.pa, in), off_x = clamped(s, 0, ln.px, in);
             if (APPLY) {
-                ra[s] = BV::template load<LOADS>(res_a, ln.c, off_a);
-                rx[s] = BV::template load<LOADS>(res_x, ln.c, off_x);
-                if (REV) n_rh[s] = BV::template load<LOADS>(res_h, ln.c, h_in ? step_off(t - 1, ln.ph) : 0u);
+                n_ra[s] = BV::template load<LOADS>(res_a, ln.c, off_a);
+                n_rx[s] = BV::template load<LOADS>(res_x, ln.c, off_x);
+                if (REV) n_rh[s] = BV::template load<LOADS>(res_h, ln.c, clamped(s, -1, ln.ph, in));
             } else {
-                ra[s] = BV::template load<0>(res_a, ln.c, off_a);
-                rx[s] = BV::template load<0>(res_x, ln.c, off_x);
+                n_ra[s] = BV::template load<0>(res_a, ln.c, off_a);
+                n_rx[s] = BV::template load<0>(res_x, ln.c, off_x);
             }
         }
     }
 
-    // Folds the issued steps to one affine pair per channel (and keeps gate and value per step for apply()).
+    // Folds the issued steps to one affine pair per channel.
     __device__ __forceinline__ void fold(int T, CT (&A)[VEC], CT (&B)[VEC], int shift = 0)
     {
         tau0 = n_tau0;
-        limit = n_limit;
-        tb = n_tb;
-        if (REV && APPLY) {
 #pragma unroll
-            for (int s = 0; s < S; s++) rh[s] = n_rh[s];
+        for (int s = 0; s < S; s++) {
+            ra[s] = n_ra[s];
+            rx[s] = n_rx[s];
+            if (REV && APPLY) rh[s] = n_rh[s];
         }
         if (RAGGED && shift != 0) {  // the last lane of a time step: its window's components into place
 #pragma unroll
@@ -308,6 +330,36 @@ struct ClSteps {
                 if (REV && APPLY) rh[s] = cl_shift_down<ST, VEC>(rh[s], shift);
             }
         }
+        if constexpr (!PACKED) {
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                V::unpack(ra[s], g[s]);
+                V::unpack(rx[s], v[s]);
+            }
+        }
+        // Steps that do not exist are the identity; the gate past the end and h[-1] are zero. The same for the whole wave.
+        const int n = count(tau0, T);
+        if (n < S || (REV && (tau0 == 0 || tau0 + S == T))) {
+            CT ones[VEC];
+#pragma unroll
+            for (int k = 0; k < VEC; k++) ones[k] = CT(1);
+            const raw_t one = V::pack(ones), zero = V::zero_raw();
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                const bool in = s < n, past = REV && s == 0 && tau0 == 0;
+                if constexpr (PACKED) {
+                    ra[s] = in ? (past ? zero : ra[s]) : one;
+                    rx[s] = in ? rx[s] : zero;
+                } else {
+#pragma unroll
+                    for (int k = 0; k < VEC; k++) {
+                        g[s][k] = in ? (past ? CT(0) : g[s][k]) : CT(1);
+                        v[s][k] = in ? v[s][k] : CT(0);
+                    }
+                }
+                if (REV && APPLY) rh[s] = tau0 + s == T - 1 ? zero : rh[s];
+            }
+        }
 #pragma unroll
         for (int k = 0; k < VEC; k++) {
             A[k] = CT(1);
@@ -315,26 +367,24 @@ struct ClSteps {
         }
 #pragma unroll
         for (int s = 0; s < S; s++) {
-            const int tau = tau0 + s;
-            const int t = REV ? T - 1 - tau : tau;
-            const bool in = tau < limit, a_in = in && (!REV || t + 1 < T);
-            CT fa[VEC], fx[VEC];
-            V::unpack(ra[s], fa);
-            V::unpack(rx[s], fx);
+            CT G[VEC], X[VEC];
+            if constexpr (PACKED) {
+                V::unpack(ra[s], G);
+                V::unpack(rx[s], X);
+                // (The compiler would keep the widened ones for apply() instead of widening again.)
+                asm volatile("" : "+v"(ra[s]), "+v"(rx[s]));
+            }
 #pragma unroll
             for (int k = 0; k < VEC; k++) {
-                g[s][k] = in ? (a_in ? fa[k] : CT(0)) : CT(1);
-                v[s][k] = in ? fx[k] : CT(0);
-                B[k] = fma_(g[s][k], B[k], v[s][k]);
-                A[k] = A[k] * g[s][k];
+                B[k] = PACKED ? fma_(G[k], B[k], X[k]) : fma_(g[s][k], B[k], v[s][k]);
+                A[k] = A[k] * (PACKED ? G[k] : g[s][k]);
             }
         }
     }
 
-    __device__ __forceinline__ void load_fold(const ClLane<ST> &ln, int T, int first_step, int limit_,
-                                              CT (&A)[VEC], CT (&B)[VEC])
+    __device__ __forceinline__ void load_fold(const ClLane<ST> &ln, int T, int first_step, CT (&A)[VEC], CT (&B)[VEC])
     {
-        issue(ln, T, first_step, limit_);
+        issue(ln, T, first_step);
         fold(T, A, B, ln.shift);
     }
 
@@ -366,6 +416,7 @@ struct ClSteps {
     // One copy of the store loop per policy, chosen once per call (the choice is the same for the whole launch).
     __device__ __forceinline__ void apply(const ClLane<ST> &ln, int T, CT (&mine)[VEC])
     {
+        if (!ln.c_ok) return;
         if constexpr (!RAGGED && sizeof(raw_t) <= 8) {
             if (ln.cached) {
                 apply_as<true>(ln, T, mine);
@@ -377,28 +428,29 @@ struct ClSteps {
 
     template <bool CACHED> __device__ __forceinline__ void apply_as(const ClLane<ST> &ln, int T, CT (&mine)[VEC])
     {
+        const int tb = base_step(tau0, T), n = count(tau0, T);
         const Base res_y0 = BV::base(ln.y0 + (int64_t)tb * ln.py0), res_y1 = BV::base(ln.y1 + (int64_t)tb * ln.py1);
+        const unsigned step_y0 = (unsigned)ln.py0 * (unsigned)sizeof(ST), step_y1 = (unsigned)ln.py1 * (unsigned)sizeof(ST);
 #pragma unroll
         for (int s = 0; s < S; s++) {
-            const int tau = tau0 + s;
-            const int t = REV ? T - 1 - tau : tau;
-            const bool in = tau < limit, h_in = in && t > 0;
-            CT out[VEC];
+            if (s < n) {
+                CT G[VEC], X[VEC], out[VEC];
+                if (PACKED) {
+                    V::unpack(ra[s], G);
+                    V::unpack(rx[s], X);
+                }
 #pragma unroll
-            for (int k = 0; k < VEC; k++) {
-                mine[k] = fma_(g[s][k], mine[k], v[s][k]);
-                out[k] = mine[k];
-            }
-            if (!REV) {
-                if (in && ln.c_ok) put<CACHED>(V::pack(out), res_y0, ln, step_off(t, ln.py0));
-            } else {
-                CT fh[VEC], ga[VEC];
-                V::unpack(rh[s], fh);
+                for (int k = 0; k < VEC; k++) {
+                    mine[k] = PACKED ? fma_(G[k], mine[k], X[k]) : fma_(g[s][k], mine[k], v[s][k]);
+                    out[k] = mine[k];
+                }
+                put<CACHED>(V::pack(out), res_y0, ln, (unsigned)rel(s) * step_y0);
+                if (REV) {
+                    CT fh[VEC], ga[VEC];
+                    V::unpack(rh[s], fh);
 #pragma unroll
-                for (int k = 0; k < VEC; k++) ga[k] = out[k] * (h_in ? fh[k] : CT(0));
-                if (in && ln.c_ok) {
-                    put<CACHED>(V::pack(out), res_y0, ln, step_off(t, ln.py0));
-                    put<CACHED>(V::pack(ga), res_y1, ln, step_off(t, ln.py1));
+                    for (int k = 0; k < VEC; k++) ga[k] = out[k] * fh[k];
+                    put<CACHED>(V::pack(ga), res_y1, ln, (unsigned)rel(s) * step_y1);
                 }
             }
         }
@@ -454,13 +506,13 @@ __device__ __forceinline__ ClLane<ST> cl_shift_lane(const ClArgs &p, int64_t bat
 template <typename ST, int VEC, bool RAGGED = false>
 __device__ __forceinline__ ClLane<ST> cl_lane(const ClArgs &p, int64_t batch_index, int group, int lane)
 {
-    const int64_t c0 = ((int64_t)group * kWave + lane) * VEC;  // first channel of this lane
+    const unsigned c0 = ((unsigned)group * kWave + (unsigned)lane) * VEC;  // first channel of this lane (C < 2^31 - 2^20)
     ClLane<ST> ln;
     ln.cached = p.cached_stores != 0;
     ln.cached_loads = p.cached_loads != 0;
-    ln.c_ok = c0 < p.C;
-    ln.shift = (RAGGED && ln.c_ok && c0 + VEC > p.C) ? (int)(c0 + VEC - p.C) : 0;  // C >= VEC: the host checks it
-    ln.c = ln.c_ok ? (unsigned)((c0 - ln.shift) * sizeof(ST)) : 0u;
+    ln.c_ok = c0 < (unsigned)p.C;
+    ln.shift = (RAGGED && ln.c_ok && c0 + VEC > (unsigned)p.C) ? (int)(c0 + VEC - (unsigned)p.C) : 0;  // C >= VEC: the host checks it
+    ln.c = ln.c_ok ? (c0 - (unsigned)ln.shift) * (unsigned)sizeof(ST) : 0u;
     ln.a = static_cast<const ST *>(p.a) + batch_index * p.sB[0];
     ln.x = static_cast<const ST *>(p.x) + batch_index * p.sB[1];
     ln.h = static_cast<const ST *>(p.h) + batch_index * p.sB[2];
@@ -522,15 +574,15 @@ __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
     // 151 / 228 -> 129 / 220 us, [32, 2048, 2048] 148 / 231 -> 131 / 222 us, [256, 1024, 1024] backward 447 -> 424 us,
     // [8, 4096, 2048] forward 93 -> 90 us. fp32 pays 30 to 120 registers for it and is level on average (+28 % to -10 %),
     // 16-byte lanes of 16-bit storage spill.
-    constexpr bool AHEAD = sizeof(ST) == 2 && VEC <= 4 && VEC * S <= 32;
+    constexpr bool AHEAD = cl_ahead<ST, VEC, S>();
     typename ClStepsOf<ST, VEC, S, REV, M, CT, false, RAGGED>::type steps;
-    if (AHEAD) steps.issue(ln, p.T, wave * S, p.T);
+    if (AHEAD) steps.issue(ln, p.T, wave * S);
     for (int it = 0; it < ntiles; it++) {
         CT *lds_A = lds + (it & 1) * 2 * plane, *lds_B = lds_A + plane;
         CT A[VEC], B[VEC], mine[VEC];
-        if (!AHEAD) steps.issue(ln, p.T, it * tile_steps + wave * S, p.T);
+        if (!AHEAD) steps.issue(ln, p.T, it * tile_steps + wave * S);
         steps.fold(p.T, A, B, ln.shift);
-        if (AHEAD && it + 1 < ntiles) steps.issue(ln, p.T, (it + 1) * tile_steps + wave * S, p.T);
+        if (AHEAD && it + 1 < ntiles) steps.issue(ln, p.T, (it + 1) * tile_steps + wave * S);
 #pragma unroll
         for (int k = 0; k < VEC; k++) mine[k] = carry[k];
         if (W > 1) {
@@ -760,7 +812,7 @@ __global__ __launch_bounds__(MAXT) void scan_cl_packed_kernel(const ClArgs p)
 // tile) its [VEC][64] published pairs; then per (row-group, super-tile) its
 // [VEC][64] pairs (SA, SB) and its [VEC][64] end values SI (encodings: Desc).
 // LDS: [W][7][VEC][64] values (per wave slot: wave pairs A, B; tile aggregates A, B;
-// super-tile SI, SA, SB).
+// super-tile SI, SA, SB); DIRECT: the first four of them.
 // ---------------------------------------------------------------------------
 template <typename CT, int VEC>
 __device__ __forceinline__ bool cl_fetch(const uint64_t *src, int lane, CT (&out)[VEC])
@@ -799,6 +851,8 @@ __device__ __forceinline__ void cl_publish_pair(uint64_t *dst, int lane, const C
     for (int k = 0; k < VEC; k++) D::store_pair(dst + (k * kWave + lane) * D::PAIR, a[k], b[k]);
 }
 
+constexpr int cl_lookback_arrays(bool direct) { return direct ? 4 : 7; }
+
 template <typename ST, int VEC, int S, bool REV, int MAXT, int M = 0, bool DIRECT = false>
 __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
 {
@@ -813,10 +867,10 @@ __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // wave-uniform: kept in a scalar register
     const int W = blockDim.x / kWave;
     const int groups = M != 0 ? p.groups : (p.C + kWave * VEC - 1) / (kWave * VEC);
-    const int64_t rowgroups = p.batch * groups;
+    const unsigned rowgroups = (unsigned)(p.batch * groups);  // below 2^31, like the grid (32 bits: 64-bit divisions are long)
     const int tpr = p.segments;              // tiles per row-group
     const int spr = (tpr + W - 1) / W;       // super-tiles per row-group
-    // LDS: per wave slot w, seven [VEC][64] arrays one after the other, so that an access is the slot's
+    // LDS: per wave slot w, its [VEC][64] arrays one after the other, so that an access is the slot's
     // base plus the lane (one register) and a constant.
     enum { exA, exB,   // pairs of this tile's waves
            tA, tB,     // aggregates of tiles 0..j-1 of the super-tile
@@ -825,7 +879,8 @@ __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
     constexpr int kVals = VEC * kWave * D::W;      // words of one [VEC][64] array of published values
     constexpr int kPairs = VEC * kWave * D::PAIR;  // ... of published pairs
     constexpr int kSup = kPairs + kVals;           // a super-tile: its pair (SA, SB), then its end value SI
-#define AT(arr, w, k) lds[((w) * 7 + (arr)) * (VEC * kWave) + (k) * kWave + lane]
+    constexpr int kArrays = cl_lookback_arrays(DIRECT);
+#define AT(arr, w, k) lds[((w) * kArrays + (arr)) * (VEC * kWave) + (k) * kWave + lane]
 
     // Row-groups of a workgroup's XCD: with p.xcd_order (time steps that are not whole 128-byte lines) a
     // contiguous run of them, so that channel groups that share a line meet in one L2 (as in scan_cl_kernel;
@@ -833,31 +888,31 @@ __global__ __launch_bounds__(MAXT) void scan_cl_lookback_kernel(const ClArgs p)
     // (xcd_order 2, any number of row-groups: XCD x = blockIdx % 8 owns the x-th run of them, of n / 8 rounded up or
     // down, and its workgroups go round that run; the host pads the grid to 8 shares of the longer run's size, so the
     // last workgroups of a shorter run's XCD have nothing to do.)
-    int64_t rg;
+    unsigned rg;
     if (p.xcd_order == 2) {
-        const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-        const int per = (int)((rowgroups + 7) / 8), rem = rowgroups % 8 == 0 ? 8 : (int)(rowgroups % 8);
-        const int mine = xcd < rem ? per : per - 1;
-        if (slot >= mine * tpr) return;
+        const unsigned xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
+        const unsigned per = (rowgroups + 7) / 8, rem = rowgroups % 8 == 0 ? 8 : rowgroups % 8;
+        const unsigned mine = xcd < rem ? per : per - 1;
+        if (slot >= mine * (unsigned)tpr) return;
         rg = (xcd < rem ? xcd * per : rem * per + (xcd - rem) * (per - 1)) + slot % mine;
     } else {
-        const int64_t rg0 = blockIdx.x % rowgroups;
-        rg = (p.xcd_order && rowgroups % 8 == 0) ? xcd_contiguous((int)rg0, (int)rowgroups) : rg0;
+        const unsigned rg0 = blockIdx.x % rowgroups;
+        rg = (p.xcd_order && rowgroups % 8 == 0) ? (unsigned)xcd_contiguous((int)rg0, (int)rowgroups) : rg0;
     }
     if (threadIdx.x == 0)
-        lds_ticket = __hip_atomic_fetch_add(reinterpret_cast<unsigned *>(p.ws + rg * kCounterStride), 1u,
+        lds_ticket = __hip_atomic_fetch_add(reinterpret_cast<unsigned *>(p.ws + (int64_t)rg * kCounterStride), 1u,
                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     const int tile = (int)__builtin_amdgcn_readfirstlane((int)lds_ticket);
-    const ClLane<ST> ln = cl_lane_of<ST, VEC, REV, false, M>(p, rg / groups, (int)(rg % groups), lane);
-    uint64_t *tiles = p.ws + rowgroups * kCounterStride + rg * (int64_t)tpr * kPairs;
-    uint64_t *supers = p.ws + rowgroups * kCounterStride + rowgroups * (int64_t)tpr * kPairs +
-                       rg * (int64_t)spr * kSup;
+    const ClLane<ST> ln = cl_lane_of<ST, VEC, REV, false, M>(p, rg / (unsigned)groups, (int)(rg % (unsigned)groups), lane);
+    uint64_t *descriptors = p.ws + (int64_t)rowgroups * kCounterStride;
+    uint64_t *tiles = descriptors + (int64_t)rg * tpr * kPairs;
+    uint64_t *supers = descriptors + (int64_t)rowgroups * tpr * kPairs + (int64_t)rg * spr * kSup;
     const int j = tile % W, m = tile / W;
 
     typename ClStepsOf<ST, VEC, S, REV, M, CT, true, false>::type cur;
     CT A[VEC], B[VEC];
-    cur.load_fold(ln, p.T, tile * W * S + wave * S, p.T, A, B);
+    cur.load_fold(ln, p.T, tile * W * S + wave * S, A, B);
 #pragma unroll
     for (int k = 0; k < VEC; k++) {
         AT(exA, wave, k) = A[k];

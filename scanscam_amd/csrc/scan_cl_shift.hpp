@@ -109,7 +109,7 @@ struct ClShiftSteps {
         return ph == 0 ? ln.c : (ph <= VEC - M ? ln.c_few : ln.c_all);
     }
 
-    __device__ __forceinline__ void issue(const ClLane<ST> &ln, int T, int first_step, int)
+    __device__ __forceinline__ void issue(const ClLane<ST> &ln, int T, int first_step)
     {
         n_first = first_step - ln.k0;
         const int lowest = REV ? T - 1 - (n_first + S - 1) - 1 : n_first;
@@ -175,9 +175,9 @@ struct ClShiftSteps {
         });
     }
 
-    __device__ __forceinline__ void load_fold(const ClLane<ST> &ln, int T, int first_step, int limit, CT (&A)[VEC], CT (&B)[VEC])
+    __device__ __forceinline__ void load_fold(const ClLane<ST> &ln, int T, int first_step, CT (&A)[VEC], CT (&B)[VEC])
     {
-        issue(ln, T, first_step, limit);
+        issue(ln, T, first_step);
         fold(T, A, B);
     }
 

@@ -112,6 +112,45 @@ def test_forced_plans(gpu, dtype):
     assert n > 90
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [1, 2, 4, 15, 16, 17, 33])
+def test_spans_that_end_inside_or_before_a_wave(gpu, dtype, T):
+    """Time steps that do not exist: a wave's last step, all but its first, whole waves of a tile, in dense tensors and in
+    views whose neighbouring memory is NaN. Bars as in test_forced_plans."""
+    bar = 1e-5 if dtype == torch.float32 else 1e-2
+    full = 4 if dtype == torch.float32 else 8
+    C = 64 * full + full
+    g = torch.Generator().manual_seed(T)
+    a = torch.rand((2, T, C), generator=g).to(dtype)
+    b, gh = (torch.randn((2, T, C), generator=g).to(dtype) for _ in range(2))
+    h = oracle.fwd(as_rows(a), as_rows(b))
+    hs = torch.from_numpy(h).mT.contiguous().to(dtype)
+    ga, gb = oracle.bwd(as_rows(a), as_rows(hs), as_rows(gh))
+
+    def view(t):  # the same values with NaN before, between and after the time steps
+        wide = torch.full((t.shape[0], T + 2, 2 * C), float("nan"), dtype=dtype, device=gpu)
+        inner = wide[:, 1:-1, C:]
+        inner.copy_(t)
+        return inner.mT
+
+    for vec in (full, full // 2, 1):
+        for steps in (4, 8, 16):
+            if vec == full and steps == 16:
+                continue
+            for mode in (hip.MODE_ROW, hip.MODE_LOOKBACK):
+                plan = hip.Plan(vec=vec, unroll=steps, waves=3 if vec < 8 else 2, mode=mode)
+                print(f"case cl spans {dtype} T={T} {plan}", flush=True)
+                results = [(hip.transposed_linear_scan_forward(a.to(gpu), b.to(gpu), plan=plan),
+                            *hip.transposed_linear_scan_backward(a.to(gpu), hs.to(gpu), gh.to(gpu), plan=plan))]
+                if T > 1:  # (one step alone is a row view)
+                    grads = hip.scan_backward(view(a), view(hs), view(gh), plan=plan)
+                    results.append((hip.scan_forward(view(a), view(b), plan=plan).mT, grads[0].mT, grads[1].mT))
+                for got_h, got_ga, got_gb in results:
+                    assert rel_err(as_rows(got_h), h) <= bar, plan
+                    assert rel_err(as_rows(got_gb), gb) <= bar, plan
+                    assert rel_err(as_rows(got_ga), ga, prev_abs(as_rows(hs))) <= bar, plan
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16, torch.float16])
 def test_element_aligned_lanes(gpu, dtype):
     """Wide lanes where C is no multiple of the lane's channels, or the tensors start at any element."""
