@@ -125,6 +125,12 @@ template <typename ST, int VEC> struct ClAccess<ST, VEC, true> {
         // No bounds: the offsets handed in are always inside the tensor.
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<ST *>(p), 0, -1, 0x00020000);
     }
+    // A base below kNowhere bytes long: what a lane stores at kNowhere or beyond is dropped by the hardware's range check.
+    static constexpr unsigned kNowhere = 0x80000000u;
+    static __device__ __forceinline__ Base bounded_base(const ST *p)
+    {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<ST *>(p), 0, (int)kNowhere, 0x00020000);
+    }
     // aux 2 = non-temporal (streamed data), 0 = the caches' normal policy.
     template <int AUX> static __device__ __forceinline__ raw_t load(Base r, unsigned lane_off, unsigned step_off)
     {
@@ -248,10 +254,12 @@ struct ClSteps {
         const int left = T - 1 - tb;
         return {tb < 0 ? -tb : 0, left < S + 1 ? left : S + 1};
     }
-    // Byte offset from the base for a tensor with `stride` elements per step.
-    static __device__ __forceinline__ unsigned clamped(int s, int d, int stride, Range r)
+    // Byte offset from the base for a tensor with `stride` elements per step. INNER (here and below): every access of the
+    // span exists.
+    template <bool INNER> static __device__ __forceinline__ unsigned clamped(int s, int d, int stride, Range r)
     {
         const unsigned step = (unsigned)stride * (unsigned)sizeof(ST);
+        if (INNER) return (unsigned)rel(s, d) * step;
         const unsigned at = (unsigned)rel(s, d) * step, least = (unsigned)r.least * step, most = (unsigned)r.most * step;
         if (!REV) return at < most ? at : most;
         if (s == 0 && d > 0) return at < most ? at : most;  // (least <= S, or the whole span does not exist and least == most)
@@ -274,24 +282,24 @@ struct ClSteps {
     static constexpr bool CHOSEN_LOADS = RAGGED && sizeof(ST) == 4 && sizeof(raw_t) == 8;
 
     // Issues every load of the wave's S steps; nothing waits for them here.
-    __device__ __forceinline__ void issue(const ClLane<ST> &ln, int T, int first_step)
+    template <bool INNER = false> __device__ __forceinline__ void issue(const ClLane<ST> &ln, int T, int first_step)
     {
         if constexpr (CHOSEN_LOADS) {
             if (ln.cached_loads) {
                 // (The compiler would merge the two copies of the loads, and drop what tells them apart.)
                 asm volatile("" ::: "memory");
-                issue_as<0>(ln, T, first_step);
+                issue_as<0, INNER>(ln, T, first_step);
                 asm volatile("" ::: "memory");
                 return;
             }
         }
-        issue_as<CACHED_LOADS ? 0 : 2>(ln, T, first_step);
+        issue_as<CACHED_LOADS ? 0 : 2, INNER>(ln, T, first_step);
     }
 
-    template <int LOADS> __device__ __forceinline__ void issue_as(const ClLane<ST> &ln, int T, int first_step)
+    template <int LOADS, bool INNER> __device__ __forceinline__ void issue_as(const ClLane<ST> &ln, int T, int first_step)
     {
         n_tau0 = first_step;
-        const int tb = base_step(first_step, T);
+        const int tb = INNER ? (REV ? T - 1 - first_step - S : first_step) : base_step(first_step, T);
         const Range in = range(tb, T);
         const Base res_a = BV::base(ln.a + (int64_t)tb * ln.pa), res_x = BV::base(ln.x + (int64_t)tb * ln.px);
         const Base res_h = BV::base(ln.h + (int64_t)tb * ln.ph);
@@ -300,11 +308,11 @@ struct ClSteps {
 #pragma unroll
         for (int s = 0; s < S; s++) {
             // The gate of step t is a[t] forwards and a[t+1] backwards.
-            const unsigned off_a = clamped(s, REV ? 1 : 0, ln.pa, in), off_x = clamped(s, 0, ln.px, in);
+            const unsigned off_a = clamped<INNER>(s, REV ? 1 : 0, ln.pa, in), off_x = clamped<INNER>(s, 0, ln.px, in);
             if (APPLY) {
                 n_ra[s] = BV::template load<LOADS>(res_a, ln.c, off_a);
                 n_rx[s] = BV::template load<LOADS>(res_x, ln.c, off_x);
-                if (REV) n_rh[s] = BV::template load<LOADS>(res_h, ln.c, clamped(s, -1, ln.ph, in));
+                if (REV) n_rh[s] = BV::template load<LOADS>(res_h, ln.c, clamped<INNER>(s, -1, ln.ph, in));
             } else {
                 n_ra[s] = BV::template load<0>(res_a, ln.c, off_a);
                 n_rx[s] = BV::template load<0>(res_x, ln.c, off_x);
@@ -313,7 +321,7 @@ struct ClSteps {
     }
 
     // Folds the issued steps to one affine pair per channel.
-    __device__ __forceinline__ void fold(int T, CT (&A)[VEC], CT (&B)[VEC], int shift = 0)
+    template <bool INNER = false> __device__ __forceinline__ void fold(int T, CT (&A)[VEC], CT (&B)[VEC], int shift = 0)
     {
         tau0 = n_tau0;
 #pragma unroll
@@ -339,7 +347,7 @@ struct ClSteps {
         }
         // Steps that do not exist are the identity; the gate past the end and h[-1] are zero. The same for the whole wave.
         const int n = count(tau0, T);
-        if (n < S || (REV && (tau0 == 0 || tau0 + S == T))) {
+        if (!INNER && (n < S || (REV && (tau0 == 0 || tau0 + S == T)))) {
             CT ones[VEC];
 #pragma unroll
             for (int k = 0; k < VEC; k++) ones[k] = CT(1);
@@ -424,6 +432,39 @@ struct ClSteps {
             }
         }
         apply_as<false>(ln, T, mine);
+    }
+
+    // The same for a span whose steps all exist, with every store on every path: lanes without channels store nowhere.
+    // (Stores under a condition are stores that may not be there: the wait for loads issued before them would have to be
+    // one for everything in flight.)
+    __device__ __forceinline__ void apply_inner(const ClLane<ST> &ln, int T, CT (&mine)[VEC])
+    {
+        using Out = ClAccess<ST, VEC, true>;
+        const int tb = REV ? T - 1 - tau0 - S : tau0;
+        const auto res_y0 = Out::bounded_base(ln.y0 + (int64_t)tb * ln.py0), res_y1 = Out::bounded_base(ln.y1 + (int64_t)tb * ln.py1);
+        const unsigned step_y0 = (unsigned)ln.py0 * (unsigned)sizeof(ST), step_y1 = (unsigned)ln.py1 * (unsigned)sizeof(ST);
+        const unsigned at = ln.c_ok ? ln.c : Out::kNowhere;
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            CT G[VEC], X[VEC], out[VEC];
+            if (PACKED) {
+                V::unpack(ra[s], G);
+                V::unpack(rx[s], X);
+            }
+#pragma unroll
+            for (int k = 0; k < VEC; k++) {
+                mine[k] = PACKED ? fma_(G[k], mine[k], X[k]) : fma_(g[s][k], mine[k], v[s][k]);
+                out[k] = mine[k];
+            }
+            Out::store(V::pack(out), res_y0, at, (unsigned)rel(s) * step_y0);
+            if (REV) {
+                CT fh[VEC], ga[VEC];
+                V::unpack(rh[s], fh);
+#pragma unroll
+                for (int k = 0; k < VEC; k++) ga[k] = out[k] * fh[k];
+                Out::store(V::pack(ga), res_y1, at, (unsigned)rel(s) * step_y1);
+            }
+        }
     }
 
     template <bool CACHED> __device__ __forceinline__ void apply_as(const ClLane<ST> &ln, int T, CT (&mine)[VEC])
@@ -541,7 +582,7 @@ template <typename ST, int VEC, int S, bool REV, typename CT, bool SPLIT, bool R
 
 // Dynamic LDS: two buffers (tiles alternate) of A and B, each [W][VEC][64] values.
 // M: channels beyond whole vectors, moved as scan_cl_shift.hpp says (0: not).
-template <typename ST, int VEC, int S, bool REV, int MAXT, bool RAGGED = false, int M = 0>
+template <typename ST, int VEC, int S, bool REV, int MAXT, bool RAGGED = false, int M = 0, bool PIPE = false>
 __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
 {
     using CT = typename ComputeOf<ST>::type;
@@ -575,14 +616,16 @@ __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
     // [8, 4096, 2048] forward 93 -> 90 us. fp32 pays 30 to 120 registers for it and is level on average (+28 % to -10 %),
     // 16-byte lanes of 16-bit storage spill.
     constexpr bool AHEAD = cl_ahead<ST, VEC, S>();
+    // PIPE: the same for 16-byte lanes of fp32 and fp64, with the stores out of the loads' way as well. Memory operations
+    // complete in order and are waited for by their number, so a wait for loads with stores behind them that may or may not
+    // have been issued is a wait for these too: AHEAD's loads are back long before the stores that the wave then waits for. In
+    // the tiles whose accesses all exist every store is issued on every path (apply_inner), the wait at the loop's head leaves
+    // them in flight, and a CU with a single workgroup moves memory while it exchanges and computes. What bounds it then is
+    // memory: fp32 [64, 2048, 1024] forwards 290 -> 264 us, 6.1 TB/s, for 94 -> 162 registers (pipe_walk() in scan_api.hip).
     typename ClStepsOf<ST, VEC, S, REV, M, CT, false, RAGGED>::type steps;
-    if (AHEAD) steps.issue(ln, p.T, wave * S);
-    for (int it = 0; it < ntiles; it++) {
+    // The waves' pairs of a tile, exchanged: the value entering this wave's span, and the carry into the next tile.
+    auto exchange = [&](int it, const CT (&A)[VEC], const CT (&B)[VEC], CT (&mine)[VEC]) {
         CT *lds_A = lds + (it & 1) * 2 * plane, *lds_B = lds_A + plane;
-        CT A[VEC], B[VEC], mine[VEC];
-        if (!AHEAD) steps.issue(ln, p.T, it * tile_steps + wave * S);
-        steps.fold(p.T, A, B, ln.shift);
-        if (AHEAD && it + 1 < ntiles) steps.issue(ln, p.T, (it + 1) * tile_steps + wave * S);
 #pragma unroll
         for (int k = 0; k < VEC; k++) mine[k] = carry[k];
         if (W > 1) {
@@ -604,8 +647,41 @@ __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
 #pragma unroll
             for (int k = 0; k < VEC; k++) carry[k] = fma_(A[k], carry[k], B[k]);
         }
-        steps.apply(ln, p.T, mine);
+    };
+    auto first_step = [&](int it) { return it * tile_steps + wave * S; };
+    auto tiles = [&](int from, int to) {
+        CT A[VEC], B[VEC], mine[VEC];
+        if (AHEAD && from < to) steps.issue(ln, p.T, first_step(from));
+        for (int it = from; it < to; it++) {
+            if (!AHEAD) steps.issue(ln, p.T, first_step(it));
+            steps.fold(p.T, A, B, ln.shift);
+            if (AHEAD && it + 1 < to) steps.issue(ln, p.T, first_step(it + 1));
+            exchange(it, A, B, mine);
+            steps.apply(ln, p.T, mine);
+        }
+    };
+    if constexpr (PIPE) {
+        const int k0 = M != 0 ? ln.k0 : 0, edge = REV ? 1 : 0;
+        // Tiles [lo, hi): all their accesses exist.
+        const int lo = (k0 + edge + tile_steps - 1) / tile_steps, hi = (p.T + k0 - edge) / tile_steps;
+        if (hi - lo >= 2) {
+            tiles(0, lo);
+            CT A[VEC], B[VEC], mine[VEC];
+            steps.template issue<true>(ln, p.T, first_step(lo));
+            auto tile = [&](int it, bool more) {
+                steps.template fold<true>(p.T, A, B);
+                if (more) steps.template issue<true>(ln, p.T, first_step(it + 1));
+                exchange(it, A, B, mine);
+                steps.apply_inner(ln, p.T, mine);
+            };
+            tile(lo, true);  // (apart from the loop: where a tile's loads are waited for, the same stores have to be behind them)
+            for (int it = lo + 1; it < hi - 1; it++) tile(it, true);
+            tile(hi - 1, false);
+            tiles(hi, ntiles);
+            return;
+        }
     }
+    tiles(0, ntiles);
 }
 
 // ---------------------------------------------------------------------------

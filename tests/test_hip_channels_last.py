@@ -112,6 +112,48 @@ def test_forced_plans(gpu, dtype):
     assert n > 90
 
 
+@pytest.mark.parametrize("dtype,C", [(torch.float32, 256), (torch.float32, 160), (torch.float32, 260), (torch.float64, 128),
+                                     (torch.float64, 70)])
+@pytest.mark.parametrize("waves", [1, 4, 8])
+def test_walks_that_load_a_tile_ahead_of_their_stores(gpu, dtype, C, waves):
+    """16-byte lanes of 8 steps: from no tile whose accesses all exist to several, and a rest of every kind; full and partial
+    last groups of channels, with memory around the outputs that has to stay as it was, and outputs in place. Partial groups
+    in as many workgroups as there are compute units walk without it, in the same arithmetic. Bars as in test_forced_plans,
+    1e-13 for fp64."""
+    bar, vec = (1e-5, 4) if dtype == torch.float32 else (1e-13, 2)
+    plan, L, code = hip.Plan(mode=hip.MODE_ROW, vec=vec, unroll=8, waves=waves), hip.lib(), hip._dtype_code(dtype)
+    groups, tile = -(-C // (64 * vec)), 8 * waves
+    stream = torch.cuda.current_stream().cuda_stream
+    for T in (tile - 1, tile + 1, 2 * tile, 2 * tile + 1, 3 * tile - 1, 3 * tile + 2, 6 * tile + 7):
+        if T < 2:
+            continue
+        g = torch.Generator().manual_seed(T)
+        batch = 240 // groups if C % (64 * vec) else 3
+        a = torch.rand((batch, T, C), generator=g, dtype=dtype).to(gpu)
+        b, gh = (torch.randn((batch, T, C), generator=g, dtype=dtype).to(gpu) for _ in range(2))
+        h = hip.transposed_linear_scan_forward(a, b, plan=plan)
+        ga, gb = hip.transposed_linear_scan_backward(a, h, gh, plan=plan)
+        for few in sorted({1, min(3, batch)}):
+            print(f"case ahead {dtype} [{few}, {T}, {C}] waves={waves}", flush=True)
+            n, pad = few * T * C, 64
+            out = [torch.full((n + 2 * pad,), 7.0, dtype=dtype, device=gpu) for _ in range(3)]
+            ptr = [t.data_ptr() + pad * t.element_size() for t in out]
+            args = (few, T, C, code, None, 0, stream, ctypes.byref(plan))
+            assert L.scanscam_scan_fwd_cl(a.data_ptr(), b.data_ptr(), ptr[0], *args) == 0
+            assert L.scanscam_scan_bwd_cl(a.data_ptr(), h.data_ptr(), gh.data_ptr(), ptr[1], ptr[2], *args) == 0
+            for got, want in zip(out, (h, ga, gb)):
+                assert bool((got[:pad] == 7).all()) and bool((got[-pad:] == 7).all())
+                assert torch.equal(got[pad:-pad].view(few, T, C), want[:few])
+            inplace = b[:few].clone()
+            assert L.scanscam_scan_fwd_cl(a.data_ptr(), inplace.data_ptr(), inplace.data_ptr(), *args) == 0
+            assert torch.equal(inplace, h[:few])
+        rows = [as_rows(t[:3]) for t in (a, b, gh, h, ga, gb)]
+        assert rel_err(rows[3], oracle.fwd(rows[0], rows[1])) <= bar
+        want_ga, want_gb = oracle.bwd(rows[0], rows[3], rows[2])
+        assert rel_err(rows[5], want_gb) <= bar
+        assert rel_err(rows[4], want_ga, prev_abs(rows[3])) <= bar
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T", [1, 2, 4, 15, 16, 17, 33])
 def test_spans_that_end_inside_or_before_a_wave(gpu, dtype, T):
