@@ -677,16 +677,20 @@ int size_cl(int64_t batch, int64_t T, int dtype, bool rev, int virtual_steps, sc
 // walk, buffers in rotation, none of them used to find the rule (profiles/walk_loads_past_stores_random_shapes.txt): fp32 forwards
 // 0.92 to 1.02 x, 0.964 x in the mean of 24 ([36, 702, 1472] 86.6 -> 79.6 us, [24, 2401, 1932] 291 -> 276), fp64 0.93 x forwards, 0.99
 // x backwards in the mean of 12 ([18, 339, 1104] 36.9 -> 31.8, [37, 307, 672] backward 63.1 -> 60.7); [64, 2048, 1024] fp32, from box
-// to box, 276 to 290 -> 264 to 270. At worst [224, 909, 512] fp32, 223 -> 231. Not taken
-//   - where 8 waves with its registers leave one workgroup per CU and there are more: fp32 [930, 174, 160] 58.8 -> 62.6 ([201,
+// to box, 276 to 290 -> 264 to 270. At worst [224, 909, 512] fp32, 223 -> 231. Two fp32 channels by 16 steps 0.91 to 1.0 x, 0.963 x
+// in the mean of 18 ([17, 840, 1504] 54.7 -> 49.6), one of fp64 by 8 steps 0.98 x in the mean of 12 ([21, 1088, 688] 71.8 -> 65.3).
+// Not taken
+//   - below three tiles, which leave fewer than two that are whole (fp64 [27, 90, 800] 11.7 -> 12.1);
+//   - where 8 waves of 32 or more words a lane leave one workgroup per CU with its registers and there are more: fp32 [930, 174, 160] 58.8 -> 62.6 ([201,
 //     238, 160], one each, 22.3 -> 20.5);
 //   - where nearly every CU has one workgroup and a time step's last group is not full, which memory's order bounds: fp32, 256 of
 //     them, [64, 2048, 1016] 345 -> 364, [64, 2048, 1008] 285 -> 297, [64, 2048, 960] 286 -> 294, 245 of them,
 //     [49, 925, 1132] 126 -> 128 (but 205, [41, 1355, 1216] 163 -> 159, and 714, [102, 591, 1680] 246 -> 234).
-bool pipe_walk(const scanscam::ClLaunch &l, int64_t C, int esize, bool rev)
+bool pipe_walk(const scanscam::ClLaunch &l, int64_t T, int64_t C, int esize, bool rev)
 {
     if (l.kind != 0 || l.group != kWave || l.ragged || l.shift != 0 || !scanscam::cl_pipe_built(esize, l.vec, l.steps, rev)) return false;
-    if (l.waves > 4 && l.grid > kComputeUnits) return false;
+    if (T < (int64_t)3 * l.waves * l.steps) return false;
+    if (l.waves > 4 && l.grid > kComputeUnits && l.vec * l.steps * esize >= 128) return false;
     return C % (kWave * l.vec) == 0 || l.grid < kComputeUnits - 20 || l.grid > kComputeUnits;
 }
 
@@ -1093,7 +1097,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         const int64_t rowgroups = batch * l.groups;
         if (clear_workspace(args.ws, words, rowgroups * kCounterStride, s) != hipSuccess) return SCANSCAM_ELAUNCH;
     }
-    l.pipe = pipe_walk(l, C, esize, rev);
+    l.pipe = pipe_walk(l, T, C, esize, rev) && !args.cached_stores;
     // (Its resources end 2 GiB past a span's base, where lanes without channels store.)
     for (int k = 0; k < 5; k++)
         if ((uint64_t)sT[k] * (uint64_t)esize * 18u + (uint64_t)C * (uint64_t)esize >= (uint64_t(1) << 31)) l.pipe = false;

@@ -616,7 +616,7 @@ __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
     // [8, 4096, 2048] forward 93 -> 90 us. fp32 pays 30 to 120 registers for it and is level on average (+28 % to -10 %),
     // 16-byte lanes of 16-bit storage spill.
     constexpr bool AHEAD = cl_ahead<ST, VEC, S>();
-    // PIPE: the same for 16-byte lanes of fp32 and fp64, with the stores out of the loads' way as well. Memory operations
+    // PIPE: the same for wide lanes of fp32 and fp64 (cl_pipe_built()), with the stores out of the loads' way as well. Memory operations
     // complete in order and are waited for by their number, so a wait for loads with stores behind them that may or may not
     // have been issued is a wait for these too: AHEAD's loads are back long before the stores that the wave then waits for. In
     // the tiles whose accesses all exist every store is issued on every path (apply_inner), the wait at the loop's head leaves

@@ -112,17 +112,18 @@ def test_forced_plans(gpu, dtype):
     assert n > 90
 
 
-@pytest.mark.parametrize("dtype,C", [(torch.float32, 256), (torch.float32, 160), (torch.float32, 260), (torch.float64, 128),
-                                     (torch.float64, 70)])
+@pytest.mark.parametrize("dtype,C,vec,steps", [(torch.float32, 256, 4, 8), (torch.float32, 160, 4, 8), (torch.float32, 260, 4, 8),
+                                               (torch.float32, 128, 2, 16), (torch.float32, 96, 2, 16), (torch.float64, 128, 2, 8),
+                                               (torch.float64, 70, 2, 8), (torch.float64, 64, 1, 8), (torch.float64, 40, 1, 8)])
 @pytest.mark.parametrize("waves", [1, 4, 8])
-def test_walks_that_load_a_tile_ahead_of_their_stores(gpu, dtype, C, waves):
-    """16-byte lanes of 8 steps: from no tile whose accesses all exist to several, and a rest of every kind; full and partial
+def test_walks_that_load_a_tile_ahead_of_their_stores(gpu, dtype, C, vec, steps, waves):
+    """From no tile whose accesses all exist to several, and a rest of every kind; full and partial
     last groups of channels, with memory around the outputs that has to stay as it was, and outputs in place. Partial groups
     in as many workgroups as there are compute units walk without it, in the same arithmetic. Bars as in test_forced_plans,
     1e-13 for fp64."""
-    bar, vec = (1e-5, 4) if dtype == torch.float32 else (1e-13, 2)
-    plan, L, code = hip.Plan(mode=hip.MODE_ROW, vec=vec, unroll=8, waves=waves), hip.lib(), hip._dtype_code(dtype)
-    groups, tile = -(-C // (64 * vec)), 8 * waves
+    bar = 1e-5 if dtype == torch.float32 else 1e-13
+    plan, L, code = hip.Plan(mode=hip.MODE_ROW, vec=vec, unroll=steps, waves=waves), hip.lib(), hip._dtype_code(dtype)
+    groups, tile = -(-C // (64 * vec)), steps * waves
     stream = torch.cuda.current_stream().cuda_stream
     for T in (tile - 1, tile + 1, 2 * tile, 2 * tile + 1, 3 * tile - 1, 3 * tile + 2, 6 * tile + 7):
         if T < 2:
