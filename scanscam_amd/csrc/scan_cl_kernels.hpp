@@ -281,7 +281,20 @@ struct ClSteps {
     static constexpr bool CACHED_LOADS = RAGGED && sizeof(ST) == 4 && sizeof(raw_t) == 16;
     static constexpr bool CHOSEN_LOADS = RAGGED && sizeof(ST) == 4 && sizeof(raw_t) == 8;
 
-    // Issues every load of the wave's S steps; nothing waits for them here.
+    // h is needed only once the scan value entering the span is known, and loads come back in the order of their issue: behind
+    // all gates and values it is on its way while the waves exchange their pairs; between them the exchange waits for it as
+    // well, and the last step's gate and value were loaded in one of fold()'s paths only, behind the waits for all the others
+    // (16-bit tiles of 16 and 64 elements). Time against the form whose accesses had conditions of their own, 12 to 20 random calls
+    // each, buffers in rotation, before -> now: tiles bf16 4 x 4 1.02 -> 0.985, fp16 1.03 -> 0.995, 4 x 16 0.975 / 0.99 -> 0.94 /
+    // 0.96, fp32 4 x 8 0.975 -> 0.95; walks fp32 4 x 8 0.99 -> 0.97, fp64 1 x 8 1.01 -> 0.99. Not in element-aligned lanes (fp32
+    // 2 x 4 1.0 -> 1.015).
+    static constexpr bool H_LAST = REV && !RAGGED;
+    // In walks of packed spans behind the fold as well, where the gates and values are back: with a whole tile's loads first and then all
+    // its stores, single tiles run slower. 8 x 8 bf16 / fp16 1.035 / 1.025 -> 0.995 / 0.99 (behind the values only: 1.015 / 1.01;
+    // [54, 64, 4032] 24.8, 26.9 between them), 4 x 16 0.97 / 0.99 -> 0.945 / 0.965; fp32 2 x 8 would lose 1 %.
+    static constexpr bool H_FOLDED = H_LAST && PACKED && !SPLIT;
+
+    // Issues every load of the wave's S steps (but h's where issue_h() follows the fold); nothing waits for them here.
     template <bool INNER = false> __device__ __forceinline__ void issue(const ClLane<ST> &ln, int T, int first_step)
     {
         if constexpr (CHOSEN_LOADS) {
@@ -312,11 +325,30 @@ struct ClSteps {
             if (APPLY) {
                 n_ra[s] = BV::template load<LOADS>(res_a, ln.c, off_a);
                 n_rx[s] = BV::template load<LOADS>(res_x, ln.c, off_x);
-                if (REV) n_rh[s] = BV::template load<LOADS>(res_h, ln.c, clamped<INNER>(s, -1, ln.ph, in));
+                if (REV && !H_LAST) n_rh[s] = BV::template load<LOADS>(res_h, ln.c, clamped<INNER>(s, -1, ln.ph, in));
             } else {
                 n_ra[s] = BV::template load<0>(res_a, ln.c, off_a);
                 n_rx[s] = BV::template load<0>(res_x, ln.c, off_x);
             }
+        }
+        if constexpr (H_LAST && !H_FOLDED) {
+            asm volatile("" ::: "memory");  // (The compiler would mix them with the others again.)
+#pragma unroll
+            for (int s = 0; s < S; s++) n_rh[s] = BV::template load<LOADS>(res_h, ln.c, clamped<INNER>(s, -1, ln.ph, in));
+        }
+    }
+
+    // H_FOLDED: h of the folded span, before its pairs are exchanged.
+    __device__ __forceinline__ void issue_h(const ClLane<ST> &ln, int T)
+    {
+        if constexpr (H_FOLDED) {
+            const int tb = base_step(tau0, T);
+            const Range in = range(tb, T);
+            const Base res_h = BV::base(ln.h + (int64_t)tb * ln.ph);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int s = 0; s < S; s++) rh[s] = BV::template load<2>(res_h, ln.c, clamped<false>(s, -1, ln.ph, in));
+            asm volatile("" ::: "memory");
         }
     }
 
@@ -328,7 +360,7 @@ struct ClSteps {
         for (int s = 0; s < S; s++) {
             ra[s] = n_ra[s];
             rx[s] = n_rx[s];
-            if (REV && APPLY) rh[s] = n_rh[s];
+            if (REV && APPLY && !H_FOLDED) rh[s] = n_rh[s];
         }
         if (RAGGED && shift != 0) {  // the last lane of a time step: its window's components into place
 #pragma unroll
@@ -345,7 +377,8 @@ struct ClSteps {
                 V::unpack(rx[s], v[s]);
             }
         }
-        // Steps that do not exist are the identity; the gate past the end and h[-1] are zero. The same for the whole wave.
+        // Steps that do not exist are the identity; the gate past the end and (H_LAST: in apply()) h[-1] are zero. The same
+        // for the whole wave.
         const int n = count(tau0, T);
         if (!INNER && (n < S || (REV && (tau0 == 0 || tau0 + S == T)))) {
             CT ones[VEC];
@@ -365,7 +398,7 @@ struct ClSteps {
                         v[s][k] = in ? v[s][k] : CT(0);
                     }
                 }
-                if (REV && APPLY) rh[s] = tau0 + s == T - 1 ? zero : rh[s];
+                if (REV && APPLY && !H_LAST) rh[s] = tau0 + s == T - 1 ? zero : rh[s];
             }
         }
 #pragma unroll
@@ -425,6 +458,11 @@ struct ClSteps {
     __device__ __forceinline__ void apply(const ClLane<ST> &ln, int T, CT (&mine)[VEC])
     {
         if (!ln.c_ok) return;
+        if (H_LAST && tau0 < T && tau0 + S >= T) {
+            const raw_t zero = V::zero_raw();
+#pragma unroll
+            for (int s = 0; s < S; s++) rh[s] = tau0 + s == T - 1 ? zero : rh[s];
+        }
         if constexpr (!RAGGED && sizeof(raw_t) <= 8) {
             if (ln.cached) {
                 apply_as<true>(ln, T, mine);
@@ -655,6 +693,7 @@ __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
         for (int it = from; it < to; it++) {
             if (!AHEAD) steps.issue(ln, p.T, first_step(it));
             steps.fold(p.T, A, B, ln.shift);
+            if constexpr (M == 0) steps.issue_h(ln, p.T);
             if (AHEAD && it + 1 < to) steps.issue(ln, p.T, first_step(it + 1));
             exchange(it, A, B, mine);
             steps.apply(ln, p.T, mine);
