@@ -221,11 +221,13 @@ struct ClSteps {
     using Base = typename BV::Base;
 
     // PACKED: 16-bit gates and values stay as they are stored from fold() to apply(), each of which widens them, in half the
-    // registers of the widened ones. In tiles of time where that lets a second workgroup of 8 waves onto a CU: 32 elements per
-    // lane backwards (130 -> 102 registers; bf16 [8, 4096, 2048] 2 x 16: 176 -> 155 us, fp16 [1, 18877, 1920] 97 -> 76 us) and 64
-    // forwards (192 -> 126; 4 x 16: 98 -> 87 us, 68 -> 58 us); 32 forwards (104 -> 72, no whole workgroup more) run 1.0 to 1.13 x
-    // and 64 backwards (222 -> 158) 1.0 to 1.09 x with it. In walks that do not load ahead, 16-byte lanes 0.94 to 1.0 x.
-    static constexpr bool PACKED = sizeof(ST) == 2 && VEC > 1 && (SPLIT ? VEC * S == (REV ? 32 : 64) : !cl_ahead<ST, VEC, S>());
+    // registers of the widened ones. In tiles of time where that lets a second workgroup of 8 waves onto a CU: 2 x 16 and 4 x 8
+    // backwards (130 -> 102 registers; bf16 [8, 4096, 2048] 2 x 16: 176 -> 155 us, fp16 [1, 18877, 1920] 97 -> 76 us) and 4 x 16
+    // forwards (192 -> 126; 98 -> 87 us, 68 -> 58 us); 8 x 4 backwards, at 128 registers either way, for its spills (18 -> 0; 0.88 x).
+    // 8 x 8 forwards would come to 129 and run 1.02 instead of 0.985 x the time before, 32 elements forwards (104 -> 72, no whole workgroup
+    // more) 1.0 to 1.13 x, 64 backwards (222 -> 158) 1.0 to 1.09 x. In walks that do not load ahead: against unpacked 4 x 16 0.94 to
+    // 1.04 x forwards (fp16 0.995 x in the mean of 20 calls, bf16, single tiles of few workgroups, 1.01), 8 x 8 backwards level.
+    static constexpr bool PACKED = sizeof(ST) == 2 && VEC > 1 && (SPLIT ? (REV ? VEC * S == 32 : VEC == 4 && S == 16) : !cl_ahead<ST, VEC, S>());
     raw_t ra[S], rx[S], rh[(REV && APPLY) ? S : 1];
     CT g[PACKED ? 1 : S][VEC], v[PACKED ? 1 : S][VEC];
     int tau0;  // scan position of the first step
