@@ -686,12 +686,17 @@ int size_cl(int64_t batch, int64_t T, int dtype, bool rev, int virtual_steps, sc
 //   - where nearly every CU has one workgroup and a time step's last group is not full, which memory's order bounds: fp32, 256 of
 //     them, [64, 2048, 1016] 345 -> 364, [64, 2048, 1008] 285 -> 297, [64, 2048, 960] 286 -> 294, 245 of them,
 //     [49, 925, 1132] 126 -> 128 (but 205, [41, 1355, 1216] 163 -> 159, and 714, [102, 591, 1680] 246 -> 234).
-bool pipe_walk(const scanscam::ClLaunch &l, int64_t T, int64_t C, int esize, bool rev)
+// `sT`: the tensors' time strides in elements; `cached`: the walk stores through the caches' normal policy, which these do not.
+bool pipe_walk(const scanscam::ClLaunch &l, int64_t T, int64_t C, int esize, bool rev, const int64_t sT[5], bool cached)
 {
     if (l.kind != 0 || l.group != kWave || l.ragged || l.shift != 0 || !scanscam::cl_pipe_built(esize, l.vec, l.steps, rev)) return false;
-    if (T < (int64_t)3 * l.waves * l.steps) return false;
+    // Two tiles whose accesses all exist, which the kernel takes for granted: a[t+1] of the first and h[t-1] of the last step do not.
+    if (T < (int64_t)3 * l.waves * l.steps + (rev ? 1 : 0)) return false;
     if (l.waves > 4 && l.grid > kComputeUnits && l.vec * l.steps * esize >= 128) return false;
-    return C % (kWave * l.vec) == 0 || l.grid < kComputeUnits - 20 || l.grid > kComputeUnits;
+    // (Its resources end 2 GiB past a span's base, where lanes without channels store.)
+    for (int k = 0; k < 5; k++)
+        if ((uint64_t)sT[k] * (uint64_t)esize * 18u + (uint64_t)C * (uint64_t)esize >= (uint64_t(1) << 31)) return false;
+    return !cached && (C % (kWave * l.vec) == 0 || l.grid < kComputeUnits - 20 || l.grid > kComputeUnits);
 }
 
 // Channels-last: the launch plan. `align`: the largest of 16, 8, 4 and the element size that every tensor's base
@@ -958,6 +963,38 @@ int shift_code_of(const scanscam_plan *plan, int64_t batch, int64_t T, int64_t C
     return free_plan ? shift_choice(batch, T, C, esize, rev, reserve) : 0;
 }
 
+// The largest of 16, 8, 4 and the element size (bytes) that every base and stride of a call's tensors is a multiple of.
+int cl_align(const void *const ptrs[5], const int64_t sB[5], const int64_t sT[5], int esize)
+{
+    int align = 16;
+    for (int k = 0; k < 5; k++)
+        while (align > esize && !(aligned_to(ptrs[k], (size_t)align) && (sB[k] * esize) % align == 0 && (sT[k] * esize) % align == 0))
+            align >>= 1;
+    return align;
+}
+
+// Whether every time step of every tensor is whole 128-byte lines.
+bool cl_lines(const void *const ptrs[5], const int64_t sB[5], const int64_t sT[5], int esize)
+{
+    for (int k = 0; k < 5; k++)
+        if ((sT[k] * esize) % 128 != 0 || !aligned_to(ptrs[k], 128) || (sB[k] * esize) % 128 != 0) return false;
+    return true;
+}
+
+// Lanes of 8 bytes or less whose time steps are no whole lines write partial lines at both ends of every
+// wave's store; non-temporal stores then cost 20 % of a plain copy's rate and stores left to the caches'
+// normal policy nothing. Measured on the kernels: 16-bit storage 8 to 35 % faster in both directions (bf16
+// [90, 2048, 514] 178 / 341 -> 139 / 298 us, [1000, 500, 130] 157 / 296 -> 120 / 202 us, [700, 300, 257] 112 / 217 ->
+// 85 / 141 us; single channels backwards lose 10 %: [260, 4000, 48]), fp32 forwards and in tiles over workgroups
+// 4 to 19 % ([8, 4096, 1000] 90 / 152 -> 83 / 128 us, [100, 3000, 300] forward 339 -> 276 us; a walk of all of T
+// backwards loses up to 11 %); on whole lines they lose 6 to 14 %, and 16-byte lanes lose 6 to 11 % either way.
+// (Element-aligned lanes of 8 bytes or less always store this way: the kernel's choice, not this flag's.)
+bool cl_cached_stores(const scanscam::ClLaunch &l, bool lines, int esize, bool rev)
+{
+    const int lane_bytes = l.vec * esize;
+    return !lines && lane_bytes <= 8 && esize <= 4 && (esize == 2 ? (lane_bytes > 2 || !rev) : (!rev || l.kind == 2));
+}
+
 int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void *y1,
            const scanscam_strides *const st[5], int64_t batch, int64_t T, int64_t C, int dtype, void *workspace,
            size_t workspace_bytes, void *stream, const scanscam_plan *plan)
@@ -972,16 +1009,14 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     const void *ptrs[5] = {a, x, rev ? h : a, y0, rev ? y1 : y0};
     const int src[5] = {0, 1, rev ? 2 : 0, 3, rev ? 4 : 3};
     int64_t sB[5], sT[5];
-    int align = 16;  // bytes every base and stride is a multiple of: 16, 8, 4 or the element size
     for (int k = 0; k < 5; k++) {
         const scanscam_strides *t = st[src[k]];
         sB[k] = batch == 1 ? 0 : (t ? t->outer : T * C);
         sT[k] = T == 1 ? 0 : (t ? t->row : C);
         if (sB[k] < 0 || sT[k] < 0 || sT[k] >= kMaxT) return SCANSCAM_EINVAL;
         if (!aligned_to(ptrs[k], (size_t)esize)) return SCANSCAM_EALIGN;
-        while (align > esize && !(aligned_to(ptrs[k], (size_t)align) && (sB[k] * esize) % align == 0 && (sT[k] * esize) % align == 0))
-            align >>= 1;
     }
+    const int align = cl_align(ptrs, sB, sT, esize);
     const bool dense = cl_dense(batch, T, C, ptrs, sB, sT);
     auto run_staged = [&](scanscam::StagedArgs st) {
         st.a = a;
@@ -1045,8 +1080,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
     args.groups = l.groups;
     args.vectors = l.vectors;
     // Time steps that are not whole 128-byte lines: neighbouring channel groups on one XCD (see the kernel).
-    bool lines = true;
-    for (int k = 0; k < 5; k++) lines = lines && (sT[k] * esize) % 128 == 0 && aligned_to(ptrs[k], 128) && (sB[k] * esize) % 128 == 0;
+    const bool lines = cl_lines(ptrs, sB, sT, esize);
     args.xcd_order = (!lines && l.grid >= 64) ? 1 : 0;
     // Tiles over workgroups: a (batch element, channel group) pair keeps its XCD over all its tiles when their number
     // is a multiple of 8. Otherwise, from 128 pairs on, the XCDs take runs of n / 8 rounded up or down and the grid is
@@ -1060,17 +1094,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
             if (l.grid >= (int64_t(1) << 31)) return SCANSCAM_EINVAL;
         }
     }
-    // Lanes of 8 bytes or less whose time steps are no whole lines write partial lines at both ends of every
-    // wave's store; non-temporal stores then cost 20 % of a plain copy's rate and stores left to the caches'
-    // normal policy nothing. Measured on the kernels: 16-bit storage 8 to 35 % faster in both directions (bf16
-    // [90, 2048, 514] 178 / 341 -> 139 / 298 us, [1000, 500, 130] 157 / 296 -> 120 / 202 us, [700, 300, 257] 112 / 217 ->
-    // 85 / 141 us; single channels backwards lose 10 %: [260, 4000, 48]), fp32 forwards and in tiles over workgroups
-    // 4 to 19 % ([8, 4096, 1000] 90 / 152 -> 83 / 128 us, [100, 3000, 300] forward 339 -> 276 us; a walk of all of T
-    // backwards loses up to 11 %); on whole lines they lose 6 to 14 %, and 16-byte lanes lose 6 to 11 % either way.
-    // (Element-aligned lanes of 8 bytes or less always store this way: the kernel's choice, not this flag's.)
-    const int lane_bytes = l.vec * esize;
-    args.cached_stores = (!lines && lane_bytes <= 8 && esize <= 4 &&
-                          (esize == 2 ? (lane_bytes > 2 || !rev) : (!rev || l.kind == 2))) ? 1 : 0;
+    args.cached_stores = cl_cached_stores(l, lines, esize, rev) ? 1 : 0;
     // Loads through the caches' normal policy in element-aligned 8-byte lanes of fp32, once the call does not fit the
     // last-level cache. Against non-temporal ones, buffers in rotation (profiles/element_aligned_loads_random_shapes.txt): 64
     // calls beyond it 0.87 to 1.02 x, 0.94 x in the mean ([16, 4096, 1999] forwards 340 -> 298 us, [256, 500, 513] backwards
@@ -1097,10 +1121,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         const int64_t rowgroups = batch * l.groups;
         if (clear_workspace(args.ws, words, rowgroups * kCounterStride, s) != hipSuccess) return SCANSCAM_ELAUNCH;
     }
-    l.pipe = pipe_walk(l, T, C, esize, rev) && !args.cached_stores;
-    // (Its resources end 2 GiB past a span's base, where lanes without channels store.)
-    for (int k = 0; k < 5; k++)
-        if ((uint64_t)sT[k] * (uint64_t)esize * 18u + (uint64_t)C * (uint64_t)esize >= (uint64_t(1) << 31)) l.pipe = false;
+    l.pipe = pipe_walk(l, T, C, esize, rev, sT, args.cached_stores != 0);
     hipError_t e = hipErrorInvalidValue;
     switch (dtype) {
     case SCANSCAM_F32: e = scanscam::launch_scan_cl<float>(args, l, rev, s); break;
@@ -1338,6 +1359,35 @@ int scanscam_predict_cl(int64_t batch, int64_t T, int64_t C, int dtype, int dire
     while (align > esize && !(batch == 1 && T == 1) && (C * esize) % align != 0) align >>= 1;
     scanscam::ClLaunch l;
     return resolve_cl(plan, batch, T, C, dtype, align, direction == SCANSCAM_BACKWARD, &l, microseconds);
+}
+
+// For tests and measurements, not part of the interface in scanscam_hip.h: whether a call walks with its loads a tile ahead, past its
+// stores (1 or 0; below zero: the negative of an error code). Tensors in the order a, x, h, y0, y1 (forwards h is a and y1 is y0),
+// bases on 128-byte borders, `sB` and `sT` their strides in elements (NULL: dense). Launches nothing.
+int scanscam_internal_walks_ahead(int64_t batch, int64_t T, int64_t C, int dtype, int direction, const int64_t *sB, const int64_t *sT,
+                                  const scanscam_plan *plan)
+{
+    const int esize = elem_size(dtype);
+    if (esize == 0) return -SCANSCAM_EDTYPE;
+    if (batch <= 0 || T <= 0 || C <= 0 || T >= kMaxT || C >= kMaxT) return -SCANSCAM_EINVAL;
+    const bool rev = direction == SCANSCAM_BACKWARD;
+    const void *const ptrs[5] = {};
+    int64_t b[5], t[5];
+    for (int k = 0; k < 5; k++) {
+        b[k] = batch == 1 ? 0 : (sB ? sB[k] : T * C);
+        t[k] = T == 1 ? 0 : (sT ? sT[k] : C);
+        if (b[k] < 0 || t[k] < 0 || t[k] >= kMaxT) return -SCANSCAM_EINVAL;
+    }
+    scanscam::ClLaunch l, shifted;
+    const int rc = resolve_cl(plan, batch, T, C, dtype, cl_align(ptrs, b, t, esize), rev, &l);
+    if (rc != SCANSCAM_OK) return -rc;
+    const bool dense = cl_dense(batch, T, C, ptrs, b, t);
+    const int parts = staged_parts_of(plan, batch, T, C, esize), code = parts > 0 ? 0 : shift_code_of(plan, batch, T, C, esize, rev, l);
+    scanscam::StagedArgs staged;
+    if (dense && ((code != 0 && resolve_shift(batch, T, C, dtype, code, &shifted)) ||
+                  (parts > 0 && resolve_staged(batch, T, C, esize, parts, &staged))))
+        return 0;
+    return pipe_walk(l, T, C, esize, rev, t, cl_cached_stores(l, cl_lines(ptrs, b, t, esize), esize, rev)) ? 1 : 0;
 }
 
 const char *scanscam_strerror(int code)

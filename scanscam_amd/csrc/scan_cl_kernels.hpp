@@ -717,27 +717,25 @@ __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
         }
     };
     if constexpr (PIPE) {
-        const int k0 = M != 0 ? ln.k0 : 0, edge = REV ? 1 : 0;
-        // Tiles [lo, hi): all their accesses exist.
-        const int lo = (k0 + edge + tile_steps - 1) / tile_steps, hi = (p.T + k0 - edge) / tile_steps;
-        if (hi - lo >= 2) {
-            tiles(0, lo);
-            CT A[VEC], B[VEC], mine[VEC];
-            steps.template issue<true>(ln, p.T, first_step(lo));
-            auto tile = [&](int it, bool more) {
-                steps.template fold<true>(p.T, A, B);
-                if (more) steps.template issue<true>(ln, p.T, first_step(it + 1));
-                exchange(it, A, B, mine);
-                steps.apply_inner(ln, p.T, mine);
-            };
-            tile(lo, true);  // (apart from the loop: where a tile's loads are waited for, the same stores have to be behind them)
-            for (int it = lo + 1; it < hi - 1; it++) tile(it, true);
-            tile(hi - 1, false);
-            tiles(hi, ntiles);
-            return;
-        }
+        constexpr int edge = REV ? 1 : 0;
+        // Tiles [lo, hi): all their accesses exist; at least two (the host's choice).
+        const int lo = (edge + tile_steps - 1) / tile_steps, hi = (p.T - edge) / tile_steps;
+        tiles(0, lo);
+        CT A[VEC], B[VEC], mine[VEC];
+        steps.template issue<true>(ln, p.T, first_step(lo));
+        auto tile = [&](int it, bool more) {
+            steps.template fold<true>(p.T, A, B);
+            if (more) steps.template issue<true>(ln, p.T, first_step(it + 1));
+            exchange(it, A, B, mine);
+            steps.apply_inner(ln, p.T, mine);
+        };
+        tile(lo, true);  // (apart from the loop: where a tile's loads are waited for, the same stores have to be behind them)
+        for (int it = lo + 1; it < hi - 1; it++) tile(it, true);
+        tile(hi - 1, false);
+        tiles(hi, ntiles);
+    } else {
+        tiles(0, ntiles);
     }
-    tiles(0, ntiles);
 }
 
 // ---------------------------------------------------------------------------

@@ -15,9 +15,25 @@ loop must miss the same criterion against float64 on that tensor, and in every
 row with a miss the kernel must be no further from float64 than twice the loop's
 own worst error in that row (plus the criterion's atol).
 """
+import ctypes
+
 import numpy as np
 
+from scanscam_amd import hip
+
 ATOL, RTOL = 1e-4, 1e-5
+
+
+def walks_ahead(batch, T, C, dtype, direction, plan=None, time_stride=None):
+    """Whether a channels-last call walks with its loads a tile ahead of its stores (no GPU needed): dense tensors on 128-byte
+    borders, or ``[batch, T, C]`` views with ``time_stride`` elements from one time step to the next."""
+    ask = hip.lib().scanscam_internal_walks_ahead
+    ask.restype = ctypes.c_int
+    ask.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int] * 2 + [ctypes.c_void_p] * 3
+    strides = [(ctypes.c_int64 * 5)(*[n] * 5) if time_stride else None for n in (T * (time_stride or 0), time_stride or 0)]
+    got = ask(batch, T, C, hip._dtype_code(dtype), direction, *strides, ctypes.byref(plan) if plan is not None else None)
+    assert got in (0, 1), got
+    return bool(got)
 
 
 def assert_reference_allclose(got, want, exact, what=""):

@@ -12,7 +12,7 @@ import pytest
 import torch
 
 import oracle
-from criteria import assert_reference_allclose
+from criteria import assert_reference_allclose, walks_ahead
 from scanscam_amd import hip
 
 pytestmark = pytest.mark.gpu
@@ -117,17 +117,16 @@ def test_forced_plans(gpu, dtype):
                                                (torch.float64, 70, 2, 8), (torch.float64, 64, 1, 8), (torch.float64, 40, 1, 8)])
 @pytest.mark.parametrize("waves", [1, 4, 8])
 def test_walks_that_load_a_tile_ahead_of_their_stores(gpu, dtype, C, vec, steps, waves):
-    """From no tile whose accesses all exist to several, and a rest of every kind; full and partial
-    last groups of channels, with memory around the outputs that has to stay as it was, and outputs in place. Partial groups
-    in as many workgroups as there are compute units walk without it, in the same arithmetic. Bars as in test_forced_plans,
-    1e-13 for fp64."""
+    """From the last call that walks without it, by one step, to one of several tiles and a rest of every kind, the kernel that
+    is meant; full and partial last groups of channels, with memory around the outputs that has to stay as it was, and outputs in
+    place over the value and over the gate. Partial groups in as many workgroups as there are compute units walk without it,
+    in the same arithmetic. Bars as in test_forced_plans, 1e-13 for fp64."""
     bar = 1e-5 if dtype == torch.float32 else 1e-13
     plan, L, code = hip.Plan(mode=hip.MODE_ROW, vec=vec, unroll=steps, waves=waves), hip.lib(), hip._dtype_code(dtype)
     groups, tile = -(-C // (64 * vec)), steps * waves
     stream = torch.cuda.current_stream().cuda_stream
-    for T in (tile - 1, tile + 1, 2 * tile, 2 * tile + 1, 3 * tile - 1, 3 * tile + 2, 6 * tile + 7):
-        if T < 2:
-            continue
+    both_ways = vec * (4 if dtype == torch.float32 else 8) == 16 and dtype == torch.float64
+    for T in (tile + 1, 3 * tile - 1, 3 * tile, 3 * tile + 1, 4 * tile - 1, 4 * tile, 4 * tile + 1, 6 * tile + 7):
         g = torch.Generator().manual_seed(T)
         batch = 240 // groups if C % (64 * vec) else 3
         a = torch.rand((batch, T, C), generator=g, dtype=dtype).to(gpu)
@@ -136,6 +135,8 @@ def test_walks_that_load_a_tile_ahead_of_their_stores(gpu, dtype, C, vec, steps,
         ga, gb = hip.transposed_linear_scan_backward(a, h, gh, plan=plan)
         for few in sorted({1, min(3, batch)}):
             print(f"case ahead {dtype} [{few}, {T}, {C}] waves={waves}", flush=True)
+            assert walks_ahead(few, T, C, dtype, hip.FORWARD, plan) == (T >= 3 * tile)
+            assert walks_ahead(few, T, C, dtype, hip.BACKWARD, plan) == (both_ways and T > 3 * tile)
             n, pad = few * T * C, 64
             out = [torch.full((n + 2 * pad,), 7.0, dtype=dtype, device=gpu) for _ in range(3)]
             ptr = [t.data_ptr() + pad * t.element_size() for t in out]
@@ -148,6 +149,10 @@ def test_walks_that_load_a_tile_ahead_of_their_stores(gpu, dtype, C, vec, steps,
             inplace = b[:few].clone()
             assert L.scanscam_scan_fwd_cl(a.data_ptr(), inplace.data_ptr(), inplace.data_ptr(), *args) == 0
             assert torch.equal(inplace, h[:few])
+            inplace = a[:few].clone()
+            assert L.scanscam_scan_fwd_cl(inplace.data_ptr(), b.data_ptr(), inplace.data_ptr(), *args) == 0
+            assert torch.equal(inplace, h[:few])
+        assert C % (64 * vec) == 0 or not walks_ahead(batch, T, C, dtype, hip.FORWARD, plan)
         rows = [as_rows(t[:3]) for t in (a, b, gh, h, ga, gb)]
         assert rel_err(rows[3], oracle.fwd(rows[0], rows[1])) <= bar
         want_ga, want_gb = oracle.bwd(rows[0], rows[3], rows[2])
@@ -155,13 +160,51 @@ def test_walks_that_load_a_tile_ahead_of_their_stores(gpu, dtype, C, vec, steps,
         assert rel_err(rows[4], want_ga, prev_abs(rows[3])) <= bar
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dtype,C,vec,steps", [(torch.float32, 256, 4, 8), (torch.float32, 224, 4, 8), (torch.float32, 96, 2, 16),
+                                               (torch.float64, 128, 2, 8), (torch.float64, 80, 2, 8), (torch.float64, 48, 1, 8)])
+def test_walks_that_load_a_tile_ahead_on_views(gpu, dtype, C, vec, steps):
+    """Halves of fused projections, read and written: the channels beside a lane's own, where lanes without channels would store,
+    and the time steps before and after stay as they were. The same values as the dense call's (the same arithmetic)."""
+    waves = 4
+    plan, L, T, batch, pad = hip.Plan(mode=hip.MODE_ROW, vec=vec, unroll=steps, waves=waves), hip.lib(), 4 * steps * waves + 3, 2, 2
+    g = torch.Generator().manual_seed(C)
+    a = torch.rand((batch, T, C), generator=g, dtype=dtype).to(gpu)
+    b, gh = (torch.randn((batch, T, C), generator=g, dtype=dtype).to(gpu) for _ in range(2))
+    h = hip.transposed_linear_scan_forward(a, b, plan=plan)
+    ga, gb = hip.transposed_linear_scan_backward(a, h, gh, plan=plan)
+    assert walks_ahead(batch, T, C, dtype, hip.FORWARD, plan, 2 * C)
+    assert walks_ahead(batch, T, C, dtype, hip.BACKWARD, plan, 2 * C) == (dtype == torch.float64 and vec == 2)
+
+    def view(t, half):
+        wide = torch.full((batch, T + 2 * pad, 2 * C), 7.0, dtype=dtype, device=gpu)
+        inner = wide[:, pad:-pad, half * C:(half + 1) * C]
+        if t is not None:
+            inner.copy_(t)
+        return wide, inner
+
+    st = ctypes.byref(hip.Strides((T + 2 * pad) * 2 * C, 2 * C))
+    tail = (batch, T, C, hip._dtype_code(dtype), None, 0, torch.cuda.current_stream().cuda_stream, ctypes.byref(plan))
+    for half in (0, 1):
+        print(f"case ahead views {dtype} {C} half={half}", flush=True)
+        ins = [view(t, half)[1] for t in (a, b, h, gh)]
+        outs = [view(None, half) for _ in range(3)]
+        va, vb, vh, vgh = (t.data_ptr() for t in ins)
+        o = [inner.data_ptr() for _, inner in outs]
+        assert L.scanscam_scan_fwd_cl_strided(va, vb, o[0], *[st] * 3, *tail) == 0
+        assert L.scanscam_scan_bwd_cl_strided(va, vh, vgh, o[1], o[2], *[st] * 5, *tail) == 0
+        for (wide, inner), want in zip(outs, (h, ga, gb)):
+            assert torch.equal(inner, want)
+            inner.fill_(7.0)
+            assert bool((wide == 7).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T", [1, 2, 4, 15, 16, 17, 33])
 def test_spans_that_end_inside_or_before_a_wave(gpu, dtype, T):
     """Time steps that do not exist: a wave's last step, all but its first, whole waves of a tile, in dense tensors and in
     views whose neighbouring memory is NaN. Bars as in test_forced_plans."""
-    bar = 1e-5 if dtype == torch.float32 else 1e-2
-    full = 4 if dtype == torch.float32 else 8
+    bar = {torch.float32: 1e-5, torch.float64: 1e-13}.get(dtype, 1e-2)
+    full = 16 // torch.empty(0, dtype=dtype).element_size()
     C = 64 * full + full
     g = torch.Generator().manual_seed(T)
     a = torch.rand((2, T, C), generator=g).to(dtype)
@@ -176,7 +219,7 @@ def test_spans_that_end_inside_or_before_a_wave(gpu, dtype, T):
         inner.copy_(t)
         return inner.mT
 
-    for vec in (full, full // 2, 1):
+    for vec in sorted({full, full // 2, 1}):
         for steps in (4, 8, 16):
             if vec == full and steps == 16:
                 continue

@@ -337,3 +337,33 @@ def test_bench_names_the_channels_last_kernel_that_runs():
     assert plan(2048, 512, 40).startswith("staged parts=") and plan(64, 2048, 1024).startswith("mode=2 vec=4 ")
     digests = {bench.kernel_sources_digest(), bench.kernel_sources_digest(bench.CHANNELS_LAST_SOURCES)}
     assert len(digests) == 2
+
+
+def test_which_walks_load_a_tile_ahead_of_their_stores():
+    """The rule's borders (the kernel takes two tiles whose accesses all exist for granted, and resources of 2 GiB)."""
+    from criteria import walks_ahead
+
+    fwd, bwd, f32, f64 = hip.FORWARD, hip.BACKWARD, torch.float32, torch.float64
+    for waves in (1, 4, 8):
+        tile = 8 * waves
+        wide, two, one = (hip.Plan(mode=hip.MODE_ROW, vec=v, unroll=s, waves=waves) for v, s in ((4, 8), (2, 8), (1, 8)))
+        for T in range(3 * tile - 2, 3 * tile + 3):
+            assert walks_ahead(3, T, 256, f32, fwd, wide) == (T >= 3 * tile)
+            assert not walks_ahead(3, T, 256, f32, bwd, wide)
+            assert walks_ahead(3, T, 128, f64, fwd, two) == (T >= 3 * tile)
+            assert walks_ahead(3, T, 128, f64, bwd, two) == (T >= 3 * tile + 1)
+            assert walks_ahead(3, T, 64, f64, fwd, one) == (T >= 3 * tile) and not walks_ahead(3, T, 64, f64, bwd, one)
+    wide, narrow = hip.Plan(mode=hip.MODE_ROW, vec=4, unroll=8, waves=4), hip.Plan(mode=hip.MODE_ROW, vec=2, unroll=16, waves=4)
+    # 18 time steps and the channels behind them within 2 GiB.
+    most = ((1 << 31) - 1 - 256 * 4) // (18 * 4)
+    for stride, ahead in ((256, True), (most - most % 4, True), (most - most % 4 + 4, False), (1 << 25, False)):
+        assert walks_ahead(2, 1000, 256, f32, fwd, wide, stride) == ahead, stride
+    # Stores through the caches (time steps that are no whole lines in 8-byte lanes of fp32), element-aligned lanes, moved channels.
+    assert walks_ahead(2, 1000, 96, f32, fwd, narrow) and not walks_ahead(2, 1000, 98, f32, fwd, narrow)
+    assert not walks_ahead(2, 1000, 257, f32, fwd, wide) and not walks_ahead(2, 1000, 256, f32, fwd, wide, 513)
+    assert not walks_ahead(64, 2048, 1001, f32, fwd) and not walks_ahead(64, 2048, 1001, f32, bwd)
+    # A last group that is not full in about one workgroup per CU; 8 waves of 32 elements a lane, more than one.
+    assert walks_ahead(200, 1000, 160, f32, fwd, wide) and not walks_ahead(236, 1000, 160, f32, fwd, wide)
+    assert not walks_ahead(256, 1000, 160, f32, fwd, wide) and walks_ahead(257, 1000, 160, f32, fwd, wide)
+    eight = hip.Plan(mode=hip.MODE_ROW, vec=4, unroll=8, waves=8)
+    assert walks_ahead(200, 1000, 160, f32, fwd, eight) and not walks_ahead(257, 1000, 160, f32, fwd, eight)
