@@ -673,19 +673,23 @@ int size_cl(int64_t batch, int64_t T, int dtype, bool rev, int virtual_steps, sc
     return SCANSCAM_OK;
 }
 
-// Whether a walk's loads run a tile ahead, past the stores (scan_cl_kernel, PIPE). GPU time of random calls whose plan is such a
-// walk, buffers in rotation, none of them used to find the rule (profiles/walk_loads_past_stores_random_shapes.txt): fp32 forwards
-// 0.92 to 1.02 x, 0.964 x in the mean of 24 ([36, 702, 1472] 86.6 -> 79.6 us, [24, 2401, 1932] 291 -> 276), fp64 0.93 x forwards, 0.99
-// x backwards in the mean of 12 ([18, 339, 1104] 36.9 -> 31.8, [37, 307, 672] backward 63.1 -> 60.7); [64, 2048, 1024] fp32, from box
-// to box, 276 to 290 -> 264 to 270. At worst [224, 909, 512] fp32, 223 -> 231. Two fp32 channels by 16 steps 0.91 to 1.0 x, 0.963 x
-// in the mean of 18 ([17, 840, 1504] 54.7 -> 49.6), one of fp64 by 8 steps 0.98 x in the mean of 12 ([21, 1088, 688] 71.8 -> 65.3).
+// Whether a walk's loads run a tile ahead, past the stores (scan_cl_kernel, PIPE). GPU time of random calls that take it, buffers in
+// rotation, none of them used to find the rule (profiles/walk_loads_past_stores_random_shapes.txt): four fp32
+// channels by 8 steps 0.95 x in the mean of 40 (0.85 to 1.01; [36, 702, 1472] 87.5 -> 79.4 us), two by 16 0.94 (0.87 to 1.0), two of fp64 by 8
+// 0.92 forwards (0.83 to 1.0), 0.98 backwards (0.92 to 1.01), single ones of fp64 0.96 in the mean of 30 (0.89 to 1.02).
 // Not taken
 //   - below three tiles, which leave fewer than two that are whole (fp64 [27, 90, 800] 11.7 -> 12.1);
 //   - where 8 waves of 32 or more words a lane leave one workgroup per CU with its registers and there are more: fp32 [930, 174, 160] 58.8 -> 62.6 ([201,
 //     238, 160], one each, 22.3 -> 20.5);
+//   - where a time step is two or four whole groups of channels, 2 or 4 KB in 16-byte lanes, from 220 workgroups on (memory's
+//     order again, as far as the sizes tell: no counter was taken): fp32 [114, 578, 1024] 149 -> 171,
+//     [234, 914, 512] 248 -> 271, [128, 2048, 512] 260 -> 271, [64, 2000, 1024] 263 -> 287, [224, 909, 512] 224 -> 233 (at 210 and 216, 0.94 and
+//     0.96 x; 8 KB steps 0.89 to 0.97 x but [32, 2048, 2048] 278 -> 286); fp64 backwards at any number, [93, 772, 256] 133 -> 136,
+//     [61, 1415, 512] 300 -> 320;
+//   - single fp64 channels, two workgroups of 4 waves per CU: 1.0 to 1.07 x, [134, 777, 180] 101.5 -> 108.8;
 //   - where nearly every CU has one workgroup and a time step's last group is not full, which memory's order bounds: fp32, 256 of
-//     them, [64, 2048, 1016] 345 -> 364, [64, 2048, 1008] 285 -> 297, [64, 2048, 960] 286 -> 294, 245 of them,
-//     [49, 925, 1132] 126 -> 128 (but 205, [41, 1355, 1216] 163 -> 159, and 714, [102, 591, 1680] 246 -> 234).
+//     them, [64, 2048, 1016] 352 -> 368, [64, 2048, 1008] 287 -> 298, [64, 2048, 960] 298 -> 307, 245 of them,
+//     [49, 925, 1132] 126 -> 128 (but 205, [41, 1355, 1216] 163 -> 151, and 714, [102, 591, 1680] 245 -> 235).
 // `sT`: the tensors' time strides in elements; `cached`: the walk stores through the caches' normal policy, which these do not.
 bool pipe_walk(const scanscam::ClLaunch &l, int64_t T, int64_t C, int esize, bool rev, const int64_t sT[5], bool cached)
 {
@@ -696,7 +700,11 @@ bool pipe_walk(const scanscam::ClLaunch &l, int64_t T, int64_t C, int esize, boo
     // (Its resources end 2 GiB past a span's base, where lanes without channels store.)
     for (int k = 0; k < 5; k++)
         if ((uint64_t)sT[k] * (uint64_t)esize * 18u + (uint64_t)C * (uint64_t)esize >= (uint64_t(1) << 31)) return false;
-    return !cached && (C % (kWave * l.vec) == 0 || l.grid < kComputeUnits - 20 || l.grid > kComputeUnits);
+    if (cached) return false;
+    const int64_t group = (int64_t)kWave * l.vec;
+    if (l.vec > 1 && (rev || l.grid >= 220) && (C == 2 * group || C == 4 * group)) return false;
+    if (l.vec == 1 && l.waves <= 4 && l.grid > kComputeUnits && l.grid <= 2 * kComputeUnits) return false;
+    return C % group == 0 || l.grid < kComputeUnits - 20 || l.grid > kComputeUnits;
 }
 
 // Channels-last: the launch plan. `align`: the largest of 16, 8, 4 and the element size that every tensor's base

@@ -676,7 +676,7 @@ __global__ __launch_bounds__(MAXT) void scan_cl_kernel(const ClArgs p)
     // have been issued is a wait for these too: AHEAD's loads are back long before the stores that the wave then waits for. In
     // the tiles whose accesses all exist every store is issued on every path (apply_inner), the wait at the loop's head leaves
     // them in flight, and a CU with a single workgroup moves memory while it exchanges and computes. What bounds it then is
-    // memory: fp32 [64, 2048, 1024] forwards 290 -> 264 us, 6.1 TB/s, for 94 -> 162 registers (pipe_walk() in scan_api.hip).
+    // memory: fp32 [36, 702, 1472] forwards 87.5 -> 79.4 us, 5.6 TB/s, for 94 -> 161 registers (pipe_walk() in scan_api.hip).
     typename ClStepsOf<ST, VEC, S, REV, M, CT, false, RAGGED>::type steps;
     // The waves' pairs of a tile, exchanged: the value entering this wave's span, and the carry into the next tile.
     auto exchange = [&](int it, const CT (&A)[VEC], const CT (&B)[VEC], CT (&mine)[VEC]) {

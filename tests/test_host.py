@@ -362,6 +362,16 @@ def test_which_walks_load_a_tile_ahead_of_their_stores():
     assert walks_ahead(2, 1000, 96, f32, fwd, narrow) and not walks_ahead(2, 1000, 98, f32, fwd, narrow)
     assert not walks_ahead(2, 1000, 257, f32, fwd, wide) and not walks_ahead(2, 1000, 256, f32, fwd, wide, 513)
     assert not walks_ahead(64, 2048, 1001, f32, fwd) and not walks_ahead(64, 2048, 1001, f32, bwd)
+    # Time steps of two or four whole groups of channels, from 220 workgroups on, backwards always; single channels, 4 waves, two per CU.
+    for C in (512, 1024):
+        least = 220 // (C // 256)
+        assert walks_ahead(least - 1, 1000, C, f32, fwd, wide) and not walks_ahead(least, 1000, C, f32, fwd, wide)
+        assert not walks_ahead(600, 1000, C, f32, fwd, wide)
+    assert all(walks_ahead(250, 1000, C, f32, fwd, wide) for C in (256, 768, 1280, 1536, 2048))
+    two, one = hip.Plan(mode=hip.MODE_ROW, vec=2, unroll=8, waves=4), hip.Plan(mode=hip.MODE_ROW, vec=1, unroll=8, waves=4)
+    assert not walks_ahead(3, 1000, 256, f64, bwd, two) and not walks_ahead(3, 1000, 512, f64, bwd, two)
+    assert walks_ahead(3, 1000, 256, f64, fwd, two) and walks_ahead(3, 1000, 384, f64, bwd, two) and walks_ahead(3, 1000, 1024, f64, bwd, two)
+    assert [walks_ahead(n, 1000, 64, f64, fwd, one) for n in (256, 257, 512, 513)] == [True, False, False, True]
     # A last group that is not full in about one workgroup per CU; 8 waves of 32 elements a lane, more than one.
     assert walks_ahead(200, 1000, 160, f32, fwd, wide) and not walks_ahead(236, 1000, 160, f32, fwd, wide)
     assert not walks_ahead(256, 1000, 160, f32, fwd, wide) and walks_ahead(257, 1000, 160, f32, fwd, wide)
