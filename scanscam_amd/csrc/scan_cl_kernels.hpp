@@ -185,11 +185,6 @@ template <typename ST, int VEC> struct ClAccess<ST, VEC, false> {
     }
 };
 
-// One wave's S consecutive time steps of a tile, for the 64*VEC channels of the workgroup.
-//   load_fold   issues all loads and folds the steps to one affine pair per channel
-//   apply       replays the steps from the scan value entering them and stores the results
-// With APPLY = false only load_fold is used, and its loads are left cacheable (the data is
-// read again later).
 // Components of a vector moved down by s places (those moved in from above are zero).
 template <typename ST, int VEC>
 __device__ __forceinline__ typename Vec<ST, VEC>::raw_t cl_shift_down(typename Vec<ST, VEC>::raw_t r, int s)
@@ -212,7 +207,10 @@ __device__ __forceinline__ typename Vec<ST, VEC>::raw_t cl_shift_down(typename V
 // Whether a walk issues the next tile's loads as soon as this tile is folded (see scan_cl_kernel).
 template <typename ST, int VEC, int S> constexpr bool cl_ahead() { return sizeof(ST) == 2 && VEC <= 4 && VEC * S <= 32; }
 
-template <typename ST, int VEC, int S, bool REV, bool APPLY, typename CT, bool SPLIT = false, bool RAGGED = false>
+// One wave's S consecutive time steps of a tile, for the 64*VEC channels of the workgroup.
+//   issue, fold, issue_h   load the steps and fold them to one affine pair per channel
+//   apply                  replays the steps from the scan value entering them and stores the results
+template <typename ST, int VEC, int S, bool REV, typename CT, bool SPLIT = false, bool RAGGED = false>
 struct ClSteps {
     using V = Vec<ST, VEC>;
     using raw_t = typename V::raw_t;
@@ -228,12 +226,12 @@ struct ClSteps {
     // more) 1.0 to 1.13 x, 64 backwards (222 -> 158) 1.0 to 1.09 x. In walks that do not load ahead: against unpacked 4 x 16 0.94 to
     // 1.04 x forwards (fp16 0.995 x in the mean of 20 calls, bf16, single tiles of few workgroups, 1.01), 8 x 8 backwards level.
     static constexpr bool PACKED = sizeof(ST) == 2 && VEC > 1 && (SPLIT ? (REV ? VEC * S == 32 : VEC == 4 && S == 16) : !cl_ahead<ST, VEC, S>());
-    raw_t ra[S], rx[S], rh[(REV && APPLY) ? S : 1];
+    raw_t ra[S], rx[S], rh[REV ? S : 1];
     CT g[PACKED ? 1 : S][VEC], v[PACKED ? 1 : S][VEC];
     int tau0;  // scan position of the first step
     // issue() may run for the next span of steps while the folded one still awaits apply(): what it brings is kept apart until
     // fold() takes it over.
-    raw_t n_ra[S], n_rx[S], n_rh[(REV && APPLY) ? S : 1];
+    raw_t n_ra[S], n_rx[S], n_rh[REV ? S : 1];
     int n_tau0;
 
     // Every access of a span lies a whole number of time steps from the span's base: step s, `d` steps later in time, lies
@@ -330,14 +328,9 @@ struct ClSteps {
         for (int s = 0; s < S; s++) {
             // The gate of step t is a[t] forwards and a[t+1] backwards.
             const unsigned off_a = clamped<INNER>(s, REV ? 1 : 0, pa, in), off_x = clamped<INNER>(s, 0, px, in);
-            if (APPLY) {
-                n_ra[s] = BV::template load<LOADS>(res_a, ln.c, off_a);
-                n_rx[s] = BV::template load<LOADS>(res_x, ln.c, off_x);
-                if (REV && !H_LAST) n_rh[s] = BV::template load<LOADS>(res_h, ln.c, clamped<INNER>(s, -1, ph, in));
-            } else {
-                n_ra[s] = BV::template load<0>(res_a, ln.c, off_a);
-                n_rx[s] = BV::template load<0>(res_x, ln.c, off_x);
-            }
+            n_ra[s] = BV::template load<LOADS>(res_a, ln.c, off_a);
+            n_rx[s] = BV::template load<LOADS>(res_x, ln.c, off_x);
+            if (REV && !H_LAST) n_rh[s] = BV::template load<LOADS>(res_h, ln.c, clamped<INNER>(s, -1, ph, in));
         }
         if constexpr (H_LAST && !H_FOLDED) {
             asm volatile("" ::: "memory");  // (The compiler would mix them with the others again.)
@@ -375,14 +368,14 @@ struct ClSteps {
         for (int s = 0; s < S; s++) {
             ra[s] = n_ra[s];
             rx[s] = n_rx[s];
-            if (REV && APPLY && !H_FOLDED) rh[s] = n_rh[s];
+            if (REV && !H_FOLDED) rh[s] = n_rh[s];
         }
         if (RAGGED && shift != 0) {  // the last lane of a time step: its window's components into place
 #pragma unroll
             for (int s = 0; s < S; s++) {
                 ra[s] = cl_shift_down<ST, VEC>(ra[s], shift);
                 rx[s] = cl_shift_down<ST, VEC>(rx[s], shift);
-                if (REV && APPLY) rh[s] = cl_shift_down<ST, VEC>(rh[s], shift);
+                if (REV) rh[s] = cl_shift_down<ST, VEC>(rh[s], shift);
             }
         }
         if constexpr (!PACKED) {
@@ -415,7 +408,7 @@ struct ClSteps {
                         v[s][k] = in ? v[s][k] : CT(0);
                     }
                 }
-                if (REV && APPLY && !H_LAST) rh[s] = tau0 + s == T - 1 ? zero : rh[s];
+                if (REV && !H_LAST) rh[s] = tau0 + s == T - 1 ? zero : rh[s];
             }
         }
 #pragma unroll
@@ -494,6 +487,7 @@ struct ClSteps {
     // one for everything in flight.)
     __device__ __forceinline__ void apply_inner(const ClLane<ST> &ln, int T, CT (&mine)[VEC])
     {
+        static_assert(!PACKED, "walks of fp32 and fp64 only");
         using Out = ClAccess<ST, VEC, true>;
         const int tb = REV ? T - 1 - tau0 - S : tau0;
         const auto res_y0 = Out::bounded_base(ln.y0 + (int64_t)tb * ln.py0), res_y1 = Out::bounded_base(ln.y1 + (int64_t)tb * ln.py1);
@@ -501,14 +495,10 @@ struct ClSteps {
         const unsigned at = ln.c_ok ? ln.c : Out::kNowhere;
 #pragma unroll
         for (int s = 0; s < S; s++) {
-            CT G[VEC], X[VEC], out[VEC];
-            if (PACKED) {
-                V::unpack(ra[s], G);
-                V::unpack(rx[s], X);
-            }
+            CT out[VEC];
 #pragma unroll
             for (int k = 0; k < VEC; k++) {
-                mine[k] = PACKED ? fma_(G[k], mine[k], X[k]) : fma_(g[s][k], mine[k], v[s][k]);
+                mine[k] = fma_(g[s][k], mine[k], v[s][k]);
                 out[k] = mine[k];
             }
             Out::store(V::pack(out), res_y0, at, (unsigned)rel(s) * step_y0);
@@ -632,7 +622,7 @@ template <typename ST, int VEC, int S, bool REV, int M, typename CT, bool SPLIT,
     using type = ClShiftSteps<ST, VEC, S, REV, M, CT, SPLIT>;
 };
 template <typename ST, int VEC, int S, bool REV, typename CT, bool SPLIT, bool RAGGED> struct ClStepsOf<ST, VEC, S, REV, 0, CT, SPLIT, RAGGED> {
-    using type = ClSteps<ST, VEC, S, REV, true, CT, SPLIT, RAGGED>;
+    using type = ClSteps<ST, VEC, S, REV, CT, SPLIT, RAGGED>;
 };
 
 // Dynamic LDS: two buffers (tiles alternate) of A and B, each [W][VEC][64] values.

@@ -172,7 +172,7 @@ constexpr bool cl_direct_built(int esize, int vec, int steps) { return esize != 
 // of 8 steps 0.95 to 1.05 x, of 16 steps 0.89 to 1.01 x).
 // fp32 backwards (119 -> 256 registers) 28 random calls run 0.957 to 1.024 x, 0.99 x in the mean, three of C = 2048 1.02 to 1.03;
 // 16-bit lanes of 8 bytes, which load ahead of their exchange already, [64, 2048, 1024] 128.6 / 214.9 -> 129.6 / 222.6 us.
-constexpr bool cl_pipe_built(int esize, int vec, int steps, bool rev) 
+constexpr bool cl_pipe_built(int esize, int vec, int steps, bool rev)
 {
     if (vec * esize == 16) return steps == 8 && (esize == 8 || (esize == 4 && !rev));
     return vec * esize == 8 && !rev && ((esize == 4 && steps == 16) || (esize == 8 && steps == 8));
