@@ -357,8 +357,9 @@ struct ClSteps {
     // forms its operands, in the other path only. Kept from seeing it, against the same kernels without: bf16 4 x 16 walks forwards
     // 1.035 -> 1.02 x the time of the form whose accesses had conditions of their own, fp32 2 x 8 walks backwards 1.01 -> 1.005, 4 x
     // 8 0.97 -> 0.96, fp16 4 x 4 tiles backwards 0.995 -> 0.98 (20 random calls each); a fp16 4 x 8 walk forwards fits 128 registers
-    // again (129). Tiles forwards and element-aligned lanes lose 0.5 to 1 % with it.
-    static constexpr bool OPAQUE = !RAGGED && (REV || !SPLIT);
+    // again (129), the element-aligned one as well, a second workgroup of 8 waves per CU: 1.065 -> 1.005 x in the mean of 16, [997, 319,
+    // 173] 84.2, 102.5 with 129, -> 84. Tiles forwards and other element-aligned lanes lose 0.5 to 1 % with it.
+    static constexpr bool OPAQUE = RAGGED ? sizeof(ST) == 2 && VEC == 4 && S == 8 && !REV : REV || !SPLIT;
 
     // Folds the issued steps to one affine pair per channel.
     template <bool INNER = false> __device__ __forceinline__ void fold(int T, CT (&A)[VEC], CT (&B)[VEC], int shift = 0)
