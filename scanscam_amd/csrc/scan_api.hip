@@ -707,6 +707,24 @@ bool pipe_walk(const scanscam::ClLaunch &l, int64_t T, int64_t C, int esize, boo
     return C % group == 0 || l.grid < kComputeUnits - 20 || l.grid > kComputeUnits;
 }
 
+// Bytes of LDS a backward walk asks for beyond its need, so that a CU holds half as many of its workgroups as its registers allow; 0
+// where none. Once more of them run than fit at once, 16-bit spans of 4 x 16 (125 registers packed, 207 unpacked: 4 workgroups
+// of 4 waves a CU or 2) and fp32 element-aligned ones of 2 x 16 (120, 136 before) lose by the better fit: bf16 [403, 120, 1360] 175 us as
+// 4, 155 as 2 a CU, [937, 118, 372] 132 and 109, fp16 [672, 47, 1852] 141 and 126; where all fit at once they gain by it ([334, 107, 144] 17.5, 20.3).
+// 44 random calls each against the unpacked form: bf16 0.96 -> 0.95 x (at most 1.23 -> 1.04), fp16 0.985 -> 0.975 (1.07 -> 1.01); fp32
+// 1.015 -> 1.0, there not where the last eighth of a single tile's waves is idle ([420, 104, 839] 158, 171).
+size_t idle_lds(const scanscam::ClLaunch &l, int64_t T, int esize, bool rev)
+{
+    if (!rev || l.kind != 0 || l.group != kWave || l.shift != 0 || l.steps != 16 || (l.waves != 4 && l.waves != 8)) return 0;
+    const bool packed = esize == 2 && l.vec == 4 && !l.ragged;
+    const bool aligned = esize == 4 && l.vec == 2 && l.ragged && T > (int64_t)l.waves * 14;
+    const int fit = l.waves > 4 ? 2 : 4;
+    if (!(packed || aligned) || l.grid <= (int64_t)fit * kComputeUnits) return 0;
+    // A CU has 160 KB: one workgroup of 8 waves, two (fp32: three) of 4.
+    const size_t share = l.waves > 4 ? 82 * 1024 : (packed ? 54 * 1024 : 41 * 1024);
+    return share > l.lds_bytes ? share - l.lds_bytes : 0;
+}
+
 // Channels-last: the launch plan. `align`: the largest of 16, 8, 4 and the element size that every tensor's base
 // and strides are multiples of (bytes). The choice itself is the cost model of scan_cl_plan.hpp: every field the
 // caller's plan leaves at zero is chosen by the smallest estimated duration; this function turns the chosen
@@ -1129,6 +1147,7 @@ int run_cl(bool rev, const void *a, const void *x, const void *h, void *y0, void
         const int64_t rowgroups = batch * l.groups;
         if (clear_workspace(args.ws, words, rowgroups * kCounterStride, s) != hipSuccess) return SCANSCAM_ELAUNCH;
     }
+    l.lds_bytes += idle_lds(l, T, esize, rev);
     l.pipe = pipe_walk(l, T, C, esize, rev, sT, args.cached_stores != 0);
     hipError_t e = hipErrorInvalidValue;
     switch (dtype) {

@@ -198,6 +198,27 @@ def test_walks_that_load_a_tile_ahead_on_views(gpu, dtype, C, vec, steps):
             assert bool((wide == 7).all())
 
 
+@pytest.mark.parametrize("dtype,C,vec,waves,batch", [(torch.bfloat16, 256, 4, 4, 1025), (torch.float16, 260, 4, 8, 257),
+                                                     (torch.float32, 129, 2, 8, 257), (torch.float32, 131, 2, 4, 513)])
+def test_walks_with_idle_lds(gpu, dtype, C, vec, waves, batch):
+    """Backward walks of more workgroups than fit at once ask for LDS that they do not use: the same values as the first few batch
+    elements alone, which do not, and the oracle's. Bars as in test_forced_plans."""
+    plan, T = hip.Plan(mode=hip.MODE_ROW, vec=vec, unroll=16, waves=waves), 16 * waves + 5
+    g = torch.Generator().manual_seed(C)
+    a = torch.rand((batch, T, C), generator=g).to(dtype).to(gpu)
+    h, gh = (torch.randn((batch, T, C), generator=g).to(dtype).to(gpu) for _ in range(2))
+    print(f"case idle lds {dtype} [{batch}, {T}, {C}] waves={waves}", flush=True)
+    got = hip.transposed_linear_scan_backward(a, h, gh, plan=plan)
+    alone = hip.transposed_linear_scan_backward(a[:3], h[:3], gh[:3], plan=plan)
+    for x, y in zip(got, alone):
+        assert torch.equal(x[:3], y)
+    last = [as_rows(t[-2:]) for t in (a, h, gh, *got)]
+    want_ga, want_gb = oracle.bwd(*last[:3])
+    bar = 1e-5 if dtype == torch.float32 else 1e-2
+    assert rel_err(last[4], want_gb) <= bar
+    assert rel_err(last[3], want_ga, prev_abs(last[1])) <= bar
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T", [1, 2, 4, 15, 16, 17, 33])
 def test_spans_that_end_inside_or_before_a_wave(gpu, dtype, T):
