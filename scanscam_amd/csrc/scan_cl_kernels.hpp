@@ -287,8 +287,8 @@ struct ClSteps {
     // (16-bit tiles of 16 and 64 elements). Time against the form whose accesses had conditions of their own, 12 to 20 random calls
     // each, buffers in rotation, before -> now: tiles bf16 4 x 4 1.02 -> 0.985, fp16 1.03 -> 0.995, 4 x 16 0.975 / 0.99 -> 0.94 /
     // 0.96, fp32 4 x 8 0.975 -> 0.95; walks fp32 4 x 8 0.99 -> 0.97, fp64 1 x 8 1.01 -> 0.99. Not in element-aligned lanes (fp32
-    // 2 x 4 1.0 -> 1.015).
-    static constexpr bool H_LAST = REV && !RAGGED;
+    // 2 x 4 1.0 -> 1.015), nor in walks of fewer steps (fp32 1 x 4 0.95 -> 0.975, 2 x 4 0.985 -> 0.99, 4 x 2 0.98 -> 0.99).
+    static constexpr bool H_LAST = REV && !RAGGED && (SPLIT || S >= 8);
     // In walks of packed spans behind the fold as well, where the gates and values are back: with a whole tile's loads first and then all
     // its stores, single tiles run slower. 8 x 8 bf16 / fp16 1.035 / 1.025 -> 0.995 / 0.99 (behind the values only: 1.015 / 1.01;
     // [54, 64, 4032] 24.8, 26.9 between them), 4 x 16 0.97 / 0.99 -> 0.945 / 0.965; fp32 2 x 8 would lose 1 %.
@@ -317,9 +317,10 @@ struct ClSteps {
         // Without this a walk keeps the products of its strides and steps, 3 S of them, in scalar registers over all its tiles: 16-bit 1 x 16
         // backwards spills 62 of them, 36 with it, 1 x 8 11 (and 73 vector registers), none with it (62). Time 0.875 -> 0.865 x that
         // of the form whose accesses had conditions of their own, 0.88 both, at worst 0.995 -> 0.985; fp32 element-aligned 2 x 8
-        // 0.995 -> 0.985 (12 to 20 random calls each). Forwards, two streams, nothing spills and element-aligned lanes lose 0.5 %.
+        // 0.995 -> 0.985 (12 to 20 random calls each). Forwards and in 4 steps nothing spills, and element-aligned lanes
+        // or fp32 1 x 4 lose 0.5 or 1 %.
         int pa = ln.pa, px = ln.px, ph = ln.ph;
-        if (REV && !INNER && !SPLIT) asm("" : "+s"(pa), "+s"(px), "+s"(ph) : "s"(first_step));
+        if (REV && !INNER && !SPLIT && S >= 8) asm("" : "+s"(pa), "+s"(px), "+s"(ph) : "s"(first_step));
         const Base res_a = BV::base(ln.a + (int64_t)tb * ln.pa), res_x = BV::base(ln.x + (int64_t)tb * ln.px);
         const Base res_h = BV::base(ln.h + (int64_t)tb * ln.ph);
         // Every load is issued unconditionally: no branch separates the loads, so all of a wave's S x streams loads are
@@ -358,8 +359,8 @@ struct ClSteps {
     // 1.035 -> 1.02 x the time of the form whose accesses had conditions of their own, fp32 2 x 8 walks backwards 1.01 -> 1.005, 4 x
     // 8 0.97 -> 0.96, fp16 4 x 4 tiles backwards 0.995 -> 0.98 (20 random calls each); a fp16 4 x 8 walk forwards fits 128 registers
     // again (129), the element-aligned one as well, a second workgroup of 8 waves per CU: 1.065 -> 1.005 x in the mean of 16, [997, 319,
-    // 173] 84.2, 102.5 with 129, -> 84. Tiles forwards and other element-aligned lanes lose 0.5 to 1 % with it.
-    static constexpr bool OPAQUE = RAGGED ? sizeof(ST) == 2 && VEC == 4 && S == 8 && !REV : REV || !SPLIT;
+    // 173] 84.2, 102.5 with 129, -> 84. Tiles forwards, other element-aligned lanes and short spans of walks lose 0.5 to 1 % with it.
+    static constexpr bool OPAQUE = RAGGED ? sizeof(ST) == 2 && VEC == 4 && S == 8 && !REV : SPLIT ? REV : (REV ? S >= 8 : VEC * S >= 32);
 
     // Folds the issued steps to one affine pair per channel.
     template <bool INNER = false> __device__ __forceinline__ void fold(int T, CT (&A)[VEC], CT (&B)[VEC], int shift = 0)
