@@ -287,8 +287,9 @@ struct ClSteps {
     // (16-bit tiles of 16 and 64 elements). Time against the form whose accesses had conditions of their own, 12 to 20 random calls
     // each, buffers in rotation, before -> now: tiles bf16 4 x 4 1.02 -> 0.985, fp16 1.03 -> 0.995, 4 x 16 0.975 / 0.99 -> 0.94 /
     // 0.96, fp32 4 x 8 0.975 -> 0.95; walks fp32 4 x 8 0.99 -> 0.97, fp64 1 x 8 1.01 -> 0.99. Not in element-aligned lanes (fp32
-    // 2 x 4 1.0 -> 1.015), nor in walks of fewer steps (fp32 1 x 4 0.95 -> 0.975, 2 x 4 0.985 -> 0.99, 4 x 2 0.98 -> 0.99).
-    static constexpr bool H_LAST = REV && !RAGGED && (SPLIT || S >= 8);
+    // 2 x 4 1.0 -> 1.015), nor in walks of fewer steps (fp32 1 x 4 0.95 -> 0.975, 2 x 4 0.985 -> 0.99, 4 x 2 0.98 -> 0.99), nor in
+    // single channels in tiles (level in the mean, [8, 4096, 512] fp32 71.8 -> 73.6 us) or fp32 walks (level, [19234, 53, 33] 167 -> 183).
+    static constexpr bool H_LAST = REV && !RAGGED && (SPLIT ? VEC > 1 : S >= 8 && (VEC > 1 || sizeof(ST) != 4));
     // In walks of packed spans behind the fold as well, where the gates and values are back: with a whole tile's loads first and then all
     // its stores, single tiles run slower. 8 x 8 bf16 / fp16 1.035 / 1.025 -> 0.995 / 0.99 (behind the values only: 1.015 / 1.01;
     // [54, 64, 4032] 24.8, 26.9 between them), 4 x 16 0.97 / 0.99 -> 0.945 / 0.965; fp32 2 x 8 would lose 1 %.
