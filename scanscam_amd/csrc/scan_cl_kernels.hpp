@@ -238,8 +238,9 @@ struct ClSteps {
     // rel(s, d) of them after it. A step that does not exist (past the row's end; backwards also a[t+1] at the first step and
     // h[t-1] at the last) reads the nearest one that does and is put right in fold(), so an access takes two scalar
     // instructions, a product with a constant and a minimum or maximum, where each step's own conditions, selects and offsets
-    // took 8 to 14 (16 x 1 fp32 elements backwards: 1662 -> 880 scalar instructions in the kernel). Over 160 random calls of 4 M
-    // elements and more, buffers in rotation, with PACKED: 0.98 x forwards (0.82 to 1.03), 0.97 x backwards (0.77 to 1.08).
+    // took 8 to 14 (16 x 1 fp32 elements backwards: 1662 -> 880 scalar instructions in the kernel). 2944 random calls, up to 20 of
+    // each kernel that the automatic plans take (profiles/channels_last_constant_steps_random_shapes.txt): 0.98 x forwards, 0.955 x
+    // backwards in the mean, with what else stands here; 85 of them above 1.02 x, bf16 4 x 16 walks forwards most often (1.03 x).
     static constexpr int rel(int s, int d = 0) { return (REV ? S - s : s) + d; }
     static __device__ __forceinline__ int base_step(int first, int T)
     {
